@@ -17,7 +17,7 @@
 // v_mfma_f32_16x16x4_f32.  Per channel chunk the input patch is staged in LDS once; the filter,
 // rewritten beforehand to [m group][chunk][tap][channel][m] in the workspace, is staged per tap
 // group.  bf16 tensors are widened while staging and rounded when stored: the arithmetic is fp32.
-#include "adh_common.h"
+#include "conv3x3_split.h"
 
 #include <algorithm>
 
@@ -601,13 +601,33 @@ static bool gen_is_3x3s2_unpadded(int dtype, const GenShape &g, bool unpadded, u
          pad_h == 1u && pad_w == 1u;
 }
 
-// conv3x3.hip: the 3x3 window at stride 1 with dilation 3 over fp32 tiles padded by 3, forward and backward-data
+// conv3x3_split.hip: the 3x3 window at stride 1 in fp32, forward and backward-data, over padded tiles and tiles without halo
+static bool gen_is_3x3_unit(int dtype, const GenShape &g) {
+  return dtype == ADH_F32 && g.kh == 3u && g.kw == 3u && g.sh == 1u && g.sw == 1u && g.dh == g.dw && g.dh <= 8u;
+}
+static Conv3x3Problem gen_3x3_problem(int which, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
+  const bool fwd = which == ADH_CONV_FWD;
+  if (!unpadded) pad_h = pad_w = 0u;
+  const uint32_t XH = g.HP - 2u * pad_h, XW = g.WP - 2u * pad_w;  // the activation's tile
+  Conv3x3Problem q = {};
+  q.num_tiles = num_tiles; q.N = g.N;
+  q.C = fwd ? g.Cin : g.Cout; q.M = fwd ? g.Cout : g.Cin;
+  q.in_H = fwd ? XH : g.OH; q.in_W = fwd ? XW : g.OW;
+  q.out_H = fwd ? g.OH : XH; q.out_W = fwd ? g.OW : XW;
+  q.stacked = unpadded;
+  q.step = XH;
+  q.dil = g.dh;
+  q.flip = !fwd;
+  q.pad_r = (int32_t)(fwd ? pad_h : 2u * g.dh - pad_h);
+  q.pad_c = (int32_t)(fwd ? pad_w : 2u * g.dw) - (fwd ? 0 : (int32_t)pad_w);
+  q.w_m_stride = fwd ? g.Cin * 9u : 9u;
+  q.w_c_stride = fwd ? 9u : g.Cin * 9u;
+  return q;
+}
+// the dilated window's filter gradient has a kernel of its own
 static bool gen_is_3x3_dilated(int dtype, const GenShape &g, bool unpadded) {
   return dtype == ADH_F32 && !unpadded && g.kh == 3u && g.kw == 3u && g.sh == 1u && g.sw == 1u && g.dh == g.dw && g.dh > 1u;
 }
-int conv3x3_dilated_try(int which, int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
-                        uint32_t W, uint32_t dil, const void *const *in_tiles, const void *w, void *const *out_tiles,
-                        float beta, hipStream_t st);
 // conv3x3_wgrad.hip: its filter gradient
 size_t conv3x3_dilated_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                                        uint32_t dil);
@@ -1202,7 +1222,9 @@ size_t conv2d_workspace(int which, int dtype, uint32_t num_tiles, uint32_t N, ui
   if (which == ADH_CONV_FWD) e = gen_plan_fwd(g, &plan, unpadded ? pad_h : 0u, unpadded ? pad_w : 0u);
   else if (which == ADH_CONV_BWD_DATA) e = gen_plan_bwd_data(g, &plan, unpadded, pad_h, pad_w);
   if (e) return 0;
-  return ((plan.wt_bytes + 255u) & ~(size_t)255u) + ((plan.part_bytes + 255u) & ~(size_t)255u);
+  const size_t bytes = ((plan.wt_bytes + 255u) & ~(size_t)255u) + ((plan.part_bytes + 255u) & ~(size_t)255u);
+  if (gen_is_3x3_unit(dtype, g)) return std::max(bytes, conv3x3_split_workspace(gen_3x3_problem(which, g, num_tiles, unpadded, pad_h, pad_w)));
+  return bytes;
 }
 
 int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t HP, uint32_t WP,
@@ -1246,11 +1268,13 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     if (e == ADH_OK && bias_tiles && bias_added) *bias_added = true;
     if (e != ADH_EUNIMPL) return e;
   }
-  if (gen_is_3x3_dilated(dtype, g, unpadded)) {
+  if (gen_is_3x3_unit(dtype, g)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
-    e = conv3x3_dilated_try(ADH_CONV_FWD, dtype, num_tiles, N, Cin, Cout, g.OH, g.OW, g.dh, x_tiles, w, y_tiles, beta,
-                            as_stream(stream));
+    Conv3x3Problem q = gen_3x3_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w);
+    q.beta = beta;
+    q.in = x_tiles; q.out = y_tiles; q.w = w;
+    e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   if (dtype == ADH_F32 && unpadded && kh == 3u && kw == 3u && sh == 2u && sw == 2u && dh == 1u && dw == 1u && pad_h == 1u &&
@@ -1295,11 +1319,13 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     e = conv1x1_try(true, num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, g.sh, dy_tiles, w, dx_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
-  if (gen_is_3x3_dilated(dtype, g, unpadded)) {
+  if (gen_is_3x3_unit(dtype, g)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
-    e = conv3x3_dilated_try(ADH_CONV_BWD_DATA, dtype, num_tiles, N, Cin, Cout, g.OH, g.OW, g.dh, dy_tiles, w, dx_tiles, beta,
-                            as_stream(stream));
+    Conv3x3Problem q = gen_3x3_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w);
+    q.beta = beta;
+    q.in = dy_tiles; q.out = dx_tiles; q.w = w;
+    e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   if (dtype == ADH_F32 && unpadded && kh == 3u && kw == 3u && sh == 2u && sw == 2u && dh == 1u && dw == 1u && pad_h == 1u &&

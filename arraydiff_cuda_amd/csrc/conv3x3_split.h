@@ -1,0 +1,35 @@
+// The 3x3 window at stride 1 in fp32, forward and backward-data: what conv3x3_split.hip gives the entry points.
+#ifndef ADH_CONV3X3_SPLIT_H
+#define ADH_CONV3X3_SPLIT_H
+
+#include "adh_common.h"
+
+namespace adh {
+
+// out[m][R][Q] = beta*out + sum over c, a, b of w * in[c][R + D*a - pad_r][Q + D*b - pad_c], D the dilation (zero outside `in`)
+struct Conv3x3Problem {
+  uint32_t num_tiles, N, C, M;  // C reduction channels, M produced channels
+  // The tiles' extents.  stacked: they are the row tiles of one tensor in rank order, whose rows are numbered through: tile t
+  // holds rows lead + t*step .. lead + (t+1)*step - 1 of it; `lead` rows precede the first tile's own and as many follow
+  // the last one's (the padded forms' outer halo row).  Otherwise every tile is a tensor of its own.
+  uint32_t in_H, in_W, out_H, out_W;
+  bool stacked;
+  uint32_t step, in_lead, out_lead;
+  int32_t pad_r, pad_c;
+  uint32_t dil;
+  bool flip;  // backward-data: the filter is walked as w[c][m][8 - tap]
+  float beta;
+  const void *const *in, *const *res;  // res (may be null): what beta adds in place of the output
+  void *const *out;
+  const void *w;
+  uint32_t w_m_stride, w_c_stride;  // of the filter's output and reduction channels
+};
+
+// fp32 sums of channel chunks that are dealt to several workgroups (0: none are)
+size_t conv3x3_split_workspace(const Conv3x3Problem &q);
+// The workspace may be null: then no chunks are dealt out.
+int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st);
+void conv3x3_split_name(const Conv3x3Problem &q, char *name, size_t name_bytes);
+
+}  // namespace adh
+#endif

@@ -1,0 +1,98 @@
+"""The fp32 3x3 convolution on the bf16 matrix cores at the sizes where its tiling can go wrong (blocks of one row and of
+many images, channels around the chunks of 32 and the groups of 16 and 64, rows that are no multiple of four, several
+row tiles in one block) against the CPU oracle, at the accuracy of fp32 arithmetic against double precision, and with
+values whose bf16 parts are not finite."""
+import numpy as np
+import pytest
+import torch
+
+from arraydiff_cuda_amd import capi
+from gpu_util import dev, host, rel_err
+
+pytestmark = pytest.mark.gpu
+
+
+def _tiles(a, K):
+    return [t.contiguous() for t in torch.chunk(a, K, dim=2)]
+
+
+@pytest.mark.parametrize("K,N,Cin,Cout,Ht,W", [
+    (1, 1, 1, 1, 1, 1), (2, 3, 31, 17, 1, 5), (3, 1, 33, 16, 2, 640), (4, 9, 32, 65, 4, 16), (4, 5, 64, 64, 2, 8), (1, 2, 65, 33, 17, 33),
+    (2, 1, 96, 130, 16, 32), (5, 2, 8, 48, 3, 12)])
+def test_unpadded_passes_vs_oracle(oracle, K, N, Cin, Cout, Ht, W):
+    rng = np.random.default_rng(810 + Cin + W)
+    H = K * Ht
+    x = rng.uniform(-1, 1, size=(N, Cin, H, W)).astype(np.float32)
+    w = (rng.standard_normal((Cout, Cin, 3, 3)) * np.sqrt(2.0 / (Cin * 9))).astype(np.float32)
+    dy = rng.standard_normal((N, Cout, H, W)).astype(np.float32)
+    xp = np.zeros((N, Cin, H + 2, W + 2), np.float32)
+    xp[:, :, 1:-1, 1:-1] = x
+    y_want, g_want = np.empty((N, Cout, H, W), np.float32), np.empty((N, Cin, H + 2, W + 2), np.float32)
+    oracle.conv_slab_fwd(xp, w, y_want)
+    oracle.conv_slab_bwd_data(w, dy, g_want)
+    g_want = g_want[:, :, 1:-1, 1:-1]
+    xs, dys = _tiles(dev(x), K), _tiles(dev(dy), K)
+    for beta in (0.0, 1.0):
+        ys, gs = [torch.ones_like(t) for t in dys], [torch.ones_like(t) for t in xs]
+        capi.check(capi.conv_unpadded_fwd_tiles(xs, dev(w), ys, N, Cin, Cout, Ht, W, beta=beta), "fwd")
+        capi.check(capi.conv_unpadded_bwd_data_tiles(dev(w), dys, gs, N, Cin, Cout, Ht, W, beta=beta), "bwd-data")
+        assert rel_err(host(torch.cat(ys, 2)), y_want + beta) <= 1e-5
+        assert rel_err(host(torch.cat(gs, 2)), g_want + beta) <= 1e-5
+
+
+def test_sums_are_as_close_to_double_precision_as_fp32_ones():
+    g = torch.Generator().manual_seed(5)
+    N, C, H, W = 2, 256, 16, 32
+    x = torch.rand((N, C, H, W), generator=g) * 2 - 1
+    w = torch.randn((C, C, 3, 3), generator=g) * (2.0 / (C * 9)) ** 0.5
+    want = torch.nn.functional.conv2d(x.double(), w.double(), padding=1)
+    y = torch.empty((N, C, H, W), device="cuda")
+    capi.check(capi.conv_unpadded_fwd_tiles([x.cuda()], w.cuda(), [y], N, C, C, H, W), "fwd")
+    err = ((y.cpu().double() - want).norm() / want.norm()).item()
+    plain = ((torch.nn.functional.conv2d(x, w, padding=1).double() - want).norm() / want.norm()).item()
+    assert err <= max(2 * plain, 1.5e-6), (err, plain)  # 2304 terms: fp32 sums in order are 1e-6 off
+
+
+def test_many_chunks_dealt_to_several_workgroups():
+    """512 channels over 2 x 8 tiles through the entry points with a workspace: sums of channel chunks added by a second kernel."""
+    K, N, C, Ht, W = 4, 3, 512, 2, 8
+    geo = (3, 3, 1, 1, 1, 1, 1, 1)
+    g = torch.Generator().manual_seed(6)
+    x = torch.rand((N, C, K * Ht, W), generator=g) * 2 - 1
+    w = torch.randn((C, C, 3, 3), generator=g) * (2.0 / (C * 9)) ** 0.5
+    want = torch.nn.functional.conv2d(x.double(), w.double(), padding=1)
+    nbytes = capi.conv2d_unpadded_workspace_bytes(capi.ADH_CONV_FWD, capi.ADH_F32, K, N, C, C, Ht, W, *geo)
+    for beta in (0.0, 1.0):
+        ys = [torch.ones((N, C, Ht, W), device="cuda") for _ in range(K)]
+        capi.check(capi.conv2d_unpadded_fwd_tiles(_tiles(x.cuda(), K), w.cuda(), ys, N, C, C, Ht, W, *geo, beta=beta,
+                                                  ws=torch.empty(nbytes // 4 + 64, device="cuda")), "fwd")
+        assert rel_err(torch.cat(ys, 2).cpu().numpy(), want.numpy() + beta) <= 1e-5
+
+
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), 3.4e38, float("nan")])
+def test_values_without_finite_bf16_parts(bad):
+    """An infinity (or a number that rounds to an infinite bf16) in the input or the filter gives what fp32 sums give: the
+    outputs it touches, and only those, are infinite, huge or NaN."""
+    N, C, H, W = 1, 40, 9, 21
+    g = torch.Generator().manual_seed(7)
+    x, w = torch.rand((N, C, H, W), generator=g) + 0.5, torch.rand((C, C, 3, 3), generator=g) * 0.1 + 0.01
+    for where in ("input", "filter"):
+        xb, wb = x.clone(), w.clone()
+        if where == "input":
+            xb[0, 3, 4, 10] = bad
+        else:
+            wb[5, 7, 1, 2] = bad
+        y = torch.empty((N, C, H, W), device="cuda")
+        capi.check(capi.conv_unpadded_fwd_tiles([xb.cuda()], wb.cuda(), [y], N, C, C, H, W), "fwd")
+        # taps in order, the zero padding as data (zero times an infinity is NaN)
+        xp = torch.nn.functional.pad(xb, (1, 1, 1, 1))
+        want = torch.zeros((N, C, H, W))
+        for a in range(3):
+            for b in range(3):
+                want = want + (xp[:, None, :, a:a + H, b:b + W] * wb[None, :, :, a, b, None, None]).sum(2)
+        got = y.cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want))
+        fine = torch.isfinite(want)
+        assert ((got[fine].double() - want[fine].double()).abs() <= 2e-6 * want[fine].double().abs()).all()
+        assert fine.any() and not torch.equal(want, torch.nn.functional.conv2d(x, w, padding=1))
