@@ -18,6 +18,7 @@
 // rewritten beforehand to [m group][chunk][tap][channel][m] in the workspace, is staged per tap
 // group.  bf16 tensors are widened while staging and rounded when stored: the arithmetic is fp32.
 #include "conv3x3_split.h"
+#include "conv3x3_wgrad_split.h"
 
 #include <algorithm>
 
@@ -1212,6 +1213,8 @@ size_t conv2d_workspace(int which, int dtype, uint32_t num_tiles, uint32_t N, ui
       bytes = std::max(bytes, conv3x3s2_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u));
     if (gen_is_thin(dtype, g, unpadded))
       bytes = std::max(bytes, conv_thin_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, kh, kw, sh, sw));
+    if (gen_is_3x3_unit(dtype, g) && g.dh == 1u)
+      bytes = std::max(bytes, conv3x3_wgrad_split_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW));
     if (gen_is_3x3_dilated(dtype, g, unpadded))
       bytes = std::max(bytes, conv3x3_dilated_wgrad_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW, g.dh));
     return (bytes + 255u) & ~(size_t)255u;
@@ -1386,6 +1389,17 @@ int conv2d_bwd_filter(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
                               workspace, st);
       if (e != ADH_EUNIMPL) return e;
     }
+  }
+  if (gen_is_3x3_unit(dtype, g) && g.dh == 1u && workspace_bytes >= conv3x3_wgrad_split_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW)) {
+    Wgrad3x3Problem q = {};
+    q.num_tiles = num_tiles; q.N = N; q.Cin = Cin; q.Cout = Cout;
+    q.x_H = g.HP - (unpadded ? 2u * pad_h : 0u); q.x_W = g.WP - (unpadded ? 2u * pad_w : 0u);
+    q.dy_H = g.OH; q.dy_W = g.OW;
+    q.stacked = unpadded;
+    q.pad_r = unpadded ? (int32_t)pad_h : 0; q.pad_c = unpadded ? (int32_t)pad_w : 0;
+    q.x = x_tiles; q.dy = dy_tiles; q.dw = dwt; q.beta = beta;
+    e = conv3x3_wgrad_split(q, workspace, st);
+    if (e != ADH_EUNIMPL) return e;
   }
   if (gen_is_3x3_dilated(dtype, g, unpadded)) {
     const size_t need = conv3x3_dilated_wgrad_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW, g.dh);

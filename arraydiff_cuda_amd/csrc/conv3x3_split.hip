@@ -39,10 +39,6 @@ constexpr uint32_t kSpChunk = 32;  // channels per staged chunk
 constexpr uint32_t kSpPP = 640;    // patch pixels per plane in LDS
 constexpr uint32_t kSpMP = 68;     // filter rows per plane: = 4 (mod 16), so that the octet planes start 64 bytes apart
 
-// memory of the device, said out loud: addresses that come out of a table in LDS would otherwise be accessed as flat ones, whose
-// loads the waits for LDS operands take in
-#define ADH_GLOBAL __attribute__((address_space(1)))
-
 struct SplitParams {
   const float *in[ADH_MAX_TILES];
   const float *res[ADH_MAX_TILES];  // what beta adds: the output itself or a residual laid out like it
@@ -63,8 +59,6 @@ struct SplitParams {
   FastDiv div_bpg, div_nbj, div_MG, div_N, div_BC, div_live, div_PPI, div_PCP, div_PPn, div_ksplit, div_in, div_out;
 };
 
-// four neighbouring values, at the alignment of one
-typedef floatx4 floatx4_u __attribute__((aligned(4)));
 __device__ __forceinline__ floatx4 load4(const ADH_GLOBAL float *p) { return *(const ADH_GLOBAL floatx4_u *)p; }
 __device__ __forceinline__ void store4(ADH_GLOBAL float *p, floatx4 v) { *(ADH_GLOBAL floatx4_u *)p = v; }
 

@@ -25,6 +25,12 @@ typedef uint32_t uintx4 __attribute__((ext_vector_type(4)));
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
 
+// Memory of the device, said out loud: addresses that come out of a table in LDS would otherwise be accessed as flat ones, whose
+// loads the waits for LDS operands take in.
+#define ADH_GLOBAL __attribute__((address_space(1)))
+// four neighbouring values, at the alignment of one
+typedef floatx4 floatx4_u __attribute__((aligned(4)));
+
 // two values' parts, packed
 __device__ __forceinline__ void split_pair(float a, float b, uint32_t &h, uint32_t &m, uint32_t &l) {
   const floatx2 v = {a, b};

@@ -1,5 +1,5 @@
-"""The fp32 3x3 convolution on the bf16 matrix cores at the sizes where its tiling can go wrong (blocks of one row and of
-many images, channels around the chunks of 32 and the groups of 16 and 64, rows that are no multiple of four, several
+"""The fp32 3x3 convolution and its filter gradient on the bf16 matrix cores at the sizes where their tiling can go wrong
+(rows shorter than a load and column tiles of every width, blocks of one row and of many images, channels around the chunks of 32 and the groups of 16 and 64, rows that are no multiple of four, several
 row tiles in one block) against the CPU oracle, at the accuracy of fp32 arithmetic against double precision, and with
 values whose bf16 parts are not finite."""
 import numpy as np
@@ -17,7 +17,7 @@ def _tiles(a, K):
 
 
 @pytest.mark.parametrize("K,N,Cin,Cout,Ht,W", [
-    (1, 1, 1, 1, 1, 1), (2, 3, 31, 17, 1, 5), (3, 1, 33, 16, 2, 640), (4, 9, 32, 65, 4, 16), (4, 5, 64, 64, 2, 8), (1, 2, 65, 33, 17, 33),
+    (1, 1, 1, 1, 1, 1), (2, 3, 31, 17, 1, 5), (1, 2, 5, 70, 9, 3), (2, 2, 40, 20, 7, 2), (1, 1, 64, 64, 5, 41), (2, 1, 33, 33, 8, 48), (3, 1, 33, 16, 2, 640), (4, 9, 32, 65, 4, 16), (4, 5, 64, 64, 2, 8), (1, 2, 65, 33, 17, 33),
     (2, 1, 96, 130, 16, 32), (5, 2, 8, 48, 3, 12)])
 def test_unpadded_passes_vs_oracle(oracle, K, N, Cin, Cout, Ht, W):
     rng = np.random.default_rng(810 + Cin + W)
@@ -30,6 +30,8 @@ def test_unpadded_passes_vs_oracle(oracle, K, N, Cin, Cout, Ht, W):
     y_want, g_want = np.empty((N, Cout, H, W), np.float32), np.empty((N, Cin, H + 2, W + 2), np.float32)
     oracle.conv_slab_fwd(xp, w, y_want)
     oracle.conv_slab_bwd_data(w, dy, g_want)
+    dw_want = np.zeros((Cout, Cin, 3, 3), np.float32)
+    oracle.conv_slab_bwd_filter(xp, dy, dw_want)
     g_want = g_want[:, :, 1:-1, 1:-1]
     xs, dys = _tiles(dev(x), K), _tiles(dev(dy), K)
     for beta in (0.0, 1.0):
@@ -38,6 +40,10 @@ def test_unpadded_passes_vs_oracle(oracle, K, N, Cin, Cout, Ht, W):
         capi.check(capi.conv_unpadded_bwd_data_tiles(dev(w), dys, gs, N, Cin, Cout, Ht, W, beta=beta), "bwd-data")
         assert rel_err(host(torch.cat(ys, 2)), y_want + beta) <= 1e-5
         assert rel_err(host(torch.cat(gs, 2)), g_want + beta) <= 1e-5
+        dw = torch.ones((Cout, Cin, 3, 3), device="cuda")
+        ws = torch.empty(capi.conv_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_F32, K, N, Cin, Cout, Ht, W) // 4, device="cuda")
+        capi.check(capi.conv_unpadded_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, Ht, W, beta=beta, ws=ws), "bwd-filter")
+        assert rel_err(host(dw), dw_want + beta) <= 1e-5
 
 
 def test_sums_are_as_close_to_double_precision_as_fp32_ones():
@@ -96,3 +102,25 @@ def test_values_without_finite_bf16_parts(bad):
         fine = torch.isfinite(want)
         assert ((got[fine].double() - want[fine].double()).abs() <= 2e-6 * want[fine].double().abs()).all()
         assert fine.any() and not torch.equal(want, torch.nn.functional.conv2d(x, w, padding=1))
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+def test_filter_gradient_of_values_without_finite_bf16_parts(bad):
+    N, Cin, Cout, H, W = 1, 20, 40, 6, 21
+    g = torch.Generator().manual_seed(8)
+    x, dy = torch.rand((N, Cin, H, W), generator=g) + 0.5, torch.rand((N, Cout, H, W), generator=g) + 0.5
+    ws = torch.empty(capi.conv_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_F32, 1, N, Cin, Cout, H, W) // 4, device="cuda")
+    for where in ("input", "gradient"):
+        xb, db = x.clone(), dy.clone()
+        (xb[0, 3, 2] if where == "input" else db[0, 30, 4])[10] = bad
+        dw = torch.empty((Cout, Cin, 3, 3), device="cuda")
+        capi.check(capi.conv_unpadded_bwd_filter_tiles([xb.cuda()], [db.cuda()], dw, N, Cin, Cout, H, W, ws=ws), "bwd-filter")
+        xp = torch.nn.functional.pad(xb, (1, 1, 1, 1))
+        want = torch.stack([torch.stack([(db[:, :, None] * xp[:, None, :, a:a + H, b:b + W]).sum((0, 3, 4)) for b in range(3)], -1)
+                            for a in range(3)], -2)
+        got = dw.cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        assert torch.equal(torch.isinf(got), torch.isinf(want))
+        fine = torch.isfinite(want)
+        assert ((got[fine].double() - want[fine].double()).abs() <= 2e-6 * want[fine].double().abs()).all()
+        assert fine.any() and not fine.all()
