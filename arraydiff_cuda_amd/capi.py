@@ -1,4 +1,5 @@
-"""ctypes binding of ``libadh.so``.  There is no fallback: if the library is missing, or a
+"""Python binding of ``libadh.so``: ctypes for every symbol (``lib()``), and functions on torch tensors whose arguments a native
+module converts (``csrc/binding.cc``).  There is no fallback: if the library is missing, or a
 call is made without a GPU, an exception is raised."""
 import ctypes
 import os
@@ -149,59 +150,65 @@ def ptr_table(ptrs):
 # ---------------------------------------------------------------------------
 # torch-tensor convenience wrappers (tests / bench).  Tensors must live on the GPU.
 # ---------------------------------------------------------------------------
+_native = None  # the module that converts the arguments and calls
+
+
+def _load_native():
+    global _native
+    import torch
+    from . import _binding
+    if not os.path.exists(LIB_PATH):
+        lib()  # raises, with what to do
+    _binding.load(LIB_PATH, torch._C._cuda_getDevice, torch._C._cuda_getCurrentRawStream)
+    _CODES.update({torch.float32: ADH_F32, torch.bfloat16: ADH_BF16})
+    _native = _binding
+    return _native
+
+
+_CODES = {}  # ADH_F32 / ADH_BF16 by torch dtype
+
+
+def _n():
+    return _native or _load_native()
+
+
 def _dt(t):
-    import torch
-    if t.dtype == torch.float32:
-        return ADH_F32
-    if t.dtype == torch.bfloat16:
-        return ADH_BF16
-    raise TypeError("dtype %s not supported" % t.dtype)
+    if _native is None:
+        _load_native()
+    code = _CODES.get(t.dtype)
+    if code is None:
+        raise TypeError("dtype %s not supported" % t.dtype)
+    return code
 
 
-def _dev(*ts):
-    for t in ts:
-        if t is not None and (not t.is_cuda or not t.is_contiguous()):
-            raise ValueError("tensors must be contiguous GPU tensors")
-
-
-def _stream():
-    import torch
-    return ctypes.c_void_p(torch.cuda.current_stream().cuda_stream)
-
-
-def _tbl(ts):
-    return ptr_table([t.data_ptr() for t in ts])
+def _ws(ws):
+    if ws is None:
+        return None, 0
+    return ws, ws.numel() * ws.element_size()
 
 
 def fill_f32(x, v):
-    _dev(x)
-    return lib().adh_fill_f32(x.numel(), v, x.data_ptr(), _stream())
+    return _n().adh_fill_f32(x.numel(), v, x)
 
 
 def add_f32(x, y):
-    _dev(x, y)
-    return lib().adh_add_f32(x.numel(), x.data_ptr(), y.data_ptr(), _stream())
+    return _n().adh_add_f32(x.numel(), x, y)
 
 
 def halo_exchange(tiles, grid_w, grid_h, p, W, H, C, N, rank=None):
-    _dev(*tiles)
-    tb, keep = _tbl(tiles)
     if rank is None:
-        return lib().adh_halo_exchange_nchw(_dt(tiles[0]), grid_w, grid_h, p, W, H, C, N, tb, _stream())
-    return lib().adh_halo_exchange_nchw_rank(_dt(tiles[0]), grid_w, grid_h, rank, p, W, H, C, N, tb, _stream())
+        return _n().adh_halo_exchange_nchw(_dt(tiles[0]), grid_w, grid_h, p, W, H, C, N, tiles)
+    return _n().adh_halo_exchange_nchw_rank(_dt(tiles[0]), grid_w, grid_h, rank, p, W, H, C, N, tiles)
 
 
 def halo_reduce(tiles, grid_w, grid_h, p, W, H, C, N, rank=None):
-    _dev(*tiles)
-    tb, keep = _tbl(tiles)
     if rank is None:
-        return lib().adh_halo_reduce_nchw(_dt(tiles[0]), grid_w, grid_h, p, W, H, C, N, tb, _stream())
-    return lib().adh_halo_reduce_nchw_rank(_dt(tiles[0]), grid_w, grid_h, rank, p, W, H, C, N, tb, _stream())
+        return _n().adh_halo_reduce_nchw(_dt(tiles[0]), grid_w, grid_h, p, W, H, C, N, tiles)
+    return _n().adh_halo_reduce_nchw_rank(_dt(tiles[0]), grid_w, grid_h, rank, p, W, H, C, N, tiles)
 
 
 def _padlike(name, p, W, H, C, N, a, b):
-    _dev(a, b)
-    return getattr(lib(), name)(_dt(a), p, W, H, C, N, a.data_ptr(), b.data_ptr(), _stream())
+    return getattr(_n(), name)(_dt(a), p, W, H, C, N, a, b)
 
 
 def halo_pad(p, W, H, C, N, x, y):
@@ -221,107 +228,65 @@ def halo_unpad_add(p, W, H, C, N, x, y):
 
 
 def halo_repad(ps, pd, W, H, C, N, x, y):
-    _dev(x, y)
-    return lib().adh_halo_repad_nchw(_dt(x), ps, pd, W, H, C, N, x.data_ptr(), y.data_ptr(), _stream())
+    return _n().adh_halo_repad_nchw(_dt(x), ps, pd, W, H, C, N, x, y)
 
 
 def slice_nchw(add, count, N, src, src_dims, src_off, dst, dst_dims, dst_off):
-    _dev(src, dst)
-    fn = lib().adh_slice_add_nchw if add else lib().adh_slice_copy_nchw
-    return fn(_dt(src), count[0], count[1], count[2], N, src.data_ptr(), src_dims[0], src_dims[1], src_dims[2],
-              src_off[0], src_off[1], src_off[2], dst.data_ptr(), dst_dims[0], dst_dims[1], dst_dims[2],
-              dst_off[0], dst_off[1], dst_off[2], _stream())
+    fn = _n().adh_slice_add_nchw if add else _n().adh_slice_copy_nchw
+    return fn(_dt(src), count[0], count[1], count[2], N, src, src_dims[0], src_dims[1], src_dims[2],
+              src_off[0], src_off[1], src_off[2], dst, dst_dims[0], dst_dims[1], dst_dims[2],
+              dst_off[0], dst_off[1], dst_off[2])
 
 
 def tiles_pack(K, p, W, H, C, N, x, tiles):
-    _dev(x, *tiles)
-    tb, keep = _tbl(tiles)
-    return lib().adh_tiles_pack_nchw(_dt(x), K, p, W, H, C, N, x.data_ptr(), tb, _stream())
+    return _n().adh_tiles_pack_nchw(_dt(x), K, p, W, H, C, N, x, tiles)
 
 
 def tiles_unpack(K, p, W, H, C, N, tiles, y):
-    _dev(y, *tiles)
-    tb, keep = _tbl(tiles)
-    return lib().adh_tiles_unpack_nchw(_dt(y), K, p, W, H, C, N, tb, y.data_ptr(), _stream())
+    return _n().adh_tiles_unpack_nchw(_dt(y), K, p, W, H, C, N, tiles, y)
 
 
 def conv_workspace_bytes(which, dtype, K, N, Cin, Cout, H, W):
     return lib().adh_conv3x3_workspace_bytes(which, dtype, K, N, Cin, Cout, H, W)
 
 
-def _ws(ws):
-    if ws is None:
-        return None, 0
-    return ws.data_ptr(), ws.numel() * ws.element_size()
-
-
 def conv_fwd_tiles(xs, w, ys, N, Cin, Cout, H, W, beta=0.0, ws=None, unexchanged=False):
     """unexchanged: xs are the row tiles of one activation in rank order whose inner halo rows have not been
     exchanged; the result equals halo_exchange followed by the ordinary forward."""
-    _dev(w, *xs, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    wp, wb = _ws(ws)
-    fn = lib().adh_conv3x3_slab_fwd_tiles_unexchanged if unexchanged else lib().adh_conv3x3_slab_fwd_tiles
-    return fn(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xt, w.data_ptr(), yt, beta,
-                                            wp, wb, _stream())
+    fn = _n().adh_conv3x3_slab_fwd_tiles_unexchanged if unexchanged else _n().adh_conv3x3_slab_fwd_tiles
+    return fn(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xs, w, ys, beta, *_ws(ws))
 
 
 def conv_bwd_data_tiles(w, dys, dxs, N, Cin, Cout, H, W, beta=0.0, ws=None, reduced=False):
     """reduced: dys are the row tiles of one gradient in rank order; the interior of every dx tile comes out as
     after backward-data followed by halo_reduce."""
-    _dev(w, *dys, *dxs)
-    dt, k1 = _tbl(dys)
-    xt, k2 = _tbl(dxs)
-    wp, wb = _ws(ws)
-    fn = lib().adh_conv3x3_slab_bwd_data_tiles_reduced if reduced else lib().adh_conv3x3_slab_bwd_data_tiles
-    return fn(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, w.data_ptr(), dt, xt, beta, wp, wb, _stream())
+    fn = _n().adh_conv3x3_slab_bwd_data_tiles_reduced if reduced else _n().adh_conv3x3_slab_bwd_data_tiles
+    return fn(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, w, dys, dxs, beta, *_ws(ws))
 
 
 def conv_unpadded_fwd_tiles(xs, w, ys, N, Cin, Cout, H, W, beta=0.0, ws=None):
     """xs, ys: the row tiles (H x W, no halo) of one tensor in rank order."""
-    _dev(w, *xs, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv3x3_unpadded_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xt, w.data_ptr(), yt, beta, wp,
-                                                wb, _stream())
+    return _n().adh_conv3x3_unpadded_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xs, w, ys, beta, *_ws(ws))
 
 
 def conv_unpadded_fwd_residual_tiles(xs, w, res, ys, N, Cin, Cout, H, W):
     """ys[t] = conv(xs, w)[t] + res[t] over tiles without halo (fp32)."""
-    _dev(w, *xs, *res, *ys)
-    xt, k1 = _tbl(xs)
-    rt, k2 = _tbl(res)
-    yt, k3 = _tbl(ys)
-    return lib().adh_conv3x3_unpadded_fwd_residual_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xt, w.data_ptr(), rt, yt,
-                                                         _stream())
+    return _n().adh_conv3x3_unpadded_fwd_residual_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xs, w, res, ys)
 
 
 def conv_unpadded_bwd_data_tiles(w, dys, dxs, N, Cin, Cout, H, W, beta=0.0, ws=None):
-    _dev(w, *dys, *dxs)
-    dt, k1 = _tbl(dys)
-    xt, k2 = _tbl(dxs)
-    wp, wb = _ws(ws)
-    return lib().adh_conv3x3_unpadded_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, w.data_ptr(), dt, xt,
-                                                     beta, wp, wb, _stream())
+    return _n().adh_conv3x3_unpadded_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, w, dys, dxs, beta,
+                                                    *_ws(ws))
 
 
 def conv_unpadded_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, H, W, beta=0.0, ws=None):
-    _dev(dw, *xs, *dys)
-    xt, k1 = _tbl(xs)
-    dt, k2 = _tbl(dys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv3x3_unpadded_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xt, dt, dw.data_ptr(),
-                                                       beta, wp, wb, _stream())
+    return _n().adh_conv3x3_unpadded_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xs, dys, dw, beta,
+                                                      *_ws(ws))
 
 
 def conv_bias_add_tiles(biases, ys, N, C, H, W):
     """ys[t][n,c,h,w] += biases[t][c]; biases are fp32 vectors of C (entries may repeat)."""
-    _dev(*biases, *ys)
-    bt, k1 = _tbl(biases)
-    yt, k2 = _tbl(ys)
-    return lib().adh_conv_bias_add_tiles(_dt(ys[0]), len(ys), N, C, H, W, bt, yt, _stream())
+    return _n().adh_conv_bias_add_tiles(_dt(ys[0]), len(ys), N, C, H, W, biases, ys)
 
 
 def conv_bwd_bias_workspace_bytes(K, N, C):
@@ -330,10 +295,7 @@ def conv_bwd_bias_workspace_bytes(K, N, C):
 
 def conv_bwd_bias_tiles(dys, db, N, C, H, W, beta=0.0, ws=None):
     """db[c] = beta*db[c] + sum over tiles, n, h, w of dys[t][n,c,h,w]."""
-    _dev(db, *dys)
-    dt, k1 = _tbl(dys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv_bwd_bias_tiles(_dt(dys[0]), len(dys), N, C, H, W, dt, db.data_ptr(), beta, wp, wb, _stream())
+    return _n().adh_conv_bwd_bias_tiles(_dt(dys[0]), len(dys), N, C, H, W, dys, db, beta, *_ws(ws))
 
 
 def conv2d_workspace_bytes(which, dtype, K, N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw):
@@ -341,41 +303,24 @@ def conv2d_workspace_bytes(which, dtype, K, N, Cin, Cout, HP, WP, kh, kw, sh, sw
 
 
 def conv2d_fwd_tiles(xs, w, ys, N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, beta=0.0, ws=None):
-    _dev(*xs, w, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_slab_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, xt,
-                                           w.data_ptr(), yt, beta, wp, wb, _stream())
+    return _n().adh_conv2d_slab_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, xs, w, ys,
+                                          beta, *_ws(ws))
 
 
 def conv2d_fwd_bias_tiles(xs, w, biases, ys, N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, beta=0.0, ws=None):
     """conv2d_fwd_tiles followed by ys[t] += biases[t] per channel, in the convolution's stores where its kernel can."""
-    _dev(*xs, w, *biases, *ys)
-    xt, k1 = _tbl(xs)
-    bt, k3 = _tbl(biases)
-    yt, k2 = _tbl(ys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_slab_fwd_bias_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, xt,
-                                                w.data_ptr(), bt, yt, beta, wp, wb, _stream())
+    return _n().adh_conv2d_slab_fwd_bias_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, xs, w,
+                                               biases, ys, beta, *_ws(ws))
 
 
 def conv2d_bwd_data_tiles(w, dys, dxs, N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, beta=0.0, ws=None):
-    _dev(w, *dys, *dxs)
-    dt, k1 = _tbl(dys)
-    gt, k2 = _tbl(dxs)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_slab_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw,
-                                                w.data_ptr(), dt, gt, beta, wp, wb, _stream())
+    return _n().adh_conv2d_slab_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw, w,
+                                               dys, dxs, beta, *_ws(ws))
 
 
 def conv2d_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw_, beta=0.0, ws=None):
-    _dev(*xs, *dys, dw)
-    xt, k1 = _tbl(xs)
-    dt, k2 = _tbl(dys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_slab_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw_,
-                                                  xt, dt, dw.data_ptr(), beta, wp, wb, _stream())
+    return _n().adh_conv2d_slab_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, HP, WP, kh, kw, sh, sw, dh, dw_, xs,
+                                                 dys, dw, beta, *_ws(ws))
 
 
 def conv2d_unpadded_workspace_bytes(which, dtype, K, N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h, pad_w):
@@ -384,36 +329,18 @@ def conv2d_unpadded_workspace_bytes(which, dtype, K, N, Cin, Cout, H, W, kh, kw,
 
 def conv2d_unpadded_fwd_tiles(xs, w, ys, N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h, pad_w, beta=0.0, ws=None):
     """Row tiles without halo, any window / stride / dilation: rows outside a tile come from its neighbours."""
-    _dev(*xs, w, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_unpadded_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h, pad_w,
-                                               xt, w.data_ptr(), yt, beta, wp, wb, _stream())
+    return _n().adh_conv2d_unpadded_fwd_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h,
+                                              pad_w, xs, w, ys, beta, *_ws(ws))
 
 
 def conv2d_unpadded_bwd_data_tiles(w, dys, dxs, N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h, pad_w, beta=0.0, ws=None):
-    _dev(w, *dys, *dxs)
-    dt, k1 = _tbl(dys)
-    gt, k2 = _tbl(dxs)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_unpadded_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw, pad_h,
-                                                    pad_w, w.data_ptr(), dt, gt, beta, wp, wb, _stream())
+    return _n().adh_conv2d_unpadded_bwd_data_tiles(_dt(dys[0]), len(dys), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw,
+                                                   pad_h, pad_w, w, dys, dxs, beta, *_ws(ws))
 
 
 def conv2d_unpadded_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw_, pad_h, pad_w, beta=0.0, ws=None):
-    _dev(*xs, *dys, dw)
-    xt, k1 = _tbl(xs)
-    dt, k2 = _tbl(dys)
-    wp, wb = _ws(ws)
-    return lib().adh_conv2d_unpadded_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw_, pad_h,
-                                                      pad_w, xt, dt, dw.data_ptr(), beta, wp, wb, _stream())
-
-
-def _opt_tbl(ts):
-    if ts is None:
-        return None, None
-    return _tbl(ts)
+    return _n().adh_conv2d_unpadded_bwd_filter_tiles(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, kh, kw, sh, sw, dh, dw_,
+                                                     pad_h, pad_w, xs, dys, dw, beta, *_ws(ws))
 
 
 def batchnorm_workspace_bytes(K, N, C):
@@ -422,173 +349,116 @@ def batchnorm_workspace_bytes(K, N, C):
 
 def batchnorm_fwd_tiles(xs, scales, shifts, ys, N, C, H, W, eps=1e-5, relu=0, out_halo=0, training=True, fixed_means=None,
                         fixed_vars=None, run_means=None, run_vars=None, save_means=None, save_invstds=None, ws=None):
-    _dev(*xs, *ys, *scales, *shifts)
-    tabs = [_tbl(xs), _tbl(scales), _tbl(shifts), _opt_tbl(fixed_means), _opt_tbl(fixed_vars), _tbl(ys), _opt_tbl(run_means),
-            _opt_tbl(run_vars), _opt_tbl(save_means), _opt_tbl(save_invstds)]
-    wp, wb = _ws(ws)
-    return lib().adh_batchnorm2d_fwd_tiles(_dt(xs[0]), 1 if training else 0, len(xs), N, C, H, W, eps, relu, out_halo,
-                                           *[t[0] for t in tabs], wp, wb, _stream())
+    return _n().adh_batchnorm2d_fwd_tiles(_dt(xs[0]), 1 if training else 0, len(xs), N, C, H, W, eps, relu, out_halo,
+                                          xs, scales, shifts, fixed_means, fixed_vars, ys, run_means, run_vars,
+                                          save_means, save_invstds, *_ws(ws))
 
 
 def batchnorm_bwd_tiles(xs, dys, scales, shifts, save_means, save_invstds, dxs, dscales, dshifts, N, C, H, W, relu=0,
                         dy_halo=0, beta_data=0.0, beta_param=0.0, ws=None):
-    _dev(*xs, *dys, *dxs)
-    tabs = [_tbl(xs), _tbl(dys), _tbl(scales), _opt_tbl(shifts), _tbl(save_means), _tbl(save_invstds), _tbl(dxs),
-            _tbl(dscales), _tbl(dshifts)]
-    wp, wb = _ws(ws)
-    return lib().adh_batchnorm2d_bwd_tiles(_dt(xs[0]), len(xs), N, C, H, W, relu, dy_halo, *[t[0] for t in tabs],
-                                           beta_data, beta_param, wp, wb, _stream())
+    return _n().adh_batchnorm2d_bwd_tiles(_dt(xs[0]), len(xs), N, C, H, W, relu, dy_halo, xs, dys, scales, shifts,
+                                          save_means, save_invstds, dxs, dscales, dshifts, beta_data, beta_param,
+                                          *_ws(ws))
 
 
 def relu_fwd(x, y):
-    _dev(x, y)
-    return lib().adh_relu_fwd(_dt(x), x.numel(), x.data_ptr(), y.data_ptr(), _stream())
+    return _n().adh_relu_fwd(_dt(x), x.numel(), x, y)
 
 
 def relu_bwd(y, dy, dx, beta=0.0):
-    _dev(y, dy, dx)
-    return lib().adh_relu_bwd(_dt(y), y.numel(), y.data_ptr(), dy.data_ptr(), dx.data_ptr(), beta, _stream())
+    return _n().adh_relu_bwd(_dt(y), y.numel(), y, dy, dx, beta)
 
 
 def sum_fwd(xs, y):
-    _dev(*xs, y)
-    xt, keep = _tbl(xs)
-    return lib().adh_sum_fwd(_dt(y), len(xs), y.numel(), xt, y.data_ptr(), _stream())
+    return _n().adh_sum_fwd(_dt(y), len(xs), y.numel(), xs, y)
 
 
 def scale_add(alpha, x, beta, y):
     """y = alpha*x + beta*y over flat fp32 tensors."""
-    _dev(x, y)
-    return lib().adh_scale_add_f32(y.numel(), alpha, x.data_ptr(), beta, y.data_ptr(), _stream())
+    return _n().adh_scale_add_f32(y.numel(), alpha, x, beta, y)
 
 
 def add_online(alpha, x, y):
     """y = y + alpha*(x - y)."""
-    _dev(x, y)
-    return lib().adh_add_online_f32(y.numel(), alpha, x.data_ptr(), y.data_ptr(), _stream())
+    return _n().adh_add_online_f32(y.numel(), alpha, x, y)
 
 
 def stat_step(rate, avg_stat, running_stat, stat):
-    _dev(avg_stat, running_stat, stat)
-    return lib().adh_stat_step_f32(stat.numel(), rate, avg_stat.data_ptr(), running_stat.data_ptr(), stat.data_ptr(),
-                                   _stream())
-
-
-def _lens(arrays):
-    return (u64 * len(arrays))(*[a.numel() for a in arrays])
+    return _n().adh_stat_step_f32(stat.numel(), rate, avg_stat, running_stat, stat)
 
 
 def flat_store(arrays, flat, offset=0):
     """Copy the arrays, in order, into consecutive ranges of `flat` starting at element `offset`."""
-    _dev(*arrays, flat)
-    t, keep = _tbl(arrays)
-    return lib().adh_flat_store_f32(len(arrays), t, _lens(arrays), offset, flat.data_ptr(), _stream())
+    return _n().adh_flat_store_f32(len(arrays), arrays, arrays, offset, flat)
 
 
 def flat_load(arrays, flat, offset=0):
     """The inverse of flat_store: consecutive ranges of `flat` into the arrays."""
-    _dev(*arrays, flat)
-    t, keep = _tbl(arrays)
-    return lib().adh_flat_load_f32(len(arrays), t, _lens(arrays), offset, flat.data_ptr(), _stream())
+    return _n().adh_flat_load_f32(len(arrays), arrays, arrays, offset, flat)
 
 
 def sgd_step(grads, param, momentum_grad, lagged_param=None, sum_grad=None, l2_reg=0.0, momentum=0.0, step_size=0.0,
              next_step_size=0.0, nesterov=False):
     """One fused optimizer update over flat fp32 vectors; grads is the list of per-rank gradient vectors."""
-    _dev(*grads, param, momentum_grad)
-    t, keep = _tbl(grads)
-    return lib().adh_sgd_step_f32(param.numel(), len(grads), t, l2_reg, momentum, step_size, next_step_size,
-                                  int(bool(nesterov)), param.data_ptr(), momentum_grad.data_ptr(),
-                                  lagged_param.data_ptr() if lagged_param is not None else None,
-                                  sum_grad.data_ptr() if sum_grad is not None else None, _stream())
+    return _n().adh_sgd_step_f32(param.numel(), len(grads), grads, l2_reg, momentum, step_size, next_step_size,
+                                 int(bool(nesterov)), param, momentum_grad, lagged_param, sum_grad)
 
 
 def pool_fwd_tiles(mode, xs, ys, N, C, HP, WP, wh, ww, sh, sw):
-    _dev(*xs, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    return lib().adh_pool2d_slab_fwd_tiles(_dt(xs[0]), mode, len(xs), N, C, HP, WP, wh, ww, sh, sw, xt, yt, _stream())
+    return _n().adh_pool2d_slab_fwd_tiles(_dt(xs[0]), mode, len(xs), N, C, HP, WP, wh, ww, sh, sw, xs, ys)
 
 
 def pool_bwd_tiles(mode, xs, ys, dys, dxs, N, C, HP, WP, wh, ww, sh, sw, beta=0.0):
-    _dev(*xs, *ys, *dys, *dxs)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    dt, k3 = _tbl(dys)
-    gt, k4 = _tbl(dxs)
-    return lib().adh_pool2d_slab_bwd_tiles(_dt(dys[0]), mode, len(dys), N, C, HP, WP, wh, ww, sh, sw, xt, yt, dt, gt,
-                                           beta, _stream())
+    return _n().adh_pool2d_slab_bwd_tiles(_dt(dys[0]), mode, len(dys), N, C, HP, WP, wh, ww, sh, sw, xs, ys, dys, dxs,
+                                          beta)
 
 
 def pool_unpadded_fwd_tiles(mode, xs, ys, N, C, H, W, wh, ww, sh, sw, pad_h, pad_w):
     """Pooling over row tiles without halo: rows outside a tile come from its neighbours, zeros outside the tensor."""
-    _dev(*xs, *ys)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _tbl(ys)
-    return lib().adh_pool2d_unpadded_fwd_tiles(_dt(xs[0]), mode, len(xs), N, C, H, W, wh, ww, sh, sw, pad_h, pad_w, xt, yt,
-                                               _stream())
+    return _n().adh_pool2d_unpadded_fwd_tiles(_dt(xs[0]), mode, len(xs), N, C, H, W, wh, ww, sh, sw, pad_h, pad_w, xs,
+                                              ys)
 
 
 def pool_unpadded_bwd_tiles(mode, xs, ys, dys, dxs, N, C, H, W, wh, ww, sh, sw, pad_h, pad_w, beta=0.0):
-    _dev(*xs, *dys, *dxs)
-    xt, k1 = _tbl(xs)
-    yt, k2 = _opt_tbl(ys)
-    dt, k3 = _tbl(dys)
-    gt, k4 = _tbl(dxs)
-    return lib().adh_pool2d_unpadded_bwd_tiles(_dt(dys[0]), mode, len(dys), N, C, H, W, wh, ww, sh, sw, pad_h, pad_w, xt, yt,
-                                               dt, gt, beta, _stream())
+    return _n().adh_pool2d_unpadded_bwd_tiles(_dt(dys[0]), mode, len(dys), N, C, H, W, wh, ww, sh, sw, pad_h, pad_w, xs,
+                                              ys, dys, dxs, beta)
 
 
 def conv_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, H, W, beta=0.0, ws=None, unexchanged=False):
-    _dev(dw, *xs, *dys)
-    xt, k1 = _tbl(xs)
-    dt, k2 = _tbl(dys)
-    wp, wb = _ws(ws)
-    fn = (lib().adh_conv3x3_slab_bwd_filter_tiles_unexchanged if unexchanged
-          else lib().adh_conv3x3_slab_bwd_filter_tiles)
-    return fn(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xt, dt, dw.data_ptr(), beta, wp, wb, _stream())
+    fn = (_n().adh_conv3x3_slab_bwd_filter_tiles_unexchanged if unexchanged
+          else _n().adh_conv3x3_slab_bwd_filter_tiles)
+    return fn(_dt(xs[0]), len(xs), N, Cin, Cout, H, W, xs, dys, dw, beta, *_ws(ws))
 
 
 def softmax_fwd(x, y):
-    _dev(x, y)
     N, C = x.shape
-    return lib().adh_softmax_fwd(C, N, x.data_ptr(), y.data_ptr(), _stream())
+    return _n().adh_softmax_fwd(C, N, x, y)
 
 
 def softmax_xent_fwd(x, label, y, loss):
-    _dev(x, label, y, loss)
     N, C = x.shape
-    return lib().adh_softmax_xent_fwd(C, N, x.data_ptr(), label.data_ptr(), y.data_ptr(), loss.data_ptr(), _stream())
+    return _n().adh_softmax_xent_fwd(C, N, x, label, y, loss)
 
 
 def softmax_nll_loss_fwd(y, label, loss):
-    _dev(y, label, loss)
     N, C = y.shape
-    return lib().adh_softmax_nll_loss_fwd(C, N, y.data_ptr(), label.data_ptr(), loss.data_ptr(), _stream())
+    return _n().adh_softmax_nll_loss_fwd(C, N, y, label, loss)
 
 
 def softmax_nll_loss_bwd(y, label, dloss, dx):
-    _dev(y, label, dloss, dx)
     N, C = y.shape
-    return lib().adh_softmax_nll_loss_bwd(C, N, y.data_ptr(), label.data_ptr(), dloss.data_ptr(), dx.data_ptr(),
-                                          _stream())
+    return _n().adh_softmax_nll_loss_bwd(C, N, y, label, dloss, dx)
 
 
 def softmax_nll_loss_bwd_scaled(y, label, dloss, dloss_all, beta, dx):
     """dx = beta*dx + dl*(y - onehot); dloss None: every example's dl is dloss_all."""
-    _dev(y, label, dx)
     N, C = y.shape
-    return lib().adh_softmax_nll_loss_bwd_scaled(C, N, y.data_ptr(), label.data_ptr(),
-                                                 None if dloss is None else dloss.data_ptr(), dloss_all, beta,
-                                                 dx.data_ptr(), _stream())
+    return _n().adh_softmax_nll_loss_bwd_scaled(C, N, y, label, dloss, dloss_all, beta, dx)
 
 
 def softmax_xent_fwd_bwd(x, label, dloss, dloss_all, y, loss, beta, dx):
-    _dev(x, label, y, loss, dx)
     N, C = x.shape
-    return lib().adh_softmax_xent_fwd_bwd(C, N, x.data_ptr(), label.data_ptr(),
-                                          None if dloss is None else dloss.data_ptr(), dloss_all, y.data_ptr(),
-                                          loss.data_ptr(), beta, dx.data_ptr(), _stream())
+    return _n().adh_softmax_xent_fwd_bwd(C, N, x, label, dloss, dloss_all, y, loss, beta, dx)
 
 
 def conv_kernel_name(which, dtype, K, N, Cin, Cout, H, W, beta=0.0):
