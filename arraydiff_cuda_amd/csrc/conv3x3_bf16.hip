@@ -8,7 +8,7 @@
 // result is rounded back to bf16 (round to nearest even).  Every product is therefore exact and every sum is in
 // fp32, i.e. the arithmetic of a bf16-input / fp32-accumulate matrix core, at the speed of the
 // fp32 path plus three streaming passes.  The filter gradient stays fp32.
-#include "adh_common.h"
+#include "conv3x3_bf16_mfma.h"
 
 namespace adh {
 
@@ -52,19 +52,60 @@ __global__ __launch_bounds__(256) void narrow_bf16_kernel(uint64_t n, const floa
   }
 }
 
-// Rows of `w_src` bf16 elements copied into rows of `w_dst` >= w_src elements (w_dst even; dst 4-byte aligned),
-// zeros behind: one thread per dword of the destination.
-__global__ __launch_bounds__(256) void repitch_bf16_kernel(uint64_t rows, uint32_t w_src, uint32_t w_dst,
-                                                          const uint16_t *__restrict__ src, uint32_t *__restrict__ dst) {
-  const uint32_t row_dwords = w_dst >> 1;
-  const uint64_t n = rows * row_dwords;
-  const uint64_t stride = (uint64_t)gridDim.x * 256u;
-  for (uint64_t i = (uint64_t)blockIdx.x * 256u + threadIdx.x; i < n; i += stride) {
-    const uint64_t r = i / row_dwords;
-    const uint32_t c = (uint32_t)(i - r * row_dwords) * 2u;
-    const uint16_t *p = src + r * w_src + c;
-    const uint32_t lo = c < w_src ? p[0] : 0u, hi = c + 1u < w_src ? p[1] : 0u;
-    dst[i] = lo | (hi << 16);
+// Rows of `w_src` bf16 elements copied into rows of `w_dst` >= w_src elements (w_dst even), zeros behind.  A thread moves
+// granules of eight elements, four of them in flight: one 16-byte load from wherever the source row starts and one store
+// (the last granule of a row: its whole dwords).  Bound by memory.
+struct RepitchParams {
+  const uint16_t *src[ADH_MAX_TILES];
+  uint16_t *dst[ADH_MAX_TILES];
+  uint32_t rows, w_src, w_dst, granules;  // granules of a destination row
+  FastDiv div_granules;
+};
+__global__ __launch_bounds__(256) void repitch_bf16_kernel(RepitchParams P) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  typedef u32x4 u32x4_src __attribute__((aligned(2)));
+  typedef u32x4 u32x4_dst __attribute__((aligned(4)));
+  constexpr int kFlight = 4;
+  const uint16_t *src = P.src[blockIdx.y];
+  uint16_t *dst = P.dst[blockIdx.y];
+  const uint32_t n = P.rows * P.granules;
+  const uint64_t elems = (uint64_t)P.rows * P.w_src;
+  for (uint32_t base = blockIdx.x * (256u * kFlight) + threadIdx.x; base < n; base += gridDim.x * (256u * kFlight)) {
+    u32x4 v[kFlight];
+    uint32_t row[kFlight], col[kFlight];
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      const uint32_t i = base + 256u * u;
+      v[u] = (u32x4){0u, 0u, 0u, 0u};
+      P.div_granules.divmod(i, row[u], col[u]);
+      col[u] *= 8u;
+      if (i >= n || col[u] >= P.w_src) continue;
+      const uint64_t at = (uint64_t)row[u] * P.w_src + col[u];
+      if (at + 8u <= elems) {
+        v[u] = *reinterpret_cast<const u32x4_src *>(src + at);
+      } else {
+        for (uint32_t e = 0; at + e < elems; ++e) v[u][e >> 1] |= (uint32_t)src[at + e] << ((e & 1u) * 16u);
+      }
+    }
+#pragma unroll
+    for (int u = 0; u < kFlight; ++u) {
+      if (base + 256u * u >= n) break;
+      // what lies behind the source row is the next row's
+      const int32_t left = (int32_t)P.w_src - (int32_t)col[u];
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        if (left <= 2 * d) v[u][d] = 0u;
+        else if (left == 2 * d + 1) v[u][d] &= 0xffffu;
+      }
+      uint16_t *o = dst + (uint64_t)row[u] * P.w_dst + col[u];
+      if (col[u] + 8u <= P.w_dst) {
+        *reinterpret_cast<u32x4_dst *>(o) = v[u];
+      } else {
+#pragma unroll
+        for (int d = 0; d < 4; ++d)
+          if (col[u] + 2u * d < P.w_dst) *reinterpret_cast<uint32_t *>(o + 2 * d) = v[u][d];
+      }
+    }
   }
 }
 
@@ -82,7 +123,7 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
                                       uint32_t W);
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree = false);
+                   hipStream_t st, bool halofree = false, bool filter_only = false);
 
 bool conv_bf16_wgrad_mfma_supported(uint32_t Cin, uint32_t Cout, uint32_t W);
 size_t conv_bf16_wgrad_mfma_workspace_bytes(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t W);
@@ -101,7 +142,24 @@ static bool wgrad_repitch_route(uint32_t Cin, uint32_t Cout, uint32_t H, uint32_
   return conv_bf16_wgrad_mfma_supported(Cin, Cout, Wd) &&
          (uint64_t)(Cin > Cout ? Cin : Cout) * (H + 2ull) * (Wd + 2ull) * 2u < (1ull << 31);
 }
-static size_t repitch_region(uint64_t elems) { return (size_t)((elems * 2u + 255u) / 256u * 256u); }
+
+int repitch_bf16_tiles(uint32_t num_tiles, uint64_t rows, uint32_t w_src, uint32_t w_dst, const void *const *src,
+                       void *const *dst, hipStream_t st) {
+  RepitchParams P;
+  for (uint32_t t = 0; t < num_tiles; ++t) {
+    P.src[t] = reinterpret_cast<const uint16_t *>(src[t]);
+    P.dst[t] = reinterpret_cast<uint16_t *>(dst[t]);
+  }
+  P.w_src = w_src;
+  P.w_dst = w_dst;
+  P.granules = (w_dst + 7u) / 8u;
+  P.rows = (uint32_t)rows;
+  P.div_granules = FastDiv(P.granules);
+  if (rows * P.granules >= (1ull << 31)) return ADH_EINVAL;
+  const uint32_t blocks = ((uint32_t)rows * P.granules + 1023u) / 1024u, most = (256u * 8u + num_tiles - 1u) / num_tiles;
+  hipLaunchKernelGGL(repitch_bf16_kernel, dim3(blocks < most ? blocks : most, num_tiles), dim3(256), 0, st, P);
+  return launch_status();
+}
 
 size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
                             uint32_t W, size_t fp32_path_bytes) {
@@ -109,7 +167,7 @@ size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t 
     return conv_bf16_wgrad_mfma_workspace_bytes(num_tiles, N, Cin, Cout, W);
   if (which == ADH_CONV_BWD_FILTER && wgrad_repitch_route(Cin, Cout, H, W)) {
     const uint32_t Wd = wgrad_wide_width(W);
-    return num_tiles * (repitch_region((uint64_t)N * Cin * (H + 2) * (Wd + 2)) + repitch_region((uint64_t)N * Cout * H * Wd)) +
+    return num_tiles * (repitch_bf16_region((uint64_t)N * Cin * (H + 2) * (Wd + 2)) + repitch_bf16_region((uint64_t)N * Cout * H * Wd)) +
            conv_bf16_wgrad_mfma_workspace_bytes(num_tiles, N, Cin, Cout, Wd);
   }
   if (which != ADH_CONV_BWD_FILTER && conv_bf16_mfma_supported(which, Cin, Cout, H, W))
@@ -226,25 +284,19 @@ int conv_bf16_filter_via_f32(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint3
     if (workspace_bytes < bf16_workspace_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, 0)) return ADH_EWORKSPACE;
     const uint64_t x_rows = (uint64_t)N * Cin * (H + 2), dy_rows = (uint64_t)N * Cout * H;
     char *ws = reinterpret_cast<char *>(workspace);
-    const void *xw[ADH_MAX_TILES];
-    const void *dyw[ADH_MAX_TILES];
+    void *xw[ADH_MAX_TILES], *dyw[ADH_MAX_TILES];
     for (uint32_t t = 0; t < num_tiles; ++t) {
       if (!x_tiles[t] || !dy_tiles[t]) return ADH_ENULL;
       if (!aligned_to(x_tiles[t], 2) || !aligned_to(dy_tiles[t], 2)) return ADH_EALIGN;
-      uint32_t *a = reinterpret_cast<uint32_t *>(ws);
-      ws += repitch_region(x_rows * (Wd + 2));
-      uint32_t *b = reinterpret_cast<uint32_t *>(ws);
-      ws += repitch_region(dy_rows * Wd);
-      hipLaunchKernelGGL(repitch_bf16_kernel, dim3(cvt_grid(x_rows * (Wd + 2) * 4u)), dim3(256), 0, st, x_rows, W + 2u, Wd + 2u,
-                         reinterpret_cast<const uint16_t *>(x_tiles[t]), a);
-      int e = launch_status();
-      if (e) return e;
-      hipLaunchKernelGGL(repitch_bf16_kernel, dim3(cvt_grid(dy_rows * Wd * 4u)), dim3(256), 0, st, dy_rows, W, Wd,
-                         reinterpret_cast<const uint16_t *>(dy_tiles[t]), b);
-      if ((e = launch_status())) return e;
-      xw[t] = a;
-      dyw[t] = b;
+      xw[t] = ws;
+      ws += repitch_bf16_region(x_rows * (Wd + 2));
+      dyw[t] = ws;
+      ws += repitch_bf16_region(dy_rows * Wd);
     }
+    int e = repitch_bf16_tiles(num_tiles, x_rows, W + 2u, Wd + 2u, x_tiles, xw, st);
+    if (e) return e;
+    e = repitch_bf16_tiles(num_tiles, dy_rows, W, Wd, dy_tiles, dyw, st);
+    if (e) return e;
     return conv_bf16_wgrad_mfma(num_tiles, N, Cin, Cout, H, Wd, xw, dyw, dw, beta, ws, st, false);
   }
   const size_t f32_bytes = adh_conv3x3_workspace_bytes(ADH_CONV_BWD_FILTER, ADH_F32, num_tiles, N, Cin, Cout, H, W);

@@ -74,6 +74,11 @@ constexpr int kStripColsK128 = 32;
 bool conv_bf16_k128_takes(const ConvBf16Params &P, uint32_t num_tiles);
 int conv_bf16_k128_launch(const ConvBf16Params &P, uint32_t gx, uint32_t groups128, hipStream_t st);
 
+// rows of w_src elements into rows of w_dst (even), zeros behind: the tiles of `src` into those of `dst`
+int repitch_bf16_tiles(uint32_t num_tiles, uint64_t rows, uint32_t w_src, uint32_t w_dst, const void *const *src,
+                       void *const *dst, hipStream_t st);
+inline size_t repitch_bf16_region(uint64_t elems) { return (size_t)((elems * 2u + 255u) / 256u * 256u); }
+
 }  // namespace adh
 
 #endif

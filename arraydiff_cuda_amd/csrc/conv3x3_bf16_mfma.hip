@@ -557,9 +557,9 @@ static int num_cus() {
 
 // Up to 64 reduction channels: any shape.  More: several launches with fp32 sums between them, which the
 // eight-wave kernels address through a buffer resource: the sums of one image have to lie inside 2 GiB.
-// (The eight-wave kernels need rows on a 4-byte boundary (forward: even width) or whole 16-byte granules
-// (backward-data: a width that is a multiple of 8) and aligned tiles; other shapes take the four-wave kernel
-// once per 64 reduction channels.)
+// (The eight-wave kernels need input rows on a 4-byte boundary (forward: even width) or whole 16-byte granules
+// (backward-data: a width that is a multiple of 8) and aligned tiles; at other widths they run over a copy of the
+// input with wider rows.  The four-wave kernel, once per 64 reduction channels, takes what is left.)
 bool conv_bf16_mfma_supported(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
   const uint32_t cred = which == ADH_CONV_FWD ? Cin : Cout;
   if (cred <= 64u) return true;
@@ -569,6 +569,20 @@ bool conv_bf16_mfma_supported(int which, uint32_t Cin, uint32_t Cout, uint32_t H
 }
 // widths whose rows the eight-wave kernels take
 static bool conv_bf16_w8_width(int which, uint32_t W) { return which == ADH_CONV_FWD ? (W % 2u) == 0u : (W % 8u) == 0u; }
+// At the other widths the input is copied into rows of the next multiple of 8, zeros behind, and the eight-wave kernels
+// run on the copy: where more than 64 channels are summed, which the four-wave kernel takes in one launch per 64 with
+// fp32 sums through memory (128 -> 128 channels, 8 images of 4 tiles of 64x255: forward 455 -> 212 us, backward-data
+// 357 -> 199, the copy included; 512 -> 512, 4 images of 14x13: 258 -> 125).  Up to 64 channels the copy costs what the
+// eight waves gain (32 channels, 8 tiles of 100x1001: 69 -> 83 us).
+static uint32_t conv_bf16_wide_row(int which, uint32_t W) { return ((which == ADH_CONV_FWD ? W + 2u : W) + 7u) & ~7u; }
+static bool conv_bf16_repitches(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
+  if (conv_bf16_w8_width(which, W) || (which == ADH_CONV_FWD ? Cin : Cout) <= 64u) return false;
+  const uint64_t rows = which == ADH_CONV_FWD ? Cin * (H + 2ull) : (uint64_t)Cout * H;
+  return rows * conv_bf16_wide_row(which, W) * 2u < (1ull << 31);
+}
+static size_t conv_bf16_repitch_bytes(int which, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
+  return repitch_bf16_region((which == ADH_CONV_FWD ? (uint64_t)N * Cin * (H + 2) : (uint64_t)N * Cout * H) * conv_bf16_wide_row(which, W));
+}
 static uint32_t conv_bf16_passes(int which, uint32_t Cin, uint32_t Cout) {
   return ((which == ADH_CONV_FWD ? Cin : Cout) + 63u) / 64u;
 }
@@ -577,9 +591,10 @@ static uint32_t conv_bf16_passes(int which, uint32_t Cin, uint32_t Cout) {
 // launch of the eight-wave kernel per 64.
 static bool conv_bf16_uses_k128(int which, uint32_t Cin, uint32_t Cout) { return Cin > 64u && Cout > 64u; }
 // (a width the eight-wave kernels do not take: one launch of the four-wave kernel per 64)
-static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint32_t W) {
+static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
   const uint32_t cred = which == ADH_CONV_FWD ? Cin : Cout;
-  if (!conv_bf16_uses_k128(which, Cin, Cout) || !conv_bf16_w8_width(which, W)) return (cred + 63u) / 64u;
+  if (!conv_bf16_uses_k128(which, Cin, Cout) || !(conv_bf16_w8_width(which, W) || conv_bf16_repitches(which, Cin, Cout, H, W)))
+    return (cred + 63u) / 64u;
   uint32_t n = 0, rem = cred;
   while (rem > 64u) {
     rem -= rem < 128u ? rem : 128u;
@@ -592,14 +607,14 @@ static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint3
 // (template arguments: old output added, sums of earlier passes read, sums written for a later pass, tiles without halo)
 const char *conv_bf16_kernel_name(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, float beta) {
   if (!conv_bf16_mfma_supported(which, Cin, Cout, H, W)) return "widen_bf16_kernel + conv3x3_f32_kernel + narrow_bf16_kernel";
-  if (!conv_bf16_w8_width(which, W)) {
+  if (!conv_bf16_w8_width(which, W) && !conv_bf16_repitches(which, Cin, Cout, H, W)) {
     if (conv_bf16_passes(which, Cin, Cout) > 1u)
       return beta != 0.f ? "conv3x3_bf16_kernel<true, false, true> + <false, true, true> per middle 64 reduction channels + <false, true, false>"
                          : "conv3x3_bf16_kernel<false, false, true> + <false, true, true> per middle 64 reduction channels + <false, true, false>";
     return beta != 0.f ? "conv3x3_bf16_kernel<true, false, false>" : "conv3x3_bf16_kernel<false, false, false>";
   }
   if (conv_bf16_uses_k128(which, Cin, Cout)) {
-    if (conv_bf16_launches(which, Cin, Cout, W) == 1u)
+    if (conv_bf16_launches(which, Cin, Cout, H, W) == 1u)
       return beta != 0.f ? "conv3x3_bf16_k128_kernel<true, false, false, false>" : "conv3x3_bf16_k128_kernel<false, false, false, false>";
     return "conv3x3_bf16_k128_kernel per 128 reduction channels (fp32 sums between the launches) + conv3x3_bf16_w8_kernel for a rest of at most 64";
   }
@@ -641,7 +656,8 @@ static size_t part_region_bytes(int which, uint32_t N, uint32_t Cin, uint32_t Co
 size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
                                       uint32_t W) {
   size_t bytes = filter_region_bytes(which, Cin, Cout);
-  if (conv_bf16_launches(which, Cin, Cout, W) > 1u) bytes += (size_t)num_tiles * part_region_bytes(which, N, Cin, Cout, H, W);
+  if (conv_bf16_launches(which, Cin, Cout, H, W) > 1u) bytes += (size_t)num_tiles * part_region_bytes(which, N, Cin, Cout, H, W);
+  if (conv_bf16_repitches(which, Cin, Cout, H, W)) bytes += num_tiles * conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W);
   return bytes;
 }
 
@@ -651,9 +667,10 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
 // and a tile's rows -1 and H are its neighbours' last and first rows (zeros at the tensor's own border): the
 // unsplit convolution with zero padding, restricted to the tile.  Only shapes the eight-wave kernel takes
 // (ADH_EUNIMPL otherwise).
+// filter_only: the workspace holds the reordered filter and no more (no copy of the input with wider rows).
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree) {
+                   hipStream_t st, bool halofree, bool filter_only) {
   ConvBf16Params P = {};
   for (uint32_t t = 0; t < num_tiles; ++t) {
     P.in[t] = reinterpret_cast<const uint16_t *>(in_tiles[t]);
@@ -683,11 +700,23 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
   P.chan0 = 0;
   P.cred_pass = P.Cred < 64u ? P.Cred : 64u;
   P.first_pass = P.last_pass = 1;
-  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, W);
+  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, H, W);
   if (launches > 1u) {
     uint8_t *part = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout);
     const size_t per_tile = part_region_bytes(which, N, Cin, Cout, H, W);
     for (uint32_t t = 0; t < num_tiles; ++t) P.part[t] = reinterpret_cast<float *>(part + t * per_tile);
+  }
+  if (!halofree && !filter_only && conv_bf16_repitches(which, Cin, Cout, H, W)) {
+    uint8_t *copy = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout) +
+                    (launches > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : 0u);
+    const size_t per_tile = conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W);
+    void *wide[ADH_MAX_TILES];
+    for (uint32_t t = 0; t < num_tiles; ++t) wide[t] = copy + t * per_tile;
+    const uint32_t w_src = P.IW;
+    P.IW = conv_bf16_wide_row(which, W);
+    const int e = repitch_bf16_tiles(num_tiles, (uint64_t)N * P.Cred * P.IH, w_src, P.IW, in_tiles, wide, st);
+    if (e) return e;
+    for (uint32_t t = 0; t < num_tiles; ++t) P.in[t] = reinterpret_cast<const uint16_t *>(wide[t]);
   }
   if (halofree && !conv_bf16_w8_takes(P, num_tiles)) return ADH_EUNIMPL;
   // the forward pass of the eight-wave kernel can read the caller's filter itself
@@ -864,7 +893,7 @@ extern "C" int adh_conv3x3_slab_fwd_tiles_static(int dtype, uint32_t num_tiles, 
   const int e = static_scratch(&ws);
   if (e) return e;
   return conv_bf16_mfma(ADH_CONV_FWD, num_tiles, N, Cin, Cout, H, W, x_pad_tiles, w, y_tiles, beta, ws, as_stream(stream),
-                        false);
+                        false, true);
 }
 
 // ---------------------------------------------------------------------------
@@ -894,6 +923,6 @@ int conv_bf16_unpadded(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
-  return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, true);
+  return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, true, false);
 }
 }  // namespace adh

@@ -687,18 +687,18 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   if (barrier_owed) phase_barrier();
 }
 
-// Shapes of the eight-wave kernel: input and output rows that start on a 4-byte boundary (input
-// rows on 16 bytes for backward-data, whose granules must lie wholly inside or outside a row),
-// images whose byte offsets fit the buffer range check's 31 bits.
+// Shapes of the eight-wave kernel: input rows that start on a 4-byte boundary (on 16 bytes for
+// backward-data, whose granules must lie wholly inside or outside a row; output rows may start
+// anywhere), images whose byte offsets fit the buffer range check's 31 bits.
 bool conv_bf16_w8_takes(const ConvBf16Params &P, uint32_t num_tiles) {
   if (P.pad ? (P.IW % 8u) != 0u : (P.IW % 2u) != 0u) return false;
   if (P.neighbour_rows && P.IH == 0u) return false;
   const uint64_t image_bytes = (uint64_t)P.Cred * P.IH * P.IW * 2u;
   if (image_bytes >= (1ull << 31)) return false;
-  if ((uint64_t)P.Cout * P.OH * P.OW * 2u >= (1ull << 31) || (P.OW % 2u) != 0u) return false;
+  if ((uint64_t)P.Cout * P.OH * P.OW * 2u >= (1ull << 31)) return false;
   const size_t a = P.pad ? 16 : 4;
   for (uint32_t t = 0; t < num_tiles; ++t)
-    if (!aligned_to(P.in[t], a) || !aligned_to(P.out[t], 4)) return false;
+    if (!aligned_to(P.in[t], a) || !aligned_to(P.out[t], 2)) return false;
   if (P.Cred > 64u) {
     // the fp32 sums between passes are addressed like the output, at four bytes an element
     if ((uint64_t)P.Cout * P.OH * P.OW * 4u >= (1ull << 31)) return false;
