@@ -1,12 +1,14 @@
-// Forward convolution of an input with very few channels (an image: 1-3) over halo-padded tiles, fp32 matrix cores:
-// the stem of a network (7x7 over RGB).  The general kernel multiplies four channels per step, so three channels
+// Convolution of an input with very few channels (an image: 1-3) over halo-padded tiles, fp32 matrix cores: the windows that
+// conv_thin_split.hip does not take (wider than eight columns, column strides from three on; for the filter gradient windows of
+// other widths than 3, 5 and 7).
+// The general kernel multiplies four channels per step, so three channels
 // waste a quarter of every step, and it stages the filter tap group by tap group between barriers.  Here the
 // reduction index is the flattened (channel, tap) pair, k = (c kh + a) kw + b < 148: the 147 pairs of a 7x7x3 window
 // are 37 steps of 4 with one pair of padding; the whole filter of 64 output channels (38 KB) and the input patch of
 // 256 output pixels (8 rows x 32 columns) are staged once, and the multiplications then run without a barrier.
 // v_mfma_f32_16x16x4_f32 takes the pixels as its row operand (a lane ends up with four neighbouring pixels of one
 // output channel); lane group g of a step reads the patch at the offset of ITS pair, kept in a register per step.
-#include "adh_common.h"
+#include "conv_thin_split.h"
 
 #include <algorithm>
 
@@ -193,6 +195,9 @@ int conv_thin_fwd_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cou
                       const void *w, void *const *y_tiles, float beta, hipStream_t st, const float *const *bias_tiles) {
   if (Cin == 0 || Cin > 3u || Cin * kh * kw > kThinK) return ADH_EUNIMPL;
   if (!aligned_to(w, 4)) return ADH_EUNIMPL;
+  const ThinProblem q = {num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, x_tiles};
+  const int e = conv_thin_split_fwd(q, w, y_tiles, beta, bias_tiles, st);
+  if (e != ADH_EUNIMPL) return e;
   bool vec = OW % 4u == 0u;
   for (uint32_t t = 0; t < num_tiles; ++t) {
     if (!aligned_to(x_tiles[t], 4) || !aligned_to(y_tiles[t], 4)) return ADH_EUNIMPL;
@@ -422,9 +427,11 @@ static bool thin_wgrad_plan(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32
 // the partial sums of conv_thin_wgrad_try (0: not a shape it serves)
 size_t conv_thin_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t HP, uint32_t WP,
                                  uint32_t OH, uint32_t OW, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw) {
+  const ThinProblem q = {num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, nullptr};
+  const size_t split_bytes = conv_thin_split_wgrad_workspace(q);
   ThinWgradPlan plan;
-  if (!thin_wgrad_plan(num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, &plan)) return 0;
-  return plan.part_bytes;
+  if (!thin_wgrad_plan(num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, &plan)) return split_bytes;
+  return std::max(split_bytes, plan.part_bytes);
 }
 
 // Filter gradient over halo-padded fp32 tiles for at most three input channels and Cin kh kw <= 160, any stride, no
@@ -432,6 +439,9 @@ size_t conv_thin_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, u
 int conv_thin_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t HP, uint32_t WP, uint32_t OH,
                         uint32_t OW, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw, const void *const *x_tiles,
                         const void *const *dy_tiles, float *dwt, float beta, void *workspace, hipStream_t st) {
+  const ThinProblem q = {num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, x_tiles};
+  const int split = conv_thin_split_wgrad(q, dy_tiles, dwt, beta, workspace, st);
+  if (split != ADH_EUNIMPL) return split;
   ThinWgradPlan plan;
   if (!thin_wgrad_plan(num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, &plan)) return ADH_EUNIMPL;
   ThinWgradParams P = {};
