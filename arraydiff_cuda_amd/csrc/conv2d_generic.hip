@@ -585,14 +585,10 @@ int conv1x1_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cou
                       uint32_t OW, uint32_t sh, uint32_t sw, const void *const *x_tiles, const void *const *dy_tiles,
                       float *dwt, float beta, void *workspace, hipStream_t st);
 
-// conv3x3s2.hip: backward-data of a 3x3 window at stride 2, padding 1, over fp32 tiles of H x W without halo
-int conv3x3s2_bwd_data_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
-                           const void *w, const void *const *dy_tiles, void *const *dx_tiles, float beta,
-                           hipStream_t st);
-
+// conv3x3s2.hip: filter gradient of a 3x3 window at stride 2, padding 1, over fp32 tiles of H x W without halo, and its
+// forward for many input channels
 int conv3x3s2_fwd_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                       const void *const *x_tiles, const void *w, void *const *y_tiles, float beta, hipStream_t st);
-
 size_t conv3x3s2_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
 int conv3x3s2_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                         const void *const *x_tiles, const void *const *dy_tiles, float *dwt, float beta, void *workspace,
@@ -605,6 +601,10 @@ static bool gen_is_3x3s2_unpadded(int dtype, const GenShape &g, bool unpadded, u
 // conv3x3_split.hip: the 3x3 window at stride 1 in fp32, forward and backward-data, over padded tiles and tiles without halo
 static bool gen_is_3x3_unit(int dtype, const GenShape &g) {
   return dtype == ADH_F32 && g.kh == 3u && g.kw == 3u && g.sh == 1u && g.sw == 1u && g.dh == g.dw && g.dh <= 8u;
+}
+// and at stride 2 over tiles of even height and width without halo
+static bool gen_is_3x3_split(int dtype, const GenShape &g, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
+  return gen_is_3x3_unit(dtype, g) || (gen_is_3x3s2_unpadded(dtype, g, unpadded, pad_h, pad_w) && g.HP % 2u == 0u && g.WP % 2u == 0u);
 }
 static Conv3x3Problem gen_3x3_problem(int which, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
   const bool fwd = which == ADH_CONV_FWD;
@@ -623,6 +623,11 @@ static Conv3x3Problem gen_3x3_problem(int which, const GenShape &g, uint32_t num
   q.pad_c = (int32_t)(fwd ? pad_w : 2u * g.dw) - (fwd ? 0 : (int32_t)pad_w);
   q.w_m_stride = fwd ? g.Cin * 9u : 9u;
   q.w_c_stride = fwd ? 9u : g.Cin * 9u;
+  if (g.sh == 2u) {
+    q.sample = fwd ? kDown : kUp;
+    q.step = g.OH;
+    q.pad_r = q.pad_c = fwd ? 1 : 0;
+  }
   return q;
 }
 // the dilated window's filter gradient has a kernel of its own
@@ -1226,7 +1231,8 @@ size_t conv2d_workspace(int which, int dtype, uint32_t num_tiles, uint32_t N, ui
   else if (which == ADH_CONV_BWD_DATA) e = gen_plan_bwd_data(g, &plan, unpadded, pad_h, pad_w);
   if (e) return 0;
   const size_t bytes = ((plan.wt_bytes + 255u) & ~(size_t)255u) + ((plan.part_bytes + 255u) & ~(size_t)255u);
-  if (gen_is_3x3_unit(dtype, g)) return std::max(bytes, conv3x3_split_workspace(gen_3x3_problem(which, g, num_tiles, unpadded, pad_h, pad_w)));
+  if (gen_is_3x3_split(dtype, g, unpadded, pad_h, pad_w))
+    return std::max(bytes, conv3x3_split_workspace(gen_3x3_problem(which, g, num_tiles, unpadded, pad_h, pad_w)));
   return bytes;
 }
 
@@ -1271,20 +1277,19 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     if (e == ADH_OK && bias_tiles && bias_added) *bias_added = true;
     if (e != ADH_EUNIMPL) return e;
   }
-  if (gen_is_3x3_unit(dtype, g)) {
+  if (gen_is_3x3s2_unpadded(dtype, g, unpadded, pad_h, pad_w)) {
+    e = gen_check_workspace(plan, workspace, workspace_bytes);
+    if (e) return e;
+    e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
+    if (e != ADH_EUNIMPL) return e;
+  }
+  if (gen_is_3x3_split(dtype, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = x_tiles; q.out = y_tiles; q.w = w;
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
-    if (e != ADH_EUNIMPL) return e;
-  }
-  if (dtype == ADH_F32 && unpadded && kh == 3u && kw == 3u && sh == 2u && sw == 2u && dh == 1u && dw == 1u && pad_h == 1u &&
-      pad_w == 1u) {
-    e = gen_check_workspace(plan, workspace, workspace_bytes);
-    if (e) return e;
-    e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   return gen_launch(dtype, &plan, num_tiles, w, workspace, workspace_bytes, as_stream(stream));
@@ -1322,20 +1327,13 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     e = conv1x1_try(true, num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, g.sh, dy_tiles, w, dx_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
-  if (gen_is_3x3_unit(dtype, g)) {
+  if (gen_is_3x3_split(dtype, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = dy_tiles; q.out = dx_tiles; q.w = w;
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
-    if (e != ADH_EUNIMPL) return e;
-  }
-  if (dtype == ADH_F32 && unpadded && kh == 3u && kw == 3u && sh == 2u && sw == 2u && dh == 1u && dw == 1u && pad_h == 1u &&
-      pad_w == 1u) {
-    e = gen_check_workspace(plan, workspace, workspace_bytes);
-    if (e) return e;
-    e = conv3x3s2_bwd_data_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, w, dy_tiles, dx_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   return gen_launch(dtype, &plan, num_tiles, w, workspace, workspace_bytes, as_stream(stream));

@@ -1,4 +1,4 @@
-// The 3x3 window at stride 1 in fp32, forward and backward-data: what conv3x3_split.hip gives the entry points.
+// The 3x3 window at stride 1, and at stride 2 over tiles without halo, in fp32, forward and backward-data: what conv3x3_split.hip gives the entry points.
 #ifndef ADH_CONV3X3_SPLIT_H
 #define ADH_CONV3X3_SPLIT_H
 
@@ -7,12 +7,16 @@
 namespace adh {
 
 // out[m][R][Q] = beta*out + sum over c, a, b of w * in[c][R + D*a - pad_r][Q + D*b - pad_c], D the dilation (zero outside `in`)
+// kDown, kUp: stride 2, padding 1, dilation 1 (tiles of even height and width), stacked without leading rows: forward from
+// tiles of 2 step rows to such of step, and backward-data from the latter to the former
+enum SplitSample { kUnit, kDown, kUp };
 struct Conv3x3Problem {
   uint32_t num_tiles, N, C, M;  // C reduction channels, M produced channels
   // The tiles' extents.  stacked: they are the row tiles of one tensor in rank order, whose rows are numbered through: tile t
   // holds rows lead + t*step .. lead + (t+1)*step - 1 of it; `lead` rows precede the first tile's own and as many follow
   // the last one's (the padded forms' outer halo row).  Otherwise every tile is a tensor of its own.
   uint32_t in_H, in_W, out_H, out_W;
+  SplitSample sample;
   bool stacked;
   uint32_t step, in_lead, out_lead;
   int32_t pad_r, pad_c;

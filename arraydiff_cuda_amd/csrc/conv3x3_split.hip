@@ -18,6 +18,11 @@
 // Row tiles of one tensor are addressed as that tensor: a patch row is divided by the tile height to find its tile, so a
 // workgroup may span tiles (a 4 x 16 tile is a quarter of a 16 x 16 image) and no halo exchange or reduction is needed.
 //
+// Measured at stride 2 (32 images, 4 tiles, forward / backward-data; v_mfma_f32 kernels before): 64 -> 128 channels on 32 x 128
+// tiles 0.236 -> 0.216 / 0.212 -> 0.143 ms, 128 -> 256 on 16 x 64 0.205 -> 0.187 / 0.192 -> 0.118 (163 TFLOP/s), 256 -> 512 on
+// 8 x 32 0.206 -> 0.181 / 0.187 -> 0.148; 48 channels on 3 tiles of 6 x 30 0.023 -> 0.013 / 0.019 -> 0.017.  A forward step has a
+// quarter of the stride-1 step's products and the same patch to load and split: that bounds it.  The next patch's loads go out
+// from the chunk's first step on (stride 1 has the registers for them from the fourth): 0.202 -> 0.187 and 0.126 -> 0.118.
 // Measured (32 images, 4 tiles without halo, forward / backward-data; v_mfma_f32 kernels before): 64 channels on 32 x 128
 // tiles 0.309 -> 0.196 / 0.182 ms (212 TFLOP/s), 128 on 16 x 64 0.297 -> 0.173, 256 on 8 x 32 0.292 -> 0.166 (232), 512 on
 // 4 x 16 0.39 -> 0.21.  Bound: the matrix pipe is busy 0.6 of the cycles; a step of 3072 matrix cycles takes 3700 to 4400
@@ -37,6 +42,8 @@ namespace adh {
 constexpr uint32_t kSpThreads = 512;
 constexpr uint32_t kSpChunk = 32;  // channels per staged chunk
 constexpr uint32_t kSpPP = 640;    // patch pixels per plane in LDS
+// a block's patch pixels; quads have few (and four sets of sums: what is staged for more pixels would be spilled)
+constexpr uint32_t split_patch(int sample) { return sample == kUp ? 384u : kSpPP; }
 constexpr uint32_t kSpMP = 68;     // filter rows per plane: = 4 (mod 16), so that the octet planes start 64 bytes apart
 
 struct SplitParams {
@@ -48,7 +55,7 @@ struct SplitParams {
   uint64_t part_tile_elems;
   uint32_t N, NI, C, M, num_tiles;
   uint32_t in_H, in_W, out_H, out_W;
-  uint32_t in_VH, out_VH;  // rows of the (stacked) tensors
+  uint32_t in_VH, grid_VH, grid_W;  // rows of the (stacked) input; what the blocks tile: output pixels, or quads of them
   uint32_t in_lead, out_lead, in_step, out_step, last_tile;
   uint32_t w_m_stride, w_c_stride;
   uint32_t BR, BC, NB, PPn;  // a block's pixels: BR x BC of NB images; patch pixels
@@ -79,15 +86,25 @@ struct SplitBlock {
 
 // VEC: a lane's results are four neighbouring pixels of one channel (pixels on the matrix rows), stored 16 bytes at a time:
 // block and output widths are multiples of four.  Otherwise four channels of one pixel, whose stores are runs of 16 pixels.
-template <int MT, int NT, bool VEC>
+//
+// SAMPLE.  Stride 2, padding 1 (tiles of even height and width):
+//   kDown, forward: the patch is (2 BR + 1) x (2 BC + 1), a row's even columns first, so that the 16 pixels of an operand are
+//     neighbours in LDS for every tap.  640 patch pixels leave 128 output pixels to a block (NT = 1).
+//   kUp, backward-data: a block owns quads, the 2 x 2 gradient pixels at (2i, 2j), which tap (1 +- a, 1 +- b) of the filter feeds
+//     from dy[i .. i + 1][j .. j + 1]: nine taps over a patch of (BR + 1) x (BC + 1), into four sets of sums.  A lane's four
+//     neighbouring quads are two rows of eight pixels.
+template <int MT, int NT, bool VEC, int SAMPLE>
 __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const SplitParams P) {
   constexpr uint32_t MW = 16u * MT;
+  constexpr int SETS = SAMPLE == kUp ? 4 : 1;  // of sums
+  constexpr uint32_t DOWN = SAMPLE == kDown ? 2u : 1u, UP = SAMPLE == kUp ? 2u : 1u;
   constexpr uint32_t SLOT = 3 * 4 * kSpMP;  // the operands of a tap
-  constexpr int XU = (4 * kSpPP + kSpThreads - 1) / kSpThreads;  // (pixel, octet) units a thread stages
+  constexpr int XU = (4 * split_patch(SAMPLE) + kSpThreads - 1) / kSpThreads;  // (pixel, octet) units a thread stages
   __shared__ __align__(16) uintx4 xl[3 * 4 * kSpPP];
   __shared__ __align__(16) uintx4 wl[3 * SLOT];
   __shared__ const float *tab[3 * ADH_MAX_TILES];  // the tiles' addresses: in, out, res
   __shared__ uint32_t not_finite;
+  constexpr int FIRST = SAMPLE == kUnit ? 3 : 0;  // step whose side work loads the next patch's first unit
   const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
 
@@ -146,8 +163,9 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     P.div_PPn.divmod(unit(j), o, p);
     P.div_PPI.divmod(p, b, e);
     P.div_PCP.divmod(e, r, c);
+    if constexpr (SAMPLE == kDown) c = c <= P.BC ? 2u * c : 2u * (c - P.BC) - 1u;
     const uint32_t img = B.img0 + b, c0 = ch * kSpChunk + o;
-    const int32_t R = (int32_t)(B.bi * P.BR + r) - P.pad_r, Q = (int32_t)(B.bj * P.BC + c) - P.pad_c;
+    const int32_t R = (int32_t)(B.bi * P.BR * DOWN + r) - P.pad_r, Q = (int32_t)(B.bj * P.BC * DOWN + c) - P.pad_c;
     const bool ok = o < 4u && c0 < P.C && img < P.NI && R >= 0 && R < (int32_t)P.in_VH && Q >= 0 && Q < (int32_t)P.in_W;
     uint32_t tile0, n;
     P.div_N.divmod(ok ? img : 0u, tile0, n);
@@ -248,9 +266,16 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     uint32_t b, e, r, c;
     P.div_live.divmod((wave * NT + q) * 16u + l16, b, e);
     P.div_BC.divmod(e, r, c);
-    pix[q] = (b < P.NB ? b * P.div_PPI.d + r * P.div_PCP.d + c : 0u) + g * kSpPP;
+    pix[q] = (b < P.NB ? b * P.div_PPI.d + r * DOWN * P.div_PCP.d + c : 0u) + g * kSpPP;
   }
-  floatx4 acc[MT][NT];
+  // where a tap of the window lies in the patch, and the set of sums that it feeds
+  auto tap_place = [&](uint32_t a, uint32_t b) {
+    if constexpr (SAMPLE == kDown) return a * P.div_PCP.d + (b == 1u ? P.BC + 1u : b / 2u);
+    else if constexpr (SAMPLE == kUp) return a / 2u * P.div_PCP.d + b / 2u;
+    else return (a * P.div_PCP.d + b) * P.dil;
+  };
+  auto tap_set = [](int t) { return SAMPLE == kUp ? (t / 3 == 1 ? 0 : 2) + (t % 3 == 1 ? 0 : 1) : 0; };
+  floatx4 acc[SETS][MT][NT];
   const uintx4 *const a_lane = wl + g * kSpMP + l16;
 
   // ---- results ----
@@ -265,11 +290,11 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     pl.img = B.img0 + b;
     pl.i = B.bi * P.BR + r;
     pl.j = B.bj * P.BC + c;
-    pl.ok = b < P.NB && pl.img < P.NI && pl.i < P.out_VH && pl.j < P.out_W;
+    pl.ok = b < P.NB && pl.img < P.NI && pl.i < P.grid_VH && pl.j < P.grid_W;
     P.div_N.divmod(pl.ok ? pl.img : 0u, tile0, n);
     const uint32_t R = pl.ok ? pl.i : P.out_lead, t = out_tile(R);
     pl.tile = tile0 + t;
-    pl.at = (size_t)n * P.M * out_plane + (size_t)(R - t * P.out_step) * P.out_W + (pl.ok ? pl.j : 0u);
+    pl.at = (size_t)n * P.M * out_plane + (size_t)((R - t * P.out_step) * UP) * P.out_W + (pl.ok ? pl.j * UP : 0u);
     return pl;
   };
   auto emit_all = [&](const SplitBlock &B) {
@@ -284,6 +309,38 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
       const bool sums = P.ksplit > 1u;
       ADH_GLOBAL float *p = (ADH_GLOBAL float *)(sums ? P.part + ((size_t)B.ks * P.num_tiles + pl.tile) * P.part_tile_elems
                                                       : const_cast<float *>(tab[ADH_MAX_TILES + pl.tile])) + o;
+      if constexpr (SAMPLE == kUp) {
+        const bool adds = !sums && P.beta != 0.f;
+        const ADH_GLOBAL float *r = (const ADH_GLOBAL float *)tab[2 * ADH_MAX_TILES + pl.tile] + o;
+#pragma unroll
+        for (int pr = 0; pr < 2; ++pr) {
+          const size_t row = pr ? (size_t)P.out_W : 0u;
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt) {
+            const floatx4 even = acc[2 * pr][mt][q], odd = acc[2 * pr + 1][mt][q];
+            if constexpr (VEC) {
+              if (!whole && m0 + mt * 16u >= P.M) continue;
+              const size_t at = (size_t)(mt * 16) * out_plane + row;
+              floatx4 lo = {even[0], odd[0], even[1], odd[1]}, hi = {even[2], odd[2], even[3], odd[3]};
+              if (adds) {
+                lo += load4(r + at);
+                hi += load4(r + at + 4);
+              }
+              store4(p + at, lo);
+              store4(p + at + 4, hi);
+            } else {
+#pragma unroll
+              for (int i = 0; i < 4; ++i) {
+                if (!whole && m0 + mt * 16u + i >= P.M) continue;
+                const size_t at = (size_t)(mt * 16 + i) * out_plane + row;
+                p[at] = adds ? even[i] + r[at] : even[i];
+                p[at + 1] = adds ? odd[i] + r[at + 1] : odd[i];
+              }
+            }
+          }
+        }
+        continue;
+      }
       if (!sums && P.beta != 0.f) {
         // (channels that do not exist read an existing one)
         const ADH_GLOBAL float *r = (const ADH_GLOBAL float *)tab[2 * ADH_MAX_TILES + pl.tile] + (pl.at + (size_t)min(m0, P.M - 1u) * out_plane);
@@ -298,24 +355,24 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
           }
         }
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[mt][q] += old[mt];
+        for (int mt = 0; mt < MT; ++mt) acc[0][mt][q] += old[mt];
       }
 #pragma unroll
       for (int mt = 0; mt < MT; ++mt) {
         if constexpr (VEC) {
-          if (whole || m0 + mt * 16u < P.M) store4(p + (size_t)(mt * 16) * out_plane, acc[mt][q]);
+          if (whole || m0 + mt * 16u < P.M) store4(p + (size_t)(mt * 16) * out_plane, acc[0][mt][q]);
         } else {
 #pragma unroll
           for (int i = 0; i < 4; ++i)
-            if (whole || m0 + mt * 16u + i < P.M) p[(size_t)(mt * 16 + i) * out_plane] = acc[mt][q][i];
+            if (whole || m0 + mt * 16u + i < P.M) p[(size_t)(mt * 16 + i) * out_plane] = acc[0][mt][q][i];
         }
       }
     }
   };
   // something staged has parts that are not finite: the wave's outputs as plain fp32 sums, straight from memory
   auto emit_plain = [&](const SplitBlock &B) {
-    for (uint32_t at = lane; at < 16u * NT * MW; at += 64u) {
-      const uint32_t m = B.mg * MW + at / (16u * NT);
+    for (uint32_t of = lane; of < 16u * NT * MW * SETS; of += 64u) {
+      const uint32_t at = of / SETS, set = of % SETS, m = B.mg * MW + at / (16u * NT);
       const Place pl = place_of(B, wave * (16u * NT) + at % (16u * NT));
       if (!pl.ok || m >= P.M) continue;
       uint32_t tile0, n;
@@ -323,7 +380,9 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
       float v = 0.f;
       for (uint32_t c = B.ch_lo * kSpChunk; c < min(B.ch_hi * kSpChunk, P.C); ++c)
         for (uint32_t t = 0; t < 9u; ++t) {
-          const int32_t R = (int32_t)(pl.i + t / 3u * P.dil) - P.pad_r, Q = (int32_t)(pl.j + t % 3u * P.dil) - P.pad_c;
+          if (SAMPLE == kUp && (uint32_t)tap_set((int)t) != set) continue;
+          const uint32_t a = SAMPLE == kUp ? t / 6u : t / 3u, b = SAMPLE == kUp ? t % 3u / 2u : t % 3u;
+          const int32_t R = (int32_t)(pl.i * DOWN + a * P.dil) - P.pad_r, Q = (int32_t)(pl.j * DOWN + b * P.dil) - P.pad_c;
           float x = 0.f;  // the padding is data: an infinite filter element times it is NaN
           if (R >= 0 && R < (int32_t)P.in_VH && Q >= 0 && Q < (int32_t)P.in_W) {
             const uint32_t ti = in_tile((uint32_t)R);
@@ -331,7 +390,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
           }
           v = __builtin_fmaf(P.w[(size_t)m * P.w_m_stride + (size_t)c * P.w_c_stride + (P.flip ? 8u - t : t)], x, v);
         }
-      const size_t o = pl.at + (size_t)m * out_plane;
+      const size_t o = pl.at + (size_t)m * out_plane + (set >> 1 ? (size_t)P.out_W : 0u) + (set & 1u);
       if (P.ksplit > 1u) {
         P.part[((size_t)B.ks * P.num_tiles + pl.tile) * P.part_tile_elems + o] = v;
       } else {
@@ -373,9 +432,11 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     }
     if (ch == B.ch_lo) {
 #pragma unroll
-      for (int mt = 0; mt < MT; ++mt)
+      for (int s = 0; s < SETS; ++s)
 #pragma unroll
-        for (int q = 0; q < NT; ++q) acc[mt][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+          for (int q = 0; q < NT; ++q) acc[s][mt][q] = floatx4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) a[0][k] = a_lane[k * 4 * kSpMP];
@@ -387,7 +448,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
       constexpr int t = decltype(step)::value;
       // two steps ahead of the multiplications: tap t2 of this chunk or of the next goes to the slot nobody reads
       constexpr int t2 = (t + 2) % 9, col = t2 % 3, row = t2 / 3;
-      uint32_t delta = ((uint32_t)((t + 1) / 3) * P.div_PCP.d + (uint32_t)((t + 1) % 3)) * P.dil;  // of the next tap
+      uint32_t delta = tap_place((t + 1) / 3, (t + 1) % 3);  // of the next tap
       asm volatile("" : "+s"(delta));  // (the nine taps' addresses are not kept in registers)
       const uintx4 *xb = xl + delta;
       // what follows group i of the step's 6 MT groups of NT multiplications
@@ -401,10 +462,10 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
           if constexpr (col == 2 && row < 2) load_wrow(B.mg, ch, row + 1);
           if constexpr (col == 2 && row == 2) load_wrow(nB.mg, nch, 0);
         }
-        if constexpr (t >= 3 && t < 3 + XU) {
-          if constexpr (i == 1) set_unit(nB, nch, t - 3);
+        if constexpr (t >= FIRST && t < FIRST + XU) {
+          if constexpr (i == 1) set_unit(nB, nch, t - FIRST);
           if constexpr (i % MT == 0 && i / MT >= 1 && i / MT <= 4) {
-            if (!idle(t - 3)) load_elems(t - 3, 2 * (i / MT) - 2, 2 * (i / MT));
+            if (!idle(t - FIRST)) load_elems(t - FIRST, 2 * (i / MT) - 2, 2 * (i / MT));
           }
         }
       };
@@ -417,10 +478,11 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
             a[cur ^ 1][k] = mt + 1 < MT ? a_lane[(t % 3) * SLOT + k * 4 * kSpMP + (mt + 1) * 16]
                                         : a_lane[((t + 1) % 3) * SLOT + k * 4 * kSpMP];
         }
+        auto &sum = acc[tap_set(t)];
         auto products = [&](auto nth, int ka, int kb) {
 #pragma unroll
           for (int q = 0; q < NT; ++q)
-            acc[mt][q] = VEC ? mfma_bf16(b[q][kb], a[cur][ka], acc[mt][q]) : mfma_bf16(a[cur][ka], b[q][kb], acc[mt][q]);
+            sum[mt][q] = VEC ? mfma_bf16(b[q][kb], a[cur][ka], sum[mt][q]) : mfma_bf16(a[cur][ka], b[q][kb], sum[mt][q]);
           __builtin_amdgcn_sched_barrier(0);
           side(std::integral_constant<int, mt * 6 + decltype(nth)::value>{});
           __builtin_amdgcn_sched_barrier(0);
@@ -483,44 +545,49 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
   P.NI = q.stacked ? q.N : q.N * q.num_tiles;
   P.in_H = q.in_H; P.in_W = q.in_W; P.out_H = q.out_H; P.out_W = q.out_W;
-  P.in_VH = q.in_H; P.out_VH = q.out_H;
+  P.in_VH = q.in_H; P.grid_VH = q.out_H; P.grid_W = q.sample == kUp ? q.in_W : q.out_W;
   P.in_step = q.in_H; P.out_step = q.out_H;
   if (q.stacked) {
-    if ((uint64_t)q.step * q.num_tiles + 2u >= (1ull << 31)) return ADH_EUNIMPL;
+    if ((uint64_t)q.step * q.num_tiles * (q.sample == kUnit ? 1u : 2u) + 2u >= (1ull << 31)) return ADH_EUNIMPL;
     P.in_lead = q.in_lead; P.out_lead = q.out_lead;
     P.in_step = P.out_step = q.step;
-    P.in_VH = q.step * q.num_tiles + 2u * q.in_lead;
-    P.out_VH = q.step * q.num_tiles + 2u * q.out_lead;
+    if (q.sample == kDown) P.in_step = 2u * q.step;
+    P.in_VH = P.in_step * q.num_tiles + 2u * q.in_lead;
+    P.grid_VH = q.step * q.num_tiles + 2u * q.out_lead;
     P.last_tile = q.num_tiles - 1u;
   }
   P.w_m_stride = q.w_m_stride; P.w_c_stride = q.w_c_stride;
   P.pad_r = q.pad_r; P.pad_c = q.pad_c; P.dil = q.dil; P.flip = q.flip ? 1 : 0;
   P.beta = q.beta;
   P.nchunks = (P.C + kSpChunk - 1u) / kSpChunk;
-  const uint32_t span = 2u * q.dil;
+  const uint32_t pixels = split_patch(q.sample);
+  // extent of the patch of n pixels, and how many pixels one of n holds
+  auto patch = [&](uint32_t n) { return q.sample == kDown ? 2u * n + 1u : q.sample == kUp ? n + 1u : n + 2u * q.dil; };
+  auto held = [&](uint32_t n) { return n < patch(1u) ? 0u : q.sample == kDown ? (n - 1u) / 2u : n - (patch(1u) - 1u); };
   double best = 1e300;
   uint32_t nbi = 0, nbj = 0;
   for (int MT = P.M <= 16u ? 1 : P.M <= 32u ? 2 : 4; MT >= 1; MT /= 2) {
     const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
-    for (int NT = 4; NT >= 1; NT /= 2) {
+    for (int NT = q.sample == kDown ? 1 : 4; NT >= 1; NT /= 2) {
+      if (q.sample == kUp && NT == 4 && MT > 1) continue;  // (four sets of sums)
       const uint32_t slots = 128u * NT;
       const double matrix = 192.0 * MT * NT;
-      const double block = P.nchunks * (9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT) + 2000.0 + 500.0 * MT * NT;
+      const double block = P.nchunks * (9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT) + 2000.0 +
+                           500.0 * MT * NT * (q.sample == kUp ? 4 : 1);
       if (block >= best) continue;
       // columns per block: whole rows, halves and so on down to eight, multiples of four where rows are
-      for (uint32_t parts = (P.out_W + 255u) / 256u; parts <= P.out_W; parts += 1u + parts / 8u) {
-        uint32_t BC = (P.out_W + parts - 1u) / parts;
+      for (uint32_t parts = (P.grid_W + 255u) / 256u; parts <= P.grid_W; parts += 1u + parts / 8u) {
+        uint32_t BC = (P.grid_W + parts - 1u) / parts;
         if (parts > 1u && BC < 8u) break;
-        if (P.out_W % 4u == 0u) BC = (BC + 3u) & ~3u;
-        const uint32_t nc = (P.out_W + BC - 1u) / BC;
-        if (BC > slots || BC + span > kSpPP) continue;
-        const uint32_t rows = kSpPP / (BC + span);
-        if (rows <= span) continue;
-        const uint32_t max_BR = std::min(std::min(P.out_VH, slots / BC), rows - span);
-        const uint32_t nr0 = (P.out_VH + max_BR - 1u) / max_BR;
-        for (uint32_t nr = nr0; nr < nr0 + 2u && nr <= P.out_VH; ++nr) {
-          const uint32_t BR = (P.out_VH + nr - 1u) / nr;
-          uint32_t NB = std::min(std::min(slots / (BR * BC), kSpPP / ((BR + span) * (BC + span))), P.NI);
+        if (P.grid_W % 4u == 0u) BC = (BC + 3u) & ~3u;
+        const uint32_t nc = (P.grid_W + BC - 1u) / BC;
+        if (BC > slots) continue;
+        const uint32_t max_BR = std::min(std::min(P.grid_VH, slots / BC), held(pixels / patch(BC)));
+        if (max_BR == 0u) continue;
+        const uint32_t nr0 = (P.grid_VH + max_BR - 1u) / max_BR;
+        for (uint32_t nr = nr0; nr < nr0 + 2u && nr <= P.grid_VH; ++nr) {
+          const uint32_t BR = (P.grid_VH + nr - 1u) / nr;
+          uint32_t NB = std::min(std::min(slots / (BR * BC), pixels / (patch(BR) * patch(BC))), P.NI);
           const uint32_t groups = (P.NI + NB - 1u) / NB;
           NB = (P.NI + groups - 1u) / groups;
           const uint64_t blocks = (uint64_t)groups * nc * nr * MG;
@@ -536,9 +603,9 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
     }
   }
   if (nbi == 0u) return ADH_EUNIMPL;
-  const uint32_t MG = (P.M + 16u * plan->MT - 1u) / (16u * plan->MT), PCP = P.BC + span, PPI = (P.BR + span) * PCP;
+  const uint32_t MG = (P.M + 16u * plan->MT - 1u) / (16u * plan->MT), PCP = patch(P.BC), PPI = patch(P.BR) * PCP;
   P.PPn = P.NB * PPI;
-  plan->vec = P.BC % 4u == 0u && P.out_W % 4u == 0u;
+  plan->vec = P.BC % 4u == 0u && P.grid_W % 4u == 0u;
   const uint64_t base = (uint64_t)((P.NI + P.NB - 1u) / P.NB) * nbi * nbj * MG;
   // Fewer blocks than half the compute units and chunks to spare: deal them to several workgroups per block (at least two
   // each) and add their sums in a second kernel (512 channels on 2 x 8 tiles, batch 32).
@@ -565,20 +632,30 @@ size_t conv3x3_split_workspace(const Conv3x3Problem &q) {
 void conv3x3_split_name(const Conv3x3Problem &q, char *name, size_t name_bytes) {
   SplitPlan plan = {};
   if (split_plan(q, false, &plan)) plan.MT = plan.NT = 0;
-  snprintf(name, name_bytes, "conv3x3_split_kernel<%d, %d, %s>", plan.MT, plan.NT, plan.vec ? "true" : "false");
+  snprintf(name, name_bytes, "conv3x3_split_kernel<%d, %d, %s, %d>", plan.MT, plan.NT, plan.vec ? "true" : "false", (int)q.sample);
 }
 
-template <int MT, int NT>
+template <int MT, int NT, int SAMPLE>
 static void launch_split(const SplitPlan &plan, hipStream_t st) {
   const dim3 grid(std::min(plan.P.xcd_chunk, 32u) * 8u), block(kSpThreads);
-  if (plan.vec) hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, true>), grid, block, 0, st, plan.P);
-  else hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, false>), grid, block, 0, st, plan.P);
+  if (plan.vec) hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, true, SAMPLE>), grid, block, 0, st, plan.P);
+  else hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, false, SAMPLE>), grid, block, 0, st, plan.P);
 }
 template <int MT>
-static void launch_split_nt(const SplitPlan &plan, hipStream_t st) {
-  if (plan.NT == 4) launch_split<MT, 4>(plan, st);
-  else if (plan.NT == 2) launch_split<MT, 2>(plan, st);
-  else launch_split<MT, 1>(plan, st);
+static void launch_split_nt(const SplitPlan &plan, SplitSample sample, hipStream_t st) {
+  if (sample == kDown) {
+    launch_split<MT, 1, kDown>(plan, st);
+  } else if (sample == kUp) {
+    if (MT == 1 && plan.NT == 4) launch_split<1, 4, kUp>(plan, st);
+    else if (plan.NT == 2) launch_split<MT, 2, kUp>(plan, st);
+    else launch_split<MT, 1, kUp>(plan, st);
+  } else if (plan.NT == 4) {
+    launch_split<MT, 4, kUnit>(plan, st);
+  } else if (plan.NT == 2) {
+    launch_split<MT, 2, kUnit>(plan, st);
+  } else {
+    launch_split<MT, 1, kUnit>(plan, st);
+  }
 }
 
 int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st) {
@@ -597,9 +674,9 @@ int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_byt
   }
   P.w = reinterpret_cast<const float *>(q.w);
   P.part = reinterpret_cast<float *>(workspace);
-  if (plan.MT == 4) launch_split_nt<4>(plan, st);
-  else if (plan.MT == 2) launch_split_nt<2>(plan, st);
-  else launch_split_nt<1>(plan, st);
+  if (plan.MT == 4) launch_split_nt<4>(plan, q.sample, st);
+  else if (plan.MT == 2) launch_split_nt<2>(plan, q.sample, st);
+  else launch_split_nt<1>(plan, q.sample, st);
   if (P.ksplit > 1u) {
     const uint32_t rb = (uint32_t)std::min<uint64_t>((P.part_tile_elems + 255u) / 256u, 2048u);
     hipLaunchKernelGGL(conv3x3_split_reduce_kernel, dim3(rb, q.num_tiles), dim3(256), 0, st, P);
