@@ -120,10 +120,10 @@ static size_t region(uint64_t elems) { return (size_t)((elems * 4u + 255u) / 256
 
 bool conv_bf16_mfma_supported(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
 size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
-                                      uint32_t W);
+                                      uint32_t W, bool may_copy);
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree = false, bool filter_only = false);
+                   hipStream_t st, bool halofree, bool may_copy);
 
 bool conv_bf16_wgrad_mfma_supported(uint32_t Cin, uint32_t Cout, uint32_t W);
 size_t conv_bf16_wgrad_mfma_workspace_bytes(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t W);
@@ -171,7 +171,7 @@ size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t 
            conv_bf16_wgrad_mfma_workspace_bytes(num_tiles, N, Cin, Cout, Wd);
   }
   if (which != ADH_CONV_BWD_FILTER && conv_bf16_mfma_supported(which, Cin, Cout, H, W))
-    return conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W);
+    return conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, true);
   const uint64_t slab = (uint64_t)N * Cin * (H + 2) * (W + 2), out = (uint64_t)N * Cout * H * W;
   const uint64_t filt = (uint64_t)Cin * Cout * 9u;
   size_t total = 0;
@@ -209,7 +209,10 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
   if (N == 0 || Cin == 0 || Cout == 0 || H == 0 || W == 0) return ADH_OK;
   if (!in_tiles || !out_tiles || !w) return ADH_ENULL;
   if (!aligned_to(w, 2)) return ADH_EALIGN;
-  const size_t need = bf16_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
+  // a workspace without room for the copy of the input at odd widths does for the kernels that need none
+  const bool mfma = conv_bf16_mfma_supported(which, Cin, Cout, H, W);
+  const size_t full = bf16_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
+  const size_t need = mfma ? conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false) : full;
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
@@ -217,12 +220,13 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
     if (!in_tiles[t] || !out_tiles[t]) return ADH_ENULL;
     if (!aligned_to(in_tiles[t], 2) || !aligned_to(out_tiles[t], 2)) return ADH_EALIGN;
   }
-  if (conv_bf16_mfma_supported(which, Cin, Cout, H, W)) {
+  if (mfma) {
     // one image is addressed through a 32-bit buffer resource
     const uint64_t cmax = Cin > Cout ? Cin : Cout;
     if (cmax * (H + 2ull) * (W + 2ull) * 2u >= (1ull << 31) || (uint64_t)Cin * Cout * 18u >= (1ull << 31))
       return ADH_EINVAL;
-    return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st);
+    return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, false,
+                          workspace_bytes >= full);
   }
   const uint64_t slab = (uint64_t)N * Cin * (H + 2) * (W + 2), outn = (uint64_t)N * Cout * H * W;
   const uint64_t in_elems = which == ADH_CONV_FWD ? slab : outn;

@@ -27,6 +27,8 @@
 // (out-of-range dwords read as zero); out-of-range columns by per-dword masks.
 #include "conv3x3_bf16_mfma.h"
 
+#include <algorithm>
+
 namespace adh {
 
 constexpr int kRingRows = 10;                         // 6 rows in use + 4 rows being written
@@ -591,9 +593,9 @@ static uint32_t conv_bf16_passes(int which, uint32_t Cin, uint32_t Cout) {
 // launch of the eight-wave kernel per 64.
 static bool conv_bf16_uses_k128(int which, uint32_t Cin, uint32_t Cout) { return Cin > 64u && Cout > 64u; }
 // (a width the eight-wave kernels do not take: one launch of the four-wave kernel per 64)
-static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
+static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, bool may_copy = true) {
   const uint32_t cred = which == ADH_CONV_FWD ? Cin : Cout;
-  if (!conv_bf16_uses_k128(which, Cin, Cout) || !(conv_bf16_w8_width(which, W) || conv_bf16_repitches(which, Cin, Cout, H, W)))
+  if (!conv_bf16_uses_k128(which, Cin, Cout) || !(conv_bf16_w8_width(which, W) || (may_copy && conv_bf16_repitches(which, Cin, Cout, H, W))))
     return (cred + 63u) / 64u;
   uint32_t n = 0, rem = cred;
   while (rem > 64u) {
@@ -653,12 +655,16 @@ static size_t part_region_bytes(int which, uint32_t N, uint32_t Cin, uint32_t Co
   const uint64_t oh = which == ADH_CONV_FWD ? H : H + 2ull, ow = which == ADH_CONV_FWD ? W : W + 2ull;
   return (size_t)((N * cout_k * oh * ow * 4u + 255u) / 256u * 256u);
 }
+// may_copy: with room for the copy of the input with wider rows where there is a route over one
 size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
-                                      uint32_t W) {
-  size_t bytes = filter_region_bytes(which, Cin, Cout);
-  if (conv_bf16_launches(which, Cin, Cout, H, W) > 1u) bytes += (size_t)num_tiles * part_region_bytes(which, N, Cin, Cout, H, W);
-  if (conv_bf16_repitches(which, Cin, Cout, H, W)) bytes += num_tiles * conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W);
-  return bytes;
+                                      uint32_t W, bool may_copy) {
+  auto sums = [&](bool copies) {
+    return conv_bf16_launches(which, Cin, Cout, H, W, copies) > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : (size_t)0;
+  };
+  size_t bytes = sums(false);
+  if (may_copy && conv_bf16_repitches(which, Cin, Cout, H, W))
+    bytes = std::max(bytes, sums(true) + num_tiles * conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W));
+  return filter_region_bytes(which, Cin, Cout) + bytes;
 }
 
 // which = ADH_CONV_FWD: in = x_pad tiles, out = y tiles; ADH_CONV_BWD_DATA: in = dy tiles,
@@ -667,10 +673,10 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
 // and a tile's rows -1 and H are its neighbours' last and first rows (zeros at the tensor's own border): the
 // unsplit convolution with zero padding, restricted to the tile.  Only shapes the eight-wave kernel takes
 // (ADH_EUNIMPL otherwise).
-// filter_only: the workspace holds the reordered filter and no more (no copy of the input with wider rows).
+// may_copy: the workspace has room for a copy of the input with wider rows.
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree, bool filter_only) {
+                   hipStream_t st, bool halofree, bool may_copy) {
   ConvBf16Params P = {};
   for (uint32_t t = 0; t < num_tiles; ++t) {
     P.in[t] = reinterpret_cast<const uint16_t *>(in_tiles[t]);
@@ -700,13 +706,13 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
   P.chan0 = 0;
   P.cred_pass = P.Cred < 64u ? P.Cred : 64u;
   P.first_pass = P.last_pass = 1;
-  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, H, W);
+  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, H, W, may_copy);
   if (launches > 1u) {
     uint8_t *part = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout);
     const size_t per_tile = part_region_bytes(which, N, Cin, Cout, H, W);
     for (uint32_t t = 0; t < num_tiles; ++t) P.part[t] = reinterpret_cast<float *>(part + t * per_tile);
   }
-  if (!halofree && !filter_only && conv_bf16_repitches(which, Cin, Cout, H, W)) {
+  if (!halofree && may_copy && conv_bf16_repitches(which, Cin, Cout, H, W)) {
     uint8_t *copy = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout) +
                     (launches > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : 0u);
     const size_t per_tile = conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W);
@@ -893,7 +899,7 @@ extern "C" int adh_conv3x3_slab_fwd_tiles_static(int dtype, uint32_t num_tiles, 
   const int e = static_scratch(&ws);
   if (e) return e;
   return conv_bf16_mfma(ADH_CONV_FWD, num_tiles, N, Cin, Cout, H, W, x_pad_tiles, w, y_tiles, beta, ws, as_stream(stream),
-                        false, true);
+                        false, false);
 }
 
 // ---------------------------------------------------------------------------
@@ -919,7 +925,7 @@ int conv_bf16_unpadded(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   if (cmax * (H + 2ull) * (W + 2ull) * 2u >= (1ull << 31) || (uint64_t)Cin * Cout * 18u >= (1ull << 31)) return ADH_EINVAL;
   if (!conv_bf16_mfma_supported(which, Cin, Cout, H, W)) return ADH_EUNIMPL;
   // the same workspace as the padded entry point of this pass (the transformed filter; the sums between passes)
-  const size_t need = conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W);
+  const size_t need = conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false);
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;

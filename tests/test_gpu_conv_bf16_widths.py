@@ -1,6 +1,10 @@
 """bf16 3x3 convolution with more than 64 reduction channels at widths that are no multiple of eight: the passes over a
 copy of the input with wider rows (rows shorter than a granule, one column off one, last strips of one column)."""
+import numpy as np
 import pytest
+import torch
+
+from arraydiff_cuda_amd import capi
 
 from test_gpu_conv_bf16 import test_bf16_conv_small_vs_oracle as check_passes_vs_oracle
 
@@ -11,3 +15,28 @@ pytestmark = pytest.mark.gpu
                                               (1, 3, 128, 128, 6, 23), (1, 1, 80, 16, 9, 97), (2, 1, 16, 80, 2, 12)])
 def test_odd_widths_vs_oracle(oracle, K, N, Cin, Cout, H, W):
     check_passes_vs_oracle(oracle, K, N, Cin, Cout, H, W)
+
+
+@pytest.mark.parametrize("which,K,N,Cin,Cout,H,W", [("fwd", 2, 2, 320, 72, 3, 7), ("bwd", 1, 3, 66, 260, 5, 9)])
+def test_a_workspace_without_room_for_the_copy(oracle, which, K, N, Cin, Cout, H, W):
+    """The reordered filter and the fp32 sums alone: the kernels that run without the copy give the same result."""
+    rng = np.random.default_rng(3)
+    bf = lambda shape: torch.from_numpy(rng.standard_normal(shape).astype(np.float32)).to(torch.bfloat16).cuda()
+    w, fwd = bf((Cout, Cin, 3, 3)), which == "fwd"
+    ins = [bf((N, Cin, H + 2, W + 2) if fwd else (N, Cout, H, W)) for _ in range(K)]
+    cred, cout = (Cin, Cout) if fwd else (Cout, Cin)
+    shape = (N, cout, H, W) if fwd else (N, cout, H + 2, W + 2)
+    small = (cout + 63) // 64 * ((cred + 63) // 64) * 9 * 2 * 64 * 32 * 2 + K * ((4 * int(np.prod(shape)) + 255) // 256 * 256)
+    full = capi.conv_workspace_bytes(capi.ADH_CONV_FWD if fwd else capi.ADH_CONV_BWD_DATA, capi.ADH_BF16, K, N, Cin, Cout, H, W)
+    assert full > small
+    got = []
+    for nbytes in (small, full):
+        outs = [torch.empty(shape, device="cuda", dtype=torch.bfloat16) for _ in range(K)]
+        ws = torch.empty(nbytes // 4, device="cuda")
+        if fwd:
+            capi.check(capi.conv_fwd_tiles(ins, w, outs, N, Cin, Cout, H, W, ws=ws), "fwd")
+        else:
+            capi.check(capi.conv_bwd_data_tiles(w, ins, outs, N, Cin, Cout, H, W, ws=ws), "bwd-data")
+        got.append(torch.cat(outs).float())
+    # both round one fp32 sum of the same products to bf16
+    assert (got[0] - got[1]).abs().max().item() <= 2 ** -7 * got[1].abs().max().item()
