@@ -20,7 +20,7 @@
 //
 // Measured at stride 2 (32 images, 4 tiles, forward / backward-data; v_mfma_f32 kernels before): 64 -> 128 channels on 32 x 128
 // tiles 0.236 -> 0.216 / 0.212 -> 0.143 ms, 128 -> 256 on 16 x 64 0.205 -> 0.187 / 0.192 -> 0.118 (163 TFLOP/s), 256 -> 512 on
-// 8 x 32 0.206 -> 0.181 / 0.187 -> 0.148; 48 channels on 3 tiles of 6 x 30 0.023 -> 0.013 / 0.019 -> 0.017.  A forward step has a
+// 8 x 32 0.206 -> 0.181 / 0.187 -> 0.131; 48 channels on 3 tiles of 6 x 30 0.023 -> 0.013 / 0.019 -> 0.014.  A forward step has a
 // quarter of the stride-1 step's products and the same patch to load and split: that bounds it.  The next patch's loads go out
 // from the chunk's first step on (stride 1 has the registers for them from the fourth): 0.202 -> 0.187 and 0.126 -> 0.118.
 // Measured (32 images, 4 tiles without halo, forward / backward-data; v_mfma_f32 kernels before): 64 channels on 32 x 128
@@ -539,7 +539,10 @@ struct SplitPlan {
 // Blocks of BR x BC output pixels (of NB images) by 16 MT channels.  The workgroups are persistent, one per compute unit, so
 // a launch takes ceil(blocks / 256) times a block.  A block's cycles, as measured in the kernel: nine steps a chunk, each a
 // SIMD's 2 * 6 * 16 * MT * NT matrix cycles (at least 1300: its barrier, staging and operand reads) and 300 more; 1500 and
-// 2000 NT a chunk for loading, splitting and changing the patch; the results.
+// 2000 NT a chunk for loading, splitting and changing the patch; the results.  Where that leaves compute units idle and there
+// is a workspace, a block's chunks are dealt to several workgroups and a second kernel adds their sums, at its launch and the
+// sums' way through memory (1.2 KB a cycle): 512 channels on 4 tiles of 2 x 8, 32 images, 130 -> 74 us; on one image of 14 x 14
+// a tile 124 -> 40; 256 -> 512 on 28 x 28, 8 images, backward-data 147 -> 95.
 static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) {
   SplitParams &P = plan->P;
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
@@ -560,6 +563,7 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
   P.pad_r = q.pad_r; P.pad_c = q.pad_c; P.dil = q.dil; P.flip = q.flip ? 1 : 0;
   P.beta = q.beta;
   P.nchunks = (P.C + kSpChunk - 1u) / kSpChunk;
+  const double out_bytes = 4.0 * P.num_tiles * P.N * P.M * P.out_H * P.out_W;
   const uint32_t pixels = split_patch(q.sample);
   // extent of the patch of n pixels, and how many pixels one of n holds
   auto patch = [&](uint32_t n) { return q.sample == kDown ? 2u * n + 1u : q.sample == kUp ? n + 1u : n + 2u * q.dil; };
@@ -572,9 +576,8 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
       if (q.sample == kUp && NT == 4 && MT > 1) continue;  // (four sets of sums)
       const uint32_t slots = 128u * NT;
       const double matrix = 192.0 * MT * NT;
-      const double block = P.nchunks * (9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT) + 2000.0 +
-                           500.0 * MT * NT * (q.sample == kUp ? 4 : 1);
-      if (block >= best) continue;
+      const double chunk = 9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT;
+      const double results = 2000.0 + 500.0 * MT * NT * (q.sample == kUp ? 4 : 1);
       // columns per block: whole rows, halves and so on down to eight, multiples of four where rows are
       for (uint32_t parts = (P.grid_W + 255u) / 256u; parts <= P.grid_W; parts += 1u + parts / 8u) {
         uint32_t BC = (P.grid_W + parts - 1u) / parts;
@@ -591,12 +594,20 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
           const uint32_t groups = (P.NI + NB - 1u) / NB;
           NB = (P.NI + groups - 1u) / groups;
           const uint64_t blocks = (uint64_t)groups * nc * nr * MG;
-          const double cost = (double)((blocks + 255u) / 256u) * block + 1e-3 * (double)blocks;
-          if (cost < best) {
-            best = cost;
-            plan->MT = MT; plan->NT = NT;
-            P.BR = BR; P.BC = BC; P.NB = NB;
-            nbi = nr; nbj = nc;
+          // chunks dealt to several workgroups per block, while all of them run at once
+          const uint64_t most = workspace ? 256u / blocks : 1u;
+          for (uint32_t cps = P.nchunks; cps >= 1u; --cps) {
+            const uint32_t ks = (P.nchunks + cps - 1u) / cps;
+            if (ks > 1u && ks > most) break;
+            const double sums = ks > 1u ? 9000.0 + out_bytes * (ks + 1) / 1200.0 : 0.0;
+            const double cost = (double)((blocks * ks + 255u) / 256u) * (cps * chunk + results) + sums + 1e-3 * (double)blocks;
+            if (cost < best) {
+              best = cost;
+              plan->MT = MT; plan->NT = NT;
+              P.BR = BR; P.BC = BC; P.NB = NB;
+              P.ksplit = ks; P.chunks_per_split = cps;
+              nbi = nr; nbj = nc;
+            }
           }
         }
       }
@@ -607,12 +618,6 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
   P.PPn = P.NB * PPI;
   plan->vec = P.BC % 4u == 0u && P.grid_W % 4u == 0u;
   const uint64_t base = (uint64_t)((P.NI + P.NB - 1u) / P.NB) * nbi * nbj * MG;
-  // Fewer blocks than half the compute units and chunks to spare: deal them to several workgroups per block (at least two
-  // each) and add their sums in a second kernel (512 channels on 2 x 8 tiles, batch 32).
-  P.ksplit = 1;
-  if (workspace && base <= 128u && P.nchunks >= 4u) P.ksplit = (uint32_t)std::min<uint64_t>(P.nchunks / 2u, 256u / base);
-  P.chunks_per_split = (P.nchunks + P.ksplit - 1u) / P.ksplit;
-  P.ksplit = (P.nchunks + P.chunks_per_split - 1u) / P.chunks_per_split;
   if (base * P.ksplit >= (1ull << 30)) return ADH_EUNIMPL;
   P.blocks = (uint32_t)(base * P.ksplit);
   P.xcd_chunk = (P.blocks + 7u) / 8u;
