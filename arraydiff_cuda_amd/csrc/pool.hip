@@ -608,6 +608,182 @@ static void launch_bwd_band(int dtype, bool max, const PoolParams &P, uint32_t b
   launch_bwd_band_u<false>(dtype, max, P, blocks, lds, st);
 }
 
+// Backward of 3x3 max pooling at stride 2, padding 1, over tiles of even height without halo and rows of whole groups of four.
+// A thread owns four columns (the two windows that start there and the next one's first column) and marches down a band of
+// window rows of the stacked tensor: a step loads two input rows, finds where the three windows of this row have their first
+// maximum (a row's own is shared by the window rows above and below it) and stores the two input rows that no later window
+// touches.  No LDS, no barrier; the next step's loads are in flight during this one's work.  Bound by memory.
+// Measured, 32 x 64 planes, 4 tiles of 64 x 256, fp32: 389 us through LDS bands (3.4 TB/s of what has to be moved), 246 here (5.5).
+struct PoolS2Params {
+  const void *x[ADH_MAX_TILES], *dy[ADH_MAX_TILES];
+  void *dx[ADH_MAX_TILES];
+  uint32_t items;  // planes x groups of columns
+  uint32_t K, H, W, OH, OW, steps;  // steps: window rows per band
+  float beta;
+  FastDiv div_groups, div_H, div_OH;
+};
+template <typename T, int V>
+__device__ __forceinline__ void load_f(const T *p, float (&f)[V]) {
+  struct alignas(V * sizeof(T)) Pack { T e[V]; };
+  const Pack v = *reinterpret_cast<const Pack *>(p);
+#pragma unroll
+  for (int i = 0; i < V; ++i) f[i] = ld_f(v.e, i);
+}
+template <typename T>
+__global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const PoolS2Params P) {
+  const uint32_t id = blockIdx.x * kPoolThreads + threadIdx.x;
+  if (id >= P.items) return;
+  uint32_t plane, c;
+  P.div_groups.divmod(id, plane, c);
+  c *= 4u;
+  const uint32_t VH = P.K * P.H, VO = P.K * P.OH;
+  // what a place beyond the row's ends or the tensor's holds is zero; it is loaded from an existing one
+  struct Row { float l[1], v[4], r[2]; };
+  const uint32_t cl = c ? c - 1u : 0u, cr = c + 4u < P.W ? c + 4u : c;
+  auto load_row = [&](uint32_t R) {
+    Row q;
+    uint32_t t, r;
+    const bool ok = R < VH;
+    P.div_H.divmod(ok ? R : 0u, t, r);
+    const T *p = reinterpret_cast<const T *>(P.x[t]) + ((size_t)plane * P.H + r) * P.W;
+    load_f<T, 4>(p + c, q.v);
+    load_f<T, 1>(p + cl, q.l);
+    load_f<T, 2>(p + cr, q.r);
+    if (!ok || c == 0u) q.l[0] = 0.f;
+    if (!ok || c + 4u >= P.W) q.r[0] = q.r[1] = 0.f;
+    if (!ok) q.v[0] = q.v[1] = q.v[2] = q.v[3] = 0.f;
+    return q;
+  };
+  struct Grad { float v[2], n[1]; };  // of the three windows
+  const uint32_t ow = c / 2u, on = ow + 2u < P.OW ? ow + 2u : ow;
+  auto load_dy = [&](uint32_t o) {
+    Grad q;
+    uint32_t t, r;
+    const bool ok = o < VO;
+    P.div_OH.divmod(ok ? o : 0u, t, r);
+    const T *p = reinterpret_cast<const T *>(P.dy[t]) + ((size_t)plane * P.OH + r) * P.OW;
+    load_f<T, 2>(p + ow, q.v);
+    load_f<T, 1>(p + on, q.n);
+    if (!ok || on == ow) q.n[0] = 0.f;
+    if (!ok) q.v[0] = q.v[1] = 0.f;
+    return q;
+  };
+  // first maximum of a row's three window columns, per window (nothing exceeds -inf: the first place, as for NaN)
+  struct Best { float b[3]; uint32_t at[3]; };
+  auto best_of = [](const Row &q) {
+    const float e[7] = {q.l[0], q.v[0], q.v[1], q.v[2], q.v[3], q.r[0], q.r[1]};
+    Best m;
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      m.b[w] = -__builtin_inff();
+      m.at[w] = 0u;
+#pragma unroll
+      for (int k = 0; k < 3; ++k)
+        if (e[2 * w + k] > m.b[w]) { m.b[w] = e[2 * w + k]; m.at[w] = (uint32_t)k; }
+    }
+    return m;
+  };
+  struct Windows { uint32_t at[3]; float g[3]; };  // where in 3 x 3, and the gradient
+  auto windows_of = [](const Best &top, const Best &mid, const Best &bot, const Grad &g) {
+    Windows q;
+#pragma unroll
+    for (int w = 0; w < 3; ++w) {
+      float b = top.b[w];
+      q.at[w] = top.at[w];
+      if (mid.b[w] > b) { b = mid.b[w]; q.at[w] = 3u + mid.at[w]; }
+      if (bot.b[w] > b) q.at[w] = 6u + bot.at[w];
+    }
+    q.g[0] = g.v[0]; q.g[1] = g.v[1]; q.g[2] = g.n[0];
+    return q;
+  };
+  // adds what row `k` (of three) of the windows gives the four columns: even windows first, as everywhere in this file
+  auto add = [](float (&f)[4], const Windows &q, uint32_t k) {
+    auto hit = [&](int w, uint32_t col) { return q.at[w] == 3u * k + col ? q.g[w] : 0.f; };
+    f[0] += hit(0, 1u);
+    f[1] += hit(0, 2u);
+    f[1] += hit(1, 0u);
+    f[2] += hit(1, 1u);
+    f[3] += hit(2, 0u);
+    f[3] += hit(1, 2u);
+  };
+  auto store_row = [&](uint32_t R, float (&f)[4]) {
+    uint32_t t, r;
+    P.div_H.divmod(R, t, r);
+    T *p = reinterpret_cast<T *>(P.dx[t]) + ((size_t)plane * P.H + r) * P.W + c;
+    if (P.beta != 0.f) {
+      float old[4];
+      load_f<T, 4>(p, old);
+#pragma unroll
+      for (int k = 0; k < 4; ++k) f[k] += old[k];
+    }
+    struct alignas(4 * sizeof(T)) Pack { T e[4]; } v;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) st_f(v.e, k, f[k]);
+    *reinterpret_cast<Pack *>(p) = v;
+  };
+
+  const uint32_t o_lo = blockIdx.y * P.steps, o_hi = min(VO + 1u, o_lo + P.steps);  // (step VO: the last input row)
+  Windows above = {{9u, 9u, 9u}, {0.f, 0.f, 0.f}};
+  Best top;
+  if (o_lo > 0u) {
+    const Row a = load_row(2u * o_lo - 3u), b = load_row(2u * o_lo - 2u), d = load_row(2u * o_lo - 1u);  // (row -1: none)
+    const Grad g = load_dy(o_lo - 1u);
+    top = best_of(d);
+    above = windows_of(best_of(a), best_of(b), top, g);
+  } else {
+    top = best_of(load_row(~0u));
+  }
+  Row r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
+  Grad g = load_dy(o_lo);
+  for (uint32_t o = o_lo; o < o_hi; ++o) {
+    const Row n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
+    const Grad ng = load_dy(o + 1u);
+    const Best bot = best_of(r1);
+    const Windows here = windows_of(top, best_of(r0), bot, g);
+    if (o > 0u) {
+      // the windows of even rows of the tile that the input row belongs to first
+      float f[4] = {0.f, 0.f, 0.f, 0.f};
+      const uint32_t t = P.div_OH.div(o - 1u);
+      if (((o - 1u - t * P.OH) & 1u) == 0u) {
+        add(f, above, 2u);
+        add(f, here, 0u);
+      } else {
+        add(f, here, 0u);
+        add(f, above, 2u);
+      }
+      store_row(2u * o - 1u, f);
+    }
+    if (o < VO) {
+      float f[4] = {0.f, 0.f, 0.f, 0.f};
+      add(f, here, 1u);
+      store_row(2u * o, f);
+    }
+    above = here;
+    top = bot;
+    r0 = n0; r1 = n1; g = ng;
+  }
+}
+// 3x3 / 2, padding 1, rows and addresses of whole groups of four (dy: of two); anything else takes the bands
+static bool pool_bwd_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
+  if (P.wh != 3u || P.ww != 3u || P.sh != 2u || P.sw != 2u || P.pad_h != 1u || P.pad_w != 1u || P.W % 4u != 0u) return false;
+  const uint64_t items = (uint64_t)P.planes * (P.W / 4u), rows = (uint64_t)P.num_tiles * P.H;
+  if (items >= (1ull << 31) || rows >= (1ull << 31)) return false;
+  for (uint32_t t = 0; t < P.num_tiles; ++t) {
+    if (!aligned_to(P.x[t], 4 * es) || !aligned_to(P.out[t], 4 * es) || !aligned_to(P.dy[t], 2 * es)) return false;
+    q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->dx[t] = P.out[t];
+  }
+  q->items = (uint32_t)items;
+  q->K = P.num_tiles; q->H = P.H; q->W = P.W; q->OH = P.OH; q->OW = P.OW;
+  q->beta = P.beta;
+  // a band of n window rows reads 2 n + 3 input rows: long ones, as long as they leave every compute unit its share of waves
+  q->steps = 32u;
+  const uint64_t waves = (items + 63u) / 64u;
+  while (q->steps > 2u && waves * (P.num_tiles * P.OH / q->steps + 1u) < 256u * 16u) q->steps /= 2u;
+  if (P.num_tiles * P.OH / q->steps >= 65535u) return false;
+  q->div_groups = FastDiv(P.W / 4u); q->div_H = FastDiv(P.H); q->div_OH = FastDiv(P.OH);
+  return true;
+}
+
 // Tiles without halo: fills the padded extents and the split's fields; the same limits as the convolution over
 // such tiles (H / sh output rows per tile must stitch, a window reaches the adjacent tiles only).
 static int pool_check_unpadded(int dtype, int mode, uint32_t num_tiles, uint32_t N, uint32_t C, uint32_t H, uint32_t W,
@@ -816,6 +992,13 @@ int adh_pool2d_unpadded_bwd_tiles(int dtype, int mode, uint32_t num_tiles, uint3
   const uint32_t band_rows =
       wh * ww > 256u ? 0u : pick_band_rows(P, num_tiles, bwd_band_aim(P, es, is_max), [&](uint32_t r) { return bwd_band_lds(P, es, is_max, r); });
   if (!band_rows) return ADH_EUNIMPL;
+  PoolS2Params q = {};
+  if (is_max && pool_bwd_max3s2(P, es, &q)) {
+    const dim3 grid((q.items + kPoolThreads - 1u) / kPoolThreads, (q.K * q.OH + q.steps) / q.steps), block(kPoolThreads);
+    if (dtype == ADH_F32) hipLaunchKernelGGL((pool_bwd_max3s2_kernel<float>), grid, block, 0, as_stream(stream), q);
+    else hipLaunchKernelGGL((pool_bwd_max3s2_kernel<uint16_t>), grid, block, 0, as_stream(stream), q);
+    return launch_status();
+  }
   set_bands(&P, band_rows);
   launch_bwd_band_u<true>(dtype, is_max, P, P.planes * num_tiles * P.bands, bwd_band_lds(P, es, is_max, band_rows),
                           as_stream(stream));
