@@ -54,7 +54,10 @@ typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 // 16 bytes at 2-byte alignment: valid for both element types (fp32 rows are 4-byte aligned)
 typedef u32x4 u32x4_unaligned __attribute__((aligned(2)));
 
-// TAIL = (W % EPT != 0): the last vector of a row is partial and is moved element-wise.
+// TAIL: W % EPT != 0 and the last vector of a row is partial and moved element-wise, which every wave does.  Only sums
+// (ADD) and rows shorter than a vector need it: otherwise the last vector ends with the row, and what it shares with the
+// one before is stored twice alike.  Measured, bf16, 8 x 128 planes, 4 tiles of 64 x 255: pack 97 -> 60 us, unpack
+// 91 -> 51.
 // STREAM = the transfer is larger than the on-package cache: loads and stores are marked
 // non-temporal so that lines are not kept (a few percent more bandwidth from HBM, but a loss
 // when the data would have stayed cache-resident, so the host decides by size).
@@ -84,7 +87,7 @@ __global__ __launch_bounds__(kBlock) void row_copy_kernel(const RowCopyParams P)
     P.div_VR.divmod(live ? v : 0u, row, vr);
     P.div_DH.divmod(row, pl, hp);
     P.div_C.divmod(pl, n, c);
-    const uint32_t w0 = vr * EPT;
+    const uint32_t w0 = TAIL ? vr * EPT : min(vr * EPT, P.W - EPT);
     cnt[k] = live ? (TAIL ? min((uint32_t)EPT, P.W - w0) : (uint32_t)EPT) : 0u;
     first[k] = vr == 0;
     const int32_t gs = (int32_t)hp + row_base;
@@ -179,7 +182,7 @@ static int launch_row_copy(int dtype, bool add, bool zero_border, RowCopyParams 
   P.div_VR = FastDiv(P.VR);
   P.div_DH = FastDiv(P.DH);
   P.div_C = FastDiv(P.C);
-  const bool tail = P.W % ept != 0;
+  const bool tail = P.W % ept != 0 && (add || P.W < ept);
   // bytes read + written by the launch; above half of the 256 MB on-package cache nothing
   // would stay resident anyway
   const uint64_t moved = 2ull * P.W * P.DH * P.C * N * n_dst * dtype_size(dtype);
