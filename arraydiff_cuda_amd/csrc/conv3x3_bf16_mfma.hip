@@ -608,7 +608,7 @@ static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint3
 // name of the kernel a bf16 forward / backward-data call over padded tiles runs, for tiles aligned to 16 bytes
 // (template arguments: old output added, sums of earlier passes read, sums written for a later pass, tiles without halo)
 const char *conv_bf16_kernel_name(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, float beta) {
-  if (!conv_bf16_mfma_supported(which, Cin, Cout, H, W)) return "widen_bf16_kernel + conv3x3_f32_kernel + narrow_bf16_kernel";
+  if (!conv_bf16_mfma_supported(which, Cin, Cout, H, W)) return "widen_bf16_kernel + conv3x3_split_kernel + narrow_bf16_kernel";
   if (!conv_bf16_w8_width(which, W) && !conv_bf16_repitches(which, Cin, Cout, H, W)) {
     if (conv_bf16_passes(which, Cin, Cout) > 1u)
       return beta != 0.f ? "conv3x3_bf16_kernel<true, false, true> + <false, true, true> per middle 64 reduction channels + <false, true, false>"
