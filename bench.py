@@ -51,6 +51,8 @@ CLOCK_RAMP_MS = 150.0
 HBM_PEAK_GBS = 8000.0
 MFMA_F32_PEAK_TFLOPS = 157.3
 MFMA_BF16_PEAK_TFLOPS = 2500.0
+# fp32 convolutions that form six bf16 products per product (three-part split)
+MFMA_SPLIT_PEAK_TFLOPS = MFMA_BF16_PEAK_TFLOPS / 6
 METRIC = "halo pack/unpack GB/s (% HBM peak); 3x3 slab-conv TFLOP/s (% MFMA peak)"
 
 
@@ -356,7 +358,7 @@ def main():
         add("conv fwd cfg2 (fp32, 4 tiles of 14(+2)x56(+2), one launch)",
             lambda: lib.adh_conv3x3_slab_fwd_tiles(capi.ADH_F32, K, N, C, C, Ht, W, tile_tbl, wt.data_ptr(), y_tbl, 0.0,
                                                    None, 0, stream),
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s",
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s",
             extra={"kernel": name2, "traffic": traffic.get(name2, (None, None))[0]})
         reps, wu = 200, 20
         add("halo pack cfg1 (unsplit -> 4 padded tiles)",
@@ -400,29 +402,29 @@ def main():
         add("conv fwd cfg3 over unexchanged tiles (4 tiles, exchange + conv in one launch)",
             lambda: lib.adh_conv3x3_slab_fwd_tiles_unexchanged(0, K, N, C, C, Ht, W, tile_tbl, wt.data_ptr(), y_tbl, 0.0,
                                                                None, 0, stream),
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("halo exchange + conv fwd cfg3 (4 tiles, two launches: what the one above replaces)",
             lambda: (lib.adh_halo_exchange_nchw(0, 1, K, p, W, Ht, C, N, tile_tbl, stream),
                      lib.adh_conv3x3_slab_fwd_tiles(0, K, N, C, C, Ht, W, tile_tbl, wt.data_ptr(), y_tbl, 0.0, None, 0,
                                                     stream))[1],
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("conv bwd-data cfg3 (4 tiles)",
             lambda: lib.adh_conv3x3_slab_bwd_data_tiles(0, K, N, C, C, Ht, W, wt.data_ptr(), dy_tbl, g_tbl, 0.0, None,
                                                         0, stream),
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("conv bwd-data cfg3 with the halo reduce folded in (4 tiles, one launch)",
             lambda: lib.adh_conv3x3_slab_bwd_data_tiles_reduced(0, K, N, C, C, Ht, W, wt.data_ptr(), dy_tbl, g_tbl, 0.0,
                                                                 None, 0, stream),
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("conv bwd-data cfg3 + halo reduce (two launches: what the one above replaces)",
             lambda: (lib.adh_conv3x3_slab_bwd_data_tiles(0, K, N, C, C, Ht, W, wt.data_ptr(), dy_tbl, g_tbl, 0.0, None, 0,
                                                          stream),
                      lib.adh_halo_reduce_nchw(0, 1, K, p, W, Ht, C, N, g_tbl, stream))[1],
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("conv bwd-filter cfg3 (4 tiles, two kernels)",
             lambda: lib.adh_conv3x3_slab_bwd_filter_tiles(0, K, N, C, C, Ht, W, tile_tbl, dy_tbl, gw.data_ptr(), 0.0,
                                                           ws.data_ptr(), ws_bytes, stream),
-            "mfma", flops_step, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", flops_step, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
 
         # config 5 sized pack / unpack: 0.5 GB, larger than the on-package cache
         Y5 = torch.empty_like(X5)
@@ -570,7 +572,7 @@ def main():
         add("reference microbench_spatial_conv: conv fwd 3x3 dilation 3 over halo 3 (fp32, 4 tiles; the 3x3 kernel with its taps three apart)",
             lambda: lib.adh_conv2d_slab_fwd_tiles(0, Kd, Nd, C, C, HPd, WPd, *geo_d, xd_tbl, wd.data_ptr(), yd_tbl, 0.0,
                                                   wsd.data_ptr(), wsd_bytes, stream),
-            "mfma", fl_d, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", fl_d, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         add("reference microbench_spatial_conv: conv bwd-filter, same shape",
             lambda: lib.adh_conv2d_slab_bwd_filter_tiles(0, Kd, Nd, C, C, HPd, WPd, *geo_d, xd_tbl, yd_tbl, gwd.data_ptr(),
                                                          0.0, wsd.data_ptr(), wsd_bytes, stream),
@@ -578,7 +580,7 @@ def main():
         add("reference microbench_spatial_conv: conv bwd-data, same shape",
             lambda: lib.adh_conv2d_slab_bwd_data_tiles(0, Kd, Nd, C, C, HPd, WPd, *geo_d, wd.data_ptr(), yd_tbl, gd_tbl,
                                                        0.0, wsd.data_ptr(), wsd_bytes, stream),
-            "mfma", fl_d, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            "mfma", fl_d, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
         del xd, yd, gd, wsd
         # tools/microbench_conv.cc:30-54: one device, N=32, 64 -> 64 channels, 3x3 over a 64(+2) x 128(+2) slab,
         # "est flops" 2*N*Co*Ci*H*W*9 = 9.66 GF (:53)
@@ -590,7 +592,7 @@ def main():
         add("reference microbench_conv: conv fwd 3x3, N=32 64->64, 64(+2)x128(+2) slab (fp32, one tile)",
             lambda: lib.adh_conv3x3_slab_fwd(0, Nc, C, C, Hc, Wc, xc.data_ptr(), wd.data_ptr(), yc_.data_ptr(), 0.0,
                                              None, 0, stream),
-            "mfma", fl_c, MFMA_F32_PEAK_TFLOPS, "TFLOP/s",
+            "mfma", fl_c, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s",
             extra={"kernel": capi.conv_kernel_name(capi.ADH_CONV_FWD, capi.ADH_F32, 1, Nc, C, C, Hc, Wc)})
         del xc, yc_
         # column halos (a K x 1 grid, src/kernels/spatial.cu:654-731): cfg1's tensor split into 4 column-tiles
@@ -675,9 +677,9 @@ def main():
             else:
                 wgf = lambda: lib.adh_conv2d_unpadded_bwd_filter_tiles(0, K, N, Ci, Co, Hu, Wu, 3, 3, su, su, 1, 1, 1, 1, xu_tbl, yu_tbl,
                                                                        gwu.data_ptr(), 0.0, wsu.data_ptr(), wsb, stream)
-            add("conv fwd over tiles without halo, fp32, N=32, 4 tiles: " + nm, f, "mfma", flop, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
-            add("conv bwd-data into tiles without halo, fp32: " + nm, b, "mfma", flop, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
-            add("conv bwd-filter over tiles without halo, fp32: " + nm, wgf, "mfma", flop, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            add("conv fwd over tiles without halo, fp32, N=32, 4 tiles: " + nm, f, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
+            add("conv bwd-data into tiles without halo, fp32: " + nm, b, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
+            add("conv bwd-filter over tiles without halo, fp32: " + nm, wgf, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS if su == 1 else MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
             del xu, yu, wu_, gwu, wsu
         # the 1x1 stride-2 projection shortcuts of the same net (matrix-product kernels of their own): the first is
         # sized by memory (priced by the bytes of the pixels it uses and writes), the third by the matrix cores
@@ -736,7 +738,7 @@ def main():
             "hbm", 2 * (packed_b + packed_b) + packed_b, HBM_PEAK_GBS, "GB/s",
             note="x and the interior of dy read twice (sums, then gradient), dx written")
         del xb, dxb
-        # slab conv of any window (fp32 matrix cores): the 7x7 stride-2 stem over halo 3 (3 -> 64 channels, 224x224 in 4
+        # slab conv of any window: the 7x7 stride-2 stem over halo 3 (3 -> 64 channels, 224x224 in 4
         # row-tiles), the stride-1 stem of the spatially-parallel net (256x256 in 4 row-tiles; forward and backward-filter
         # of both by the kernels for at most three input channels) and a stride-2 3x3 (64 -> 128 channels) over cfg1's tiles
         for label, Ci, Co, Hs, Ws, ph, geo in (("7x7 s2 stem 3->64, 4 tiles of 62x230", 3, 64, 56, 224, 3, (7, 7, 2, 2, 1, 1)),
@@ -760,7 +762,7 @@ def main():
             add("general conv fwd " + label,
                 lambda: lib.adh_conv2d_slab_fwd_tiles(0, K, N, Ci, Co, HPs, WPs, *geo, xg_tbl, wg.data_ptr(), yg_tbl, 0.0,
                                                       wsg.data_ptr(), wsg_bytes, stream),
-                "mfma", fl, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+                "mfma", fl, MFMA_SPLIT_PEAK_TFLOPS if Ci <= 3 else MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
             add("general conv bwd-data " + label,
                 lambda: lib.adh_conv2d_slab_bwd_data_tiles(0, K, N, Ci, Co, HPs, WPs, *geo, wg.data_ptr(), yg_tbl, gg_tbl,
                                                            0.0, wsg.data_ptr(), wsg_bytes, stream),
@@ -768,7 +770,7 @@ def main():
             add("general conv bwd-filter " + label,
                 lambda: lib.adh_conv2d_slab_bwd_filter_tiles(0, K, N, Ci, Co, HPs, WPs, *geo, xg_tbl, yg_tbl, gwg.data_ptr(),
                                                              0.0, wsg.data_ptr(), wsg_bytes, stream),
-                "mfma", fl, MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+                "mfma", fl, MFMA_SPLIT_PEAK_TFLOPS if Ci <= 3 else MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
             del xg, yg, gg, wsg
 
         # the optimizer's flat vectors at ResNet-18's parameter count (11.69 M floats), gradients of 4 ranks
