@@ -4,7 +4,7 @@
 // gradient on that of conv3x3_bf16_wgrad.hip (at a width that is no multiple of 8 over copies of the
 // tensors with wider rows, made here).  What those do not take (images or sums beyond the 2 GiB a
 // buffer resource addresses) goes the route below: the bf16 slabs, filter and (for beta = 1) outputs
-// are widened to fp32 in the caller's workspace, the fp32 MFMA kernels run on the copies, and the
+// are widened to fp32 in the caller's workspace, the fp32 kernels run on the copies, and the
 // result is rounded back to bf16 (round to nearest even).  Every product is therefore exact and every sum is in
 // fp32, i.e. the arithmetic of a bf16-input / fp32-accumulate matrix core, at the speed of the
 // fp32 path plus three streaming passes.  The filter gradient stays fp32.
