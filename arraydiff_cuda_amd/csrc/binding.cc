@@ -12,6 +12,8 @@
 #include <torch/csrc/autograd/python_variable.h>
 
 #include <array>
+#include <exception>
+#include <memory>
 #include <tuple>
 #include <type_traits>
 #include <utility>
@@ -32,6 +34,7 @@ struct Tables {
   }
 };
 
+// (the tensor's methods throw, for instance where it has no storage: call() turns that into a Python error)
 const at::Tensor *gpu_tensor(PyObject *o) {
   if (!THPVariable_Check(o)) {
     PyErr_Format(PyExc_TypeError, "expected a tensor, got %s", Py_TYPE(o)->tp_name);
@@ -60,6 +63,11 @@ bool address_of(PyObject *o, uint64_t *p) {
   return true;
 }
 
+struct Release {
+  void operator()(PyObject *o) const { Py_DECREF(o); }
+};
+using Reference = std::unique_ptr<PyObject, Release>;
+
 template <typename T>
 bool convert(PyObject *o, T *v, Tables &tables) {
   if constexpr (std::is_floating_point_v<T>) {
@@ -78,13 +86,13 @@ bool convert(PyObject *o, T *v, Tables &tables) {
         *v = nullptr;
         return true;
       }
-      PyObject *seq = PySequence_Fast(o, "expected a sequence of tensors");
+      const Reference seq(PySequence_Fast(o, "expected a sequence of tensors"));
       if (!seq) return false;
       std::vector<uint64_t> &table = tables.next();
-      const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq);
+      const Py_ssize_t n = PySequence_Fast_GET_SIZE(seq.get());
       bool ok = true;
       for (Py_ssize_t i = 0; ok && i < n; ++i) {
-        PyObject *item = PySequence_Fast_GET_ITEM(seq, i);
+        PyObject *item = PySequence_Fast_GET_ITEM(seq.get(), i);
         uint64_t p = 0;
         if (lengths) {
           const at::Tensor *t = gpu_tensor(item);
@@ -95,7 +103,6 @@ bool convert(PyObject *o, T *v, Tables &tables) {
         }
         table.push_back(p);
       }
-      Py_DECREF(seq);
       if (!ok) return false;
       *v = reinterpret_cast<T>(table.data());
     }
@@ -122,7 +129,15 @@ PyObject *call(int (*fn)(A...), PyObject *const *args, std::index_sequence<I...>
   static thread_local Tables tables;
   tables.used = 0;
   std::tuple<A...> values;
-  if (!(convert(args[I], &std::get<I>(values), tables) && ...)) return nullptr;
+  try {
+    if (!(convert(args[I], &std::get<I>(values), tables) && ...)) return nullptr;
+  } catch (const c10::Error &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what_without_backtrace());
+    return nullptr;
+  } catch (const std::exception &e) {
+    PyErr_SetString(PyExc_RuntimeError, e.what());
+    return nullptr;
+  }
   if (!stream_of_torch(&std::get<sizeof...(I)>(values))) return nullptr;
   int rc;
   Py_BEGIN_ALLOW_THREADS

@@ -1,6 +1,7 @@
 """The native argument conversion refuses what a launch could not take before it reaches the library."""
 import pytest
 import torch
+from torch._subclasses.fake_tensor import FakeTensorMode
 
 from arraydiff_cuda_amd import capi
 
@@ -13,3 +14,10 @@ from arraydiff_cuda_amd import capi
 def test_refused_arguments(call, error):
     with pytest.raises(error):
         call()
+
+
+@pytest.mark.parametrize("call", [lambda t: capi.relu_fwd(t, t), lambda t: capi.sum_fwd([t], t)])
+def test_a_tensor_without_an_address_raises(call):
+    """Under vmap a tensor has no storage: torch's C++ exception arrives as a Python one."""
+    with FakeTensorMode(), pytest.raises(RuntimeError, match="storage"):
+        torch.vmap(lambda t: (call(t), t)[1])(torch.empty(3, 4, device="cuda"))
