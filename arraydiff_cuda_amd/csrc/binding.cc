@@ -1,9 +1,9 @@
 // Python calls of the C ABI with torch tensors as arguments (the module arraydiff_cuda_amd._binding).
 //
 // Every function declared in adh_capi.h that launches work on tensors is callable under its own name with its own
-// arguments but the last: the stream is torch's current one.  A device pointer is a tensor (contiguous, on the GPU), None
-// or an address, a table of device pointers a sequence of tensors, and a table of lengths the sequence of tensors whose
-// lengths they are.  The conversions are chosen by the parameters' C types.
+// arguments but the last: the stream is torch's current one.  A device pointer is a tensor (contiguous, on the GPU) or None, a
+// table of device pointers a sequence of tensors, and a table of lengths the sequence of tensors whose lengths they are.  The
+// conversions are chosen by the parameters' C types.
 // A small launch costs what its caller spends on the host: with ctypes, an exchange of the halos of four 14x56 tiles and
 // its backward took 18.0 us, of which the two kernels are 6; here the pair takes 6.7 us, and the fused softmax loss over
 // 256x1000 11.5 us instead of 23.8.
@@ -49,14 +49,6 @@ const at::Tensor *gpu_tensor(PyObject *o) {
 }
 
 bool address_of(PyObject *o, uint64_t *p) {
-  if (o == Py_None) {
-    *p = 0;
-    return true;
-  }
-  if (PyLong_Check(o)) {
-    *p = PyLong_AsUnsignedLongLong(o);
-    return !PyErr_Occurred();
-  }
   const at::Tensor *t = gpu_tensor(o);
   if (!t) return false;
   *p = reinterpret_cast<uint64_t>(t->data_ptr());
@@ -79,7 +71,7 @@ bool convert(PyObject *o, T *v, Tables &tables) {
     constexpr bool lengths = std::is_same_v<std::remove_const_t<P>, uint64_t>;
     if constexpr (!std::is_pointer_v<P> && !lengths) {
       uint64_t p = 0;
-      if (!address_of(o, &p)) return false;
+      if (o != Py_None && !address_of(o, &p)) return false;
       *v = reinterpret_cast<T>(p);
     } else {
       if (o == Py_None) {
