@@ -543,6 +543,9 @@ struct SplitPlan {
 // is a workspace, a block's chunks are dealt to several workgroups and a second kernel adds their sums, at its launch and the
 // sums' way through memory (1.2 KB a cycle): 512 channels on 4 tiles of 2 x 8, 32 images, 130 -> 74 us; on one image of 14 x 14
 // a tile 124 -> 40; 256 -> 512 on 28 x 28, 8 images, backward-data 147 -> 95.
+// The choice is made anew on every call, so tiles that cannot win are passed over by their least number of blocks before they are
+// priced: 64 channels on 4 x 32 x 128 5.8 -> 1.2 us of host time, on 8 x 128 x 2048 10.8 -> 1.6, the median of random shapes
+// 3.9 -> 1.5, with the same choices.
 static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) {
   SplitParams &P = plan->P;
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
@@ -570,6 +573,7 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
   auto held = [&](uint32_t n) { return n < patch(1u) ? 0u : q.sample == kDown ? (n - 1u) / 2u : n - (patch(1u) - 1u); };
   double best = 1e300;
   uint32_t nbi = 0, nbj = 0;
+  const uint64_t grid_rows = (uint64_t)P.NI * P.grid_VH, grid_pixels = grid_rows * P.grid_W;
   for (int MT = P.M <= 16u ? 1 : P.M <= 32u ? 2 : 4; MT >= 1; MT /= 2) {
     const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
     for (int NT = q.sample == kDown ? 1 : 4; NT >= 1; NT /= 2) {
@@ -578,36 +582,51 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
       const double matrix = 192.0 * MT * NT;
       const double chunk = 9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT;
       const double results = 2000.0 + 500.0 * MT * NT * (q.sample == kUp ? 4 : 1);
+      // What `blocks` blocks cost, their chunks undealt or (where they leave compute units idle) as dealt at best.  It grows with
+      // their number, so that tiles whose least possible number costs more than the best plan so far are passed over.
+      auto undealt = [&](uint64_t blocks) { return (double)((blocks + 255u) / 256u) * (P.nchunks * chunk + results) + 1e-3 * (double)blocks; };
+      auto dealt = [&](uint64_t blocks, uint32_t cps, uint32_t ks) {
+        return cps * chunk + results + 9000.0 + out_bytes * (ks + 1) / 1200.0 + 1e-3 * (double)blocks;
+      };
+      auto worse = [&](uint64_t least) {
+        if (undealt(least) < best) return false;
+        const uint64_t most = workspace ? 256u / least : 1u;
+        return most < 2u || dealt(least, (uint32_t)((P.nchunks + most - 1u) / most), 2u) >= best;
+      };
+      if (worse((grid_pixels + slots - 1u) / slots * MG)) continue;
       // columns per block: whole rows, halves and so on down to eight, multiples of four where rows are
       for (uint32_t parts = (P.grid_W + 255u) / 256u; parts <= P.grid_W; parts += 1u + parts / 8u) {
         uint32_t BC = (P.grid_W + parts - 1u) / parts;
         if (parts > 1u && BC < 8u) break;
         if (P.grid_W % 4u == 0u) BC = (BC + 3u) & ~3u;
-        const uint32_t nc = (P.grid_W + BC - 1u) / BC;
         if (BC > slots) continue;
-        const uint32_t max_BR = std::min(std::min(P.grid_VH, slots / BC), held(pixels / patch(BC)));
+        const uint32_t nc = (P.grid_W + BC - 1u) / BC, rows = slots / BC;
+        if (worse((grid_rows + rows - 1u) / rows * nc * MG)) continue;
+        const uint32_t patch_BC = patch(BC), max_BR = std::min(std::min(P.grid_VH, rows), held(pixels / patch_BC));
         if (max_BR == 0u) continue;
         const uint32_t nr0 = (P.grid_VH + max_BR - 1u) / max_BR;
         for (uint32_t nr = nr0; nr < nr0 + 2u && nr <= P.grid_VH; ++nr) {
           const uint32_t BR = (P.grid_VH + nr - 1u) / nr;
-          uint32_t NB = std::min(std::min(slots / (BR * BC), pixels / (patch(BR) * patch(BC))), P.NI);
+          uint32_t NB = std::min(std::min(rows / BR, pixels / (patch(BR) * patch_BC)), P.NI);
           const uint32_t groups = (P.NI + NB - 1u) / NB;
-          NB = (P.NI + groups - 1u) / groups;
           const uint64_t blocks = (uint64_t)groups * nc * nr * MG;
+          auto keep = [&](double cost, uint32_t ks, uint32_t cps) {
+            if (cost >= best) return;
+            best = cost;
+            plan->MT = MT; plan->NT = NT;
+            P.BR = BR; P.BC = BC; P.NB = (P.NI + groups - 1u) / groups;
+            P.ksplit = ks; P.chunks_per_split = cps;
+            nbi = nr; nbj = nc;
+          };
+          keep(undealt(blocks), 1u, P.nchunks);
           // chunks dealt to several workgroups per block, while all of them run at once
           const uint64_t most = workspace ? 256u / blocks : 1u;
-          for (uint32_t cps = P.nchunks; cps >= 1u; --cps) {
-            const uint32_t ks = (P.nchunks + cps - 1u) / cps;
-            if (ks > 1u && ks > most) break;
-            const double sums = ks > 1u ? 9000.0 + out_bytes * (ks + 1) / 1200.0 : 0.0;
-            const double cost = (double)((blocks * ks + 255u) / 256u) * (cps * chunk + results) + sums + 1e-3 * (double)blocks;
-            if (cost < best) {
-              best = cost;
-              plan->MT = MT; plan->NT = NT;
-              P.BR = BR; P.BC = BC; P.NB = NB;
-              P.ksplit = ks; P.chunks_per_split = cps;
-              nbi = nr; nbj = nc;
-            }
+          if (most < 2u) continue;
+          uint32_t ks = 1;
+          for (uint32_t cps = P.nchunks - 1u; cps >= 1u; --cps) {
+            ks = (P.nchunks + cps - 1u) / cps;
+            if (ks > most) break;
+            keep(dealt(blocks, cps, ks), ks, cps);
           }
         }
       }

@@ -3,6 +3,7 @@ validation that returns before any device work is exercised without a GPU."""
 import ctypes
 import os
 import re
+import time
 
 from arraydiff_cuda_amd import capi
 
@@ -82,3 +83,22 @@ def test_bf16_conv_workspace_holds_the_sums_of_every_route_that_needs_them():
     for which in (capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA):
         filt, part = need(which, 2, 1, 128, 128, 9, 72)
         assert l.adh_conv3x3_workspace_bytes(which, capi.ADH_BF16, 2, 1, 128, 128, 9, 72) == filt
+
+
+def test_the_choice_of_a_tile_is_made_in_microseconds():
+    """Every fp32 3x3 call chooses its tile anew: the search has to cost little beside a launch (it took 10 us and more for wide
+    rows while every tile was priced).  The best of many repetitions, with room for a slow host."""
+    l = capi.lib()
+    name = ctypes.create_string_buffer(256)
+    kernels = {(4, 32, 64, 64, 32, 128): b"<4, 4, true, 0>", (4, 32, 512, 512, 4, 16): b"<4, 2, true, 0>", (8, 2, 64, 64, 128, 2048): b"<4, 4, true, 0>",
+               (7, 3, 272, 40, 61, 1013): b"<4, 4, false, 0>", (4, 32, 64, 64, 14, 56): b"<4, 4, true, 0>"}
+    for (K, N, Cin, Cout, H, W), kernel in kernels.items():
+        args = [capi.ADH_CONV_FWD, capi.ADH_F32, K, N, Cin, Cout, H, W, 0.0, name, 256]
+        best = 1e9
+        for _ in range(50):
+            t = time.perf_counter()
+            for _ in range(20):
+                assert l.adh_conv3x3_kernel_name(*args) == capi.ADH_OK
+            best = min(best, (time.perf_counter() - t) / 20)
+        assert name.value == b"conv3x3_split_kernel" + kernel
+        assert best < 6e-6, (K, N, Cin, Cout, H, W, best)
