@@ -12,6 +12,10 @@
 //   * x rows go through a ring of 2 RS + 2 rows and dy rows through two buffers: a step brings RS new rows of each.  The rows
 //     of the next step are split and stored while this one is multiplied, and the ones after those are on their way in
 //     registers; the two waves of a SIMD take turns, one staging while the other multiplies.  One barrier a step.
+//   * What is multiplied need not be there: a step may reach past dy's last column or row, where dy is zero and x is whatever lies
+//     beside it, and an infinity's parts are not all finite.  Either way (zero times a NaN, inf - inf) the sum comes out as NaN:
+//     sums that are NaN are computed over again in plain fp32 from the pixels that exist.  (Noting such values as they are
+//     staged takes instructions and registers in the loop.)
 //   * The halves' sums are added through LDS, the workgroups' by a second kernel in a fixed order (reproducible).
 // Row tiles of one tensor are addressed as that tensor (as in conv3x3_split.hip).
 //
@@ -50,7 +54,7 @@ template <int OT, int CT>
 __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(const WgradSplitParams P) {
   constexpr uint32_t CO = 32u * OT, CI = 32u * CT;
   __shared__ __align__(16) char lds[kWsLdsBytes];
-  __shared__ uint32_t not_finite;
+  __shared__ uint32_t nan_sums;
   char *const dyl = lds + 3u * P.x_part_bytes;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -63,7 +67,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   uint32_t s = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
   const uint32_t s_end = (uint32_t)((uint64_t)P.total_steps * (split + 1u) / P.splits);
 
-  if (tid == 0u) not_finite = 0u;
+  if (tid == 0u) nan_sums = 0u;
   lds_barrier();
 
   // the run that the workgroup stands in: an image (pair) and a column tile of it
@@ -157,9 +161,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   };
   // slot0: ring slot of x row x0; buf: the dy buffer
   auto store = [&](uint32_t slot0, uint32_t nx, uint32_t buf, uint32_t nd) {
-    float mx = 0.f;
     auto put = [&](floatx4 y, char *p, uint32_t stride) {
-      mx = max_abs(max_abs(mx, y[0], y[1]), y[2], y[3]);
       uint32_t part[3][2];
       split_pair(y[0], y[1], part[0][0], part[1][0], part[2][0]);
       split_pair(y[2], y[3], part[0][1], part[1][1], part[2][1]);
@@ -184,14 +186,12 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
     }
     if (wave < nx && lane < CI) {
       if (!c_tail_ok) tail[0] = tail[1] = 0.f;
-      mx = max_abs(mx, tail[0], tail[1]);
       uint32_t part[3];
       split_pair(tail[0], tail[1], part[0], part[1], part[2]);
       char *p = lds + (slot_of(wave) * (CI * P.XP) + lane * P.XP + P.TW) * 2u;
 #pragma unroll
       for (int k = 0; k < 3; ++k) *reinterpret_cast<uint32_t *>(p + k * P.x_part_bytes) = part[k];
     }
-    if (mx >= kSplitLimit) not_finite = 1u;
   };
 
   // ---- this lane group's octet of a step: row io of the step, octet qo of the row ----
@@ -299,37 +299,6 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   // ---- the halves' sums, then to the workspace ----
   lds_barrier();
   constexpr uint32_t kTile = 9u * 256u;
-  if (not_finite != 0u) {
-    // plain fp32 sums, straight from memory; sums land where the second half's would
-    s = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
-    float *out = P.part + (size_t)blockIdx.x * (4u * OT * CT * kTile);
-    for (uint32_t at = tid; at < 4u * OT * CT * kTile; at += kWsThreads) {
-      const uint32_t i = at & 3u, ln = at >> 2 & 63u, rest = at >> 8, tap = rest % 9u, ct = rest / 9u % CT, ot = rest / 9u / CT % OT;
-      const uint32_t wt = rest / 9u / CT / OT;
-      const uint32_t co = co0 + ((wt & 1u) * OT + ot) * 16u + (ln >> 4) * 4u + i, ci = ci0 + ((wt >> 1) * CT + ct) * 16u + (ln & 15u);
-      float sum = 0.f;
-      if (co < P.Cout && ci < P.Cin)
-        for (uint32_t st = s; st < s_end; ++st) {
-          uint32_t run, rs, img, ctile;
-          P.div_row_steps.divmod(st, run, rs);
-          P.div_cols.divmod(run, img, ctile);
-          P.div_N.divmod(img, tile0, n);
-          for (uint32_t R = rs * P.RS; R < min((rs + 1u) * P.RS, P.dy_VH); ++R)
-            for (uint32_t Q = ctile * P.TW; Q < min((ctile + 1u) * P.TW, P.dy_W); ++Q) {
-              const int32_t xr = (int32_t)(R + tap / 3u) - P.pad_r, xc = (int32_t)(Q + tap % 3u) - P.pad_c;
-              float xe = 0.f;
-              if (xr >= 0 && xr < (int32_t)P.x_VH && xc >= 0 && xc < (int32_t)P.x_W) {
-                const Row w = row_of((uint32_t)xr, true);
-                xe = P.x[w.tile][((size_t)n * P.Cin + ci) * x_plane + (size_t)w.r * P.x_W + (uint32_t)xc];
-              }
-              const Row w = row_of(R, false);
-              sum = __builtin_fmaf(P.dy[w.tile][((size_t)n * P.Cout + co) * dy_plane + (size_t)w.r * P.dy_W + Q], xe, sum);
-            }
-        }
-      out[at] = sum;
-    }
-    return;
-  }
   floatx4 *const other = reinterpret_cast<floatx4 *>(lds) + (wave & 3u) * (OT * CT * 9u * 64u) + lane;
   if (half != 0u) {
 #pragma unroll
@@ -340,15 +309,51 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
         for (int t = 0; t < 9; ++t) other[((ot * CT + ct) * 9 + t) * 64] = acc[ot][ct][t];
   }
   lds_barrier();
+  float *const part = P.part + (size_t)blockIdx.x * (4u * OT * CT * kTile);
   if (half == 0u) {
-    ADH_GLOBAL float *out = (ADH_GLOBAL float *)P.part + (size_t)blockIdx.x * (4u * OT * CT * kTile) + (size_t)wave * (OT * CT * kTile) + lane * 4u;
+    ADH_GLOBAL float *out = (ADH_GLOBAL float *)part + (size_t)wave * (OT * CT * kTile) + lane * 4u;
+    bool nan = false;
 #pragma unroll
     for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
       for (int ct = 0; ct < CT; ++ct)
 #pragma unroll
-        for (int t = 0; t < 9; ++t)
-          *(ADH_GLOBAL floatx4_u *)(out + ((ot * CT + ct) * 9 + t) * 256) = acc[ot][ct][t] + other[((ot * CT + ct) * 9 + t) * 64];
+        for (int t = 0; t < 9; ++t) {
+          const floatx4 sum = acc[ot][ct][t] + other[((ot * CT + ct) * 9 + t) * 64];
+          nan |= __builtin_isunordered(sum[0], sum[1]) || __builtin_isunordered(sum[2], sum[3]);
+          *(ADH_GLOBAL floatx4_u *)(out + ((ot * CT + ct) * 9 + t) * 256) = sum;
+        }
+    if (nan) nan_sums = 1u;
+  }
+  __syncthreads();
+  if (nan_sums == 0u) return;
+  // sums that are NaN once more in plain fp32, straight from memory
+  s = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
+  for (uint32_t at = tid; at < 4u * OT * CT * kTile; at += kWsThreads) {
+    if (part[at] == part[at]) continue;
+    const uint32_t i = at & 3u, ln = at >> 2 & 63u, rest = at >> 8, tap = rest % 9u, ct = rest / 9u % CT, ot = rest / 9u / CT % OT;
+    const uint32_t wt = rest / 9u / CT / OT;
+    const uint32_t co = co0 + ((wt & 1u) * OT + ot) * 16u + (ln >> 4) * 4u + i, ci = ci0 + ((wt >> 1) * CT + ct) * 16u + (ln & 15u);
+    float sum = 0.f;
+    if (co < P.Cout && ci < P.Cin)
+      for (uint32_t st = s; st < s_end && sum == sum; ++st) {  // (a NaN stays one)
+        uint32_t run, rs, img, ctile;
+        P.div_row_steps.divmod(st, run, rs);
+        P.div_cols.divmod(run, img, ctile);
+        P.div_N.divmod(img, tile0, n);
+        for (uint32_t R = rs * P.RS; R < min((rs + 1u) * P.RS, P.dy_VH) && sum == sum; ++R)
+          for (uint32_t Q = ctile * P.TW; Q < min((ctile + 1u) * P.TW, P.dy_W) && sum == sum; ++Q) {
+            const int32_t xr = (int32_t)(R + tap / 3u) - P.pad_r, xc = (int32_t)(Q + tap % 3u) - P.pad_c;
+            float xe = 0.f;
+            if (xr >= 0 && xr < (int32_t)P.x_VH && xc >= 0 && xc < (int32_t)P.x_W) {
+              const Row w = row_of((uint32_t)xr, true);
+              xe = P.x[w.tile][((size_t)n * P.Cin + ci) * x_plane + (size_t)w.r * P.x_W + (uint32_t)xc];
+            }
+            const Row w = row_of(R, false);
+            sum = __builtin_fmaf(P.dy[w.tile][((size_t)n * P.Cout + co) * dy_plane + (size_t)w.r * P.dy_W + Q], xe, sum);
+          }
+      }
+    part[at] = sum;
   }
 }
 

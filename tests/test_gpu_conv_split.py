@@ -124,3 +124,38 @@ def test_filter_gradient_of_values_without_finite_bf16_parts(bad):
         fine = torch.isfinite(want)
         assert ((got[fine].double() - want[fine].double()).abs() <= 2e-6 * want[fine].double().abs()).all()
         assert fine.any() and not fine.all()
+
+
+@pytest.mark.parametrize("bad", [float("inf"), float("nan")])
+@pytest.mark.parametrize("halo", [False, True])
+@pytest.mark.parametrize("K,H,W", [(1, 6, 56), (1, 7, 21), (3, 5, 32), (1, 9, 8), (2, 1, 13)])
+def test_filter_gradient_of_a_bad_value_at_the_border(K, H, W, halo, bad):
+    """A step of the kernel multiplies pixels past the last column and row of dy, which are zero, with what x has beside them: a
+    NaN there belongs to the taps that reach it from a pixel that exists, and to no other."""
+    N, Cin, Cout = 2, 20, 40
+    g = torch.Generator().manual_seed(9)
+    p = 1 if halo else 0
+    x, dy = torch.rand((K, N, Cin, H + 2 * p, W + 2 * p), generator=g) + 0.5, torch.rand((K, N, Cout, H, W), generator=g) + 0.5
+    ws = torch.empty(capi.conv_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_F32, K, N, Cin, Cout, H, W) // 4, device="cuda")
+    fn = capi.conv_bwd_filter_tiles if halo else capi.conv_unpadded_bwd_filter_tiles
+    for row, col in ((0, -1), (-1, 0), (-1, -1), (H // 2, W // 2), (0, 0), (0, -2), (-2, 0)):
+        if not (-x.shape[3] <= row and -x.shape[4] <= col):
+            continue
+        xb = x.clone()
+        xb[K - 1, 1, 3, row, col] = bad
+        dw = torch.empty((Cout, Cin, 3, 3), device="cuda")
+        capi.check(fn(list(xb.cuda()), list(dy.cuda()), dw, N, Cin, Cout, H, W, ws=ws), "bwd-filter")
+        if halo:
+            xp, d, h = xb.transpose(0, 1).reshape(N, K, Cin, H + 2, W + 2), dy.transpose(0, 1), H
+        else:  # the row tiles of one tensor
+            h = K * H
+            xp = torch.nn.functional.pad(torch.cat(list(xb), 2), (1, 1, 1, 1))[:, None]
+            d = torch.cat(list(dy), 2)[:, None]
+        want = torch.stack([torch.stack([(d.double()[:, :, :, None] * xp.double()[:, :, None, :, a:a + h, b:b + W]).sum((0, 1, 4, 5))
+                                         for b in range(3)], -1) for a in range(3)], -2)
+        got = dw.cpu()
+        assert torch.equal(torch.isnan(got), torch.isnan(want)), (row, col)
+        assert torch.equal(torch.isinf(got), torch.isinf(want)), (row, col)
+        fine = torch.isfinite(want)
+        # positive sums of K N H W terms, each addition rounded once
+        assert ((got[fine].double() - want[fine]).abs() <= (K * N * H * W + 4) * 2.0 ** -24 * want[fine]).all() and fine.any()
