@@ -1396,7 +1396,7 @@ int conv2d_bwd_filter(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
     q.stacked = unpadded;
     q.pad_r = unpadded ? (int32_t)pad_h : 0; q.pad_c = unpadded ? (int32_t)pad_w : 0;
     q.x = x_tiles; q.dy = dy_tiles; q.dw = dwt; q.beta = beta;
-    e = conv3x3_wgrad_split(q, workspace, st);
+    e = conv3x3_wgrad_split(q, workspace, workspace_bytes, st);
     if (e != ADH_EUNIMPL) return e;
   }
   if (gen_is_3x3_dilated(dtype, g, unpadded)) {

@@ -9,6 +9,7 @@
 // fp32, i.e. the arithmetic of a bf16-input / fp32-accumulate matrix core, at the speed of the
 // fp32 path plus three streaming passes.  The filter gradient stays fp32.
 #include "conv3x3_bf16_mfma.h"
+#include "conv3x3_wgrad_split.h"
 
 namespace adh {
 
@@ -184,10 +185,6 @@ size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t 
 
 using namespace adh;
 
-// fp32 kernels of the other translation units
-extern "C" size_t adh_conv3x3_workspace_bytes(int which, int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin,
-                                              uint32_t Cout, uint32_t H, uint32_t W);
-
 namespace adh {
 
 static int widen(uint64_t n, const void *src, float *dst, hipStream_t st) {
@@ -303,9 +300,7 @@ int conv_bf16_filter_via_f32(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint3
     if (e) return e;
     return conv_bf16_wgrad_mfma(num_tiles, N, Cin, Cout, H, Wd, xw, dyw, dw, beta, ws, st, false);
   }
-  const size_t f32_bytes = adh_conv3x3_workspace_bytes(ADH_CONV_BWD_FILTER, ADH_F32, num_tiles, N, Cin, Cout, H, W);
-  if (f32_bytes == 0) return ADH_EUNIMPL;
-  const size_t need = bf16_workspace_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, f32_bytes);
+  const size_t need = bf16_workspace_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, conv3x3_wgrad_split_least_workspace(Cin, Cout));
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;

@@ -442,7 +442,7 @@ static int wgrad_entry(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, 
   if ((uint64_t)Cin * Cout * 9u >= (1ull << 31)) return ADH_EINVAL;
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 4)) return ADH_EALIGN;
-  if (workspace_bytes < conv3x3_wgrad_split_workspace(num_tiles, N, Cin, Cout, H, W)) return ADH_EWORKSPACE;
+  if (workspace_bytes < conv3x3_wgrad_split_least_workspace(Cin, Cout)) return ADH_EWORKSPACE;
   for (uint32_t t = 0; t < num_tiles; ++t) {
     if (!x_pad_tiles[t] || !dy_tiles[t]) return ADH_ENULL;
     if (!aligned_to(x_pad_tiles[t], 4) || !aligned_to(dy_tiles[t], 4)) return ADH_EALIGN;
@@ -455,7 +455,7 @@ static int wgrad_entry(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, 
   q.neighbours = rows_from_neighbours && !unpadded;
   q.pad_r = q.pad_c = unpadded ? 1 : 0;
   q.x = x_pad_tiles; q.dy = dy_tiles; q.dw = dw; q.beta = beta;
-  return conv3x3_wgrad_split(q, workspace, st);
+  return conv3x3_wgrad_split(q, workspace, workspace_bytes, st);
 }
 
 int adh_conv3x3_slab_bwd_filter_tiles(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout,

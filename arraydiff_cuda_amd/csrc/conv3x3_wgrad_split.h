@@ -22,7 +22,10 @@ struct Wgrad3x3Problem {
 
 // enough for every form (padded, unexchanged, without halo) of the layer whose tiles' interiors are H x W
 size_t conv3x3_wgrad_split_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
-int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, hipStream_t st);
+// the least that it runs with: in a smaller workspace than the above the pixels are dealt to fewer workgroups, below a workgroup
+// per channel group the groups are launched in turn
+size_t conv3x3_wgrad_split_least_workspace(uint32_t Cin, uint32_t Cout);
+int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st);
 
 }  // namespace adh
 #endif

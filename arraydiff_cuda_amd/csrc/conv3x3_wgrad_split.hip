@@ -45,7 +45,7 @@ struct WgradSplitParams {
   int32_t pad_r, pad_c, neighbours;
   uint32_t TW, logQ, RS, NR, XP, DP;        // logQ: log2 of a row's groups of four columns; pitches in pixels
   uint32_t x_part_bytes, dy_part_bytes;     // bytes of one part of the ring and of the dy buffers
-  uint32_t col_tiles, row_steps, total_steps, splits, ci_groups;
+  uint32_t col_tiles, row_steps, total_steps, splits, ci_groups, group0;
   float beta;
   FastDiv div_row_steps, div_cols, div_N, div_step, div_splits, div_cig;
 };
@@ -62,7 +62,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
 
   uint32_t group, split, cog, cig;
   P.div_splits.divmod(blockIdx.x, group, split);
-  P.div_cig.divmod(group, cog, cig);
+  P.div_cig.divmod(P.group0 + group, cog, cig);
   const uint32_t co0 = cog * CO, ci0 = cig * CI;
   uint32_t s = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
   const uint32_t s_end = (uint32_t)((uint64_t)P.total_steps * (split + 1u) / P.splits);
@@ -375,7 +375,7 @@ __global__ __launch_bounds__(256) void conv3x3_wgrad_split_reduce_kernel(const W
   for (int k = 1; k < 16; ++k) sum += sums[k][threadIdx.x];
   const uint32_t ln = e & 63u, rest = e >> 6, tap = rest % 9u, ct = rest / 9u % CT, ot = rest / 9u / CT % OT, wt = rest / 9u / CT / OT;
   uint32_t cog, cig;
-  P.div_cig.divmod(group, cog, cig);
+  P.div_cig.divmod(P.group0 + group, cog, cig);
   const uint32_t co = cog * (32u * OT) + ((wt & 1u) * OT + ot) * 16u + (ln >> 4) * 4u, ci = cig * (32u * CT) + ((wt >> 1) * CT + ct) * 16u + (ln & 15u);
   if (ci >= P.Cin) return;
 #pragma unroll
@@ -396,20 +396,30 @@ static uint32_t ws_max_splits(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
   return (uint32_t)std::max<uint64_t>(1u, std::min<uint64_t>(most, 256u / groups));
 }
 
+// a workgroup's sums
+size_t conv3x3_wgrad_split_least_workspace(uint32_t Cin, uint32_t Cout) {
+  return (size_t)ws_channel_tiles(Cout) * ws_channel_tiles(Cin) * 4u * 9u * 256u * 4u;
+}
 size_t conv3x3_wgrad_split_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
   const uint32_t ot = ws_channel_tiles(Cout), ct = ws_channel_tiles(Cin);
   const uint64_t groups = (uint64_t)((Cout + 32u * ot - 1u) / (32u * ot)) * ((Cin + 32u * ct - 1u) / (32u * ct));
-  return (size_t)groups * ws_max_splits(num_tiles, N, Cin, Cout, H, W) * 4u * ot * ct * 9u * 256u * 4u;
+  return (size_t)groups * ws_max_splits(num_tiles, N, Cin, Cout, H, W) * conv3x3_wgrad_split_least_workspace(Cin, Cout);
 }
 
+// at_once: channel groups whose sums the workspace holds
 template <int OT, int CT>
-static int launch_wgrad_split(const WgradSplitParams &P, uint32_t groups, hipStream_t st) {
-  hipLaunchKernelGGL((conv3x3_wgrad_split_kernel<OT, CT>), dim3(groups * P.splits), dim3(kWsThreads), 0, st, P);
-  hipLaunchKernelGGL((conv3x3_wgrad_split_reduce_kernel<OT, CT>), dim3(groups * (4u * OT * CT * 9u * 64u / 16u)), dim3(256), 0, st, P);
-  return launch_status();
+static int launch_wgrad_split(WgradSplitParams P, uint32_t groups, uint32_t at_once, hipStream_t st) {
+  for (P.group0 = 0u; P.group0 < groups; P.group0 += at_once) {
+    const uint32_t n = std::min(at_once, groups - P.group0);
+    hipLaunchKernelGGL((conv3x3_wgrad_split_kernel<OT, CT>), dim3(n * P.splits), dim3(kWsThreads), 0, st, P);
+    hipLaunchKernelGGL((conv3x3_wgrad_split_reduce_kernel<OT, CT>), dim3(n * (4u * OT * CT * 9u * 64u / 16u)), dim3(256), 0, st, P);
+    const int e = launch_status();
+    if (e) return e;
+  }
+  return ADH_OK;
 }
 
-int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, hipStream_t st) {
+int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st) {
   WgradSplitParams P = {};
   for (uint32_t t = 0; t < q.num_tiles; ++t) {
     P.x[t] = reinterpret_cast<const float *>(q.x[t]);
@@ -454,11 +464,15 @@ int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, hipStream_t s
   P.ci_groups = (q.Cin + 32u * CT - 1u) / (32u * CT);
   const uint32_t groups = P.ci_groups * ((q.Cout + 32u * OT - 1u) / (32u * OT));
   P.splits = std::min(ws_max_splits(q.num_tiles, q.N, q.Cin, q.Cout, q.dy_H, q.dy_W), P.total_steps);
+  const uint64_t room = workspace_bytes / conv3x3_wgrad_split_least_workspace(q.Cin, q.Cout);  // for workgroups' sums
+  if (room == 0u) return ADH_EWORKSPACE;
+  const uint32_t at_once = (uint32_t)std::min<uint64_t>(groups, room);
+  P.splits = (uint32_t)std::min<uint64_t>(P.splits, room / at_once);
   if ((uint64_t)groups * P.splits >= (1ull << 24)) return ADH_EUNIMPL;
   P.div_row_steps = FastDiv(P.row_steps); P.div_cols = FastDiv(P.col_tiles);
   P.div_N = FastDiv(q.N); P.div_step = FastDiv(P.step); P.div_splits = FastDiv(P.splits); P.div_cig = FastDiv(P.ci_groups);
-  if (OT == 2u) return CT == 2u ? launch_wgrad_split<2, 2>(P, groups, st) : launch_wgrad_split<2, 1>(P, groups, st);
-  return CT == 2u ? launch_wgrad_split<1, 2>(P, groups, st) : launch_wgrad_split<1, 1>(P, groups, st);
+  if (OT == 2u) return CT == 2u ? launch_wgrad_split<2, 2>(P, groups, at_once, st) : launch_wgrad_split<2, 1>(P, groups, at_once, st);
+  return CT == 2u ? launch_wgrad_split<1, 2>(P, groups, at_once, st) : launch_wgrad_split<1, 1>(P, groups, at_once, st);
 }
 
 }  // namespace adh

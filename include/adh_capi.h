@@ -266,6 +266,8 @@ int adh_conv3x3_unpadded_bwd_filter_tiles(int dtype, uint32_t num_tiles, uint32_
  * dw[co,ci,kh,kw] = beta*dw + sum_{tiles,n,h,w} dy[n,co,h,w] * x_pad[n,ci,h+kh,w+kw]
  * (the sum over tiles is what ParallelSGDOptimizer's ncclReduce did across ranks,
  * include/arraydiff/optimize.hh:443-451).  dw is always fp32.  Deterministic.
+ * ADH_F32: a workspace below adh_conv3x3_workspace_bytes is taken down to one workgroup's sums (147,456 bytes; half
+ * of it for each side of at most 32 channels): fewer workgroups share the pixels then, or the channel groups run in turn.
  * ADH_BF16: the matrix-core kernel reads rows of whole 16-byte granules; at a width that is no multiple
  * of 8 the rows of x_pad and dy are first copied into the workspace at the next such width with zeros
  * behind (a zero dy adds nothing to any tap), one more pass over both tensors. */

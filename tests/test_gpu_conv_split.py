@@ -159,3 +159,26 @@ def test_filter_gradient_of_a_bad_value_at_the_border(K, H, W, halo, bad):
         fine = torch.isfinite(want)
         # positive sums of K N H W terms, each addition rounded once
         assert ((got[fine].double() - want[fine]).abs() <= (K * N * H * W + 4) * 2.0 ** -24 * want[fine]).all() and fine.any()
+
+
+@pytest.mark.parametrize("K,N,Cin,Cout,H,W", [(5, 4, 128, 64, 7, 7), (1, 1, 65, 65, 3, 5), (2, 3, 20, 100, 9, 33), (1, 2, 40, 30, 4, 4), (1, 1, 3, 5, 2, 2)])
+def test_filter_gradient_in_a_small_workspace(K, N, Cin, Cout, H, W):
+    """A workspace below the query's answer: fewer workgroups share the pixels, then the channel groups run in turn."""
+    g = torch.Generator().manual_seed(10)
+    x, dy = torch.rand((N, Cin, K * H, W), generator=g) * 2 - 1, torch.randn((N, Cout, K * H, W), generator=g)
+    want = torch.nn.grad.conv2d_weight(x.double(), (Cout, Cin, 3, 3), dy.double(), padding=1).numpy()
+    xs, dys = _tiles(x.cuda(), K), _tiles(dy.cuda(), K)
+    unit = 4 * 9 * 1024 * (2 if Cin > 32 else 1) * (2 if Cout > 32 else 1)  # a workgroup's sums
+    groups = -(-Cin // 64) * -(-Cout // 64)
+    full = capi.conv_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_F32, K, N, Cin, Cout, H, W)
+    for nbytes in {unit, groups * unit - 4, groups * unit, 2 * groups * unit + 4, full // 2, full}:
+        if not unit <= nbytes <= full:
+            continue
+        ws = torch.full((nbytes // 4 + 64,), 7.0, device="cuda")
+        dw = torch.ones((Cout, Cin, 3, 3), device="cuda")
+        capi.check(capi.conv_unpadded_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, H, W, beta=1.0, ws=ws[:nbytes // 4]), "bwd-filter")
+        assert rel_err(host(dw), want + 1.0) <= 1e-5, nbytes
+        assert (ws[nbytes // 4:] == 7.0).all()
+    dw = torch.ones((Cout, Cin, 3, 3), device="cuda")
+    small = torch.empty(unit // 4 - 1, device="cuda")
+    assert capi.conv_unpadded_bwd_filter_tiles(xs, dys, dw, N, Cin, Cout, H, W, ws=small) == capi.ADH_EWORKSPACE
