@@ -649,7 +649,7 @@ size_t conv_thin_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, u
                                  uint32_t OH, uint32_t OW, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw);
 int conv_thin_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t HP, uint32_t WP, uint32_t OH,
                         uint32_t OW, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw, const void *const *x_tiles,
-                        const void *const *dy_tiles, float *dwt, float beta, void *workspace, hipStream_t st);
+                        const void *const *dy_tiles, float *dwt, float beta, void *workspace, size_t workspace_bytes, hipStream_t st);
 static bool gen_is_thin(int dtype, const GenShape &g, bool unpadded) {
   return dtype == ADH_F32 && !unpadded && g.dh == 1u && g.dw == 1u && g.Cin <= 3u && (g.kh > 1u || g.kw > 1u);
 }
@@ -1380,13 +1380,9 @@ int conv2d_bwd_filter(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
     }
   }
   if (gen_is_thin(dtype, g, unpadded)) {
-    const size_t need = conv_thin_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, kh, kw, sh, sw);
-    if (need != 0) {
-      if (workspace_bytes < need) return ADH_EWORKSPACE;
-      e = conv_thin_wgrad_try(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, kh, kw, sh, sw, x_tiles, dy_tiles, dwt, beta,
-                              workspace, st);
-      if (e != ADH_EUNIMPL) return e;
-    }
+    e = conv_thin_wgrad_try(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, kh, kw, sh, sw, x_tiles, dy_tiles, dwt, beta,
+                            workspace, workspace_bytes, st);
+    if (e != ADH_EUNIMPL) return e;
   }
   if (gen_is_3x3_unit(dtype, g) && g.dh == 1u && workspace_bytes >= conv3x3_wgrad_split_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW)) {
     Wgrad3x3Problem q = {};

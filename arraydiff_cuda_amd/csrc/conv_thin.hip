@@ -435,15 +435,16 @@ size_t conv_thin_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, u
 }
 
 // Filter gradient over halo-padded fp32 tiles for at most three input channels and Cin kh kw <= 160, any stride, no
-// dilation.  `workspace` holds conv_thin_wgrad_workspace bytes.  ADH_EUNIMPL: not served; nothing launched.
+// dilation.  ADH_EUNIMPL: not served, or not in a workspace below conv_thin_wgrad_workspace; nothing launched.
 int conv_thin_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t HP, uint32_t WP, uint32_t OH,
                         uint32_t OW, uint32_t kh, uint32_t kw, uint32_t sh, uint32_t sw, const void *const *x_tiles,
-                        const void *const *dy_tiles, float *dwt, float beta, void *workspace, hipStream_t st) {
+                        const void *const *dy_tiles, float *dwt, float beta, void *workspace, size_t workspace_bytes, hipStream_t st) {
   const ThinProblem q = {num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, x_tiles};
-  const int split = conv_thin_split_wgrad(q, dy_tiles, dwt, beta, workspace, st);
+  const int split = conv_thin_split_wgrad(q, dy_tiles, dwt, beta, workspace, workspace_bytes, st);
   if (split != ADH_EUNIMPL) return split;
   ThinWgradPlan plan;
-  if (!thin_wgrad_plan(num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, &plan)) return ADH_EUNIMPL;
+  if (!thin_wgrad_plan(num_tiles, N, Cin, Cout, HP, WP, OH, OW, kh, kw, sh, sw, &plan) || workspace_bytes < plan.part_bytes)
+    return ADH_EUNIMPL;
   ThinWgradParams P = {};
   for (uint32_t t = 0; t < num_tiles; ++t) {
     if (!aligned_to(x_tiles[t], 4) || !aligned_to(dy_tiles[t], 4)) return ADH_EUNIMPL;

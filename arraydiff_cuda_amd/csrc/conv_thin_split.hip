@@ -684,9 +684,12 @@ size_t conv_thin_split_wgrad_workspace(const ThinProblem &q) {
   return (size_t)P.splits * P.M * P.KK * sizeof(float);
 }
 
-int conv_thin_split_wgrad(const ThinProblem &q, const void *const *dy_tiles, float *dw, float beta, void *workspace, hipStream_t st) {
+int conv_thin_split_wgrad(const ThinProblem &q, const void *const *dy_tiles, float *dw, float beta, void *workspace,
+                          size_t workspace_bytes, hipStream_t st) {
   ThinSplitWgradParams P = {};
   if (!thin_split_wgrad_plan(q, &P)) return ADH_EUNIMPL;
+  P.splits = (uint32_t)std::min<uint64_t>(P.splits, workspace_bytes / ((uint64_t)P.M * P.KK * sizeof(float)));
+  if (P.splits == 0u) return ADH_EUNIMPL;
   for (uint32_t t = 0; t < q.num_tiles; ++t) {
     if (!aligned_to(q.x[t], 4) || !aligned_to(dy_tiles[t], 4)) return ADH_EUNIMPL;
     P.x[t] = reinterpret_cast<const float *>(q.x[t]);

@@ -81,3 +81,21 @@ def test_values_without_finite_bf16_parts(bad, s):
         capi.check(capi.conv2d_bwd_filter_tiles([xb.cuda()], [db.cuda()], dw, N, Cin, Cout, HP, WP, *geo,
                                                 ws=_ws(capi.ADH_CONV_BWD_FILTER, 1, N, Cin, Cout, HP, WP, geo)), "bwd-filter")
         same(dw.cpu(), torch.stack([(db[:, :, None] * xt[:, None]).sum((0, 3, 4)) for xt in taps(xb)], -1).reshape(Cout, Cin, k, k))
+
+
+@pytest.mark.parametrize("K,N,Cin,Cout,OH,OW,k,s,nbytes", [(4, 3, 3, 64, 9, 18, 7, 1, 1474560), (4, 4, 3, 64, 12, 1, 7, 2, 655360),
+                                                           (3, 4, 3, 64, 16, 4, 3, 2, 196608), (1, 3, 3, 64, 1, 6, 3, 2, 16384)])
+def test_filter_gradient_in_a_small_workspace(K, N, Cin, Cout, OH, OW, k, s, nbytes):
+    """A workspace below the query's answer but enough for the general kernel: fewer workgroups share the pixels."""
+    HP, WP, geo = (OH - 1) * s + k, (OW - 1) * s + k, (k, k, s, s, 1, 1)
+    g = torch.Generator().manual_seed(11)
+    xs = [torch.rand((N, Cin, HP, WP), generator=g) * 2 - 1 for _ in range(K)]
+    dys = [torch.randn((N, Cout, OH, OW), generator=g) for _ in range(K)]
+    want = torch.nn.grad.conv2d_weight(torch.cat(xs).double(), (Cout, Cin, k, k), torch.cat(dys).double(), stride=s).numpy()
+    assert nbytes < capi.conv2d_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_F32, K, N, Cin, Cout, HP, WP, *geo)
+    ws = torch.full((nbytes // 4 + 64,), 7.0, device="cuda")
+    dw = torch.ones((Cout, Cin, k, k), device="cuda")
+    capi.check(capi.conv2d_bwd_filter_tiles([x.cuda() for x in xs], [d.cuda() for d in dys], dw, N, Cin, Cout, HP, WP, *geo, beta=1.0,
+                                            ws=ws[:nbytes // 4]), "bwd-filter")
+    assert (ws[nbytes // 4:] == 7.0).all()
+    assert rel_err(host(dw), want + 1.0) <= 1e-5
