@@ -147,19 +147,24 @@ static bool wgrad_repitch_route(uint32_t Cin, uint32_t Cout, uint32_t H, uint32_
 int repitch_bf16_tiles(uint32_t num_tiles, uint64_t rows, uint32_t w_src, uint32_t w_dst, const void *const *src,
                        void *const *dst, hipStream_t st) {
   RepitchParams P;
-  for (uint32_t t = 0; t < num_tiles; ++t) {
-    P.src[t] = reinterpret_cast<const uint16_t *>(src[t]);
-    P.dst[t] = reinterpret_cast<uint16_t *>(dst[t]);
-  }
   P.w_src = w_src;
   P.w_dst = w_dst;
   P.granules = (w_dst + 7u) / 8u;
-  P.rows = (uint32_t)rows;
   P.div_granules = FastDiv(P.granules);
-  if (rows * P.granules >= (1ull << 31)) return ADH_EINVAL;
-  const uint32_t blocks = ((uint32_t)rows * P.granules + 1023u) / 1024u, most = (256u * 8u + num_tiles - 1u) / num_tiles;
-  hipLaunchKernelGGL(repitch_bf16_kernel, dim3(blocks < most ? blocks : most, num_tiles), dim3(256), 0, st, P);
-  return launch_status();
+  // the kernel counts a launch's granules in 32 bits
+  const uint64_t most_rows = ((1ull << 31) - 1u) / P.granules;
+  for (uint64_t row = 0; row < rows; row += most_rows) {
+    for (uint32_t t = 0; t < num_tiles; ++t) {
+      P.src[t] = reinterpret_cast<const uint16_t *>(src[t]) + row * w_src;
+      P.dst[t] = reinterpret_cast<uint16_t *>(dst[t]) + row * w_dst;
+    }
+    P.rows = (uint32_t)(rows - row < most_rows ? rows - row : most_rows);
+    const uint32_t blocks = (P.rows * P.granules + 1023u) / 1024u, most = (256u * 8u + num_tiles - 1u) / num_tiles;
+    hipLaunchKernelGGL(repitch_bf16_kernel, dim3(blocks < most ? blocks : most, num_tiles), dim3(256), 0, st, P);
+    const int e = launch_status();
+    if (e) return e;
+  }
+  return ADH_OK;
 }
 
 size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,

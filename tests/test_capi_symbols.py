@@ -5,6 +5,9 @@ import os
 import re
 import time
 
+import pytest
+import torch
+
 from arraydiff_cuda_amd import capi
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
@@ -83,6 +86,19 @@ def test_bf16_conv_workspace_holds_the_sums_of_every_route_that_needs_them():
     for which in (capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA):
         filt, part = need(which, 2, 1, 128, 128, 9, 72)
         assert l.adh_conv3x3_workspace_bytes(which, capi.ADH_BF16, 2, 1, 128, 128, 9, 72) == filt
+
+
+@pytest.mark.skipif(torch.cuda.is_available(), reason="the call would be launched, on addresses that are none")
+def test_bf16_filter_gradient_takes_copies_beyond_32_bit_counts():
+    """2^31 granules and more of an odd width's copy (tiles above 34 GB) are no error of the arguments: without a GPU it is the
+    launch that fails."""
+    l = capi.lib()
+    K, N, Cin, Cout, H, W = 1, 1 << 14, 512, 8, 1022, 13  # 2^33 rows of three granules
+    xs, keep = capi.ptr_table([0x10000])
+    nbytes = l.adh_conv3x3_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_BF16, K, N, Cin, Cout, H, W)
+    assert nbytes > 1 << 34
+    rc = l.adh_conv3x3_slab_bwd_filter_tiles(capi.ADH_BF16, K, N, Cin, Cout, H, W, xs, xs, 0x10000, 0.0, 0x10000, nbytes, None)
+    assert rc > 0
 
 
 def test_the_choice_of_a_tile_is_made_in_microseconds():
