@@ -124,7 +124,7 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
                                       uint32_t W, bool may_copy);
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree, bool may_copy);
+                   size_t workspace_bytes, hipStream_t st, bool halofree);
 
 bool conv_bf16_wgrad_mfma_supported(uint32_t Cin, uint32_t Cout, uint32_t W);
 size_t conv_bf16_wgrad_mfma_workspace_bytes(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t W);
@@ -211,10 +211,10 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
   if (N == 0 || Cin == 0 || Cout == 0 || H == 0 || W == 0) return ADH_OK;
   if (!in_tiles || !out_tiles || !w) return ADH_ENULL;
   if (!aligned_to(w, 2)) return ADH_EALIGN;
-  // a workspace without room for the copy of the input at odd widths does for the kernels that need none
+  // a workspace without room for copies of the input at odd widths does for the kernels that need none
   const bool mfma = conv_bf16_mfma_supported(which, Cin, Cout, H, W);
-  const size_t full = bf16_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
-  const size_t need = mfma ? conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false) : full;
+  const size_t need = mfma ? conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false)
+                           : bf16_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
@@ -227,8 +227,7 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
     const uint64_t cmax = Cin > Cout ? Cin : Cout;
     if (cmax * (H + 2ull) * (W + 2ull) * 2u >= (1ull << 31) || (uint64_t)Cin * Cout * 18u >= (1ull << 31))
       return ADH_EINVAL;
-    return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, false,
-                          workspace_bytes >= full);
+    return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, workspace_bytes, st, false);
   }
   const uint64_t slab = (uint64_t)N * Cin * (H + 2) * (W + 2), outn = (uint64_t)N * Cout * H * W;
   const uint64_t in_elems = which == ADH_CONV_FWD ? slab : outn;

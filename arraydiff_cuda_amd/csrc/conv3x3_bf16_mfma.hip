@@ -655,15 +655,39 @@ static size_t part_region_bytes(int which, uint32_t N, uint32_t Cin, uint32_t Co
   const uint64_t oh = which == ADH_CONV_FWD ? H : H + 2ull, ow = which == ADH_CONV_FWD ? W : W + 2ull;
   return (size_t)((N * cout_k * oh * ow * 4u + 255u) / 256u * 256u);
 }
-// may_copy: with room for the copy of the input with wider rows where there is a route over one
+// The copies with wider rows are made and used some images at a time, those of every tile or, where an image of each is too much,
+// of some tiles: as many as fit, one at least.  A workspace may hold 512 MiB of them (and their fp32 sums) and does with 64.
+// 128 -> 128 channels, 8 images of 4 tiles of 64x255 (136 MB of copies), forward: 207 us at once, 226 in 128 MiB, 277 in 64, 358
+// in 32, and 455 without copies; 32 images 836, 826 in 512 MiB, 864 in 256; 512 -> 64, 64 images of 6 tiles of 64x33 (1.2 GB)
+// 1830, 2130 in 512 MiB: the images of a turn have to go round the compute units.
+constexpr uint64_t kMostCopies = 512ull << 20, kLeastCopies = 64ull << 20;
+struct CopyTurn {
+  uint32_t tiles, images;
+  uint64_t bytes;
+};
+static CopyTurn conv_bf16_copy_turn(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
+                                    uint64_t room) {
+  const bool sums = conv_bf16_launches(which, Cin, Cout, H, W) > 1u;
+  auto bytes = [&](uint32_t images) {
+    return (uint64_t)conv_bf16_repitch_bytes(which, images, Cin, Cout, H, W) + (sums ? part_region_bytes(which, images, Cin, Cout, H, W) : 0u);
+  };
+  CopyTurn t = {num_tiles, N, 0u};
+  if (bytes(1u) * num_tiles > room) {
+    t.tiles = (uint32_t)std::max<uint64_t>(1u, room / bytes(1u));
+    t.images = 1u;
+  } else {
+    const uint32_t most = (uint32_t)std::min<uint64_t>(N, room / (bytes(1u) * num_tiles)), turns = (N + most - 1u) / most;
+    t.images = (N + turns - 1u) / turns;
+  }
+  t.bytes = t.tiles * bytes(t.images);
+  return t;
+}
+// may_copy: with room for copies of the input with wider rows where there is a route over them
 size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
                                       uint32_t W, bool may_copy) {
-  auto sums = [&](bool copies) {
-    return conv_bf16_launches(which, Cin, Cout, H, W, copies) > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : (size_t)0;
-  };
-  size_t bytes = sums(false);
+  size_t bytes = conv_bf16_launches(which, Cin, Cout, H, W, false) > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : (size_t)0;
   if (may_copy && conv_bf16_repitches(which, Cin, Cout, H, W))
-    bytes = std::max(bytes, sums(true) + num_tiles * conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W));
+    bytes = std::max<size_t>(bytes, conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, kMostCopies).bytes);
   return filter_region_bytes(which, Cin, Cout) + bytes;
 }
 
@@ -673,10 +697,10 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
 // and a tile's rows -1 and H are its neighbours' last and first rows (zeros at the tensor's own border): the
 // unsplit convolution with zero padding, restricted to the tile.  Only shapes the eight-wave kernel takes
 // (ADH_EUNIMPL otherwise).
-// may_copy: the workspace has room for a copy of the input with wider rows.
-int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
-                   const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                   hipStream_t st, bool halofree, bool may_copy) {
+// may_copy: the workspace has room for copies of the tiles with wider rows.  filter_ready: it holds the reordered filter already.
+static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
+                               const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
+                               hipStream_t st, bool halofree, bool may_copy, bool filter_ready) {
   ConvBf16Params P = {};
   for (uint32_t t = 0; t < num_tiles; ++t) {
     P.in[t] = reinterpret_cast<const uint16_t *>(in_tiles[t]);
@@ -728,7 +752,7 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
   // the forward pass of the eight-wave kernel can read the caller's filter itself
   const bool direct = which == ADH_CONV_FWD && (Cin % 64u) == 0u && aligned_to(w, 16) && (P.IW % 2u) == 0u;
   int e = ADH_OK;
-  if (!direct) {
+  if (!direct && !filter_ready) {
     const uint32_t total = groups * P.passes * kWtGroupElems;
     hipLaunchKernelGGL(conv3x3_bf16_filter_kernel, dim3((total + 255u) / 256u), dim3(256), 0, st,
                        reinterpret_cast<const uint16_t *>(w), reinterpret_cast<uint16_t *>(workspace), Cin, Cout,
@@ -832,6 +856,33 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
   return conv_bf16_w4_launch(P, gx, groups, st);
 }
 
+int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
+                   const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
+                   size_t workspace_bytes, hipStream_t st, bool halofree) {
+  const uint64_t room = workspace_bytes > filter_region_bytes(which, Cin, Cout) ? workspace_bytes - filter_region_bytes(which, Cin, Cout) : 0u;
+  if (halofree || !conv_bf16_repitches(which, Cin, Cout, H, W) ||
+      room < conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, kLeastCopies).bytes)
+    return conv_bf16_mfma_some(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, halofree, false, false);
+  const CopyTurn turn = conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, std::min<uint64_t>(room, kMostCopies));
+  const uint64_t slab = (H + 2ull) * (W + 2ull) * 2u, inner = (uint64_t)H * W * 2u;  // bytes of a channel
+  const uint64_t in_image = which == ADH_CONV_FWD ? Cin * slab : Cout * inner, out_image = which == ADH_CONV_FWD ? Cout * inner : Cin * slab;
+  bool filter_ready = false;
+  for (uint32_t t = 0; t < num_tiles; t += turn.tiles)
+    for (uint32_t n = 0; n < N; n += turn.images) {
+      const uint32_t tiles = std::min(turn.tiles, num_tiles - t), images = std::min(turn.images, N - n);
+      const void *in[ADH_MAX_TILES];
+      void *out[ADH_MAX_TILES];
+      for (uint32_t k = 0; k < tiles; ++k) {
+        in[k] = reinterpret_cast<const char *>(in_tiles[t + k]) + n * in_image;
+        out[k] = reinterpret_cast<char *>(out_tiles[t + k]) + n * out_image;
+      }
+      const int e = conv_bf16_mfma_some(which, tiles, images, Cin, Cout, H, W, in, w, out, beta, workspace, st, false, true, filter_ready);
+      if (e) return e;
+      filter_ready = true;
+    }
+  return ADH_OK;
+}
+
 }  // namespace adh
 
 // ---------------------------------------------------------------------------
@@ -898,8 +949,8 @@ extern "C" int adh_conv3x3_slab_fwd_tiles_static(int dtype, uint32_t num_tiles, 
   void *ws = nullptr;
   const int e = static_scratch(&ws);
   if (e) return e;
-  return conv_bf16_mfma(ADH_CONV_FWD, num_tiles, N, Cin, Cout, H, W, x_pad_tiles, w, y_tiles, beta, ws, as_stream(stream),
-                        false, false);
+  return conv_bf16_mfma(ADH_CONV_FWD, num_tiles, N, Cin, Cout, H, W, x_pad_tiles, w, y_tiles, beta, ws, kStaticScratchBytes,
+                        as_stream(stream), false);
 }
 
 // ---------------------------------------------------------------------------
@@ -929,6 +980,6 @@ int conv_bf16_unpadded(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
-  return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, true, false);
+  return conv_bf16_mfma(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, workspace_bytes, st, true);
 }
 }  // namespace adh

@@ -147,10 +147,11 @@ int adh_tiles_unpack_nchw(int dtype, uint32_t K, uint32_t halo_pad, uint32_t W, 
  *     with the sums in registers when there are also more than 64 output channels (fp32 sums pass through
  *     the workspace only between such launches: 256 channels are two), else 64 per launch;
  *   - more than 64 reduction channels at any other width (odd; backward-data at a width that is no multiple
- *     of 8): the same kernels over a copy of the input with rows of the next multiple of 8 in the workspace
- *     (128 -> 128 channels on 64 x 255 tiles 740-790 TFLOP/s, the copy included).  In a workspace that holds the
- *     reordered filter and the fp32 sums but not the copy: the four-wave matrix-core kernel once per 64
- *     reduction channels, 340-430 TFLOP/s there.  Tiles off the alignment above take that kernel too when the
+ *     of 8): the same kernels over copies of the input with rows of the next multiple of 8 in the workspace
+ *     (128 -> 128 channels on 64 x 255 tiles 740-790 TFLOP/s, the copies included), made for as many images at a
+ *     time as it holds: the query asks for 512 MiB at most, 64 MiB (or one image) do with slower turns.  In a
+ *     workspace that holds the reordered filter and the fp32 sums but not that: the four-wave matrix-core kernel
+ *     once per 64 reduction channels, 340-430 TFLOP/s there.  Tiles off the alignment above take that kernel too when the
  *     reduction needs more than one launch anyway; where the width promises ONE launch of 128 channels the
  *     workspace has no room for the sums and the call returns ADH_EALIGN;
  *   - the sums of one image beyond 2 GiB (Cout * H * W * 4 bytes): the tensors are widened to fp32 in the

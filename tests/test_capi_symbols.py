@@ -88,6 +88,20 @@ def test_bf16_conv_workspace_holds_the_sums_of_every_route_that_needs_them():
         assert l.adh_conv3x3_workspace_bytes(which, capi.ADH_BF16, 2, 1, 128, 128, 9, 72) == filt
 
 
+def test_bf16_conv_workspace_does_not_hold_every_copy_of_an_odd_width():
+    """The copies of the input with wider rows, and their sums, are made some images at a time: 512 MiB of them, or one image."""
+    l = capi.lib()
+    for (K, N, Cin, Cout, H, W) in [(6, 128, 1, 512, 64, 33), (8, 64, 128, 128, 64, 255), (2, 3, 512, 1, 128, 501), (2, 40, 512, 512, 128, 501)]:
+        for which in (capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA):
+            cred, cout = (Cin, Cout) if which == capi.ADH_CONV_FWD else (Cout, Cin)
+            oh, ow = (H, W) if which == capi.ADH_CONV_FWD else (H + 2, W + 2)
+            filt = ((cout + 63) // 64) * ((cred + 63) // 64) * 9 * 2 * 64 * 32 * 2
+            sums = (N * cout * oh * ow * 4 + 255) // 256 * 256
+            image = cred * (H + 2) * ((W + 2 + 7) // 8 * 8) * 2 + cout * oh * ow * 4 + 512
+            got = l.adh_conv3x3_workspace_bytes(which, capi.ADH_BF16, K, N, Cin, Cout, H, W)
+            assert got <= filt + max(K * sums, 512 << 20, image), (which, K, N, Cin, Cout, H, W, got)
+
+
 @pytest.mark.skipif(torch.cuda.is_available(), reason="the call would be launched, on addresses that are none")
 def test_bf16_filter_gradient_takes_copies_beyond_32_bit_counts():
     """2^31 granules and more of an odd width's copy (tiles above 34 GB) are no error of the arguments: without a GPU it is the

@@ -40,3 +40,41 @@ def test_a_workspace_without_room_for_the_copy(oracle, which, K, N, Cin, Cout, H
         got.append(torch.cat(outs).float())
     # both round one fp32 sum of the same products to bf16
     assert (got[0] - got[1]).abs().max().item() <= 2 ** -7 * got[1].abs().max().item()
+
+
+@pytest.mark.parametrize("which,K,N,Cin,Cout,H,W", [("fwd", 2, 9, 320, 66, 64, 255), ("bwd", 2, 5, 66, 320, 64, 255),  # images in turn
+                                                    ("fwd", 3, 2, 320, 65, 64, 501),  # two tiles, then one
+                                                    ("bwd", 2, 1, 1, 144, 120, 2043)])  # a tile at a time, each larger than the least room
+def test_copies_in_turn(which, K, N, Cin, Cout, H, W):
+    """A workspace with room for some of the copies: every image's bits are those of a call for it alone, and nothing is written
+    past the workspace."""
+    fwd = which == "fwd"
+    g = torch.Generator(device="cuda").manual_seed(4)
+    bf = lambda shape: torch.randn(shape, generator=g, device="cuda").to(torch.bfloat16)
+    w = bf((Cout, Cin, 3, 3))
+    ins = [bf((N, Cin, H + 2, W + 2) if fwd else (N, Cout, H, W)) for _ in range(K)]
+    olds = [bf((N, Cout, H, W) if fwd else (N, Cin, H + 2, W + 2)) for _ in range(K)]
+    code = capi.ADH_CONV_FWD if fwd else capi.ADH_CONV_BWD_DATA
+    query = lambda k, n: capi.conv_workspace_bytes(code, capi.ADH_BF16, k, n, Cin, Cout, H, W)
+
+    def run(ins, outs, n, nbytes):
+        ws = torch.full((nbytes // 4 + 64,), 7.0, device="cuda")
+        if fwd:
+            capi.check(capi.conv_fwd_tiles(ins, w, outs, n, Cin, Cout, H, W, beta=1.0, ws=ws[:nbytes // 4]), "fwd")
+        else:
+            capi.check(capi.conv_bwd_data_tiles(w, ins, outs, n, Cin, Cout, H, W, beta=1.0, ws=ws[:nbytes // 4]), "bwd-data")
+        assert (ws[nbytes // 4:] == 7.0).all()
+
+    cred, cout, oh, ow = (Cin, Cout, H, W) if fwd else (Cout, Cin, H + 2, W + 2)
+    filt = ((cout + 63) // 64) * ((cred + 63) // 64) * 9 * 2 * 64 * 32 * 2
+    sums = K * ((N * cout * oh * ow * 4 + 255) // 256 * 256)
+    least = filt + max(sums, 64 << 20, query(1, 1) - filt)
+    got, all_at_once = [t.clone() for t in olds], [t.clone() for t in olds]
+    run(ins, all_at_once, N, query(K, N))
+    run(ins, got, N, least)
+    for k in range(K):
+        assert torch.equal(got[k], all_at_once[k])
+        for n in range(N):
+            alone = olds[k][n:n + 1].clone()
+            run([ins[k][n:n + 1].clone()], [alone], 1, query(1, 1))
+            assert torch.equal(got[k][n:n + 1], alone), (k, n)
