@@ -13,6 +13,8 @@
 //     three slots: one barrier a step, and the first operands of a step are fetched in the one before.
 //   * What a step has to do besides multiplying is dealt out between its groups of NT MFMAs.  Done in one piece at the
 //     step's start, both waves of a SIMD stood in it at once (212 TFLOP/s, 256 channels on 8 x 32 tiles; 232 dealt out).
+//   * The products below h*h are summed apart from it, or for some taps, as the registers allow (LOW below): additions at the
+//     size of the whole sum, six a tap, would cost digits that fp32 sums have.
 //   * The workgroups are persistent and the sequence of chunks runs on across their blocks: the next block's first patch
 //     and filter rows arrive during the last steps of this one.
 // Row tiles of one tensor are addressed as that tensor: a patch row is divided by the tile height to find its tile, so a
@@ -44,6 +46,7 @@ constexpr uint32_t kSpChunk = 32;  // channels per staged chunk
 constexpr uint32_t kSpPP = 640;    // patch pixels per plane in LDS
 // a block's patch pixels; quads have few (and four sets of sums: what is staged for more pixels would be spilled)
 constexpr uint32_t split_patch(int sample) { return sample == kUp ? 384u : kSpPP; }
+constexpr int kLowApart = 10;
 constexpr uint32_t kSpMP = 68;     // filter rows per plane: = 4 (mod 16), so that the octet planes start 64 bytes apart
 
 struct SplitParams {
@@ -93,7 +96,12 @@ struct SplitBlock {
 //   kUp, backward-data: a block owns quads, the 2 x 2 gradient pixels at (2i, 2j), which tap (1 +- a, 1 +- b) of the filter feeds
 //     from dy[i .. i + 1][j .. j + 1]: nine taps over a patch of (BR + 1) x (BC + 1), into four sets of sums.  A lane's four
 //     neighbouring quads are two rows of eight pixels.
-template <int MT, int NT, bool VEC, int SAMPLE>
+//
+// LOW.  Six products of parts go into a sum per tap and chunk, and each addition is rounded at the size of the sum; all but h*h
+// are below 2^-8 of it.  kLowApart: they have sums of their own, added at the block's end, and cost no digit.  Where registers
+// are short, the small products of LOW of the nine taps are summed up from zero and added at once; 0: every product is added
+// by itself.  The choice hangs on the channels alone, so that all tiles give the same bits (split_low).
+template <int MT, int NT, bool VEC, int SAMPLE, int LOW>
 __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const SplitParams P) {
   constexpr uint32_t MW = 16u * MT;
   constexpr int SETS = SAMPLE == kUp ? 4 : 1;  // of sums
@@ -104,6 +112,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   __shared__ __align__(16) uintx4 wl[3 * SLOT];
   __shared__ const float *tab[3 * ADH_MAX_TILES];  // the tiles' addresses: in, out, res
   __shared__ uint32_t not_finite;
+  constexpr bool APART = LOW == kLowApart;
   constexpr int FIRST = SAMPLE == kUnit ? 3 : 0;  // step whose side work loads the next patch's first unit
   const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
@@ -276,6 +285,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   };
   auto tap_set = [](int t) { return SAMPLE == kUp ? (t / 3 == 1 ? 0 : 2) + (t % 3 == 1 ? 0 : 1) : 0; };
   floatx4 acc[SETS][MT][NT];
+  floatx4 low[APART ? SETS : 1][APART ? MT : 1][NT];
   const uintx4 *const a_lane = wl + g * kSpMP + l16;
 
   // ---- results ----
@@ -437,6 +447,14 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
         for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
           for (int q = 0; q < NT; ++q) acc[s][mt][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (APART) {
+#pragma unroll
+        for (int s = 0; s < SETS; ++s)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int q = 0; q < NT; ++q) low[s][mt][q] = floatx4{0.f, 0.f, 0.f, 0.f};
+      }
     }
 #pragma unroll
     for (int k = 0; k < 3; ++k) a[0][k] = a_lane[k * 4 * kSpMP];
@@ -479,12 +497,24 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
                                         : a_lane[((t + 1) % 3) * SLOT + k * 4 * kSpMP];
         }
         auto &sum = acc[tap_set(t)];
-        auto products = [&](auto nth, int ka, int kb) {
+        constexpr bool ONCE = !APART && (LOW == 9 || (t < 2 * LOW && t % 2 == 0));  // this tap's small products are added once
+        auto products = [&](auto group, int ka, int kb) {
+          constexpr int nth = decltype(group)::value;
 #pragma unroll
-          for (int q = 0; q < NT; ++q)
-            sum[mt][q] = VEC ? mfma_bf16(b[q][kb], a[cur][ka], sum[mt][q]) : mfma_bf16(a[cur][ka], b[q][kb], sum[mt][q]);
+          for (int q = 0; q < NT; ++q) {
+            floatx4 &to = (APART || ONCE) && ka + kb > 0 ? low[APART ? tap_set(t) : 0][APART ? mt : 0][q] : sum[mt][q];
+            if (ONCE && nth == 0) to = floatx4{0.f, 0.f, 0.f, 0.f};
+            to = VEC ? mfma_bf16(b[q][kb], a[cur][ka], to) : mfma_bf16(a[cur][ka], b[q][kb], to);
+          }
+          if constexpr (ONCE && nth == 5) {
+#pragma unroll
+            for (int q = 0; q < NT; ++q) {
+              sum[mt][q] += low[0][0][q];
+              asm volatile("" : "+v"(sum[mt][q]));  // (stays where it is: moved about, the sums are spilled)
+            }
+          }
           __builtin_amdgcn_sched_barrier(0);
-          side(std::integral_constant<int, mt * 6 + decltype(nth)::value>{});
+          side(std::integral_constant<int, mt * 6 + nth>{});
           __builtin_amdgcn_sched_barrier(0);
         };
         auto refill = [&](int kb) {  // the last use of this part of the pixels is behind: fetch the next tap's
@@ -500,13 +530,21 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
         products(std::integral_constant<int, 2>{}, 0, 1);
         refill(1);
         products(std::integral_constant<int, 3>{}, 2, 0);
-        products(std::integral_constant<int, 4>{}, 1, 0);
-        products(std::integral_constant<int, 5>{}, 0, 0);
+        products(std::integral_constant<int, 4>{}, ONCE ? 0 : 1, 0);  // (the small products' sum is waited for, not h*h's)
+        products(std::integral_constant<int, 5>{}, ONCE ? 1 : 0, 0);
         refill(0);
       });
       if (t < 8) lds_barrier();
     });
     if (last) {
+      if constexpr (APART) {
+#pragma unroll
+        for (int s = 0; s < SETS; ++s)
+#pragma unroll
+          for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+            for (int q = 0; q < NT; ++q) acc[s][mt][q] += low[s][mt][q];
+      }
       settle_x();
       if (not_finite == 0u) emit_all(B);
       else emit_plain(B);
@@ -529,9 +567,22 @@ __global__ __launch_bounds__(256) void conv3x3_split_reduce_kernel(const SplitPa
 
 // ---- host side ----
 
+// How the small products are summed (see LOW), by the relative error against double precision over that of sums of
+// v_mfma_f32_16x16x4_f32, for inputs that are uniform in [-1, 1] / normal and rectified.  64 channels: each product by itself 0.83 / 1.12,
+// four taps at once 0.68 / 0.91, nine 0.35 / 0.43, apart 0.30 / 0.34; 16 channels, whose chunk has as many additions for half the
+// terms: 1.11 / 1.46, 0.93 / 1.23, 0.43 / 0.55, 0.33 / 0.38; one channel, by itself 2.2 / 1.8, apart 0.51 / 0.64.  Backward-data at
+// stride 2: 64 channels by itself 0.37 / 0.37, 16 channels 0.96 / 0.98, three 1.95 / 1.47.
+// 64 -> 64 channels on 32 x 128 tiles (32 images, 4 tiles): by itself 215 us, four taps 215, nine 235, apart (half the tile, for the
+// registers) 260.
+static int split_low(SplitSample sample, uint32_t C, uint32_t nchunks) {
+  if (sample == kDown) return kLowApart;  // (one set of sums, and the registers for two)
+  if (sample == kUp) return C < 16u ? kLowApart : 0;
+  return C <= 4u ? kLowApart : 8u * C >= 7u * kSpChunk * nchunks ? 4 : 9;
+}
+
 struct SplitPlan {
   SplitParams P;
-  int MT, NT;
+  int MT, NT, low;
   bool vec;
   size_t part_bytes;
 };
@@ -566,6 +617,7 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
   P.pad_r = q.pad_r; P.pad_c = q.pad_c; P.dil = q.dil; P.flip = q.flip ? 1 : 0;
   P.beta = q.beta;
   P.nchunks = (P.C + kSpChunk - 1u) / kSpChunk;
+  plan->low = split_low(q.sample, P.C, P.nchunks);
   const double out_bytes = 4.0 * P.num_tiles * P.N * P.M * P.out_H * P.out_W;
   const uint32_t pixels = split_patch(q.sample);
   // extent of the patch of n pixels, and how many pixels one of n holds
@@ -578,6 +630,7 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
     const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
     for (int NT = q.sample == kDown ? 1 : 4; NT >= 1; NT /= 2) {
       if (q.sample == kUp && NT == 4 && MT > 1) continue;  // (four sets of sums)
+      if (plan->low == kLowApart && (q.sample == kUnit ? NT != 2 : q.sample == kUp && MT * NT > 2)) continue;  // (the registers)
       const uint32_t slots = 128u * NT;
       const double matrix = 192.0 * MT * NT;
       const double chunk = 9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT;
@@ -656,29 +709,32 @@ size_t conv3x3_split_workspace(const Conv3x3Problem &q) {
 void conv3x3_split_name(const Conv3x3Problem &q, char *name, size_t name_bytes) {
   SplitPlan plan = {};
   if (split_plan(q, false, &plan)) plan.MT = plan.NT = 0;
-  snprintf(name, name_bytes, "conv3x3_split_kernel<%d, %d, %s, %d>", plan.MT, plan.NT, plan.vec ? "true" : "false", (int)q.sample);
+  snprintf(name, name_bytes, "conv3x3_split_kernel<%d, %d, %s, %d, %d>", plan.MT, plan.NT, plan.vec ? "true" : "false", (int)q.sample, plan.low);
 }
 
-template <int MT, int NT, int SAMPLE>
+template <int MT, int NT, int SAMPLE, int LOW>
 static void launch_split(const SplitPlan &plan, hipStream_t st) {
   const dim3 grid(std::min(plan.P.xcd_chunk, 32u) * 8u), block(kSpThreads);
-  if (plan.vec) hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, true, SAMPLE>), grid, block, 0, st, plan.P);
-  else hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, false, SAMPLE>), grid, block, 0, st, plan.P);
+  if (plan.vec) hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, true, SAMPLE, LOW>), grid, block, 0, st, plan.P);
+  else hipLaunchKernelGGL((conv3x3_split_kernel<MT, NT, false, SAMPLE, LOW>), grid, block, 0, st, plan.P);
 }
 template <int MT>
 static void launch_split_nt(const SplitPlan &plan, SplitSample sample, hipStream_t st) {
+  const bool apart = plan.low == kLowApart;
   if (sample == kDown) {
-    launch_split<MT, 1, kDown>(plan, st);
+    launch_split<MT, 1, kDown, kLowApart>(plan, st);
   } else if (sample == kUp) {
-    if (MT == 1 && plan.NT == 4) launch_split<1, 4, kUp>(plan, st);
-    else if (plan.NT == 2) launch_split<MT, 2, kUp>(plan, st);
-    else launch_split<MT, 1, kUp>(plan, st);
+    if (MT == 1 && plan.NT == 4) launch_split<1, 4, kUp, 0>(plan, st);
+    else if (plan.NT == 2) apart ? launch_split<1, 2, kUp, kLowApart>(plan, st) : launch_split<MT, 2, kUp, 0>(plan, st);
+    else apart ? launch_split<MT == 4 ? 2 : MT, 1, kUp, kLowApart>(plan, st) : launch_split<MT, 1, kUp, 0>(plan, st);
+  } else if (apart) {
+    launch_split<MT, 2, kUnit, kLowApart>(plan, st);
   } else if (plan.NT == 4) {
-    launch_split<MT, 4, kUnit>(plan, st);
+    plan.low == 4 ? launch_split<MT, 4, kUnit, 4>(plan, st) : launch_split<MT, 4, kUnit, 9>(plan, st);
   } else if (plan.NT == 2) {
-    launch_split<MT, 2, kUnit>(plan, st);
+    plan.low == 4 ? launch_split<MT, 2, kUnit, 4>(plan, st) : launch_split<MT, 2, kUnit, 9>(plan, st);
   } else {
-    launch_split<MT, 1, kUnit>(plan, st);
+    plan.low == 4 ? launch_split<MT, 1, kUnit, 4>(plan, st) : launch_split<MT, 1, kUnit, 9>(plan, st);
   }
 }
 

@@ -34,7 +34,8 @@ __device__ __forceinline__ floatx4 buffer_load4(__amdgpu_buffer_rsrc_t r, uint32
 //   * A workgroup of four waves owns 16 MT x (1 or 2) output channels; the filter stays in registers (4 MT x Q x 3) over all the
 //     tiles of 8x32 (16 x 16; half at stride 2) pixels it walks.  Two workgroups per compute unit: one stages while the
 //     other multiplies, and a tile's values are on their way in registers while the one before is multiplied.
-//   * Per pair of 16-pixel units and step a wave reads 6 operands for 12 MT MFMAs.
+//   * Per pair of 16-pixel units and step a wave reads 6 operands for 12 MT MFMAs.  The products below h*h have sums of their own:
+//     in one sum the error against double precision was 0.82 (rectified inputs 1.12, 3x3 1.35) of the v_mfma_f32 kernel's, now 0.31 (0.37, 0.48).
 // Measured (64 channels; the v_mfma_f32 kernel of conv_thin.hip before): 7x7 over 3 channels, 32 images of 4 tiles of 64x256 398 -> 261 us
 // (151 TFLOP/s), 7x7 / 2 on 56x112 236 -> 115; 3x3, 16 images of 32x128 75 -> 27; one image of 14x14 36 -> 10 (37 filter values a thread
 // loaded in two batches instead of one by one: 19 -> 10).  Bound by the matrix cores, busy for 150 us of the first; a wave
@@ -225,7 +226,7 @@ __global__ __launch_bounds__(kTsThreads, 2) void conv_thin_split_fwd_kernel(cons
     }
     // a pair of units: its sums (false: below the last row), and their way out
     uint32_t row[2], col[2];
-    floatx4 acc[2][MT];
+    floatx4 acc[2][MT];  // h*h of the parts; the small products have sums of their own, whose additions cost no digit of these
     auto sum = [&](uint32_t pi) {
       uint32_t at[2], key[2];
 #pragma unroll
@@ -237,10 +238,11 @@ __global__ __launch_bounds__(kTsThreads, 2) void conv_thin_split_fwd_kernel(cons
         key[u] = r * P.sh + 2u * cu;
       }
       if (pi >= P.pairs || row[0] >= P.OH) return false;
+      floatx4 low[2][MT];
 #pragma unroll
       for (int u = 0; u < 2; ++u)
 #pragma unroll
-        for (int mt = 0; mt < MT; ++mt) acc[u][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
+        for (int mt = 0; mt < MT; ++mt) acc[u][mt] = low[u][mt] = floatx4{0.f, 0.f, 0.f, 0.f};
       uint32_t zero = 0u;  // (opaque: an address per step, worked out once for all tiles, is more registers than there are)
       asm volatile("" : "+v"(zero));
 #pragma unroll
@@ -260,8 +262,15 @@ __global__ __launch_bounds__(kTsThreads, 2) void conv_thin_split_fwd_kernel(cons
 #pragma unroll
           for (int u = 0; u < 2; ++u)
 #pragma unroll
-            for (int mt = 0; mt < MT; ++mt) acc[u][mt] = mfma_bf16(b[u][xp[k]], wreg[mt][q][wpt[k]], acc[u][mt]);
+            for (int mt = 0; mt < MT; ++mt) {
+              floatx4 &to = k < 5 ? low[u][mt] : acc[u][mt];
+              to = mfma_bf16(b[u][xp[k]], wreg[mt][q][wpt[k]], to);
+            }
       }
+#pragma unroll
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int mt = 0; mt < MT; ++mt) acc[u][mt] += low[u][mt];
       return true;
     };
     // a lane holds pixels 4 g .. 4 g + 3 of each unit for channel l16 of each channel tile

@@ -4,9 +4,12 @@
 // bf16 values, x = h + m + l: each is the rounding of what the ones before it leave, 8 + 8 + 8 significant bits.  Products
 // of bf16 values are exact in the matrix cores and their sums are fp32.  Of the nine products of two such sums the six down
 // to h*l, l*h and m*m are formed; the other three are below 2^-24 of |x*w|, less than the rounding of one fp32 product.
-// Measured against double precision on dot products of 64, 576 and 4608 terms (uniform times normal values) the relative
-// error is 1.1e-7, 3.6e-7 and 1.08e-6, where v_mfma_f32_16x16x4_f32 has 1.4e-7, 4.3e-7 and 1.22e-6: the matrix core rounds
-// once per 32 terms and product, the fp32 one once per term.  All nine products change no digit of these.
+// The matrix core rounds its sum once per 32 terms and product, the fp32 one once per term.  Six roundings at the size of the
+// sum are more than fp32's where few of the 32 terms exist, and where many are zero (rectified inputs); five of them belong
+// to products that are below 2^-8 of the sixth.  The kernels therefore sum those by themselves as far as registers allow.
+// Relative error against double precision over that of v_mfma_f32_16x16x4_f32 sums, uniform / rectified inputs:
+// convolution 0.68 / 0.91 at full chunks of 32 channels, 0.3 - 0.5 at others, 0.3 - 0.6 at stride 2 and in the stem; the filter
+// gradients, whose terms are pixels and always many, 0.6 - 0.8 / 0.8 - 1.0 with all six in one sum.
 // Values to take care of: one whose leading part is not finite (an infinity, or a number within half a bf16 step of the
 // largest one) has inf - inf = NaN in its parts, and a NaN times the zero of a place that does not exist is one.  The kernels
 // note such values, or sums that came out as NaN, and compute what they touch over again in plain fp32 from what exists.

@@ -120,8 +120,8 @@ def test_the_choice_of_a_tile_is_made_in_microseconds():
     rows while every tile was priced).  The best of many repetitions, with room for a slow host."""
     l = capi.lib()
     name = ctypes.create_string_buffer(256)
-    kernels = {(4, 32, 64, 64, 32, 128): b"<4, 4, true, 0>", (4, 32, 512, 512, 4, 16): b"<4, 2, true, 0>", (8, 2, 64, 64, 128, 2048): b"<4, 4, true, 0>",
-               (7, 3, 272, 40, 61, 1013): b"<4, 4, false, 0>", (4, 32, 64, 64, 14, 56): b"<4, 4, true, 0>"}
+    kernels = {(4, 32, 64, 64, 32, 128): b"<4, 4, true, 0, 4>", (4, 32, 512, 512, 4, 16): b"<4, 2, true, 0, 4>", (8, 2, 64, 64, 128, 2048): b"<4, 4, true, 0, 4>",
+               (7, 3, 272, 40, 61, 1013): b"<4, 4, false, 0, 4>", (4, 32, 64, 64, 14, 56): b"<4, 4, true, 0, 4>"}
     for (K, N, Cin, Cout, H, W), kernel in kernels.items():
         args = [capi.ADH_CONV_FWD, capi.ADH_F32, K, N, Cin, Cout, H, W, 0.0, name, 256]
         best = 1e9
