@@ -586,7 +586,7 @@ int conv1x1_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cou
                       float *dwt, float beta, void *workspace, hipStream_t st);
 
 // conv3x3s2.hip: filter gradient of a 3x3 window at stride 2, padding 1, over fp32 tiles of H x W without halo, and its
-// forward for many input channels
+// forward for launches that would leave the split kernel's last round idle
 int conv3x3s2_fwd_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                       const void *const *x_tiles, const void *w, void *const *y_tiles, float beta, hipStream_t st);
 size_t conv3x3s2_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
@@ -1277,18 +1277,20 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     if (e == ADH_OK && bias_tiles && bias_added) *bias_added = true;
     if (e != ADH_EUNIMPL) return e;
   }
-  if (gen_is_3x3s2_unpadded(dtype, g, unpadded, pad_h, pad_w)) {
-    e = gen_check_workspace(plan, workspace, workspace_bytes);
-    if (e) return e;
-    e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
-    if (e != ADH_EUNIMPL) return e;
-  }
   if (gen_is_3x3_split(dtype, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = x_tiles; q.out = y_tiles; q.w = w;
+    // Stride 2: the two kernels stand as 0.85 - 0.91 to 1 in time where the split one's rounds are full, from 64 to 1024 channels
+    // on either side; its blocks are coarse, and with more than an eighth of the rounds idle the fp32 one is ahead (of full
+    // rounds: 9/16 1.08 - 1.13, 3/4 1.08 - 1.15, 5/6 1.06, 9/10 0.97 - 1.0).  A single round is the split one's: 0.15 - 0.85 with
+    // chunks dealt out.
+    if (g.sh == 2u && conv3x3_split_idles(q)) {
+      e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
+      if (e != ADH_EUNIMPL) return e;
+    }
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }

@@ -706,6 +706,13 @@ size_t conv3x3_split_workspace(const Conv3x3Problem &q) {
   return split_plan(q, true, &plan) ? 0u : (plan.part_bytes + 255u) & ~(size_t)255u;
 }
 
+bool conv3x3_split_idles(const Conv3x3Problem &q) {
+  SplitPlan plan = {};
+  if (split_plan(q, false, &plan)) return false;
+  const uint32_t rounds = (plan.P.blocks + 255u) / 256u;
+  return rounds > 1u && (rounds * 256u - plan.P.blocks) * 8u > rounds * 256u;
+}
+
 void conv3x3_split_name(const Conv3x3Problem &q, char *name, size_t name_bytes) {
   SplitPlan plan = {};
   if (split_plan(q, false, &plan)) plan.MT = plan.NT = 0;

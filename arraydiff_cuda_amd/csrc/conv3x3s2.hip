@@ -1,5 +1,5 @@
-// 3x3 convolution at stride 2 with padding 1 over row tiles WITHOUT halo, fp32 matrix cores: forward from 512 input channels on,
-// and backward-filter (the other cases are conv3x3_split.hip's).
+// 3x3 convolution at stride 2 with padding 1 over row tiles WITHOUT halo, fp32 matrix cores: forward (where
+// conv3x3_split.hip's larger blocks would leave its last round idle) and backward-filter.
 #include "adh_common.h"
 
 #include <algorithm>
@@ -220,9 +220,6 @@ int conv3x3s2_fwd_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cou
   const uint32_t OH = H / 2u, OW = W / 2u;
   uint32_t QR, QC, NBI;
   if (!s2_quads(OH, OW, &QR, &QC, &NBI)) return ADH_EUNIMPL;
-  // The kernel of the bf16 matrix cores is faster below: 128 -> 256 channels on 16x64 tiles 187 us (the general kernel 205),
-  // 256 -> 512 on 8x32 182 (this one 206); 512 -> 512 on 4x16 158 (this one 130).
-  if (Cin < 512u) return ADH_EUNIMPL;
   if (!aligned_to(w, 16) || Cin % 4u != 0u) return ADH_EUNIMPL;
   for (uint32_t t = 0; t < num_tiles; ++t)
     if (!aligned_to(y_tiles[t], 16) || !aligned_to(x_tiles[t], 4)) return ADH_EUNIMPL;

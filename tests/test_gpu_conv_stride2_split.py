@@ -91,3 +91,17 @@ def test_values_without_finite_bf16_parts(bad):
             fine = torch.isfinite(want)
             assert ((got[fine].double() - want[fine].double()).abs() <= 2e-6 * want[fine].double().abs()).all()
             assert fine.any()
+
+
+@pytest.mark.parametrize("Cin,Cout", [(8, 320), (12, 384), (512, 128), (5, 576)])
+def test_forward_on_either_side_of_the_line_between_the_kernels(Cin, Cout):
+    """24 images of 16 x 16 results are 48 blocks per 64 channels: 240 and 96 (one round), 288 and 432 (two, of which 224 and 80 idle)."""
+    g = torch.Generator().manual_seed(14)
+    x, w = torch.rand((24, Cin, 32, 32), generator=g) * 2 - 1, torch.randn((Cout, Cin, 3, 3), generator=g) * (2.0 / (9 * Cin)) ** 0.5
+    want = torch.nn.functional.conv2d(x.double(), w.double(), stride=2, padding=1)
+    geo = (3, 3, 2, 2, 1, 1, 1, 1)
+    for beta in (0.0, 1.0):
+        y = torch.ones((24, Cout, 16, 16), device="cuda")
+        ws = torch.empty(capi.conv2d_unpadded_workspace_bytes(capi.ADH_CONV_FWD, capi.ADH_F32, 1, 24, Cin, Cout, 32, 32, *geo) // 4, device="cuda")
+        capi.check(capi.conv2d_unpadded_fwd_tiles([x.cuda()], w.cuda(), [y], 24, Cin, Cout, 32, 32, *geo, beta=beta, ws=ws), "fwd")
+        assert ((y.cpu().double() - want - beta).abs().max() / want.abs().max()).item() <= 1e-5
