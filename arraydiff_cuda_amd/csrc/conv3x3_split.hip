@@ -21,13 +21,13 @@
 // workgroup may span tiles (a 4 x 16 tile is a quarter of a 16 x 16 image) and no halo exchange or reduction is needed.
 //
 // Measured at stride 2 (32 images, 4 tiles, forward / backward-data; v_mfma_f32 kernels before): 64 -> 128 channels on 32 x 128
-// tiles 0.236 -> 0.216 / 0.212 -> 0.143 ms, 128 -> 256 on 16 x 64 0.205 -> 0.187 / 0.192 -> 0.118 (163 TFLOP/s), 256 -> 512 on
-// 8 x 32 0.206 -> 0.181 / 0.187 -> 0.131; 48 channels on 3 tiles of 6 x 30 0.023 -> 0.013 / 0.019 -> 0.014.  A forward step has a
+// tiles 0.214 -> 0.188 / 0.212 -> 0.130 ms, 128 -> 256 on 16 x 64 0.205 -> 0.182 / 0.192 -> 0.118 (163 TFLOP/s), 256 -> 512 on
+// 8 x 32 0.206 -> 0.179 / 0.187 -> 0.132; 48 channels on 3 tiles of 6 x 30 0.023 -> 0.013 / 0.019 -> 0.014.  A forward step has a
 // quarter of the stride-1 step's products and the same patch to load and split: that bounds it.  The next patch's loads go out
 // from the chunk's first step on (stride 1 has the registers for them from the fourth): 0.202 -> 0.187 and 0.126 -> 0.118.
 // Measured (32 images, 4 tiles without halo, forward / backward-data; v_mfma_f32 kernels before): 64 channels on 32 x 128
-// tiles 0.309 -> 0.196 / 0.182 ms (212 TFLOP/s), 128 on 16 x 64 0.297 -> 0.173, 256 on 8 x 32 0.292 -> 0.166 (232), 512 on
-// 4 x 16 0.39 -> 0.21.  Bound: the matrix pipe is busy 0.6 of the cycles; a step of 3072 matrix cycles takes 3700 to 4400
+// tiles 0.309 -> 0.209 / 0.197 ms (196 TFLOP/s), 128 on 16 x 64 0.297 -> 0.182, 256 on 8 x 32 0.292 -> 0.175 (221), 512 on
+// 4 x 16 0.39 -> 0.215 / 0.212.  Bound: the matrix pipe is busy 0.6 of the cycles; a step of 3072 matrix cycles takes 3700 to 4400
 // (the loads' address arithmetic and the splitting compete for issue slots), the patch's change of chunk 4500, and a block's
 // results leave at the rate of the memory, all workgroups at once.
 #include "conv3x3_split.h"

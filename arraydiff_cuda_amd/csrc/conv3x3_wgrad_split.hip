@@ -19,8 +19,8 @@
 //   * The halves' sums are added through LDS, the workgroups' by a second kernel in a fixed order (reproducible).
 // Row tiles of one tensor are addressed as that tensor (as in conv3x3_split.hip).
 //
-// Measured (32 images, 4 tiles without halo; the v_mfma_f32 kernel before): 64 channels on 32 x 128 tiles 0.351 -> 0.201 ms
-// (193 TFLOP/s), 128 on 16 x 64 0.354 -> 0.193, 256 on 8 x 32 0.361 -> 0.195, 512 on 4 x 16 0.456 -> 0.21 (0.61 through the
+// Measured (32 images, 4 tiles without halo; the v_mfma_f32 kernel before): 64 channels on 32 x 128 tiles 0.351 -> 0.197 ms
+// (196 TFLOP/s), 128 on 16 x 64 0.354 -> 0.193, 256 on 8 x 32 0.361 -> 0.195, 512 on 4 x 16 0.456 -> 0.21 (0.61 through the
 // general entry point before).  Staging: with rows, channels and tiles worked out per group of four values the kernel took
 // 0.45 ms; a thread's channel and column fixed and a wave's row uniform it is a load, a split and three writes.  Bound: a
 // step of 6912 matrix cycles takes about 12000, the splitting and the shifts (a third of the issue slots) and the clock,

@@ -7,7 +7,7 @@
 // gradient vectors of all ranks onto rank 0 (ncclReduce, optimize.hh:443-451), (3) runs three
 // to five whole-vector axpy kernels (src/kernels/array.cu:97-124) for l2, momentum and the
 // parameter update, and (4) copies the result back into every array (load_val).  Here
-//   (1), (4) are one launch per vector: a segment table travels in the kernel arguments;
+//   (1), (4) are one launch per 48 arrays of a vector: a segment table travels in the kernel arguments;
 //   (2), (3) are ONE pass: the kernel reads the K gradient vectors, the parameters and the
 //            momentum once and writes momentum, parameters and the lagged copy once.
 // All of it is HBM-bound streaming; 16-byte accesses, nothing staged.

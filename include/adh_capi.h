@@ -271,7 +271,8 @@ int adh_conv3x3_unpadded_bwd_filter_tiles(int dtype, uint32_t num_tiles, uint32_
  * of it for each side of at most 32 channels): fewer workgroups share the pixels then, or the channel groups run in turn.
  * ADH_BF16: the matrix-core kernel reads rows of whole 16-byte granules; at a width that is no multiple
  * of 8 the rows of x_pad and dy are first copied into the workspace at the next such width with zeros
- * behind (a zero dy adds nothing to any tap), one more pass over both tensors. */
+ * behind, one more pass over both tensors (a zero dy adds nothing to any tap, unless what it meets in the last two
+ * columns of x_pad is not finite). */
 int adh_conv3x3_slab_bwd_filter(int dtype, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                                 const void *x_pad, const void *dy, float *dw, float beta,
                                 void *workspace, size_t workspace_bytes, void *stream);
