@@ -630,7 +630,8 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
     const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
     for (int NT = q.sample == kDown ? 1 : 4; NT >= 1; NT /= 2) {
       if (q.sample == kUp && NT == 4 && MT > 1) continue;  // (four sets of sums)
-      if (plan->low == kLowApart && (q.sample == kUnit ? NT != 2 : q.sample == kUp && MT * NT > 2)) continue;  // (the registers)
+      // (what the registers hold of two sets of sums: at stride 1 the largest such tile of each height)
+      if (plan->low == kLowApart && (q.sample == kUnit ? NT != (MT == 1 ? 4 : 2) : q.sample == kUp && NT > 1 && MT * NT > 2)) continue;
       const uint32_t slots = 128u * NT;
       const double matrix = 192.0 * MT * NT;
       const double chunk = 9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT;
@@ -733,9 +734,9 @@ static void launch_split_nt(const SplitPlan &plan, SplitSample sample, hipStream
   } else if (sample == kUp) {
     if (MT == 1 && plan.NT == 4) launch_split<1, 4, kUp, 0>(plan, st);
     else if (plan.NT == 2) apart ? launch_split<1, 2, kUp, kLowApart>(plan, st) : launch_split<MT, 2, kUp, 0>(plan, st);
-    else apart ? launch_split<MT == 4 ? 2 : MT, 1, kUp, kLowApart>(plan, st) : launch_split<MT, 1, kUp, 0>(plan, st);
+    else apart ? launch_split<MT, 1, kUp, kLowApart>(plan, st) : launch_split<MT, 1, kUp, 0>(plan, st);
   } else if (apart) {
-    launch_split<MT, 2, kUnit, kLowApart>(plan, st);
+    launch_split<MT, MT == 1 ? 4 : 2, kUnit, kLowApart>(plan, st);
   } else if (plan.NT == 4) {
     plan.low == 4 ? launch_split<MT, 4, kUnit, 4>(plan, st) : launch_split<MT, 4, kUnit, 9>(plan, st);
   } else if (plan.NT == 2) {
