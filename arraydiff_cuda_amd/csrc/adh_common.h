@@ -44,6 +44,33 @@ __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
   return (uint16_t)(u >> 16);
 }
 
+// A thread's vector (16 bytes, or one element) at element alignment.  STREAM: non-temporal, for data that the on-package
+// cache would not keep anyway.  Reads of 537 MB reach 6.9 to 7.1 TB/s that way against 5.7 to 6.4, whatever the order and the
+// loads in flight.
+template <bool STREAM, typename V, typename T>
+__device__ __forceinline__ V load_vec(const T *p) {
+  typedef uint32_t Raw __attribute__((ext_vector_type(4), aligned(2)));
+  V v;
+  if constexpr (STREAM && sizeof(V) == 16) {
+    const Raw r = __builtin_nontemporal_load(reinterpret_cast<const Raw *>(p));
+    __builtin_memcpy(&v, &r, 16);
+  } else {
+    v = *reinterpret_cast<const V *>(p);
+  }
+  return v;
+}
+template <bool STREAM, typename V, typename T>
+__device__ __forceinline__ void store_vec(T *p, const V &v) {
+  typedef uint32_t Raw __attribute__((ext_vector_type(4), aligned(2)));
+  if constexpr (STREAM && sizeof(V) == 16) {
+    Raw r;
+    __builtin_memcpy(&r, &v, 16);
+    __builtin_nontemporal_store(r, reinterpret_cast<Raw *>(p));
+  } else {
+    *reinterpret_cast<V *>(p) = v;
+  }
+}
+
 __device__ __forceinline__ float elem_add(float a, float b) { return a + b; }
 __device__ __forceinline__ uint16_t elem_add(uint16_t a, uint16_t b) {
   return f32_to_bf16_bits(bf16_bits_to_f32(a) + bf16_bits_to_f32(b));

@@ -16,9 +16,15 @@
 // Backward mirrors it: reduce sum dy' and sum dy'*(x - mean) (dy' = dy masked by the rectifier, dy read
 // from the interior of the padded gradient tile when the forward wrote a padded tile); apply works out
 // the parameter gradients and three coefficients, then dx = beta*dx + k1*dy' + k2*(x - mean) + k3.
+//
+// Measured, fp32, 64 channels, 32 images, 4 tiles of 64 x 256 (537 MB a tensor), before (temporal accesses, one group in
+// flight, coefficients before the loads) -> now: reduce 123 -> 86 us (6.2 TB/s), backward 225 -> 165 to 190; apply 240 -> 207,
+// backward 320 -> 283 (5.7 TB/s).  bf16, 100 channels, 9 images, 4 tiles of 14 x 333 (before: element by element): reduce 23 -> 10.6,
+// backward 31 -> 16.6; apply 25 -> 22, backward 56 -> 34.
 #include "adh_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace adh {
 
@@ -37,7 +43,8 @@ struct BnParams {
   float *o2[ADH_MAX_TILES];               // forward: saved mean
   float *o3[ADH_MAX_TILES];               // forward: saved 1/sqrt(var + eps)
   float *partial;                         // [tile][c][split][2]
-  uint32_t N, C, H, W, HW, p, split, n_per_split, tiles, groups_per_plane, slots_log2, planes_per_pass;
+  uint32_t N, C, H, W, HW, p, split, n_per_split, tiles, groups_per_plane, slots_log2, along, planes_per_pass;
+  uint32_t run;  // elements that lie side by side in both tensors of a pass: the plane, or (padded gradient) a row
   float eps, beta, beta_param;  // beta: input-gradient accumulation; beta_param: parameter-gradient accumulation
   int relu;
   FastDiv div_C, div_N, div_split, div_groups, div_cols;  // div_groups: the 16-byte groups of a plane; div_cols: row length of the index that a kernel splits into (row, column)
@@ -79,60 +86,66 @@ __device__ __forceinline__ float2 block_sum2(float a, float b) {
 
 // grid: tiles * C * split.  BWD = false: sums of (x - K), (x - K)^2.  BWD = true: sums of dy', dy' * (x - mean)
 // (dy' = dy where a*(x - mean) + shift > 0 when the rectifier was fused, else dy), dy at the interior of a tile padded by p.
-// VEC > 1: H*W (and, backward, W) are whole numbers of VEC-element groups, one 16-byte access per group.
-template <typename T, bool BWD, int VEC>
+// A run of P.run elements (a row of a padded gradient, else the whole plane) is whole groups of VEC; the last group ends
+// with the run and leaves out what it shares with the one before.
+// Four groups a thread are loaded before the first is added: with one, the loads in flight bound it (DRAM latency).
+template <typename T, bool BWD, int VEC, bool STREAM>
 __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P) {
   typedef BnVec<T, VEC> Vec;
+  constexpr int U = 4;
   uint32_t tc, sp, tile, c;
   P.div_split.divmod(blockIdx.x, tc, sp);
   P.div_C.divmod(tc, tile, c);
   const T *x = reinterpret_cast<const T *>(P.x[tile]);
+  const T *dy = reinterpret_cast<const T *>(P.dy[tile]);
   const uint32_t n0 = sp * P.n_per_split, n1 = min(P.N, n0 + P.n_per_split);
-  const uint32_t groups = P.HW / (uint32_t)VEC;
+  const uint32_t WP = P.W + 2u * P.p, HPp = P.H + 2u * P.p;
+  // (forward: the channel's first element, so that the sums stay small next to the variance)
+  const float mean = BWD ? P.mean_in[tile][c] : bn_ld(x, (size_t)c * P.HW);
+  const float a = BWD && P.relu ? P.scale[tile][c] * P.second_in[tile][c] : 0.f;
+  const float b = BWD && P.relu ? P.shift[tile][c] : 0.f;
   float s1 = 0.f, s2 = 0.f;
-  if (!BWD) {
-    const float K = bn_ld(x, (size_t)c * P.HW);
-    // the groups of the split's planes are numbered through: a plane of a few groups (a late layer's 4 x 16 tile
-    // is 16 of them) would otherwise leave most of the workgroup idle for one load latency per plane
-    // (P.planes_per_pass planes at a time keep the running number below 2^31: one pass but for gigantic planes)
-    for (uint32_t nb = n0; nb < n1; nb += P.planes_per_pass) {
-      const uint32_t items = min(P.planes_per_pass, n1 - nb) * groups;
-      for (uint32_t it = threadIdx.x; it < items; it += kBnThreads) {
-        uint32_t nr, i;
-        P.div_groups.divmod(it, nr, i);
-        const T *pl = x + ((size_t)(nb + nr) * P.C + c) * P.HW;
-        const Vec xv = *reinterpret_cast<const Vec *>(pl + (size_t)i * VEC);
+  // the groups of the split's planes are numbered through: a plane of a few groups (a late layer's 4 x 16 tile
+  // is 16 of them) would otherwise leave most of the workgroup idle for one load latency per plane
+  // (P.planes_per_pass planes at a time keep the running number below 2^31: one pass but for gigantic planes)
+  for (uint32_t nb = n0; nb < n1; nb += P.planes_per_pass) {
+    const uint32_t items = min(P.planes_per_pass, n1 - nb) * P.groups_per_plane;
+    for (uint32_t it0 = threadIdx.x; it0 < items; it0 += U * kBnThreads) {
+      Vec xv[U], dv[U];
+      uint32_t skip[U];
 #pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-          const float v = bn_f(xv.v[k]) - K;
-          s1 += v;
-          s2 += v * v;
-        }
-      }
-    }
-  } else {
-    const T *dy = reinterpret_cast<const T *>(P.dy[tile]);
-    const uint32_t WP = P.W + 2u * P.p, HPp = P.H + 2u * P.p;
-    const float a = P.relu ? P.scale[tile][c] * P.second_in[tile][c] : 0.f;
-    const float mean = P.mean_in[tile][c];
-    const float b = P.relu ? P.shift[tile][c] : 0.f;
-    for (uint32_t nb = n0; nb < n1; nb += P.planes_per_pass) {
-      const uint32_t items = min(P.planes_per_pass, n1 - nb) * groups;
-      for (uint32_t it = threadIdx.x; it < items; it += kBnThreads) {
+      for (int u = 0; u < U; ++u) {
+        const uint32_t it = it0 + (uint32_t)u * kBnThreads;
         uint32_t nr, i, h, w;
-        P.div_groups.divmod(it, nr, i);
-        P.div_cols.divmod(i, h, w);  // groups per row
-        const T *pl = x + ((size_t)(nb + nr) * P.C + c) * P.HW;
-        const T *dl = dy + ((size_t)(nb + nr) * P.C + c) * HPp * WP + (size_t)P.p * WP + P.p;
-        const Vec xv = *reinterpret_cast<const Vec *>(pl + (size_t)i * VEC);
-        const Vec dv = *reinterpret_cast<const Vec *>(dl + (size_t)h * WP + w * VEC);
-#pragma unroll
-        for (int k = 0; k < VEC; ++k) {
-          const float xc = bn_f(xv.v[k]) - mean;
-          float d = bn_f(dv.v[k]);
+        P.div_groups.divmod(it < items ? it : it0, nr, i);
+        P.div_cols.divmod(i, h, w);  // groups of a run
+        const uint32_t at = min(w * VEC, P.run - VEC);
+        skip[u] = it < items ? w * VEC - at : VEC;
+        const size_t plane = (size_t)(nb + nr) * P.C + c;
+        xv[u] = load_vec<STREAM, Vec>(x + plane * P.HW + (size_t)h * P.run + at);
+        if (BWD) dv[u] = load_vec<STREAM, Vec>(dy + plane * HPp * WP + (size_t)(h + P.p) * WP + P.p + at);
+      }
+      auto add = [&](int u, int k) {
+        const float xc = bn_f(xv[u].v[k]) - mean;
+        if (BWD) {
+          float d = bn_f(dv[u].v[k]);
           if (P.relu && !(a * xc + b > 0.f)) d = 0.f;
           s1 += d;
           s2 += d * xc;
+        } else {
+          s1 += xc;
+          s2 += xc * xc;
+        }
+      };
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        if (skip[u] == 0u) {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k) add(u, k);
+        } else {
+#pragma unroll
+          for (int k = 0; k < VEC; ++k)
+            if ((uint32_t)k >= skip[u]) add(u, k);
         }
       }
     }
@@ -144,32 +157,54 @@ __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P)
   }
 }
 
-// The five numbers the apply pass needs for one (tile, channel), worked out by ONE thread of every apply
-// workgroup that touches the channel (the sums of the splits are added in double, in split order, so every
-// workgroup gets the same bits).  `publish`: this thread also writes the channel's statistics (forward) or
-// parameter gradients (backward); exactly one thread per (tile, channel) in the grid is told to.
+// What the numbers of one (tile, channel) are worked out from; `v`: the first of the sums that this lane adds.
+struct BnCoefIn {
+  float scale, shift, mean, second;
+  float2 v;
+};
+template <typename T, int MODE>
+__device__ __forceinline__ BnCoefIn bn_coef_load(const BnParams &P, uint32_t tile, uint32_t c, uint32_t lane) {
+  BnCoefIn in = {P.scale[tile][c], P.shift[tile][c], 0.f, 0.f, make_float2(0.f, 0.f)};
+  in.mean = MODE == 0 ? bn_ld(reinterpret_cast<const T *>(P.x[tile]), (size_t)c * P.HW) : P.mean_in[tile][c];
+  if (MODE != 0) in.second = P.second_in[tile][c];
+  if (MODE != 1 && lane < P.split)
+    in.v = *reinterpret_cast<const float2 *>(P.partial + (((size_t)tile * P.C + c) * P.split + lane) * 2u);
+  return in;
+}
+
+// The five numbers the apply pass needs for one (tile, channel), worked out by `lanes` threads of every apply workgroup
+// that touches the channel (the sums of the splits are added in double, in an order that hangs on `lanes` alone, the same
+// over the launch, so every workgroup gets the same bits); the first of them writes cf.  `publish`: it also writes the
+// channel's statistics (forward) or parameter gradients (backward); exactly one per (tile, channel) in the grid is told to.
 //   MODE 0, training forward : cf = { a = scale / sqrt(var + eps), mean, shift }
 //   MODE 1, inference        : the same from the fixed statistics
 //   MODE 2, backward         : cf = { k1 = a, k2, k3, mean, shift };  dx = k1 dy' + k2 (x - mean) + k3
 template <typename T, int MODE>
-__device__ void bn_plane_coef(const BnParams &P, uint32_t tile, uint32_t c, bool publish, float *cf) {
-  const size_t tc = (size_t)tile * P.C + c;
+__device__ __forceinline__ void bn_plane_coef(const BnParams &P, const BnCoefIn &in, uint32_t tile, uint32_t c, uint32_t lane,
+                                              uint32_t lanes, bool publish, float *cf) {
+  const float scale = in.scale, shift = in.shift, K = in.mean, saved = in.second;
   if (MODE == 1) {
-    const double invstd = 1.0 / sqrt((double)P.second_in[tile][c] + (double)P.eps);
-    cf[0] = (float)((double)P.scale[tile][c] * invstd);
-    cf[1] = P.mean_in[tile][c];
-    cf[2] = P.shift[tile][c];
+    if (lane != 0u) return;
+    const double invstd = 1.0 / sqrt((double)saved + (double)P.eps);
+    cf[0] = (float)((double)scale * invstd);
+    cf[1] = K;
+    cf[2] = shift;
     return;
   }
-  double s1 = 0.0, s2 = 0.0;
-  for (uint32_t sp = 0; sp < P.split; ++sp) {
-    s1 += (double)P.partial[(tc * P.split + sp) * 2u];
-    s2 += (double)P.partial[(tc * P.split + sp) * 2u + 1u];
+  double s1 = (double)in.v.x, s2 = (double)in.v.y;
+  for (uint32_t sp = lane + lanes; sp < P.split; sp += lanes) {
+    const float2 v = *reinterpret_cast<const float2 *>(P.partial + (((size_t)tile * P.C + c) * P.split + sp) * 2u);
+    s1 += (double)v.x;
+    s2 += (double)v.y;
   }
+  for (uint32_t o = lanes >> 1; o > 0u; o >>= 1) {
+    s1 += __shfl_xor(s1, (int)o);
+    s2 += __shfl_xor(s2, (int)o);
+  }
+  if (lane != 0u) return;
   const double m = (double)P.N * (double)P.HW;
   if (MODE == 0) {
-    const double K = (double)bn_ld(reinterpret_cast<const T *>(P.x[tile]), (size_t)c * P.HW);
-    const double d = s1 / m, mean = K + d;
+    const double d = s1 / m, mean = (double)K + d;
     double var = s2 / m - d * d;
     if (var < 0.0) var = 0.0;
     const double invstd = 1.0 / sqrt(var + (double)P.eps);
@@ -179,99 +214,122 @@ __device__ void bn_plane_coef(const BnParams &P, uint32_t tile, uint32_t c, bool
       if (P.o2[tile]) P.o2[tile][c] = (float)mean;
       if (P.o3[tile]) P.o3[tile][c] = (float)invstd;
     }
-    cf[0] = (float)((double)P.scale[tile][c] * invstd);
+    cf[0] = (float)((double)scale * invstd);
     cf[1] = (float)mean;
-    cf[2] = P.shift[tile][c];
+    cf[2] = shift;
   } else {
-    const double mean = P.mean_in[tile][c], invstd = P.second_in[tile][c], scale = P.scale[tile][c];
+    const double invstd = saved;
     const double dshift = s1, dscale = s2 * invstd;  // sum dy' * (x - mean) * invstd
     if (publish) {
       P.o0[tile][c] = (float)((P.beta_param != 0.f ? (double)P.o0[tile][c] : 0.0) + dscale);
       P.o1[tile][c] = (float)((P.beta_param != 0.f ? (double)P.o1[tile][c] : 0.0) + dshift);
     }
     // dx = a * (dy' - dshift/m - xhat * dscale/m),  xhat = (x - mean) * invstd
-    const double a = scale * invstd;
+    const double a = (double)scale * invstd;
     cf[0] = (float)a;
     cf[1] = (float)(-a * invstd * dscale / m);
     cf[2] = (float)(-a * dshift / m);
-    cf[3] = (float)mean;
-    cf[4] = P.shift[tile][c];  // the rectifier's mask needs the forward output's sign
+    cf[3] = K;
+    cf[4] = shift;  // the rectifier's mask needs the forward output's sign
   }
 }
 
-// a thread moves VEC consecutive elements of the padded output
-// plane (forward: any shape, the last partial group element by element) or of the packed gradient plane (backward:
-// VEC > 1 needs H*W and W to be whole numbers of groups)
-// MODE as in bn_plane_coef: the first U threads of the workgroup work out the coefficients of its U planes
-// (there is no separate finalize launch), everyone else picks them up from LDS.
-template <typename T, int MODE, int VEC>
+// a thread moves U groups of VEC consecutive elements, all loads before the first store: of the packed gradient plane's runs
+// (backward: P.run elements, the last group ending with the run; what it shares with the one before is left to that, so
+// that dx may be x or dy), of an unpadded output plane in the same way, or of a padded one (element by element where a
+// group is not inside one row).
+// The loads go out before the coefficients are worked out (MODE as in bn_plane_coef; there is no separate finalize
+// launch): the chain of loads, sums and a square root is as long as theirs.  What that needs is loaded before them, so
+// that it does not wait for them.
+// Work split (bn_apply_grid): a plane of at most 128 groups takes 1 << P.slots_log2 = 16 .. 128 threads and the workgroup's
+// parts take U planes each; a larger plane takes the whole workgroup, band by band (blockIdx.y): the same group of U
+// planes a thread, or (P.along, backward) U groups of one plane.
+template <typename T, int MODE, int VEC, bool STREAM>
 __global__ __launch_bounds__(kBnThreads) void bn_apply_kernel(const BnParams P) {
   typedef BnVec<T, VEC> Vec;
   constexpr bool BWD = MODE == 2;
-  constexpr int U = 4;  // planes per thread: a thread moves the same group of each, all loads before the first store
-  // A plane of at most 128 groups (the late layers' tiles) takes P.slots = 16 .. 128 threads, and the workgroup's
-  // 256 / P.slots parts take U planes each; a larger plane takes the whole workgroup, band by band (blockIdx.y).
+  constexpr uint32_t U = 4;
   __shared__ float cf_s[U * 16][8];
   const uint32_t WP = P.W + 2u * P.p, HPp = P.H + 2u * P.p;
   const uint32_t total = HPp * WP;
   const uint32_t planes = P.tiles * P.N * P.C;
   const uint32_t parts = kBnThreads >> P.slots_log2;
   const uint32_t part = threadIdx.x >> P.slots_log2;
-  if (threadIdx.x < (uint32_t)U * parts) {
-    const uint32_t pl = blockIdx.x * U * parts + threadIdx.x;
-    if (pl < planes) {
+  const bool along = BWD && P.along;
+  const uint32_t per_block = along ? 1u : U * parts;  // planes
+  const uint32_t gi = blockIdx.y * (along ? U * kBnThreads : kBnThreads) + (threadIdx.x & ((1u << P.slots_log2) - 1u));  // group within a plane
+  const uint32_t lanes = min(8u, kBnThreads / per_block), ci = threadIdx.x / lanes, clane = threadIdx.x - ci * lanes;
+  uint32_t c_tile = 0, c_n = 0, c_c = 0;
+  const bool c_live = ci < per_block && blockIdx.x * per_block + ci < planes;
+  BnCoefIn coef_in;
+  if (c_live) {
+    uint32_t tn;
+    P.div_C.divmod(blockIdx.x * per_block + ci, tn, c_c);
+    P.div_N.divmod(tn, c_tile, c_n);
+    coef_in = bn_coef_load<T, MODE>(P, c_tile, c_c, clane);
+  }
+  Vec xv[U], dv[U], old[U];
+  T *out_u[U];
+  bool live[U];
+  uint32_t skip[U], mask = (1u << VEC) - 1u, out_off = 0;
+#pragma unroll
+  for (uint32_t u = 0; u < U; ++u) live[u] = false;
+  if (BWD) {
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t pl = along ? blockIdx.x : (blockIdx.x * parts + part) * U + u;
+      const uint32_t g = along ? gi + u * kBnThreads : gi;
+      live[u] = pl < planes && g < P.groups_per_plane;
+      if (!live[u]) continue;
+      uint32_t tn, c, tile, n, h, w;
+      P.div_C.divmod(pl, tn, c);
+      P.div_N.divmod(tn, tile, n);
+      P.div_cols.divmod(g, h, w);  // groups of a run
+      const uint32_t at = min(w * VEC, P.run - VEC);
+      skip[u] = w * VEC - at;
+      const size_t plane = (size_t)n * P.C + c, off = plane * P.HW + (size_t)h * P.run + at;
+      out_u[u] = reinterpret_cast<T *>(P.out[tile]) + off;
+      xv[u] = load_vec<STREAM, Vec>(reinterpret_cast<const T *>(P.x[tile]) + off);
+      dv[u] = load_vec<STREAM, Vec>(reinterpret_cast<const T *>(P.dy[tile]) + plane * total + (size_t)(h + P.p) * WP + P.p + at);
+      if (P.beta != 0.f) old[u] = load_vec<false, Vec>(out_u[u]);
+    }
+  } else if (gi < P.groups_per_plane) {
+    // where the group sits is the same for every plane
+    uint32_t r = 0, col = 0, in_off;
+    bool whole = true;
+    if (P.p == 0u && total >= (uint32_t)VEC) {  // the last group ends with the plane
+      in_off = out_off = min(gi * VEC, total - VEC);
+    } else {
+      P.div_cols.divmod(gi * VEC, r, col);
+      whole = r - P.p < P.H && col >= P.p && col + VEC <= P.p + P.W;  // inside one interior row
+      in_off = (r - P.p) * P.W + (col - P.p);
+      out_off = gi * VEC;
+      if (!whole) {
+        mask = 0u;
+        uint32_t rr = r, cc = col;
+#pragma unroll
+        for (int k = 0; k < VEC; ++k) {
+          if (rr - P.p < P.H && cc - P.p < P.W) mask |= 1u << k;
+          if (++cc == WP) {
+            cc = 0;
+            ++rr;
+          }
+        }
+      }
+    }
+#pragma unroll
+    for (uint32_t u = 0; u < U; ++u) {
+      const uint32_t pl = (blockIdx.x * parts + part) * U + u;
+      live[u] = pl < planes;
+      if (!live[u]) continue;
+      skip[u] = gi * VEC - out_off;
       uint32_t tn, c, tile, n;
       P.div_C.divmod(pl, tn, c);
       P.div_N.divmod(tn, tile, n);
-      bn_plane_coef<T, MODE>(P, tile, c, blockIdx.y == 0u && n == 0u, cf_s[threadIdx.x]);
-    }
-  }
-  __syncthreads();
-  const uint32_t gi = blockIdx.y * kBnThreads + (threadIdx.x & ((1u << P.slots_log2) - 1u));  // group of VEC elements within a plane
-  if (gi >= P.groups_per_plane) return;
-  // where the group sits is the same for every plane
-  uint32_t r = 0, col = 0, in_off = 0, mask = 0;
-  bool whole = false;
-  if (!BWD) {
-    P.div_cols.divmod(gi * VEC, r, col);
-    whole = VEC > 1 && r - P.p < P.H && col >= P.p && col + VEC <= P.p + P.W;  // inside one interior row
-    in_off = (r - P.p) * P.W + (col - P.p);
-    if (!whole) {
-      uint32_t rr = r, cc = col;
-#pragma unroll
-      for (int k = 0; k < VEC; ++k) {
-        if (rr - P.p < P.H && cc - P.p < P.W) mask |= 1u << k;
-        if (++cc == WP) {
-          cc = 0;
-          ++rr;
-        }
-      }
-    } else {
-      mask = (1u << VEC) - 1u;
-    }
-  } else {
-    uint32_t h, w;
-    P.div_cols.divmod(gi, h, w);  // groups per row
-    in_off = h * WP + w * VEC;     // within the interior of the padded gradient plane
-  }
-  Vec xv[U], dv[U], old[U];
-  const float *cf_u[U];
-  T *out_u[U];
-  bool live[U];
-#pragma unroll
-  for (int u = 0; u < U; ++u) {
-    const uint32_t pl = (blockIdx.x * parts + part) * U + u;
-    live[u] = pl < planes;
-    if (!live[u]) continue;
-    uint32_t tn, c, tile, n;
-    P.div_C.divmod(pl, tn, c);
-    P.div_N.divmod(tn, tile, n);
-    cf_u[u] = cf_s[part * U + u];
-    const T *x = reinterpret_cast<const T *>(P.x[tile]) + ((size_t)n * P.C + c) * P.HW;
-    if (!BWD) {
-      out_u[u] = reinterpret_cast<T *>(P.out[tile]) + ((size_t)n * P.C + c) * total;
+      const T *x = reinterpret_cast<const T *>(P.x[tile]) + ((size_t)n * P.C + c) * P.HW;
+      out_u[u] = reinterpret_cast<T *>(P.out[tile]) + ((size_t)n * P.C + c) * total + out_off;
       if (whole) {
-        xv[u] = *reinterpret_cast<const Vec *>(x + in_off);
+        xv[u] = load_vec<STREAM, Vec>(x + in_off);
       } else {
         uint32_t rr = r, cc = col;
 #pragma unroll
@@ -283,18 +341,14 @@ __global__ __launch_bounds__(kBnThreads) void bn_apply_kernel(const BnParams P) 
           }
         }
       }
-    } else {
-      const T *dy = reinterpret_cast<const T *>(P.dy[tile]) + ((size_t)n * P.C + c) * total + (size_t)P.p * WP + P.p;
-      out_u[u] = reinterpret_cast<T *>(P.out[tile]) + ((size_t)n * P.C + c) * P.HW;
-      xv[u] = *reinterpret_cast<const Vec *>(x + (size_t)gi * VEC);
-      dv[u] = *reinterpret_cast<const Vec *>(dy + in_off);
-      if (P.beta != 0.f) old[u] = *reinterpret_cast<const Vec *>(out_u[u] + (size_t)gi * VEC);
     }
   }
+  if (c_live) bn_plane_coef<T, MODE>(P, coef_in, c_tile, c_c, clane, lanes, blockIdx.y == 0u && c_n == 0u, cf_s[ci]);
+  __syncthreads();
 #pragma unroll
-  for (int u = 0; u < U; ++u) {
+  for (uint32_t u = 0; u < U; ++u) {
     if (!live[u]) continue;
-    const float *cf = cf_u[u];
+    const float *cf = cf_s[along ? 0u : part * U + u];
     Vec out;
     if (!BWD) {
       const float a = cf[0], mean = cf[1], b = cf[2];
@@ -307,14 +361,6 @@ __global__ __launch_bounds__(kBnThreads) void bn_apply_kernel(const BnParams P) 
         }
         bn_t(out.v[k], v);
       }
-      const uint32_t o = gi * VEC;
-      if (o + VEC <= total) {
-        *reinterpret_cast<Vec *>(out_u[u] + o) = out;
-      } else {
-#pragma unroll
-        for (int k = 0; k < VEC; ++k)
-          if (o + k < total) out_u[u][o + k] = out.v[k];
-      }
     } else {
       const float k1 = cf[0], k2 = cf[1], k3 = cf[2], mean = cf[3], b = cf[4];
 #pragma unroll
@@ -326,7 +372,13 @@ __global__ __launch_bounds__(kBnThreads) void bn_apply_kernel(const BnParams P) 
         if (P.beta != 0.f) g += bn_f(old[u].v[k]);
         bn_t(out.v[k], g);
       }
-      *reinterpret_cast<Vec *>(out_u[u] + (size_t)gi * VEC) = out;
+    }
+    if (skip[u] == 0u && (BWD || out_off + VEC <= total)) {
+      store_vec<STREAM, Vec>(out_u[u], out);
+    } else {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k)
+        if ((uint32_t)k >= skip[u] && (BWD || out_off + k < total)) out_u[u][k] = out.v[k];
     }
   }
 }
@@ -391,8 +443,9 @@ static int bn_common(int dtype, uint32_t num_tiles, uint32_t N, uint32_t C, uint
   return ADH_OK;
 }
 
-// sets the apply kernel's work split and returns its grid: x = groups of four planes, y = bands of 256 groups of a plane
-static dim3 bn_apply_grid(BnParams *P, uint32_t groups_per_plane) {
+// sets the apply kernel's work split and returns its grid.  Four groups of one plane (along) where a plane has as many: two
+// tensors read and one written at the same place of four planes 64 KB apart took 311 us, of one plane 271.
+static dim3 bn_apply_grid(BnParams *P, uint32_t groups_per_plane, bool backward) {
   P->groups_per_plane = groups_per_plane;
   P->div_N = FastDiv(P->N);
   // threads per plane: the whole workgroup, or for planes of at most 128 groups the power of two that holds them
@@ -401,9 +454,39 @@ static dim3 bn_apply_grid(BnParams *P, uint32_t groups_per_plane) {
     P->slots_log2 = 4;
     while ((1u << P->slots_log2) < groups_per_plane) ++P->slots_log2;
   }
-  const uint64_t planes = (uint64_t)P->tiles * P->N * P->C;
-  const uint64_t per_block = 4u * (kBnThreads >> P->slots_log2);
-  return dim3((uint32_t)((planes + per_block - 1u) / per_block), (groups_per_plane + kBnThreads - 1u) / kBnThreads);
+  const uint32_t planes = P->tiles * P->N * P->C, along = 4u * kBnThreads;
+  P->along = backward && groups_per_plane >= along;
+  if (P->along) return dim3(planes, (groups_per_plane + along - 1u) / along);
+  const uint32_t per_block = 4u * (kBnThreads >> P->slots_log2);
+  return dim3((planes + per_block - 1u) / per_block, (groups_per_plane + kBnThreads - 1u) / kBnThreads);
+}
+
+// A plane is `runs` runs of `run` elements, each read as groups of `vec`.  False: one element at a time is read, where the
+// last groups, stored element by element, are more than an eighth of all (5.6 us against 8.9 for the backward pass over
+// bf16 planes of 22).
+static bool bn_runs(BnParams *P, uint32_t run, uint32_t runs, uint32_t vec) {
+  const bool wide = run % vec == 0u || run >= 8u * vec;
+  const uint32_t groups = wide ? (run + vec - 1u) / vec : run;
+  P->run = run;
+  P->groups_per_plane = groups * runs;
+  P->div_cols = FastDiv(groups);
+  P->div_groups = FastDiv(P->groups_per_plane);
+  P->planes_per_pass = std::max(1u, 0x7fffffffu / P->groups_per_plane);
+  return wide;
+}
+
+// `bytes`: what a pass reads.  Non-temporal where the on-package cache (256 MB) cannot keep it for the second pass.
+static bool bn_stream(uint64_t bytes) { return bytes > (256ull << 20); }
+
+template <typename F>
+static void bn_launch(bool stream_data, int dtype, F f) {
+  if (dtype == ADH_F32) {
+    if (stream_data) f(std::true_type{}, 0.f);
+    else f(std::false_type{}, 0.f);
+  } else {
+    if (stream_data) f(std::true_type{}, uint16_t(0));
+    else f(std::false_type{}, uint16_t(0));
+  }
 }
 
 }  // namespace adh
@@ -452,32 +535,26 @@ int adh_batchnorm2d_fwd_tiles(int dtype, int training, uint32_t num_tiles, uint3
   }
   P.eps = eps;
   P.relu = relu ? 1 : 0;
-  P.div_cols = FastDiv(W + 2u * out_halo);  // the apply kernel walks the padded output plane
   hipStream_t st = as_stream(stream);
-  const uint32_t tc = num_tiles * C;
-  const uint32_t vec = (uint32_t)(16 / dtype_size(dtype));
-  const bool wide = (H * W) % vec == 0;  // the statistics pass reads whole 16-byte groups
-  P.div_groups = FastDiv(wide ? H * W / vec : H * W);
-  P.planes_per_pass = std::max(1u, 0x7fffffffu / (wide ? H * W / vec : H * W));
+  const uint32_t tc = num_tiles * C, vec = (uint32_t)(16 / es);
   const uint32_t gpp = ((H + 2u * out_halo) * (W + 2u * out_halo) + vec - 1u) / vec;
   if ((gpp + kBnThreads - 1u) / kBnThreads > 65535u) return ADH_EINVAL;  // grid.y
+  const bool stream_data = bn_stream((uint64_t)tc * N * H * W * es);
   if (training) {
-    if (dtype == ADH_F32) {
-      if (wide) hipLaunchKernelGGL((bn_reduce_kernel<float, false, 4>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
-      else hipLaunchKernelGGL((bn_reduce_kernel<float, false, 1>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
-    } else {
-      if (wide) hipLaunchKernelGGL((bn_reduce_kernel<uint16_t, false, 8>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
-      else hipLaunchKernelGGL((bn_reduce_kernel<uint16_t, false, 1>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
-    }
+    const bool wide = bn_runs(&P, H * W, 1u, vec);  // the statistics pass
+    bn_launch(stream_data, dtype, [&](auto s, auto t) {
+      typedef decltype(t) T;
+      if (wide) hipLaunchKernelGGL((bn_reduce_kernel<T, false, 16 / sizeof(T), s>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
+      else hipLaunchKernelGGL((bn_reduce_kernel<T, false, 1, false>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
+    });
   }
-  const dim3 grid = bn_apply_grid(&P, gpp);
-  if (training) {
-    if (dtype == ADH_F32) hipLaunchKernelGGL((bn_apply_kernel<float, 0, 4>), grid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_apply_kernel<uint16_t, 0, 8>), grid, dim3(kBnThreads), 0, st, P);
-  } else {
-    if (dtype == ADH_F32) hipLaunchKernelGGL((bn_apply_kernel<float, 1, 4>), grid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_apply_kernel<uint16_t, 1, 8>), grid, dim3(kBnThreads), 0, st, P);
-  }
+  P.div_cols = FastDiv(W + 2u * out_halo);  // the apply kernel walks the padded output plane
+  const dim3 grid = bn_apply_grid(&P, gpp, false);
+  bn_launch(stream_data, dtype, [&](auto s, auto t) {
+    typedef decltype(t) T;
+    if (training) hipLaunchKernelGGL((bn_apply_kernel<T, 0, 16 / sizeof(T), s>), grid, dim3(kBnThreads), 0, st, P);
+    else hipLaunchKernelGGL((bn_apply_kernel<T, 1, 16 / sizeof(T), s>), grid, dim3(kBnThreads), 0, st, P);
+  });
   return launch_status();
 }
 
@@ -514,32 +591,24 @@ int adh_batchnorm2d_bwd_tiles(int dtype, uint32_t num_tiles, uint32_t N, uint32_
     P.o1[t] = dshift_tiles[t];
   }
   P.relu = relu ? 1 : 0;
-  // the reduce and apply kernels walk the packed plane in groups of `vec` elements when rows are whole groups
-  const uint32_t vec = (uint32_t)(16 / dtype_size(dtype));
-  const bool wide = W % vec == 0;
-  P.div_cols = FastDiv(wide ? W / vec : W);
-  P.div_groups = FastDiv(wide ? H * W / vec : H * W);
-  P.planes_per_pass = std::max(1u, 0x7fffffffu / (wide ? H * W / vec : H * W));
   hipStream_t st = as_stream(stream);
-  const uint32_t tc = num_tiles * C;
-  if (((wide ? H * W / vec : H * W) + kBnThreads - 1u) / kBnThreads > 65535u) return ADH_EINVAL;  // grid.y
-  const dim3 rgrid(tc * P.split), agrid = bn_apply_grid(&P, wide ? H * W / vec : H * W);
+  const uint32_t tc = num_tiles * C, vec = (uint32_t)(16 / es);
+  const bool wide = dy_halo ? bn_runs(&P, W, H, vec) : bn_runs(&P, H * W, 1u, vec);
+  if ((P.groups_per_plane + kBnThreads - 1u) / kBnThreads > 65535u) return ADH_EINVAL;  // grid.y
+  const bool stream_data = bn_stream((uint64_t)tc * N * H * W * es * 2u);
   P.beta = beta_data;
   P.beta_param = beta_param;
-  if (dtype == ADH_F32) {
-    if (wide) hipLaunchKernelGGL((bn_reduce_kernel<float, true, 4>), rgrid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_reduce_kernel<float, true, 1>), rgrid, dim3(kBnThreads), 0, st, P);
-  } else {
-    if (wide) hipLaunchKernelGGL((bn_reduce_kernel<uint16_t, true, 8>), rgrid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_reduce_kernel<uint16_t, true, 1>), rgrid, dim3(kBnThreads), 0, st, P);
-  }
-  if (dtype == ADH_F32) {
-    if (wide) hipLaunchKernelGGL((bn_apply_kernel<float, 2, 4>), agrid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_apply_kernel<float, 2, 1>), agrid, dim3(kBnThreads), 0, st, P);
-  } else {
-    if (wide) hipLaunchKernelGGL((bn_apply_kernel<uint16_t, 2, 8>), agrid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_apply_kernel<uint16_t, 2, 1>), agrid, dim3(kBnThreads), 0, st, P);
-  }
+  const dim3 rgrid(tc * P.split), agrid = bn_apply_grid(&P, P.groups_per_plane, true);
+  bn_launch(stream_data, dtype, [&](auto s, auto t) {
+    typedef decltype(t) T;
+    if (wide) {
+      hipLaunchKernelGGL((bn_reduce_kernel<T, true, 16 / sizeof(T), s>), rgrid, dim3(kBnThreads), 0, st, P);
+      hipLaunchKernelGGL((bn_apply_kernel<T, 2, 16 / sizeof(T), s>), agrid, dim3(kBnThreads), 0, st, P);
+    } else {
+      hipLaunchKernelGGL((bn_reduce_kernel<T, true, 1, false>), rgrid, dim3(kBnThreads), 0, st, P);
+      hipLaunchKernelGGL((bn_apply_kernel<T, 2, 1, false>), agrid, dim3(kBnThreads), 0, st, P);
+    }
+  });
   return launch_status();
 }
 
