@@ -11,6 +11,7 @@
 //             dx coalesced.  y is not read: the maximum is recomputed from the staged input.
 // Direct kernels (rows too wide for LDS, windows of more than 256 elements): one thread per
 //   output (forward) or per padded element (backward), window reads served by the caches.
+// 3x3 / 2 max pooling over tiles without halo has kernels of its own (pool_fwd_max3s2_kernel, pool_bwd_max3s2_kernel).
 // Tiles without halo (the UNP instances of the banded kernels): the tiles are the row tiles of one tensor in rank
 //   order; a block stages its band of the PADDED tile into LDS element by element, reading rows outside the
 //   tile from the neighbouring tiles and zeros outside the tensor, and then works as over a padded tile.
@@ -21,6 +22,7 @@
 #include "adh_common.h"
 
 #include <algorithm>
+#include <type_traits>
 
 namespace adh {
 
@@ -608,73 +610,173 @@ static void launch_bwd_band(int dtype, bool max, const PoolParams &P, uint32_t b
   launch_bwd_band_u<false>(dtype, max, P, blocks, lds, st);
 }
 
-// Backward of 3x3 max pooling at stride 2, padding 1, over tiles of even height without halo and rows of whole groups of four.
-// A thread owns four columns (the two windows that start there and the next one's first column) and marches down a band of
-// window rows of the stacked tensor: a step loads two input rows, finds where the three windows of this row have their first
-// maximum (a row's own is shared by the window rows above and below it) and stores the two input rows that no later window
-// touches.  No LDS, no barrier; the next step's loads are in flight during this one's work.  Bound by memory.
-// Measured, 32 x 64 planes, 4 tiles of 64 x 256, fp32: 389 us through LDS bands (3.4 TB/s of what has to be moved), 246 here (5.5).
+// 3x3 max pooling at stride 2, padding 1, over tiles of even height without halo (rows of at least one group of columns).
+// A thread owns NC columns (16 bytes of a row) and marches down a band of window rows of the stacked tensor.  No LDS, no
+// barrier; the next step's loads are in flight during this one's work (and have arrived before its stores go out, or the
+// next step would wait for those too: 82 against 102 us).  Bound by memory.  Bands of 32 window rows; 8: 8 % slower, 64: no faster.
+// Measured against the LDS bands, which stage rows that are no whole 16-byte groups one element at a time: 18 x 482 planes of
+// 6 x 350, fp32: forward 33 -> 19.5 us, backward 82 -> 41; bf16, 36 x 100 planes of 14 x 333: 31 -> 13, 62 -> 35.  32 x 64 planes,
+// 4 tiles of 48 x 128, fp32: forward 80 -> 43, and at 64 x 256: forward 126 -> 138, backward 389 -> 247; bf16: 127 -> 83, 194
+// (four columns a thread) -> 145.
 struct PoolS2Params {
   const void *x[ADH_MAX_TILES], *dy[ADH_MAX_TILES];
-  void *dx[ADH_MAX_TILES];
+  void *out[ADH_MAX_TILES];  // y (forward) or dx
   uint32_t items;  // planes x groups of columns
   uint32_t K, H, W, OH, OW, steps;  // steps: window rows per band
   float beta;
   FastDiv div_groups, div_H, div_OH;
 };
 template <typename T, int V>
+struct __attribute__((packed, aligned(sizeof(T)))) S2Pack { T e[V]; };
+template <bool STREAM, int V, typename T>
 __device__ __forceinline__ void load_f(const T *p, float (&f)[V]) {
-  struct alignas(V * sizeof(T)) Pack { T e[V]; };
-  const Pack v = *reinterpret_cast<const Pack *>(p);
+  const S2Pack<T, V> v = load_vec<STREAM, S2Pack<T, V>>(p);
 #pragma unroll
   for (int i = 0; i < V; ++i) f[i] = ld_f(v.e, i);
 }
-template <typename T>
-__global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const PoolS2Params P) {
+// f[k] = f[k + s], zero beyond the end
+template <int V>
+__device__ __forceinline__ void shift_down(float (&f)[V], uint32_t s) {
+#pragma unroll
+  for (int b = 1; b < V; b *= 2)
+#pragma unroll
+    for (int k = 0; k < V; ++k) {
+      const float v = k + b < V ? f[k + b] : 0.f;
+      f[k] = s & (uint32_t)b ? v : f[k];
+    }
+}
+// Columns c - 1 .. c + NC + 1 of row R of the stacked tensor; what a place beyond the row's ends or the tensor's holds is zero
+// (it is loaded from an existing one).  TAILS: rows are no whole groups; the last group's vector ends with the row.
+template <int NC>
+struct S2Row { float l[1], v[NC], r[2]; };
+template <typename T, int NC, bool TAILS, bool STREAM, bool RIGHT>
+__device__ __forceinline__ S2Row<NC> s2_load_row(const PoolS2Params &P, uint32_t plane, uint32_t c, uint32_t R) {
+  S2Row<NC> q;
+  uint32_t t, r;
+  const bool ok = R < P.K * P.H;
+  P.div_H.divmod(ok ? R : 0u, t, r);
+  const T *p = reinterpret_cast<const T *>(P.x[t]) + ((size_t)plane * P.H + r) * P.W;
+  const uint32_t at = TAILS ? min(c, P.W - NC) : c, cr = min(c + NC, P.W - 2u);
+  load_f<STREAM, NC>(p + at, q.v);
+  load_f<false, 1>(p + (c ? c - 1u : 0u), q.l);
+  if (RIGHT) load_f<false, 2>(p + cr, q.r);
+  if (TAILS) shift_down(q.v, c - at);
+  if (!ok || c == 0u) q.l[0] = 0.f;
+  if (RIGHT) {
+    if (TAILS && cr + 1u == c + NC) q.r[0] = q.r[1];
+    if (!ok || c + NC >= P.W) q.r[0] = 0.f;
+    if (!ok || c + NC + 1u >= P.W) q.r[1] = 0.f;
+  }
+  if (!ok)
+#pragma unroll
+    for (int k = 0; k < NC; ++k) q.v[k] = 0.f;
+  return q;
+}
+template <typename T, bool TAILS, int V>
+__device__ __forceinline__ void s2_store(T *p, const float (&f)[V], uint32_t count, bool stream) {
+  S2Pack<T, V> v;
+#pragma unroll
+  for (int k = 0; k < V; ++k) st_f(v.e, k, f[k]);
+  if (!TAILS || count >= (uint32_t)V) {
+    if (stream) store_vec<true>(p, v);
+    else store_vec<false>(p, v);
+  } else {
+#pragma unroll
+    for (int k = 0; k < V - 1; ++k)
+      if ((uint32_t)k < count) p[k] = v.e[k];
+  }
+}
+
+// waits for what is on its way to these registers: before a step's stores, so that the next step does not wait for those
+template <int V>
+__device__ __forceinline__ void arrived(const float (&f)[V]) {
+#pragma unroll
+  for (int k = 0; k < V; ++k) asm volatile("" ::"v"(f[k]));
+}
+
+template <typename T, bool TAILS, bool STREAM>
+__global__ __launch_bounds__(kPoolThreads) void pool_fwd_max3s2_kernel(const PoolS2Params P) {
+  constexpr int NC = 16 / sizeof(T), NW = NC / 2;
   const uint32_t id = blockIdx.x * kPoolThreads + threadIdx.x;
   if (id >= P.items) return;
   uint32_t plane, c;
   P.div_groups.divmod(id, plane, c);
-  c *= 4u;
-  const uint32_t VH = P.K * P.H, VO = P.K * P.OH;
-  // what a place beyond the row's ends or the tensor's holds is zero; it is loaded from an existing one
-  struct Row { float l[1], v[4], r[2]; };
-  const uint32_t cl = c ? c - 1u : 0u, cr = c + 4u < P.W ? c + 4u : c;
-  auto load_row = [&](uint32_t R) {
-    Row q;
-    uint32_t t, r;
-    const bool ok = R < VH;
-    P.div_H.divmod(ok ? R : 0u, t, r);
-    const T *p = reinterpret_cast<const T *>(P.x[t]) + ((size_t)plane * P.H + r) * P.W;
-    load_f<T, 4>(p + c, q.v);
-    load_f<T, 1>(p + cl, q.l);
-    load_f<T, 2>(p + cr, q.r);
-    if (!ok || c == 0u) q.l[0] = 0.f;
-    if (!ok || c + 4u >= P.W) q.r[0] = q.r[1] = 0.f;
-    if (!ok) q.v[0] = q.v[1] = q.v[2] = q.v[3] = 0.f;
-    return q;
+  c *= NC;
+  auto load_row = [&](uint32_t R) { return s2_load_row<T, NC, TAILS, STREAM, false>(P, plane, c, R); };
+  struct Best { float b[NW]; };
+  auto best_of = [](const S2Row<NC> &q) {  // nothing exceeds -inf, as for NaN
+    Best m;
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      const float e[3] = {w ? q.v[2 * w - 1] : q.l[0], q.v[2 * w], q.v[2 * w + 1]};
+      m.b[w] = -__builtin_inff();
+#pragma unroll
+      for (int k = 0; k < 3; ++k) m.b[w] = e[k] > m.b[w] ? e[k] : m.b[w];
+    }
+    return m;
   };
-  struct Grad { float v[2], n[1]; };  // of the three windows
-  const uint32_t ow = c / 2u, on = ow + 2u < P.OW ? ow + 2u : ow;
+  const uint32_t VO = P.K * P.OH, o_lo = blockIdx.y * P.steps, o_hi = min(VO, o_lo + P.steps);
+  if (o_lo >= o_hi) return;
+  Best top = best_of(load_row(2u * o_lo - 1u));  // (row -1: none)
+  S2Row<NC> r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
+  for (uint32_t o = o_lo; o < o_hi; ++o) {
+    const S2Row<NC> n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
+    const Best mid = best_of(r0), bot = best_of(r1);
+    float f[NW];
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      f[w] = mid.b[w] > top.b[w] ? mid.b[w] : top.b[w];
+      f[w] = bot.b[w] > f[w] ? bot.b[w] : f[w];
+    }
+    arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l);
+    uint32_t t, r;
+    P.div_OH.divmod(o, t, r);
+    s2_store<T, TAILS, NW>(reinterpret_cast<T *>(P.out[t]) + ((size_t)plane * P.OH + r) * P.OW + c / 2u, f, P.OW - c / 2u, false);
+    top = bot;
+    r0 = n0; r1 = n1;
+  }
+}
+
+// A step loads two input rows, finds where the windows of this row that touch the thread's columns (the last one with its
+// first column only) have their first maximum (a row's own is shared by the window rows above and below it) and stores the
+// two input rows that no later window touches.
+template <typename T, bool TAILS, bool STREAM>
+__global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const PoolS2Params P) {
+  constexpr int NC = 16 / sizeof(T), NW = NC / 2;
+  const uint32_t id = blockIdx.x * kPoolThreads + threadIdx.x;
+  if (id >= P.items) return;
+  uint32_t plane, c;
+  P.div_groups.divmod(id, plane, c);
+  c *= NC;
+  const uint32_t VO = P.K * P.OH;
+  auto load_row = [&](uint32_t R) { return s2_load_row<T, NC, TAILS, STREAM, true>(P, plane, c, R); };
+  struct Grad { float v[NW], n[1]; };  // of the windows
+  const uint32_t ow = c / 2u, ow_at = TAILS ? min(ow, P.OW - NW) : ow, on = ow + NW < P.OW ? ow + NW : ow;
   auto load_dy = [&](uint32_t o) {
     Grad q;
     uint32_t t, r;
     const bool ok = o < VO;
     P.div_OH.divmod(ok ? o : 0u, t, r);
     const T *p = reinterpret_cast<const T *>(P.dy[t]) + ((size_t)plane * P.OH + r) * P.OW;
-    load_f<T, 2>(p + ow, q.v);
-    load_f<T, 1>(p + on, q.n);
+    load_f<false, NW>(p + ow_at, q.v);
+    load_f<false, 1>(p + on, q.n);
+    if (TAILS) shift_down(q.v, ow - ow_at);
     if (!ok || on == ow) q.n[0] = 0.f;
-    if (!ok) q.v[0] = q.v[1] = 0.f;
+    if (!ok)
+#pragma unroll
+      for (int k = 0; k < NW; ++k) q.v[k] = 0.f;
     return q;
   };
   // first maximum of a row's three window columns, per window (nothing exceeds -inf: the first place, as for NaN)
-  struct Best { float b[3]; uint32_t at[3]; };
-  auto best_of = [](const Row &q) {
-    const float e[7] = {q.l[0], q.v[0], q.v[1], q.v[2], q.v[3], q.r[0], q.r[1]};
+  struct Best { float b[NW + 1]; uint32_t at[NW + 1]; };
+  auto best_of = [](const S2Row<NC> &q) {
+    float e[NC + 3];
+    e[0] = q.l[0]; e[NC + 1] = q.r[0]; e[NC + 2] = q.r[1];
+#pragma unroll
+    for (int k = 0; k < NC; ++k) e[k + 1] = q.v[k];
     Best m;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
+    for (int w = 0; w <= NW; ++w) {
       m.b[w] = -__builtin_inff();
       m.at[w] = 0u;
 #pragma unroll
@@ -683,94 +785,90 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
     }
     return m;
   };
-  struct Windows { uint32_t at[3]; float g[3]; };  // where in 3 x 3, and the gradient
+  struct Windows { uint32_t at[NW + 1]; float g[NW + 1]; };  // where in 3 x 3, and the gradient
   auto windows_of = [](const Best &top, const Best &mid, const Best &bot, const Grad &g) {
     Windows q;
 #pragma unroll
-    for (int w = 0; w < 3; ++w) {
+    for (int w = 0; w <= NW; ++w) {
       float b = top.b[w];
       q.at[w] = top.at[w];
       if (mid.b[w] > b) { b = mid.b[w]; q.at[w] = 3u + mid.at[w]; }
       if (bot.b[w] > b) q.at[w] = 6u + bot.at[w];
+      q.g[w] = w < NW ? g.v[w < NW ? w : 0] : g.n[0];
     }
-    q.g[0] = g.v[0]; q.g[1] = g.v[1]; q.g[2] = g.n[0];
     return q;
   };
-  // adds what row `k` (of three) of the windows gives the four columns: even windows first, as everywhere in this file
-  auto add = [](float (&f)[4], const Windows &q, uint32_t k) {
+  // adds what row `k` (of three) of the windows gives the columns: even windows first, as everywhere in this file
+  auto add = [](float (&f)[NC], const Windows &q, uint32_t k) {
     auto hit = [&](int w, uint32_t col) { return q.at[w] == 3u * k + col ? q.g[w] : 0.f; };
-    f[0] += hit(0, 1u);
-    f[1] += hit(0, 2u);
-    f[1] += hit(1, 0u);
-    f[2] += hit(1, 1u);
-    f[3] += hit(2, 0u);
-    f[3] += hit(1, 2u);
+#pragma unroll
+    for (int w = 0; w < NW; ++w) {
+      f[2 * w] += hit(w, 1u);
+      const int even = w & 1 ? w + 1 : w, odd = w & 1 ? w : w + 1;  // column 2 w + 1 is the third of window w, the first of w + 1
+      f[2 * w + 1] += hit(even, even == w ? 2u : 0u);
+      f[2 * w + 1] += hit(odd, odd == w ? 2u : 0u);
+    }
   };
-  auto store_row = [&](uint32_t R, float (&f)[4]) {
+  auto store_row = [&](uint32_t R, float (&f)[NC]) {
     uint32_t t, r;
     P.div_H.divmod(R, t, r);
-    T *p = reinterpret_cast<T *>(P.dx[t]) + ((size_t)plane * P.H + r) * P.W + c;
+    T *p = reinterpret_cast<T *>(P.out[t]) + ((size_t)plane * P.H + r) * P.W + c;
     if (P.beta != 0.f) {
-      float old[4];
-      load_f<T, 4>(p, old);
 #pragma unroll
-      for (int k = 0; k < 4; ++k) f[k] += old[k];
+      for (int k = 0; k < NC; ++k)
+        if (!TAILS || c + (uint32_t)k < P.W) f[k] += ld_f(p, k);
     }
-    struct alignas(4 * sizeof(T)) Pack { T e[4]; } v;
-#pragma unroll
-    for (int k = 0; k < 4; ++k) st_f(v.e, k, f[k]);
-    *reinterpret_cast<Pack *>(p) = v;
+    s2_store<T, TAILS, NC>(p, f, P.W - c, STREAM);
   };
 
   const uint32_t o_lo = blockIdx.y * P.steps, o_hi = min(VO + 1u, o_lo + P.steps);  // (step VO: the last input row)
-  Windows above = {{9u, 9u, 9u}, {0.f, 0.f, 0.f}};
+  Windows above;
   Best top;
   if (o_lo > 0u) {
-    const Row a = load_row(2u * o_lo - 3u), b = load_row(2u * o_lo - 2u), d = load_row(2u * o_lo - 1u);  // (row -1: none)
+    const S2Row<NC> a = load_row(2u * o_lo - 3u), b = load_row(2u * o_lo - 2u), d = load_row(2u * o_lo - 1u);  // (row -1: none)
     const Grad g = load_dy(o_lo - 1u);
     top = best_of(d);
     above = windows_of(best_of(a), best_of(b), top, g);
   } else {
     top = best_of(load_row(~0u));
+#pragma unroll
+    for (int w = 0; w <= NW; ++w) { above.at[w] = 9u; above.g[w] = 0.f; }
   }
-  Row r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
+  S2Row<NC> r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
   Grad g = load_dy(o_lo);
   for (uint32_t o = o_lo; o < o_hi; ++o) {
-    const Row n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
+    const S2Row<NC> n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
     const Grad ng = load_dy(o + 1u);
     const Best bot = best_of(r1);
     const Windows here = windows_of(top, best_of(r0), bot, g);
-    if (o > 0u) {
-      // the windows of even rows of the tile that the input row belongs to first
-      float f[4] = {0.f, 0.f, 0.f, 0.f};
-      const uint32_t t = P.div_OH.div(o - 1u);
-      if (((o - 1u - t * P.OH) & 1u) == 0u) {
-        add(f, above, 2u);
-        add(f, here, 0u);
-      } else {
-        add(f, here, 0u);
-        add(f, above, 2u);
-      }
-      store_row(2u * o - 1u, f);
+    float f0[NC] = {}, f1[NC] = {};  // rows 2 o - 1 and 2 o
+    // the windows of even rows of the tile that the input row belongs to first
+    const uint32_t before = o > 0u ? o - 1u : 0u;
+    if (((before - P.div_OH.div(before) * P.OH) & 1u) == 0u) {
+      add(f0, above, 2u);
+      add(f0, here, 0u);
+    } else {
+      add(f0, here, 0u);
+      add(f0, above, 2u);
     }
-    if (o < VO) {
-      float f[4] = {0.f, 0.f, 0.f, 0.f};
-      add(f, here, 1u);
-      store_row(2u * o, f);
-    }
+    add(f1, here, 1u);
+    arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l); arrived(n0.r); arrived(n1.r); arrived(ng.v); arrived(ng.n);
+    if (o > 0u) store_row(2u * o - 1u, f0);
+    if (o < VO) store_row(2u * o, f1);
     above = here;
     top = bot;
     r0 = n0; r1 = n1; g = ng;
   }
 }
-// 3x3 / 2, padding 1, rows and addresses of whole groups of four (dy: of two); anything else takes the bands
-static bool pool_bwd_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
-  if (P.wh != 3u || P.ww != 3u || P.sh != 2u || P.sw != 2u || P.pad_h != 1u || P.pad_w != 1u || P.W % 4u != 0u) return false;
-  const uint64_t items = (uint64_t)P.planes * (P.W / 4u), rows = (uint64_t)P.num_tiles * P.H;
+
+// 3x3 / 2, padding 1, rows of at least a group of columns; anything else takes the bands
+static bool pool_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
+  const uint32_t nc = (uint32_t)(16u / es), groups = (P.W + nc - 1u) / nc;
+  if (P.wh != 3u || P.ww != 3u || P.sh != 2u || P.sw != 2u || P.pad_h != 1u || P.pad_w != 1u || P.W < nc) return false;
+  const uint64_t items = (uint64_t)P.planes * groups, rows = (uint64_t)P.num_tiles * P.H;
   if (items >= (1ull << 31) || rows >= (1ull << 31)) return false;
   for (uint32_t t = 0; t < P.num_tiles; ++t) {
-    if (!aligned_to(P.x[t], 4 * es) || !aligned_to(P.out[t], 4 * es) || !aligned_to(P.dy[t], 2 * es)) return false;
-    q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->dx[t] = P.out[t];
+    q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->out[t] = P.out[t];
   }
   q->items = (uint32_t)items;
   q->K = P.num_tiles; q->H = P.H; q->W = P.W; q->OH = P.OH; q->OW = P.OW;
@@ -780,8 +878,27 @@ static bool pool_bwd_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
   const uint64_t waves = (items + 63u) / 64u;
   while (q->steps > 2u && waves * (P.num_tiles * P.OH / q->steps + 1u) < 256u * 16u) q->steps /= 2u;
   if (P.num_tiles * P.OH / q->steps >= 65535u) return false;
-  q->div_groups = FastDiv(P.W / 4u); q->div_H = FastDiv(P.H); q->div_OH = FastDiv(P.OH);
+  q->div_groups = FastDiv(groups); q->div_H = FastDiv(P.H); q->div_OH = FastDiv(P.OH);
   return true;
+}
+// non-temporal accesses where the input is larger than the on-package cache
+template <bool FWD>
+static int launch_max3s2(int dtype, const PoolParams &P, const PoolS2Params &q, hipStream_t st) {
+  const size_t es = dtype_size(dtype);
+  const bool tails = q.W % (16u / es) != 0u, stream = (uint64_t)P.planes * q.K * q.H * q.W * es > (256ull << 20);
+  const dim3 grid((q.items + kPoolThreads - 1u) / kPoolThreads, (q.K * q.OH + q.steps) / q.steps), block(kPoolThreads);
+  auto go = [&](auto tl, auto sm) {
+    auto kernel = [&](auto t) {
+      typedef decltype(t) T;
+      if constexpr (FWD) hipLaunchKernelGGL((pool_fwd_max3s2_kernel<T, tl, sm>), grid, block, 0, st, q);
+      else hipLaunchKernelGGL((pool_bwd_max3s2_kernel<T, tl, sm>), grid, block, 0, st, q);
+    };
+    if (dtype == ADH_F32) kernel(0.f);
+    else kernel(uint16_t(0));
+  };
+  if (tails) stream ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  else stream ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+  return launch_status();
 }
 
 // Tiles without halo: fills the padded extents and the split's fields; the same limits as the convolution over
@@ -954,6 +1071,8 @@ int adh_pool2d_unpadded_fwd_tiles(int dtype, int mode, uint32_t num_tiles, uint3
   pool_unpadded_vectors(&P, es, num_tiles, false);
   const uint32_t band_rows = pick_band_rows(P, num_tiles, kPoolBandBytes, [&](uint32_t r) { return fwd_band_lds(P, es, r); });
   if (!band_rows) return ADH_EUNIMPL;  // rows too wide for a band in LDS: use the padded entry points
+  PoolS2Params q = {};
+  if (mode == ADH_POOL_MAX && pool_max3s2(P, es, &q)) return launch_max3s2<true>(dtype, P, q, as_stream(stream));
   set_bands(&P, band_rows);
   launch_fwd_band_u<true>(dtype, mode == ADH_POOL_MAX, P, P.planes * num_tiles * P.bands, fwd_band_lds(P, es, band_rows),
                           as_stream(stream));
@@ -993,12 +1112,7 @@ int adh_pool2d_unpadded_bwd_tiles(int dtype, int mode, uint32_t num_tiles, uint3
       wh * ww > 256u ? 0u : pick_band_rows(P, num_tiles, bwd_band_aim(P, es, is_max), [&](uint32_t r) { return bwd_band_lds(P, es, is_max, r); });
   if (!band_rows) return ADH_EUNIMPL;
   PoolS2Params q = {};
-  if (is_max && pool_bwd_max3s2(P, es, &q)) {
-    const dim3 grid((q.items + kPoolThreads - 1u) / kPoolThreads, (q.K * q.OH + q.steps) / q.steps), block(kPoolThreads);
-    if (dtype == ADH_F32) hipLaunchKernelGGL((pool_bwd_max3s2_kernel<float>), grid, block, 0, as_stream(stream), q);
-    else hipLaunchKernelGGL((pool_bwd_max3s2_kernel<uint16_t>), grid, block, 0, as_stream(stream), q);
-    return launch_status();
-  }
+  if (is_max && pool_max3s2(P, es, &q)) return launch_max3s2<false>(dtype, P, q, as_stream(stream));
   set_bands(&P, band_rows);
   launch_bwd_band_u<true>(dtype, is_max, P, P.planes * num_tiles * P.bands, bwd_band_lds(P, es, is_max, band_rows),
                           as_stream(stream));

@@ -1,7 +1,7 @@
 """Backward of 3x3 max pooling at stride 2 over tiles without halo, rows of whole groups of four: the kernel that keeps its
 windows in registers, at the sizes where it can go wrong (one group of columns, tiles of two rows, an odd number of window rows
-per tile, bands of every length), against the oracle's pooling of the unsplit padded tensor; the alignment that leaves it to
-the banded kernel; ties, infinities and NaN against that kernel."""
+per tile, bands of every length), against the oracle's pooling of the unsplit padded tensor; ties, infinities and NaN with
+tiles off their alignment (test_gpu_pool_max3s2_widths.py: against the banded kernel)."""
 import pytest
 import torch
 
@@ -18,7 +18,7 @@ def test_vs_unsplit_oracle(oracle, K, N, C, Ht, W):
 
 
 def _backward(xs, dys, shape, offset=0):
-    """offset: elements by which the gradient tiles are off their alignment, where the banded kernel serves the call."""
+    """offset: elements by which the gradient tiles are off their alignment."""
     N, C, Ht, W = shape
     gs = [torch.empty(N * C * Ht * W + offset, device="cuda", dtype=xs[0].dtype)[offset:].view(shape) for _ in xs]
     capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, xs, None, dys, gs, *shape, 3, 3, 2, 2, 1, 1), "bwd")

@@ -1,0 +1,69 @@
+"""3x3 max pooling at stride 2 over tiles without halo at any row length, forward and backward, by the kernels that keep
+their windows in registers: every remainder of a group of columns (4 fp32, 8 bf16), rows of one group, bit for bit against the
+banded kernels, which serve the same pooling over one halo-padded tile."""
+import pytest
+import torch
+import torch.nn.functional as F
+
+from arraydiff_cuda_amd import capi
+
+pytestmark = pytest.mark.gpu
+
+WINDOW = (3, 3, 2, 2)
+
+
+def _inputs(dtype, K, N, C, Ht, W, seed):
+    """Values of few levels, so that most windows have ties, and some special ones."""
+    g = torch.Generator().manual_seed(seed)
+    x = torch.randint(-2, 3, (N, C, Ht * K, W), generator=g).float()
+    special = torch.tensor([float("inf"), -float("inf"), float("nan"), torch.finfo(dtype).min, -0.0])
+    where = torch.rand(x.shape, generator=g) < 0.2
+    x[where] = special[torch.randint(0, 5, (int(where.sum()),), generator=g)]
+    dy = torch.randn((N, C, Ht * K // 2, (W - 1) // 2 + 1), generator=g)
+    return x.to(dtype).cuda(), dy.to(dtype).cuda()
+
+
+def _same(a, b):
+    return torch.equal(a.nan_to_num(nan=123.0), b.nan_to_num(nan=123.0)) and torch.equal(torch.signbit(a), torch.signbit(b))
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("W", [4, 5, 6, 7, 8, 9, 10, 11, 12, 13, 14, 15, 16, 17, 31, 255, 350, 515])
+@pytest.mark.parametrize("K,Ht", [(1, 6), (3, 8)])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_same_as_the_banded_kernels(dtype, W, K, Ht, beta):
+    N, C, H, OW = 2, 3, Ht * K, (W - 1) // 2 + 1
+    x, dy = _inputs(dtype, K, N, C, Ht, W, W)
+    xs = [t.contiguous() for t in x.chunk(K, 2)]
+    dys = [t.contiguous() for t in dy.chunk(K, 2)]
+    ys = [torch.full_like(t, 7.0) for t in dys]
+    old = torch.randint(-4, 5, x.shape, generator=torch.Generator().manual_seed(9)).to(dtype).cuda()
+    dxs = [t.clone().contiguous() for t in old.chunk(K, 2)]
+    capi.check(capi.pool_unpadded_fwd_tiles(capi.ADH_POOL_MAX, xs, ys, N, C, Ht, W, *WINDOW, 1, 1), "forward")
+    capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, xs, None, dys, dxs, N, C, Ht, W, *WINDOW, 1, 1, beta=beta), "backward")
+    padded = F.pad(x, (1, 1, 1, 1))
+    want_y, want_dx = torch.empty((N, C, H // 2, OW), device="cuda", dtype=dtype), F.pad(old, (1, 1, 1, 1))
+    capi.check(capi.pool_fwd_tiles(capi.ADH_POOL_MAX, [padded], [want_y], N, C, H + 2, W + 2, *WINDOW), "padded forward")
+    capi.check(capi.pool_bwd_tiles(capi.ADH_POOL_MAX, [padded], [want_y], [dy], [want_dx], N, C, H + 2, W + 2, *WINDOW, beta=beta), "padded backward")
+    assert _same(torch.cat(ys, 2), want_y)
+    assert _same(torch.cat(dxs, 2), want_dx[:, :, 1:-1, 1:-1])
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_larger_than_the_cache(dtype):
+    """Where the accesses are non-temporal."""
+    N, C, Ht, W, K = 2, 33, 512 if dtype is torch.float32 else 1024, 1100, 2
+    x, dy = _inputs(dtype, K, N, C, Ht, W, 3)
+    assert x.numel() * x.element_size() > 256 << 20
+    xs = [t.contiguous() for t in x.chunk(K, 2)]
+    dys = [t.contiguous() for t in dy.chunk(K, 2)]
+    ys, dxs = [torch.empty_like(t) for t in dys], [torch.empty_like(t) for t in xs]
+    capi.check(capi.pool_unpadded_fwd_tiles(capi.ADH_POOL_MAX, xs, ys, N, C, Ht, W, *WINDOW, 1, 1), "forward")
+    capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, xs, None, dys, dxs, N, C, Ht, W, *WINDOW, 1, 1), "backward")
+    for n in range(N):  # one image is small enough for the cache
+        small, sdy = [t[n:n + 1].contiguous() for t in xs], [t[n:n + 1].contiguous() for t in dys]
+        y1, d1 = [torch.empty_like(t) for t in sdy], [torch.empty_like(t) for t in small]
+        capi.check(capi.pool_unpadded_fwd_tiles(capi.ADH_POOL_MAX, small, y1, 1, C, Ht, W, *WINDOW, 1, 1), "forward")
+        capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, small, None, sdy, d1, 1, C, Ht, W, *WINDOW, 1, 1), "backward")
+        for t in range(K):
+            assert _same(ys[t][n:n + 1], y1[t]) and _same(dxs[t][n:n + 1], d1[t])
