@@ -19,8 +19,8 @@
 //
 // Measured, fp32, 64 channels, 32 images, 4 tiles of 64 x 256 (537 MB a tensor), before (temporal accesses, one group in
 // flight, coefficients before the loads) -> now: reduce 123 -> 86 us (6.2 TB/s), backward 225 -> 165 to 190; apply 240 -> 207,
-// backward 320 -> 283 (5.7 TB/s).  bf16, 100 channels, 9 images, 4 tiles of 14 x 333 (before: element by element): reduce 23 -> 10.6,
-// backward 31 -> 16.6; apply 25 -> 22, backward 56 -> 34.
+// backward 320 -> 283 (5.7 TB/s).  bf16, 100 channels, 9 images, 4 tiles of 14 x 333, both passes: 135 -> 87 (the backward apply pass
+// 56 -> 34: its groups no longer end where rows do; the sums stay element by element, eight in flight).
 #include "adh_common.h"
 
 #include <algorithm>
@@ -47,7 +47,7 @@ struct BnParams {
   uint32_t run;  // elements that lie side by side in both tensors of a pass: the plane, or (padded gradient) a row
   float eps, beta, beta_param;  // beta: input-gradient accumulation; beta_param: parameter-gradient accumulation
   int relu;
-  FastDiv div_C, div_N, div_split, div_groups, div_cols;  // div_groups: the 16-byte groups of a plane; div_cols: row length of the index that a kernel splits into (row, column)
+  FastDiv div_C, div_N, div_split, div_groups, div_cols;  // div_groups: what a plane is numbered by; div_cols: row length of the index that a kernel splits into (row, column)
 };
 
 __device__ __forceinline__ float bn_ld(const float *p, size_t i) { return p[i]; }
@@ -86,13 +86,13 @@ __device__ __forceinline__ float2 block_sum2(float a, float b) {
 
 // grid: tiles * C * split.  BWD = false: sums of (x - K), (x - K)^2.  BWD = true: sums of dy', dy' * (x - mean)
 // (dy' = dy where a*(x - mean) + shift > 0 when the rectifier was fused, else dy), dy at the interior of a tile padded by p.
-// A run of P.run elements (a row of a padded gradient, else the whole plane) is whole groups of VEC; the last group ends
-// with the run and leaves out what it shares with the one before.
-// Four groups a thread are loaded before the first is added: with one, the loads in flight bound it (DRAM latency).
+// VEC > 1: H*W (and, backward, W) are whole numbers of VEC-element groups, one 16-byte access per group.
+// U groups a thread are loaded before the first is added (with one, the latency of a load bounds it), and are added in the
+// order of a thread that takes one at a time: what a sum rounds to decides where activations tie in a pooling window.
 template <typename T, bool BWD, int VEC, bool STREAM>
 __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P) {
   typedef BnVec<T, VEC> Vec;
-  constexpr int U = 4;
+  constexpr int U = VEC > 1 ? 4 : 8;
   uint32_t tc, sp, tile, c;
   P.div_split.divmod(blockIdx.x, tc, sp);
   P.div_C.divmod(tc, tile, c);
@@ -104,31 +104,33 @@ __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P)
   const float mean = BWD ? P.mean_in[tile][c] : bn_ld(x, (size_t)c * P.HW);
   const float a = BWD && P.relu ? P.scale[tile][c] * P.second_in[tile][c] : 0.f;
   const float b = BWD && P.relu ? P.shift[tile][c] : 0.f;
+  const uint32_t groups = P.HW / (uint32_t)VEC;
   float s1 = 0.f, s2 = 0.f;
   // the groups of the split's planes are numbered through: a plane of a few groups (a late layer's 4 x 16 tile
   // is 16 of them) would otherwise leave most of the workgroup idle for one load latency per plane
   // (P.planes_per_pass planes at a time keep the running number below 2^31: one pass but for gigantic planes)
   for (uint32_t nb = n0; nb < n1; nb += P.planes_per_pass) {
-    const uint32_t items = min(P.planes_per_pass, n1 - nb) * P.groups_per_plane;
-    for (uint32_t it0 = threadIdx.x; it0 < items; it0 += U * kBnThreads) {
-      Vec xv[U], dv[U];
-      uint32_t skip[U];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint32_t it = it0 + (uint32_t)u * kBnThreads;
-        uint32_t nr, i, h, w;
-        P.div_groups.divmod(it < items ? it : it0, nr, i);
-        P.div_cols.divmod(i, h, w);  // groups of a run
-        const uint32_t at = min(w * VEC, P.run - VEC);
-        skip[u] = it < items ? w * VEC - at : VEC;
-        const size_t plane = (size_t)(nb + nr) * P.C + c;
-        xv[u] = load_vec<STREAM, Vec>(x + plane * P.HW + (size_t)h * P.run + at);
-        if (BWD) dv[u] = load_vec<STREAM, Vec>(dy + plane * HPp * WP + (size_t)(h + P.p) * WP + P.p + at);
+    const uint32_t items = min(P.planes_per_pass, n1 - nb) * groups;
+    auto load = [&](uint32_t it, Vec &xv, Vec &dv) {
+      uint32_t nr, i;
+      P.div_groups.divmod(it, nr, i);
+      const size_t plane = (size_t)(nb + nr) * P.C + c;
+      xv = load_vec<STREAM, Vec>(x + plane * P.HW + (size_t)i * VEC);
+      if (!BWD) return;
+      if (P.p == 0u) {
+        dv = load_vec<STREAM, Vec>(dy + plane * P.HW + (size_t)i * VEC);
+      } else {
+        uint32_t h, w;
+        P.div_cols.divmod(i, h, w);  // groups per row
+        dv = load_vec<STREAM, Vec>(dy + plane * HPp * WP + (size_t)(h + P.p) * WP + P.p + w * VEC);
       }
-      auto add = [&](int u, int k) {
-        const float xc = bn_f(xv[u].v[k]) - mean;
+    };
+    auto add = [&](const Vec &xv, const Vec &dv) {
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) {
+        const float xc = bn_f(xv.v[k]) - mean;
         if (BWD) {
-          float d = bn_f(dv[u].v[k]);
+          float d = bn_f(dv.v[k]);
           if (P.relu && !(a * xc + b > 0.f)) d = 0.f;
           s1 += d;
           s2 += d * xc;
@@ -136,18 +138,25 @@ __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P)
           s1 += xc;
           s2 += xc * xc;
         }
-      };
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        if (skip[u] == 0u) {
-#pragma unroll
-          for (int k = 0; k < VEC; ++k) add(u, k);
-        } else {
-#pragma unroll
-          for (int k = 0; k < VEC; ++k)
-            if ((uint32_t)k >= skip[u]) add(u, k);
-        }
       }
+    };
+    Vec xv[U], dv[U];
+    uint32_t it = threadIdx.x;
+    for (; it + (U - 1u) * kBnThreads < items; it += U * kBnThreads) {
+#pragma unroll
+      for (int u = 0; u < U; ++u) load(it + (uint32_t)u * kBnThreads, xv[u], dv[u]);
+#pragma unroll
+      for (int u = 0; u < U; ++u) add(xv[u], dv[u]);
+    }
+    if (it < items) {  // the rest: loaded from existing places, added where it exists
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u) {
+        const uint32_t i = it + (uint32_t)u * kBnThreads;
+        load(i < items ? i : it, xv[u], dv[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < U - 1; ++u)
+        if (it + (uint32_t)u * kBnThreads < items) add(xv[u], dv[u]);
     }
   }
   const float2 r = block_sum2(s1, s2);
@@ -461,17 +470,22 @@ static dim3 bn_apply_grid(BnParams *P, uint32_t groups_per_plane, bool backward)
   return dim3((planes + per_block - 1u) / per_block, (groups_per_plane + kBnThreads - 1u) / kBnThreads);
 }
 
-// A plane is `runs` runs of `run` elements, each read as groups of `vec`.  False: one element at a time is read, where the
-// last groups, stored element by element, are more than an eighth of all (5.6 us against 8.9 for the backward pass over
-// bf16 planes of 22).
+// The reduce pass numbers a plane's `rows` rows of `items` (groups of elements) through.
+static void bn_items(BnParams *P, uint32_t items, uint32_t rows) {
+  P->div_cols = FastDiv(items);
+  P->div_groups = FastDiv(items * rows);
+  P->planes_per_pass = std::max(1u, 0x7fffffffu / (items * rows));
+}
+
+// The backward apply pass: a plane is `runs` runs of `run` elements, each moved as groups of `vec`.  False: one element at a
+// time, where the last groups, stored element by element, are more than an eighth of all (5.6 us against 8.9 over bf16
+// planes of 22).
 static bool bn_runs(BnParams *P, uint32_t run, uint32_t runs, uint32_t vec) {
   const bool wide = run % vec == 0u || run >= 8u * vec;
   const uint32_t groups = wide ? (run + vec - 1u) / vec : run;
   P->run = run;
   P->groups_per_plane = groups * runs;
   P->div_cols = FastDiv(groups);
-  P->div_groups = FastDiv(P->groups_per_plane);
-  P->planes_per_pass = std::max(1u, 0x7fffffffu / P->groups_per_plane);
   return wide;
 }
 
@@ -541,7 +555,8 @@ int adh_batchnorm2d_fwd_tiles(int dtype, int training, uint32_t num_tiles, uint3
   if ((gpp + kBnThreads - 1u) / kBnThreads > 65535u) return ADH_EINVAL;  // grid.y
   const bool stream_data = bn_stream((uint64_t)tc * N * H * W * es);
   if (training) {
-    const bool wide = bn_runs(&P, H * W, 1u, vec);  // the statistics pass
+    const bool wide = H * W % vec == 0u;  // the statistics pass reads whole 16-byte groups
+    bn_items(&P, H * W / (wide ? vec : 1u), 1u);
     bn_launch(stream_data, dtype, [&](auto s, auto t) {
       typedef decltype(t) T;
       if (wide) hipLaunchKernelGGL((bn_reduce_kernel<T, false, 16 / sizeof(T), s>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
@@ -593,21 +608,27 @@ int adh_batchnorm2d_bwd_tiles(int dtype, uint32_t num_tiles, uint32_t N, uint32_
   P.relu = relu ? 1 : 0;
   hipStream_t st = as_stream(stream);
   const uint32_t tc = num_tiles * C, vec = (uint32_t)(16 / es);
-  const bool wide = dy_halo ? bn_runs(&P, W, H, vec) : bn_runs(&P, H * W, 1u, vec);
+  const bool rwide = W % vec == 0u;  // the sums are of whole 16-byte groups of a row
+  const bool awide = dy_halo ? bn_runs(&P, W, H, vec) : bn_runs(&P, H * W, 1u, vec);
   if ((P.groups_per_plane + kBnThreads - 1u) / kBnThreads > 65535u) return ADH_EINVAL;  // grid.y
   const bool stream_data = bn_stream((uint64_t)tc * N * H * W * es * 2u);
   P.beta = beta_data;
   P.beta_param = beta_param;
-  const dim3 rgrid(tc * P.split), agrid = bn_apply_grid(&P, P.groups_per_plane, true);
+  const uint32_t apply_groups = P.groups_per_plane;
+  const FastDiv apply_cols = P.div_cols;
+  bn_items(&P, W / (rwide ? vec : 1u), H);
+  const dim3 rgrid(tc * P.split);
   bn_launch(stream_data, dtype, [&](auto s, auto t) {
     typedef decltype(t) T;
-    if (wide) {
-      hipLaunchKernelGGL((bn_reduce_kernel<T, true, 16 / sizeof(T), s>), rgrid, dim3(kBnThreads), 0, st, P);
-      hipLaunchKernelGGL((bn_apply_kernel<T, 2, 16 / sizeof(T), s>), agrid, dim3(kBnThreads), 0, st, P);
-    } else {
-      hipLaunchKernelGGL((bn_reduce_kernel<T, true, 1, false>), rgrid, dim3(kBnThreads), 0, st, P);
-      hipLaunchKernelGGL((bn_apply_kernel<T, 2, 1, false>), agrid, dim3(kBnThreads), 0, st, P);
-    }
+    if (rwide) hipLaunchKernelGGL((bn_reduce_kernel<T, true, 16 / sizeof(T), s>), rgrid, dim3(kBnThreads), 0, st, P);
+    else hipLaunchKernelGGL((bn_reduce_kernel<T, true, 1, false>), rgrid, dim3(kBnThreads), 0, st, P);
+  });
+  P.div_cols = apply_cols;
+  const dim3 agrid = bn_apply_grid(&P, apply_groups, true);
+  bn_launch(stream_data, dtype, [&](auto s, auto t) {
+    typedef decltype(t) T;
+    if (awide) hipLaunchKernelGGL((bn_apply_kernel<T, 2, 16 / sizeof(T), s>), agrid, dim3(kBnThreads), 0, st, P);
+    else hipLaunchKernelGGL((bn_apply_kernel<T, 2, 1, false>), agrid, dim3(kBnThreads), 0, st, P);
   });
   return launch_status();
 }
