@@ -861,12 +861,14 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
   }
 }
 
-// 3x3 / 2, padding 1, rows of at least a group of columns; anything else takes the bands
+// 3x3 / 2, padding 1, rows of at least a group of columns; anything else takes the bands, and so do the smallest tensors: a
+// thread's chain of loads is longer than a band's (16 to 20 k pixels: 4.1 us a pass there, 5 to 9 here; 72 k: the other way round)
 static bool pool_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
   const uint32_t nc = (uint32_t)(16u / es), groups = (P.W + nc - 1u) / nc;
   if (P.wh != 3u || P.ww != 3u || P.sh != 2u || P.sw != 2u || P.pad_h != 1u || P.pad_w != 1u || P.W < nc) return false;
   const uint64_t items = (uint64_t)P.planes * groups, rows = (uint64_t)P.num_tiles * P.H;
   if (items >= (1ull << 31) || rows >= (1ull << 31)) return false;
+  if (P.planes * rows * P.W < (1u << 15)) return false;
   for (uint32_t t = 0; t < P.num_tiles; ++t) {
     q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->out[t] = P.out[t];
   }
