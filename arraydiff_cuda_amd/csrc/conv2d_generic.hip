@@ -18,6 +18,7 @@
 // rewritten beforehand to [m group][chunk][tap][channel][m] in the workspace, is staged per tap
 // group.  bf16 tensors are widened while staging and rounded when stored: the arithmetic is fp32.
 #include "conv3x3_split.h"
+#include "conv_bf16_patch.h"
 #include "conv3x3_wgrad_split.h"
 
 #include <algorithm>
@@ -627,6 +628,26 @@ static Conv3x3Problem gen_3x3_problem(int which, const GenShape &g, uint32_t num
     q.sample = fwd ? kDown : kUp;
     q.step = g.OH;
     q.pad_r = q.pad_c = fwd ? 1 : 0;
+  }
+  return q;
+}
+// conv_bf16_patch.hip: bf16 tensors, forward and backward-data.  3x3 windows at stride 1 and (over tiles of even height and width
+// without halo) 2; 1x1 windows at stride 1 and 2 (backward-data: even heights and widths).  The number of taps, or 0.
+static int gen_patch_taps(int which, int dtype, const GenShape &g, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
+  if (dtype != ADH_BF16 || g.sh != g.sw || g.sh > 2u) return 0;
+  if (g.kh == 1u && g.kw == 1u) {
+    if (unpadded && (pad_h || pad_w)) return 0;
+    return g.sh == 1u || which == ADH_CONV_FWD || (g.HP % 2u == 0u && g.WP % 2u == 0u) ? 1 : 0;
+  }
+  return gen_is_3x3_split(ADH_F32, g, unpadded, pad_h, pad_w) ? 9 : 0;
+}
+static Conv3x3Problem gen_patch_problem(int which, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w, int taps) {
+  Conv3x3Problem q = gen_3x3_problem(which, g, num_tiles, unpadded, pad_h, pad_w);
+  if (taps == 1) {  // (its tiles are independent)
+    q.stacked = false;
+    q.pad_r = q.pad_c = 0;
+    q.w_m_stride = which == ADH_CONV_FWD ? g.Cin : 1u;
+    q.w_c_stride = which == ADH_CONV_FWD ? 1u : g.Cin;
   }
   return q;
 }
@@ -1294,6 +1315,15 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
+  if (const int taps = gen_patch_taps(ADH_CONV_FWD, dtype, g, unpadded, pad_h, pad_w)) {
+    e = gen_check_workspace(plan, workspace, workspace_bytes);
+    if (e) return e;
+    Conv3x3Problem q = gen_patch_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w, taps);
+    q.beta = beta;
+    q.in = x_tiles; q.out = y_tiles; q.w = w;
+    e = conv_bf16_patch(q, taps, workspace, workspace_bytes, 1e30, as_stream(stream));
+    if (e != ADH_EUNIMPL) return e;
+  }
   return gen_launch(dtype, &plan, num_tiles, w, workspace, workspace_bytes, as_stream(stream));
 }
 
@@ -1336,6 +1366,15 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     q.beta = beta;
     q.in = dy_tiles; q.out = dx_tiles; q.w = w;
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
+    if (e != ADH_EUNIMPL) return e;
+  }
+  if (const int taps = gen_patch_taps(ADH_CONV_BWD_DATA, dtype, g, unpadded, pad_h, pad_w)) {
+    e = gen_check_workspace(plan, workspace, workspace_bytes);
+    if (e) return e;
+    Conv3x3Problem q = gen_patch_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w, taps);
+    q.beta = beta;
+    q.in = dy_tiles; q.out = dx_tiles; q.w = w;
+    e = conv_bf16_patch(q, taps, workspace, workspace_bytes, 1e30, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   return gen_launch(dtype, &plan, num_tiles, w, workspace, workspace_bytes, as_stream(stream));
