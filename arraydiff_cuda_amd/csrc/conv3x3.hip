@@ -15,8 +15,8 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
 // The problem of a pass whose tiles' interiors are H x W.  rows_from_neighbours: the tiles are the row tiles of one tensor
 // in rank order; over padded tiles (forward) the inner halo rows are then the neighbours' interior rows, and (backward-data)
 // what a halo reduce would add is part of the sums.  unpadded: neither side carries a halo.
-static Conv3x3Problem conv3x3_problem(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
-                                      bool rows_from_neighbours, bool unpadded) {
+Conv3x3Problem conv3x3_problem(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
+                               bool rows_from_neighbours, bool unpadded) {
   const bool fwd = which == ADH_CONV_FWD;
   const uint32_t halo = unpadded ? 0u : 2u;
   Conv3x3Problem q = {};
@@ -67,6 +67,8 @@ static int conv_direct(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   return conv3x3_split(q, nullptr, 0, st);
 }
 
+// the patches' kernel name, where they serve the call
+bool conv_bf16_takes_patches(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, char *name, size_t name_bytes);
 const char *conv_bf16_kernel_name(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, float beta);
 int conv_bf16_unpadded(int which, int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                        const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
@@ -84,6 +86,7 @@ int adh_conv3x3_kernel_name(int which, int dtype, uint32_t num_tiles, uint32_t N
   if (which != ADH_CONV_FWD && which != ADH_CONV_BWD_DATA) return ADH_EINVAL;
   if (num_tiles == 0 || N == 0 || Cin == 0 || Cout == 0 || H == 0 || W == 0) return ADH_EINVAL;
   if (dtype == ADH_BF16) {
+    if (conv_bf16_takes_patches(which, num_tiles, N, Cin, Cout, H, W, name, name_bytes)) return ADH_OK;
     snprintf(name, name_bytes, "%s", conv_bf16_kernel_name(which, Cin, Cout, H, W, beta));
     return ADH_OK;
   }

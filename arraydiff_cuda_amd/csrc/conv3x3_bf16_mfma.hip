@@ -25,9 +25,11 @@
 //
 // Out-of-range rows, channels and buffer ends are handled by the buffer resource's range check
 // (out-of-range dwords read as zero); out-of-range columns by per-dword masks.
+#include "conv_bf16_patch.h"
 #include "conv3x3_bf16_mfma.h"
 
 #include <algorithm>
+#include <cmath>
 
 namespace adh {
 
@@ -856,9 +858,44 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
   return conv_bf16_w4_launch(P, gx, groups, st);
 }
 
+// Strips or patches: strips are ahead on large images of 64 or 128 channels (64 -> 64 on 8 tiles of 128 x 2048 258 against 578 us, 128 ->
+// 128 on 4 tiles of 64 x 256 109 and 190), patches where a launch is small, the channels are no whole 64, or more than one launch of
+// strips would follow another (21 -> 400 on 6 tiles of 6 x 171, backward-data, 372 against 25 us; 566 random shapes: 2.25 times as fast
+// over all, 2.48 with this choice, 2.51 with the better of both each time).
+// What the strips' launches take, fitted to those shapes (rms error 20 %): each its start and its waves' steps; padded to whole 64 (or
+// 128) channels and 64 (32) columns the multiplications; the copies of odd rows, and the sums between launches.
+static double conv_bf16_strips_us(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, bool halofree) {
+  const bool fwd = which == ADH_CONV_FWD, wide = conv_bf16_uses_k128(which, Cin, Cout);
+  const double images = (double)num_tiles * N, C = fwd ? Cin : Cout, M = fwd ? Cout : Cin;
+  const double oh = H + (fwd || halofree ? 0.0 : 2.0), ow = W + (fwd || halofree ? 0.0 : 2.0), ih = H + (fwd && !halofree ? 2.0 : 0.0), iw = W + (fwd && !halofree ? 2.0 : 0.0);
+  const double unit = wide ? 128.0 : 64.0, cols = wide ? 32.0 : 64.0, launches = std::ceil(C / unit), groups = std::ceil(M / unit);
+  const double flops = images * oh * std::ceil(ow / cols) * cols * 18.0 * launches * groups * unit * unit;
+  const double steps = std::ceil(std::max(1.0, images * std::ceil(ow / 64.0) * std::ceil(oh / 4.0) * std::ceil(M / 64.0) / 256.0));
+  double us = launches * (wide ? 22.7 : 18.2) + (wide ? 0.49e-9 : 0.81e-9) * flops + 0.69 * steps * std::ceil(C / 64.0);
+  if (!halofree && W % 8u != 0u) us += 0.74e-6 * images * C * ih * iw;
+  return us + 2e-6 * (launches - 1.0) * images * M * oh * ow;
+}
+constexpr double kPatchAhead = 1.15;  // by which patches have to be expected ahead
+
+bool conv_bf16_takes_patches(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, char *name, size_t name_bytes) {
+  return conv_bf16_mfma_supported(which, Cin, Cout, H, W) &&
+         conv_bf16_patch_name(conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, false), 9, conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false),
+                              conv_bf16_strips_us(which, num_tiles, N, Cin, Cout, H, W, false) / kPatchAhead, name, name_bytes);
+}
+
 int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                    const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
                    size_t workspace_bytes, hipStream_t st, bool halofree) {
+  // (tiles off the alignment that the strips want: what is refused there stays refused)
+  bool aligned = true;
+  for (uint32_t t = 0; t < num_tiles; ++t) aligned = aligned && aligned_to(in_tiles[t], 16);
+  if (aligned) {
+    Conv3x3Problem q = conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, halofree);
+    q.beta = beta;
+    q.in = in_tiles; q.out = out_tiles; q.w = w;
+    const int e = conv_bf16_patch(q, 9, workspace, workspace_bytes, conv_bf16_strips_us(which, num_tiles, N, Cin, Cout, H, W, halofree) / kPatchAhead, st);
+    if (e != ADH_EUNIMPL) return e;
+  }
   const uint64_t room = workspace_bytes > filter_region_bytes(which, Cin, Cout) ? workspace_bytes - filter_region_bytes(which, Cin, Cout) : 0u;
   if (halofree || !conv_bf16_repitches(which, Cin, Cout, H, W) ||
       room < conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, kLeastCopies).bytes)

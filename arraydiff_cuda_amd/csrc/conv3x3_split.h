@@ -29,6 +29,10 @@ struct Conv3x3Problem {
   uint32_t w_m_stride, w_c_stride;  // of the filter's output and reduction channels
 };
 
+// The problem of the 3x3 entry points (conv3x3.hip).
+Conv3x3Problem conv3x3_problem(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
+                               bool rows_from_neighbours, bool unpadded);
+
 // fp32 sums of channel chunks that are dealt to several workgroups (0: none are)
 size_t conv3x3_split_workspace(const Conv3x3Problem &q);
 // The workspace may be null: then no chunks are dealt out.

@@ -107,3 +107,81 @@ def test_1x1_stride_2_over_odd_tiles(H, W):
 def test_many_blocks():
     _check(2, 8, 96, 160, 32, 64, 3, 2)
     _check(2, 8, 96, 160, 16, 60, 3, 1)
+
+
+def _check_3x3(K, N, Ci, Co, H, W, halo, beta=0.0, skew=0, spoil=None):
+    """The entry points of the 3x3 window, over padded tiles (backward-data: the whole padded slab) or tiles without halo."""
+    g = torch.Generator().manual_seed(Ci * 7 + Co + W)
+    bf = lambda t: t.to(torch.bfloat16)
+    w = bf(torch.randn((Co, Ci, 3, 3), generator=g) * (2.0 / (Ci * 9)) ** 0.5)
+    if spoil:
+        spoil(w)
+    if halo:
+        xs = [bf(torch.rand((N, Ci, H + 2, W + 2), generator=g) * 2 - 1) for _ in range(K)]
+        dys = [bf(torch.randn((N, Co, H, W), generator=g)) for _ in range(K)]
+        ins = [x.double().requires_grad_() for x in xs]
+        ys64 = [F.conv2d(x, w.double()) for x in ins]
+        torch.autograd.backward(ys64, [d.double() for d in dys])
+        dx64 = [x.grad for x in ins]
+    else:
+        x, dy = bf(torch.rand((N, Ci, H * K, W), generator=g) * 2 - 1), bf(torch.randn((N, Co, H * K, W), generator=g))
+        x64 = x.double().requires_grad_()
+        y = F.conv2d(x64, w.double(), padding=1)
+        y.backward(dy.double())
+        xs, dys, ys64, dx64 = x.chunk(K, 2), dy.chunk(K, 2), y.detach().chunk(K, 2), x64.grad.chunk(K, 2)
+
+    def put(t):  # `skew` elements off alignment
+        d = torch.empty(t.numel() + skew, device="cuda", dtype=torch.bfloat16)[skew:].view(t.shape)
+        return d.copy_(t)
+    old_y, old_x = [bf(torch.randn(t.shape, generator=g)) for t in ys64], [bf(torch.randn(t.shape, generator=g)) for t in dx64]
+    wd, xd, dyd, ys, dxs = put(w), [put(t) for t in xs], [put(t) for t in dys], [put(t) for t in old_y], [put(t) for t in old_x]
+    size = (N, Ci, Co, H, W)
+    ws = [torch.empty(capi.conv_workspace_bytes(q, capi.ADH_BF16, K, *size) // 4 + 64, device="cuda") for q in (capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA)]
+    fwd, bwd = (capi.conv_fwd_tiles, capi.conv_bwd_data_tiles) if halo else (capi.conv_unpadded_fwd_tiles, capi.conv_unpadded_bwd_data_tiles)
+    capi.check(fwd(xd, wd, ys, *size, beta=beta, ws=ws[0]), "forward")
+    capi.check(bwd(wd, dyd, dxs, *size, beta=beta, ws=ws[1]), "backward-data")
+    for got, want, old in list(zip(ys, ys64, old_y)) + list(zip(dxs, dx64, old_x)):
+        want, got = want.detach() + (old.double() if beta else 0.0), got.cpu().double()
+        # (of a spoiled channel the kernels also multiply the padding's zeros; the others have to be as ever)
+        fine = want.isfinite().all(3, keepdim=True).all(2, keepdim=True).all(0, keepdim=True).expand_as(want)
+        scale = want[fine].abs()
+        err = (got - want)[fine].abs()
+        assert bool((err <= 2.0 ** -8 * 1.001 * scale + 2e-5 * (1 + scale.max())).all()), err.max()
+
+
+def _patches(which, K, N, Ci, Co, H, W):
+    return "patch_kernel" in capi.conv_kernel_name(which, capi.ADH_BF16, K, N, Ci, Co, H, W)
+
+
+@pytest.mark.parametrize("Ci,Co", CHANNELS + [(224, 16), (16, 224), (97, 300)])
+@pytest.mark.parametrize("halo", [True, False])
+def test_small_3x3_channels(Ci, Co, halo):
+    assert _patches(capi.ADH_CONV_FWD, 2, 3, Ci, Co, 5, 16) and _patches(capi.ADH_CONV_BWD_DATA, 2, 3, Ci, Co, 5, 16)
+    _check_3x3(2, 3, Ci, Co, 5, 16, halo)
+
+
+@pytest.mark.parametrize("W", [1, 2, 3, 7, 8, 9, 31, 64, 65, 250, 515])
+def test_small_3x3_widths(W):
+    _check_3x3(2, 2, 24, 40, 6, W, True, beta=1.0)
+
+
+@pytest.mark.parametrize("halo", [True, False])
+def test_the_filter_in_order_first(halo):
+    """Large enough a launch to put the filter in order, with partial groups of 64 channels on both sides."""
+    for which in (capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA):
+        assert capi.conv_kernel_name(which, capi.ADH_BF16, 4, 8, 76, 140, 32, 40).endswith("9, true>")
+    _check_3x3(4, 8, 76, 140, 32, 40, halo)
+
+
+@pytest.mark.parametrize("skew", [1, 3])
+def test_tiles_off_alignment(skew):
+    _check_3x3(2, 3, 20, 24, 5, 17, True, skew=skew)
+
+
+def test_an_infinite_filter_element_stays_in_its_channel():
+    def spoil(w):
+        w[3, 17, 1, 1] = float("inf")  # channels of a partial chunk
+        w[5, 19, 0, 2] = float("nan")
+    for halo in (True, False):
+        _check_3x3(2, 2, 20, 24, 6, 16, halo, spoil=spoil)
+        _check_3x3(2, 2, 33, 24, 6, 16, halo, spoil=spoil)  # (a chunk of one channel)
