@@ -19,6 +19,7 @@
 // group.  bf16 tensors are widened while staging and rounded when stored: the arithmetic is fp32.
 #include "conv3x3_split.h"
 #include "conv_bf16_patch.h"
+#include "conv_s2_wgrad.h"
 #include "conv3x3_wgrad_split.h"
 
 #include <algorithm>
@@ -586,14 +587,10 @@ int conv1x1_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cou
                       uint32_t OW, uint32_t sh, uint32_t sw, const void *const *x_tiles, const void *const *dy_tiles,
                       float *dwt, float beta, void *workspace, hipStream_t st);
 
-// conv3x3s2.hip: filter gradient of a 3x3 window at stride 2, padding 1, over fp32 tiles of H x W without halo, and its
-// forward for launches that would leave the split kernel's last round idle
+// conv3x3s2.hip: forward of a 3x3 window at stride 2, padding 1, over fp32 tiles of H x W without halo, for launches that would leave
+// the split kernel's last round idle
 int conv3x3s2_fwd_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                       const void *const *x_tiles, const void *w, void *const *y_tiles, float beta, hipStream_t st);
-size_t conv3x3s2_wgrad_workspace(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
-int conv3x3s2_wgrad_try(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
-                        const void *const *x_tiles, const void *const *dy_tiles, float *dwt, float beta, void *workspace,
-                        hipStream_t st);
 static bool gen_is_3x3s2_unpadded(int dtype, const GenShape &g, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
   return dtype == ADH_F32 && unpadded && g.kh == 3u && g.kw == 3u && g.sh == 2u && g.sw == 2u && g.dh == 1u && g.dw == 1u &&
          pad_h == 1u && pad_w == 1u;
@@ -640,6 +637,15 @@ static int gen_patch_taps(int which, int dtype, const GenShape &g, bool unpadded
     return g.sh == 1u || which == ADH_CONV_FWD || (g.HP % 2u == 0u && g.WP % 2u == 0u) ? 1 : 0;
   }
   return gen_is_3x3_split(ADH_F32, g, unpadded, pad_h, pad_w) ? 9 : 0;
+}
+// conv_s2_wgrad.hip: the filter gradient at stride 2 over tiles of even height and width without halo, 3x3 in either type and 1x1 in
+// bf16 (conv1x1.hip has fp32's).  Whether the shape is such a one.
+static bool gen_s2_wgrad_problem(int dtype, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w, S2WgradProblem *q) {
+  if (!unpadded || g.sh != 2u || g.sw != 2u || g.HP % 2u != 0u || g.WP % 2u != 0u) return false;
+  const bool three = gen_is_3x3s2_unpadded(ADH_F32, g, unpadded, pad_h, pad_w);
+  if (!three && (dtype != ADH_BF16 || g.kh != 1u || g.kw != 1u || pad_h != 0u || pad_w != 0u)) return false;
+  *q = S2WgradProblem{dtype, three ? 9 : 1, num_tiles, g.N, g.Cin, g.Cout, g.OH, g.OW, nullptr, nullptr, nullptr, 0.f};
+  return true;
 }
 static Conv3x3Problem gen_patch_problem(int which, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w, int taps) {
   Conv3x3Problem q = gen_3x3_problem(which, g, num_tiles, unpadded, pad_h, pad_w);
@@ -1235,8 +1241,9 @@ size_t conv2d_workspace(int which, int dtype, uint32_t num_tiles, uint32_t N, ui
     size_t bytes = wp.partial_bytes;
     if (gen_is_pointwise_wgrad(dtype, g, unpadded, pad_h, pad_w))
       bytes = std::max(bytes, conv1x1_wgrad_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW));
-    if (gen_is_3x3s2_unpadded(dtype, g, unpadded, pad_h, pad_w))
-      bytes = std::max(bytes, conv3x3s2_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u));
+    S2WgradProblem s2;
+    if (gen_s2_wgrad_problem(dtype, g, num_tiles, unpadded, pad_h, pad_w, &s2))
+      bytes = std::max(bytes, std::max(conv_s2_wgrad_workspace(s2), conv_s2_wgrad_required(s2)));
     if (gen_is_thin(dtype, g, unpadded))
       bytes = std::max(bytes, conv_thin_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, kh, kw, sh, sw));
     if (gen_is_3x3_unit(dtype, g) && g.dh == 1u)
@@ -1444,13 +1451,12 @@ int conv2d_bwd_filter(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
       if (e != ADH_EUNIMPL) return e;
     }
   }
-  if (gen_is_3x3s2_unpadded(dtype, g, unpadded, pad_h, pad_w)) {
-    const size_t need = conv3x3s2_wgrad_workspace(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u);
-    if (need != 0) {
-      if (workspace_bytes < need) return ADH_EWORKSPACE;
-      e = conv3x3s2_wgrad_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, dy_tiles, dwt, beta, workspace, st);
-      if (e != ADH_EUNIMPL) return e;
-    }
+  S2WgradProblem s2;
+  if (gen_s2_wgrad_problem(dtype, g, num_tiles, unpadded, pad_h, pad_w, &s2)) {
+    if (workspace_bytes < conv_s2_wgrad_required(s2)) return ADH_EWORKSPACE;
+    s2.x = x_tiles; s2.dy = dy_tiles; s2.dw = dwt; s2.beta = beta;
+    e = conv_s2_wgrad(s2, workspace, workspace_bytes, st);
+    if (e != ADH_EUNIMPL) return e;
   }
   plan.P.partial = reinterpret_cast<float *>(workspace);
   if (dtype == ADH_F32) launch_wgrad_gen<float>(plan, st);
