@@ -1,8 +1,8 @@
 // bf16 entry of the 3x3 slab convolution: bf16 tensors in HBM, fp32 accumulation.
 //
 // Forward and backward-data run on the bf16 matrix-core kernels of conv3x3_bf16_mfma.hip, the filter
-// gradient on that of conv3x3_bf16_wgrad.hip (at a width that is no multiple of 8 over copies of the
-// tensors with wider rows, made here).  What those do not take (images or sums beyond the 2 GiB a
+// gradient on that of conv3x3_wgrad_steps.hip or of conv3x3_bf16_wgrad.hip (at a width that is no multiple
+// of 8 over copies of the tensors with wider rows, made here).  What those do not take (images or sums beyond the 2 GiB a
 // buffer resource addresses) goes the route below: the bf16 slabs, filter and (for beta = 1) outputs
 // are widened to fp32 in the caller's workspace, the fp32 kernels run on the copies, and the
 // result is rounded back to bf16 (round to nearest even).  Every product is therefore exact and every sum is in
@@ -10,6 +10,9 @@
 // fp32 path plus three streaming passes.  The filter gradient stays fp32.
 #include "conv3x3_bf16_mfma.h"
 #include "conv3x3_wgrad_split.h"
+#include "conv3x3_wgrad_steps.h"
+
+#include <algorithm>
 
 namespace adh {
 
@@ -128,6 +131,7 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
 
 bool conv_bf16_wgrad_mfma_supported(uint32_t Cin, uint32_t Cout, uint32_t W);
 size_t conv_bf16_wgrad_mfma_workspace_bytes(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t W);
+double conv_bf16_wgrad_mfma_us(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W);
 int conv_bf16_wgrad_mfma(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                          const void *const *x_tiles, const void *const *dy_tiles, float *dw, float beta,
                          void *workspace, hipStream_t st, bool unpadded);
@@ -167,8 +171,32 @@ int repitch_bf16_tiles(uint32_t num_tiles, uint64_t rows, uint32_t w_src, uint32
   return ADH_OK;
 }
 
-size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
-                            uint32_t W, size_t fp32_path_bytes) {
+static StepsWgradProblem wgrad_problem(bool stacked, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
+  return StepsWgradProblem{ADH_BF16, stacked, num_tiles, N, Cin, Cout, H, W, nullptr, nullptr, nullptr, 0.f};
+}
+static int wgrad_steps(StepsWgradProblem q, const void *const *x_tiles, const void *const *dy_tiles, float *dw, float beta, void *workspace,
+                       size_t workspace_bytes, hipStream_t st) {
+  q.x = x_tiles;
+  q.dy = dy_tiles;
+  q.dw = dw;
+  q.beta = beta;
+  return conv3x3_wgrad_steps(q, workspace, workspace_bytes, st);
+}
+// Whether conv3x3_wgrad_steps.hip is expected to be faster than conv3x3_bf16_wgrad.hip, which walks whole columns of an image 64 wide:
+// that one where such strips fill the chip and are long (64 channels on 32 images of 4 tiles of 32 x 128: 49 us against 62), the steps where they
+// do not, where channels are few or the filter is large (512 on 4 x 16: 591 -> 71), and at odd widths, which they
+// take as they are (128 on 8 images of 4 tiles of 64 x 255: 247 -> 168).
+static bool takes_steps(const StepsWgradProblem &q) {
+  const uint32_t Wd = (q.W + 7u) & ~7u;
+  double strips = conv_bf16_wgrad_mfma_us(q.num_tiles, q.N, q.Cin, q.Cout, q.H, Wd);
+  if (Wd != q.W) strips += 8.0 + 0.106e-6 * 4.0 * q.num_tiles * q.N * ((double)q.Cin * (q.H + 2.0) * (Wd + 2.0) + (double)q.Cout * q.H * Wd);
+  const double steps = conv3x3_wgrad_steps_us(q);
+  return steps > 0.0 && steps < strips;
+}
+
+// what a call has to bring
+static size_t bf16_required_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
+                                  uint32_t W, size_t fp32_path_bytes) {
   if (which == ADH_CONV_BWD_FILTER && conv_bf16_wgrad_mfma_supported(Cin, Cout, W))
     return conv_bf16_wgrad_mfma_workspace_bytes(num_tiles, N, Cin, Cout, W);
   if (which == ADH_CONV_BWD_FILTER && wgrad_repitch_route(Cin, Cout, H, W)) {
@@ -184,6 +212,14 @@ size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t 
   if (which == ADH_CONV_BWD_FILTER) total = num_tiles * (region(slab) + region(out));
   else total = num_tiles * (region(slab) + region(out)) + region(filt);
   return total + (fp32_path_bytes + 255u) / 256u * 256u;
+}
+size_t bf16_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
+                            uint32_t W, size_t fp32_path_bytes) {
+  size_t bytes = bf16_required_bytes(which, num_tiles, N, Cin, Cout, H, W, fp32_path_bytes);
+  if (which == ADH_CONV_BWD_FILTER)
+    for (bool stacked : {false, true})
+      bytes = std::max(bytes, conv3x3_wgrad_steps_workspace(wgrad_problem(stacked, num_tiles, N, Cin, Cout, H, W)));
+  return bytes;
 }
 
 }  // namespace adh
@@ -214,7 +250,7 @@ int conv_bf16_via_f32(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
   // a workspace without room for copies of the input at odd widths does for the kernels that need none
   const bool mfma = conv_bf16_mfma_supported(which, Cin, Cout, H, W);
   const size_t need = mfma ? conv_bf16_mfma_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, false)
-                           : bf16_workspace_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
+                           : bf16_required_bytes(which, num_tiles, N, Cin, Cout, H, W, 0);
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
@@ -270,6 +306,7 @@ int conv_bf16_filter_via_f32(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint3
     return adh_conv3x3_slab_bwd_filter_tiles(ADH_F32, num_tiles, N, Cin, Cout, H, W, x_tiles, dy_tiles, dw, beta,
                                              workspace, workspace_bytes, st);
   if (!x_tiles || !dy_tiles) return ADH_ENULL;
+  const StepsWgradProblem steps = wgrad_problem(false, num_tiles, N, Cin, Cout, H, W);
   if (conv_bf16_wgrad_mfma_supported(Cin, Cout, W)) {
     if (!workspace) return ADH_ENULL;
     if (!aligned_to(workspace, 256) || !aligned_to(dw, 4)) return ADH_EALIGN;
@@ -280,13 +317,14 @@ int conv_bf16_filter_via_f32(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint3
       if (!x_tiles[t] || !dy_tiles[t]) return ADH_ENULL;
       if (!aligned_to(x_tiles[t], 2) || !aligned_to(dy_tiles[t], 2)) return ADH_EALIGN;
     }
+    if (takes_steps(steps)) return wgrad_steps(steps, x_tiles, dy_tiles, dw, beta, workspace, workspace_bytes, st);
     return conv_bf16_wgrad_mfma(num_tiles, N, Cin, Cout, H, W, x_tiles, dy_tiles, dw, beta, workspace, st, false);
   }
   if (wgrad_repitch_route(Cin, Cout, H, W)) {
     const uint32_t Wd = wgrad_wide_width(W);
     if (!workspace) return ADH_ENULL;
     if (!aligned_to(workspace, 256) || !aligned_to(dw, 4)) return ADH_EALIGN;
-    if (workspace_bytes < bf16_workspace_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, 0)) return ADH_EWORKSPACE;
+    if (workspace_bytes < bf16_required_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, 0)) return ADH_EWORKSPACE;
     const uint64_t x_rows = (uint64_t)N * Cin * (H + 2), dy_rows = (uint64_t)N * Cout * H;
     char *ws = reinterpret_cast<char *>(workspace);
     void *xw[ADH_MAX_TILES], *dyw[ADH_MAX_TILES];
@@ -298,13 +336,14 @@ int conv_bf16_filter_via_f32(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint3
       dyw[t] = ws;
       ws += repitch_bf16_region(dy_rows * Wd);
     }
+    if (takes_steps(steps)) return wgrad_steps(steps, x_tiles, dy_tiles, dw, beta, workspace, workspace_bytes, st);
     int e = repitch_bf16_tiles(num_tiles, x_rows, W + 2u, Wd + 2u, x_tiles, xw, st);
     if (e) return e;
     e = repitch_bf16_tiles(num_tiles, dy_rows, W, Wd, dy_tiles, dyw, st);
     if (e) return e;
     return conv_bf16_wgrad_mfma(num_tiles, N, Cin, Cout, H, Wd, xw, dyw, dw, beta, ws, st, false);
   }
-  const size_t need = bf16_workspace_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, conv3x3_wgrad_split_least_workspace(Cin, Cout));
+  const size_t need = bf16_required_bytes(ADH_CONV_BWD_FILTER, num_tiles, N, Cin, Cout, H, W, conv3x3_wgrad_split_least_workspace(Cin, Cout));
   if (!workspace) return ADH_ENULL;
   if (!aligned_to(workspace, 256)) return ADH_EALIGN;
   if (workspace_bytes < need) return ADH_EWORKSPACE;
@@ -366,5 +405,7 @@ extern "C" int adh_conv3x3_unpadded_bwd_filter_tiles(int dtype, uint32_t num_til
     if (!x_tiles[t] || !dy_tiles[t]) return ADH_ENULL;
     if (!aligned_to(x_tiles[t], 16) || !aligned_to(dy_tiles[t], 2)) return ADH_EALIGN;
   }
+  const StepsWgradProblem steps = wgrad_problem(true, num_tiles, N, Cin, Cout, H, W);
+  if (takes_steps(steps)) return wgrad_steps(steps, x_tiles, dy_tiles, dw, beta, workspace, workspace_bytes, as_stream(stream));
   return conv_bf16_wgrad_mfma(num_tiles, N, Cin, Cout, H, W, x_tiles, dy_tiles, dw, beta, workspace, as_stream(stream), true);
 }

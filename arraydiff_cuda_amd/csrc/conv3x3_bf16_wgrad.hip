@@ -1,5 +1,5 @@
-// Filter gradient of the 3x3 slab convolution on the bf16 matrix cores, for up to 64 input and
-// 64 output channels and image widths that are a multiple of eight:
+// Filter gradient of the 3x3 slab convolution on the bf16 matrix cores, for image widths that are a multiple of eight, where strips of
+// 64 columns fill the chip (conv3x3_wgrad_steps.hip takes the other layers):
 //   dw[co][ci][kh][kw] = sum over images, rows h, columns w of dy[co][h][w] * x_pad[ci][h+kh][w+kw]
 //
 // The reduction runs over pixels, and eight neighbouring pixels of a channel row are 16
@@ -372,6 +372,15 @@ static uint64_t wgrad_bf16_items(uint32_t num_tiles, uint32_t N, uint32_t W) {
 size_t conv_bf16_wgrad_mfma_workspace_bytes(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t W) {
   const size_t pairs = (size_t)((Cin + 63u) / 64u) * ((Cout + 63u) / 64u);
   return pairs * wgrad_bf16_blocks(wgrad_bf16_items(num_tiles, N, W)) * kWgPartialFloats * sizeof(float);
+}
+
+// Expected time in us, from 158 layers of 16 to 512 channels (rms error 7 %): rows one after the other in as many rounds as there are
+// workgroups (of 112 KB of LDS) per compute unit, and the partials' way to memory and back.
+double conv_bf16_wgrad_mfma_us(uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
+  const uint64_t items = wgrad_bf16_items(num_tiles, N, W), blocks = items < 256u ? items : 256u;
+  const uint64_t pairs = (uint64_t)((Cin + 63u) / 64u) * ((Cout + 63u) / 64u), wg = blocks * pairs, per = (items + blocks - 1u) / blocks;
+  const double rounds = per * (0.8 * ((wg + 255u) / 256u) + 0.2 * wg / 256.0);
+  return 9.3 + rounds * (0.886 * (H + 2.0) + 0.7) + 0.29e-6 * sizeof(float) * kWgPartialFloats * wg;
 }
 
 // Arguments are validated by the caller (pointers, alignment, workspace size, extents > 0).

@@ -25,20 +25,17 @@
 #include <algorithm>
 #include <cmath>
 
-#include "split_bf16.h"
+#include "wgrad_sums.h"
 
 namespace adh {
 
-struct S2WgParams {
+struct S2WgParams : WgradSums {
   const void *x[ADH_MAX_TILES], *dy[ADH_MAX_TILES];
-  float *part;  // [channel group][split][wave][ot][tap][lane][4]
-  float *dw;
-  uint32_t N, Cin, Cout;
+  uint32_t N;
   uint32_t dy_H, dy_W, x_H, x_W, dy_VH, last_tile;
   uint32_t logT, TW, RS, NR, swizzle;  // TW = 1 << logT; swizzle: dy's octets of channel c are exchanged by c >> swizzle
-  uint32_t row_steps, total_steps, splits, ci_groups;
-  float beta;
-  FastDiv div_row_steps, div_cols, div_H, div_splits, div_cig;
+  uint32_t row_steps, total_steps, ci_groups;
+  FastDiv div_row_steps, div_cols, div_H, div_splits;
 };
 
 constexpr uint32_t s2wg_ring(uint32_t rs, int taps) { return taps == 9 ? 4u * rs + 1u : 2u * rs; }
@@ -376,37 +373,6 @@ __global__ __launch_bounds__(64 * WO * WC, 2) void conv_s2_wgrad_kernel(const S2
   }
 }
 
-// dw = beta*dw + the splits' sums.  Sixteen lanes take sixteen neighbouring groups of four sums and 16 slices of the splits
-// each (slice j: splits j, j + 16, ..); the slices are then added in order: a fixed order, so the result has fixed bits.  In
-// double: as many fp32 additions of ever larger sums cost half a digit.
-template <int TAPS, int OT, int WO, int WC>
-__global__ __launch_bounds__(256) void conv_s2_wgrad_reduce_kernel(const S2WgParams P) {
-  typedef double doublex4 __attribute__((ext_vector_type(4)));
-  __shared__ doublex4 sums[16][16];
-  constexpr uint32_t kQuads = WO * WC * OT * TAPS * 64u;  // of a channel group
-  const uint32_t quad = blockIdx.x * 16u + (threadIdx.x & 15u), slice = threadIdx.x >> 4;
-  const uint32_t group = quad / kQuads, e = quad - group * kQuads;
-  const floatx4 *p = reinterpret_cast<const floatx4 *>(P.part) + (size_t)group * P.splits * kQuads + e;
-  doublex4 sum = {0.0, 0.0, 0.0, 0.0};
-  for (uint32_t k = slice; k < P.splits; k += 16u) sum += __builtin_convertvector(*reinterpret_cast<const floatx4 *>(p + (size_t)k * kQuads), doublex4);
-  sums[slice][threadIdx.x & 15u] = sum;
-  __syncthreads();
-  if (slice != 0u) return;
-#pragma unroll
-  for (int k = 1; k < 16; ++k) sum += sums[k][threadIdx.x];
-  const uint32_t ln = e & 63u, rest = e >> 6, tap = rest % TAPS, ot = rest / TAPS % OT, wt = rest / TAPS / OT;
-  uint32_t cog, cig;
-  P.div_cig.divmod(group, cog, cig);
-  const uint32_t co = cog * (16u * OT * WO) + ((wt % WO) * OT + ot) * 16u + (ln >> 4) * 4u, ci = cig * (16u * WC) + (wt / WO) * 16u + (ln & 15u);
-  if (ci >= P.Cin) return;
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    if (co + i >= P.Cout) break;
-    float *d = P.dw + ((size_t)(co + i) * P.Cin + ci) * TAPS + tap;
-    *d = (float)(P.beta != 0.f ? (double)*d + sum[i] : sum[i]);
-  }
-}
-
 // ---- host side ----
 
 struct S2WgPlan {
@@ -484,7 +450,7 @@ size_t conv_s2_wgrad_required(const S2WgradProblem &q) {
 template <typename T, int TAPS, int OT, int WO, int WC>
 static void launch_s2wg(const S2WgPlan &plan, hipStream_t st) {
   hipLaunchKernelGGL((conv_s2_wgrad_kernel<T, TAPS, OT, WO, WC>), dim3(plan.groups * plan.P.splits), dim3(64 * WO * WC), 0, st, plan.P);
-  hipLaunchKernelGGL((conv_s2_wgrad_reduce_kernel<TAPS, OT, WO, WC>), dim3(plan.groups * (WO * WC * OT * TAPS * 64u / 16u)), dim3(256), 0, st, plan.P);
+  hipLaunchKernelGGL((wgrad_sums_kernel<TAPS, OT, WO, WC>), dim3(plan.groups * (WO * WC * OT * TAPS * 64u / 16u)), dim3(256), 0, st, static_cast<const WgradSums &>(plan.P));
 }
 template <typename T, int TAPS>
 static void launch_s2wg_channels(const S2WgPlan &plan, hipStream_t st) {
