@@ -2,9 +2,9 @@
 //   dw[co][ci][a][b] = beta*dw + sum over images, R, Q of dy[co][R][Q] * x[ci][R + a - pad_r][Q + b - pad_c]
 //
 // Mapping.  Per tap D[co][ci] += A[co][pixel] B[pixel][ci] on v_mfma_f32_16x16x32_bf16, k = 32 pixels: four octets of
-// neighbouring pixels of a row.  Both tensors lie in LDS as they do in memory, [channel][pixel] (no transposition), in three
-// parts; an operand is one ds_read_b128, and the window's second and third columns come from the same octet and the dword
-// after it by v_alignbit.
+// neighbouring pixels of a row.  Both tensors lie in LDS as [row][octet][channel] (octet_swap), in three parts; an operand is one
+// ds_read_b128, and the window's second and third columns come from the same octet and the next one's first columns (a
+// ds_read_b64: 4.3 cycles, a dword 8) by v_alignbit.
 //   * A workgroup of eight waves, one per compute unit, owns 32*OT output channels x 32*CT input channels x nine taps and a
 //     run of steps; a step is RS rows of TW columns (2 x 32, 4 x 16 or 8 x 8), half of its octets for each half of the
 //     waves.  A wave keeps 16*OT x 16*CT x 9 sums: at OT = CT = 2 a step is 216 MFMAs
@@ -21,9 +21,10 @@
 //
 // Measured (32 images, 4 tiles without halo; the v_mfma_f32 kernel before): 64 channels on 32 x 128 tiles 0.351 -> 0.197 ms
 // (196 TFLOP/s), 128 on 16 x 64 0.354 -> 0.193, 256 on 8 x 32 0.361 -> 0.195, 512 on 4 x 16 0.456 -> 0.21 (0.61 through the
-// general entry point before).  Staging: with rows, channels and tiles worked out per group of four values the kernel took
+// general entry point before); with [octet][channel] rows in place of [channel][pixel] ones, where bank conflicts took 0.41 of all cycles,
+// 0.181, 0.173, 0.175, 0.192, and 1.08 times as fast in the mean of 115 layers (176 -> 16 channels on 3 tiles of 7 x 391 116 -> 91 us).  Staging: with rows, channels and tiles worked out per group of four values the kernel took
 // 0.45 ms; a thread's channel and column fixed and a wave's row uniform it is a load, a split and three writes.  Bound: a
-// step of 6912 matrix cycles takes about 12000, the splitting and the shifts (a third of the issue slots) and the clock,
+// step of 6912 matrix cycles takes about 11000, the splitting and the shifts (a third of the issue slots) and the clock,
 // which the power limit holds at 1.8 - 2.1 GHz; and on short layers the workgroups' sums, 38 MB written and read back.
 #include "conv3x3_wgrad_split.h"
 
@@ -43,7 +44,8 @@ struct WgradSplitParams {
   uint32_t N, Cin, Cout, num_tiles;
   uint32_t x_H, x_W, dy_H, dy_W, x_VH, dy_VH, step, last_tile;
   int32_t pad_r, pad_c, neighbours;
-  uint32_t TW, logQ, RS, NR, XP, DP;        // logQ: log2 of a row's groups of four columns; pitches in pixels
+  uint32_t TW, logQ, RS, NR;                // logQ: log2 of a row's groups of four columns
+  uint32_t x_row_bytes, dy_row_bytes;       // of one part of a row of x (with the octet behind it) and of dy
   uint32_t x_part_bytes, dy_part_bytes;     // bytes of one part of the ring and of the dy buffers
   uint32_t col_tiles, row_steps, total_steps, splits, ci_groups, group0;
   float beta;
@@ -92,6 +94,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   const uint32_t x_rows = kWsThreads / (CI << P.logQ), dy_rows = kWsThreads / (CO << P.logQ);  // per 512 groups
   const uint32_t x_row = (wave * 64u) >> P.logQ >> (CT == 2 ? 6 : 5), dy_row = (wave * 64u) >> P.logQ >> (OT == 2 ? 6 : 5);
   const bool c_x_ok = ci0 + c_x < P.Cin, c_dy_ok = co0 + c_dy < P.Cout, c_tail_ok = lane < CI && ci0 + lane < P.Cin;
+  const uint32_t x_to = ((q >> 1) * CI + (c_x ^ octet_swap(q >> 1))) * 16u + (q & 1u) * 8u, dy_to = ((q >> 1) * CO + (c_dy ^ octet_swap(q >> 1))) * 16u + (q & 1u) * 8u;
   const size_t x_chan = (size_t)(c_x_ok ? ci0 + c_x : 0u) * x_plane, dy_chan = (size_t)(c_dy_ok ? co0 + c_dy : 0u) * dy_plane;
   const size_t tail_chan = (size_t)(c_tail_ok ? ci0 + lane : 0u) * x_plane;
   // columns by which four loaded values lie left of the wanted ones (they are loaded inside the row); 4: none exists
@@ -175,20 +178,20 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
       const uint32_t i = (uint32_t)j * x_rows + x_row;
-      if (i < nx) put(moved(vx[j], x_shift), lds + (slot_of(i) * (CI * P.XP) + c_x * P.XP + 4u * q) * 2u, P.x_part_bytes);
+      if (i < nx) put(moved(vx[j], x_shift), lds + slot_of(i) * P.x_row_bytes + x_to, P.x_part_bytes);
       __builtin_amdgcn_sched_barrier(0);
     }
 #pragma unroll
     for (int j = 0; j < DR; ++j) {
       const uint32_t i = (uint32_t)j * dy_rows + dy_row;
-      if (i < nd) put(moved(vd[j], dy_shift), dyl + ((buf * P.RS + i) * (CO * P.DP) + c_dy * P.DP + 4u * q) * 2u, P.dy_part_bytes);
+      if (i < nd) put(moved(vd[j], dy_shift), dyl + (buf * P.RS + i) * P.dy_row_bytes + dy_to, P.dy_part_bytes);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (wave < nx && lane < CI) {
       if (!c_tail_ok) tail[0] = tail[1] = 0.f;
       uint32_t part[3];
       split_pair(tail[0], tail[1], part[0], part[1], part[2]);
-      char *p = lds + (slot_of(wave) * (CI * P.XP) + lane * P.XP + P.TW) * 2u;
+      char *p = lds + slot_of(wave) * P.x_row_bytes + ((P.TW >> 3) * CI + (lane ^ octet_swap(P.TW >> 3))) * 16u;
 #pragma unroll
       for (int k = 0; k < 3; ++k) *reinterpret_cast<uint32_t *>(p + k * P.x_part_bytes) = part[k];
     }
@@ -196,8 +199,8 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
 
   // ---- this lane group's octet of a step: row io of the step, octet qo of the row ----
   const uint32_t oct = half * 4u + g, io = oct >> (P.logQ - 1u), qo = oct & ((1u << (P.logQ - 1u)) - 1u);
-  const uint32_t b_base = ((wc * CT * 16u + l16) * P.XP + 8u * qo) * 2u;
-  const uint32_t a_base = ((io * CO + wo * OT * 16u + l16) * P.DP + 8u * qo) * 2u;
+  const uint32_t b_base = (qo * CI + wc * CT * 16u + (l16 ^ octet_swap(qo))) * 16u, e_base = ((qo + 1u) * CI + wc * CT * 16u + (l16 ^ octet_swap(qo + 1u))) * 16u;
+  const uint32_t a_base = io * P.dy_row_bytes + (qo * CO + wo * OT * 16u + (l16 ^ octet_swap(qo))) * 16u;
 
   floatx4 acc[OT][CT][9];
 #pragma unroll
@@ -214,17 +217,17 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
     for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
       for (int k = 0; k < 3; ++k)
-        a[ot][k] = *reinterpret_cast<const uintx4 *>(dyl + k * P.dy_part_bytes + a_base + (ot * 16u + buf * P.RS * CO) * P.DP * 2u);
-    struct Operand { uintx4 d; uint32_t e; };
+        a[ot][k] = *reinterpret_cast<const uintx4 *>(dyl + k * P.dy_part_bytes + a_base + ot * 256u + buf * P.RS * P.dy_row_bytes);
+    struct Operand { uintx4 d; uintx2 e; };  // an octet, the next one's first columns
     Operand b[2][3];
     auto fetch = [&](int set, int r, int ct) {
       uint32_t slot = base + io + (uint32_t)r;
       slot -= slot >= P.NR ? P.NR : 0u;
-      const char *p = lds + slot * (CI * P.XP * 2u) + b_base + ct * (16u * P.XP * 2u);
+      const char *p = lds + slot * P.x_row_bytes + ct * 256u;
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        b[set][k].d = *reinterpret_cast<const uintx4 *>(p + k * P.x_part_bytes);
-        b[set][k].e = *reinterpret_cast<const uint32_t *>(p + k * P.x_part_bytes + 16u);
+        b[set][k].d = *reinterpret_cast<const uintx4 *>(p + b_base + k * P.x_part_bytes);
+        b[set][k].e = *reinterpret_cast<const uintx2 *>(p + e_base + k * P.x_part_bytes);
       }
     };
     fetch(0, 0, 0);
@@ -235,8 +238,9 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
       uintx4 w[3][3];  // part, window column
 #pragma unroll
       for (int k = 0; k < 3; ++k) {
-        const uintx4 d = b[cur][k].d;
-        const uint32_t e = b[cur][k].e;
+        uintx4 d = b[cur][k].d;
+        asm("" : "+v"(d));  // (the compiler would read the shifted columns from LDS again, dword by dword)
+        const uint32_t e = b[cur][k].e[0];
         w[k][0] = d;
         w[k][1] = uintx4{__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
                          __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(e, d[3], 16)};
@@ -450,12 +454,14 @@ int conv3x3_wgrad_split(const Wgrad3x3Problem &q, void *workspace, size_t worksp
     const double cost = (double)NI * ((q.dy_W + TW - 1u) / TW) * ((P.dy_VH + RS - 1u) / RS + 0.75) * (logQ == 3u ? 1.0 : logQ == 2u ? 1.05 : 1.25);
     if (cost < best) {
       best = cost;
-      P.logQ = logQ; P.TW = TW; P.RS = RS; P.XP = TW + 8u; P.DP = TW;
+      P.logQ = logQ; P.TW = TW; P.RS = RS;
     }
   }
   P.NR = 2u * P.RS + 2u;
-  P.x_part_bytes = P.NR * 32u * CT * P.XP * 2u;
-  P.dy_part_bytes = 2u * P.RS * 32u * OT * P.DP * 2u;
+  P.x_row_bytes = (P.TW / 8u + 1u) * 32u * CT * 16u;
+  P.dy_row_bytes = P.TW / 8u * 32u * OT * 16u;
+  P.x_part_bytes = P.NR * P.x_row_bytes;
+  P.dy_part_bytes = 2u * P.RS * P.dy_row_bytes;
   P.col_tiles = (q.dy_W + P.TW - 1u) / P.TW;
   P.row_steps = (P.dy_VH + P.RS - 1u) / P.RS;
   const uint64_t total = (uint64_t)NI * P.col_tiles * P.row_steps;

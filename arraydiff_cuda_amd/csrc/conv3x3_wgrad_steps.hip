@@ -32,11 +32,11 @@ namespace adh {
 
 struct StepsParams : WgradSums {
   const void *x[ADH_MAX_TILES], *dy[ADH_MAX_TILES];
-  uint32_t N, stacked;
+  uint32_t N, stacked, by_xcd;
   uint32_t H, W, x_H, x_W;         // a tile's dy and x
   uint32_t rows, x_rows;           // of a plane (an image; stacked: of all tiles): of dy and x
   uint32_t row_steps, cols, total_steps, ci_groups;
-  FastDiv div_row_steps, div_cols, div_H, div_N, div_groups;
+  FastDiv div_row_steps, div_cols, div_H, div_N, div_groups, div_splits;
 };
 
 // k blocks (of 32 pixels) a step, the widest step
@@ -48,10 +48,6 @@ constexpr uint32_t steps_narrowest(bool few) { return few ? 16u : 8u; }
 // of one part: x rows with an octet behind them (whose first two columns exist), dy rows, twice
 constexpr uint32_t steps_x_bytes(uint32_t tw, uint32_t ci, uint32_t kb) { return steps_ring(kb * 32u / tw) * (tw / 8u + 1u) * ci * 16u; }
 constexpr uint32_t steps_dy_bytes(uint32_t co, uint32_t kb) { return 2u * kb * 4u * co * 16u; }
-// Rows lie in LDS as [octet of columns][channel].  An octet's channels are exchanged by this: the writes of a channel's octets
-// spread over the banks, and the reads (the hardware takes eight channels of one octet with the other eight of the next) don't meet.
-__device__ __forceinline__ uint32_t steps_swap(uint32_t octet) { return (octet & 3u) | ((octet & 4u) ? 12u : 0u); }
-
 // How THREADS threads take a row's units of eight columns, columns first, then channels, then rows (a wave's units are of one row):
 // unit j of a thread is channel pass j % passes of row (j / passes) * rows + the thread's.
 template <uint32_t THREADS, uint32_t U, uint32_t C>
@@ -126,10 +122,9 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
   const uint32_t wo = wave % WO, wc = wave / WO;
 
-  // Workgroups go to the eight XCDs in turn; an XCD takes neighbouring splits of all channel groups, which share rows.
   uint32_t group, split, cog, cig;
-  const uint32_t xcd = blockIdx.x & 7u, per = gridDim.x >> 3, more = gridDim.x & 7u;
-  P.div_groups.divmod(xcd * per + min(xcd, more) + (blockIdx.x >> 3), split, group);
+  if (P.by_xcd) xcd_order(P.div_groups, split, group);
+  else P.div_splits.divmod(blockIdx.x, group, split);
   P.div_cig.divmod(group, cog, cig);
   const uint32_t co0 = cog * CO, ci0 = cig * CI;
   const uint32_t s_begin = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
@@ -141,8 +136,8 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
 
   const XUnits xu(tid, wave);
   const DyUnits du(tid, wave);
-  const uint32_t q8 = 8u * xu.q, swap = steps_swap(xu.q), tail_c = tid % CI, tail_row = tid / CI;
-  const uint32_t tail_to = (U * CI + (tail_c ^ steps_swap(U))) * 16u;
+  const uint32_t q8 = 8u * xu.q, swap = octet_swap(xu.q), tail_c = tid % CI, tail_row = tid / CI;
+  const uint32_t tail_to = (U * CI + (tail_c ^ octet_swap(U))) * 16u;
 
   // a step: row step rs of a run (an image's column tile), whether the run's rows begin with it
   struct Step {
@@ -321,7 +316,7 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
     // this lane group's octet of k block kb: row io of the step, octet qo of the row
     auto row_of = [&](uint32_t kb) { return U >= 4u ? kb * 4u / U : kb * (4u / U) + g / U; };
     auto octet_of = [&](uint32_t kb) { return U >= 4u ? kb * 4u % U + g : g % U; };
-    auto lane_at = [&](uint32_t octet, uint32_t C, uint32_t c0) { return (octet * C + c0 + (l16 ^ steps_swap(octet))) * 16u; };
+    auto lane_at = [&](uint32_t octet, uint32_t C, uint32_t c0) { return (octet * C + c0 + (l16 ^ octet_swap(octet))) * 16u; };
     auto read_dy = [&](uint32_t kb, uintx4 (&v)[OT][PARTS]) {
       const char *p = dyl + (buf * RS + row_of(kb)) * (U * CO * 16u) + lane_at(octet_of(kb), CO, wo * OT * 16u);
 #pragma unroll
@@ -515,6 +510,9 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   }
   if (best == 1e300 || (uint64_t)groups * P.splits >= (1ull << 22)) return false;
   plan->us = steps_us(cost, plan->TW, groups, P.splits, P.total_steps, plan->split_bytes);
+  // From half of what the XCDs' caches hold (8 x 4 MB): 240 -> 16 channels on 4 tiles of 20 x 104, 81 MB, 85 -> 59 us, 1.08 in the mean from 32 MB,
+  // 1.02 from 16; smaller ones lose 1 to 4 % (up to 16 %), as the partial sums' order suits the second kernel less.
+  P.by_xcd = (uint64_t)q.num_tiles * q.N * q.H * q.W * (q.Cin + q.Cout) * (parts == 3 ? 4u : 2u) > (16ull << 20) ? 1u : 0u;
   P.div_row_steps = FastDiv(P.row_steps); P.div_cols = FastDiv(P.cols); P.div_H = FastDiv(q.stacked ? P.H : 1u << 31); P.div_N = FastDiv(P.N);
   P.div_cig = FastDiv(P.ci_groups);
   return true;
@@ -557,7 +555,7 @@ int conv3x3_wgrad_steps(const StepsWgradProblem &q, void *workspace, size_t work
   if (!steps_plan(q, &plan) || workspace_bytes < plan.split_bytes) return ADH_EUNIMPL;
   StepsParams &P = plan.P;
   P.splits = (uint32_t)std::min<uint64_t>(P.splits, workspace_bytes / plan.split_bytes);
-  P.div_groups = FastDiv(plan.groups);
+  P.div_groups = FastDiv(plan.groups); P.div_splits = FastDiv(P.splits);
   for (uint32_t t = 0; t < q.num_tiles; ++t) {
     P.x[t] = q.x[t];
     P.dy[t] = q.dy[t];
