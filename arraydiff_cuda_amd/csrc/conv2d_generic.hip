@@ -19,6 +19,7 @@
 // group.  bf16 tensors are widened while staging and rounded when stored: the arithmetic is fp32.
 #include "conv3x3_split.h"
 #include "conv_bf16_patch.h"
+#include "conv_f32_patch.h"
 #include "conv_s2_wgrad.h"
 #include "conv3x3_wgrad_split.h"
 
@@ -628,10 +629,10 @@ static Conv3x3Problem gen_3x3_problem(int which, const GenShape &g, uint32_t num
   }
   return q;
 }
-// conv_bf16_patch.hip: bf16 tensors, forward and backward-data.  3x3 windows at stride 1 and (over tiles of even height and width
+// conv_bf16_patch.hip, conv_f32_patch.hip: forward and backward-data.  3x3 windows at stride 1 and (over tiles of even height and width
 // without halo) 2; 1x1 windows at stride 1 and 2 (backward-data: even heights and widths).  The number of taps, or 0.
-static int gen_patch_taps(int which, int dtype, const GenShape &g, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
-  if (dtype != ADH_BF16 || g.sh != g.sw || g.sh > 2u) return 0;
+static int gen_patch_taps(int which, const GenShape &g, bool unpadded, uint32_t pad_h, uint32_t pad_w) {
+  if (g.sh != g.sw || g.sh > 2u) return 0;
   if (g.kh == 1u && g.kw == 1u) {
     if (unpadded && (pad_h || pad_w)) return 0;
     return g.sh == 1u || which == ADH_CONV_FWD || (g.HP % 2u == 0u && g.WP % 2u == 0u) ? 1 : 0;
@@ -1296,6 +1297,13 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     if (e) return e;
     e = conv1x1_try(false, num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, g.sh, x_tiles, w, y_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
+    if (gen_patch_taps(ADH_CONV_FWD, g, unpadded, pad_h, pad_w) == 1) {
+      Conv3x3Problem q = gen_patch_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w, 1);
+      q.beta = beta;
+      q.in = x_tiles; q.out = y_tiles; q.w = w;
+      e = conv_f32_patch(q, 1, as_stream(stream));
+      if (e != ADH_EUNIMPL) return e;
+    }
   }
   if (gen_is_thin(dtype, g, unpadded)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
@@ -1311,6 +1319,10 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = x_tiles; q.out = y_tiles; q.w = w;
+    if (conv_f32_patch_ahead(q, workspace != nullptr)) {
+      e = conv_f32_patch(q, 9, as_stream(stream));
+      if (e != ADH_EUNIMPL) return e;
+    }
     // Stride 2: the two kernels stand as 0.85 - 0.91 to 1 in time where the split one's rounds are full, from 64 to 1024 channels
     // on either side; its blocks are coarse, and with more than an eighth of the rounds idle the fp32 one is ahead (of full
     // rounds: 9/16 1.08 - 1.13, 3/4 1.08 - 1.15, 5/6 1.06, 9/10 0.97 - 1.0).  A single round is the split one's: 0.15 - 0.85 with
@@ -1322,7 +1334,7 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
-  if (const int taps = gen_patch_taps(ADH_CONV_FWD, dtype, g, unpadded, pad_h, pad_w)) {
+  if (const int taps = dtype != ADH_BF16 ? 0 : gen_patch_taps(ADH_CONV_FWD, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
     Conv3x3Problem q = gen_patch_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w, taps);
@@ -1365,6 +1377,13 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     if (e) return e;
     e = conv1x1_try(true, num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, g.sh, dy_tiles, w, dx_tiles, beta, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
+    if (gen_patch_taps(ADH_CONV_BWD_DATA, g, unpadded, pad_h, pad_w) == 1) {
+      Conv3x3Problem q = gen_patch_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w, 1);
+      q.beta = beta;
+      q.in = dy_tiles; q.out = dx_tiles; q.w = w;
+      e = conv_f32_patch(q, 1, as_stream(stream));
+      if (e != ADH_EUNIMPL) return e;
+    }
   }
   if (gen_is_3x3_split(dtype, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
@@ -1372,10 +1391,14 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = dy_tiles; q.out = dx_tiles; q.w = w;
+    if (conv_f32_patch_ahead(q, workspace != nullptr)) {
+      e = conv_f32_patch(q, 9, as_stream(stream));
+      if (e != ADH_EUNIMPL) return e;
+    }
     e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
-  if (const int taps = gen_patch_taps(ADH_CONV_BWD_DATA, dtype, g, unpadded, pad_h, pad_w)) {
+  if (const int taps = dtype != ADH_BF16 ? 0 : gen_patch_taps(ADH_CONV_BWD_DATA, g, unpadded, pad_h, pad_w)) {
     e = gen_check_workspace(plan, workspace, workspace_bytes);
     if (e) return e;
     Conv3x3Problem q = gen_patch_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w, taps);

@@ -3,6 +3,7 @@
 //   forward       : in = x, out = y,  Wt(o=co,k=ci,a,b) = w[co][ci][a][b]
 //   backward-data : in = dy, out = dx, Wt(o=ci,k=co,a,b) = w[co][ci][2-a][2-b]; over padded tiles dx is the WHOLE padded slab
 #include "conv3x3_split.h"
+#include "conv_f32_patch.h"
 
 #include <stdio.h>
 
@@ -64,6 +65,11 @@ static int conv_direct(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   Conv3x3Problem q = conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, rows_from_neighbours, unpadded);
   q.beta = res_tiles ? 1.f : beta;
   q.in = in_tiles; q.out = out_tiles; q.res = res_tiles; q.w = w;
+  // (of the plain form, for all forms of a layer: their sums have the same bits)
+  if (conv_f32_patch_ahead(conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, unpadded), false)) {
+    const int e = conv_f32_patch(q, 9, st);
+    if (e != ADH_EUNIMPL) return e;
+  }
   return conv3x3_split(q, nullptr, 0, st);
 }
 
@@ -91,7 +97,8 @@ int adh_conv3x3_kernel_name(int which, int dtype, uint32_t num_tiles, uint32_t N
     return ADH_OK;
   }
   if (dtype != ADH_F32) return ADH_EINVAL;
-  conv3x3_split_name(conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, false), name, name_bytes);
+  const Conv3x3Problem q = conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, false);
+  if (!conv_f32_patch_ahead(q, false) || !conv_f32_patch_name(q, 9, name, name_bytes)) conv3x3_split_name(q, name, name_bytes);
   return ADH_OK;
 }
 

@@ -584,6 +584,7 @@ struct SplitPlan {
   SplitParams P;
   int MT, NT, low;
   bool vec;
+  double cycles;  // expected
   size_t part_bytes;
 };
 
@@ -687,6 +688,7 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
     }
   }
   if (nbi == 0u) return ADH_EUNIMPL;
+  plan->cycles = best;
   const uint32_t MG = (P.M + 16u * plan->MT - 1u) / (16u * plan->MT), PCP = patch(P.BC), PPI = patch(P.BR) * PCP;
   P.PPn = P.NB * PPI;
   plan->vec = P.BC % 4u == 0u && P.grid_W % 4u == 0u;
@@ -705,6 +707,11 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
 size_t conv3x3_split_workspace(const Conv3x3Problem &q) {
   SplitPlan plan = {};
   return split_plan(q, true, &plan) ? 0u : (plan.part_bytes + 255u) & ~(size_t)255u;
+}
+
+double conv3x3_split_us(const Conv3x3Problem &q, bool workspace) {
+  SplitPlan plan = {};
+  return split_plan(q, workspace, &plan) ? 1e300 : plan.cycles / 2100.0;
 }
 
 bool conv3x3_split_idles(const Conv3x3Problem &q) {

@@ -19,36 +19,16 @@
 // to 7 %, half the tile (no spilled registers) 4 to 40 %.
 #include "conv_bf16_patch.h"
 
+#include "conv_patch_plan.h"
+
 #include <stdio.h>
 
 #include <algorithm>
+#include <cmath>
 
 #include "split_bf16.h"
 
 namespace adh {
-
-constexpr uint32_t kPtThreads = 256;
-// pixels of a patch plane in LDS
-constexpr uint32_t pt_pixels(int sample, int taps, int nt) {
-  return taps == 1 ? 64u * nt + 16u : sample == kDown ? 640u : nt == 4 ? 640u : nt == 2 ? 384u : 256u;
-}
-
-struct PatchParams {
-  const uint16_t *in[ADH_MAX_TILES];
-  uint16_t *out[ADH_MAX_TILES];
-  const uint16_t *w;  // the caller's, or (READY) in the order of the LDS: [64 m][chunk][tap][octet][m][8 channels]
-  uint32_t N, NI, C, M, num_tiles;
-  uint32_t in_H, in_W, out_H, out_W;
-  uint32_t in_VH, grid_VH, grid_W;  // rows of the (stacked) input; what the blocks tile: output pixels, or quads of them
-  uint32_t in_lead, out_lead, in_step, out_step, last_tile;
-  uint32_t w_m_stride, w_c_stride;
-  uint32_t BR, BC, NB, pitch, image;  // a block's pixels: BR x BC of NB images; pixels of a patch row, of an image's patch
-  uint32_t nchunks, blocks, xcd_chunk;
-  int32_t pad_r, pad_c, flip;
-  uint32_t dil;
-  float beta;
-  FastDiv div_bpg, div_nbj, div_MG, div_N, div_BC, div_live, div_pairs, div_pairs_img, div_pairs_row, div_in, div_out;
-};
 
 typedef uint32_t pt_u32 __attribute__((aligned(2)));
 typedef uintx4 pt_u32x4 __attribute__((aligned(2)));
@@ -113,7 +93,7 @@ __global__ __launch_bounds__(kPtThreads) void conv_bf16_patch_filter_kernel(cons
 template <int MT, int NT, int SAMPLE, int TAPS, bool READY>
 __global__ __launch_bounds__(kPtThreads, 2) void conv_bf16_patch_kernel(const PatchParams P) {
   constexpr uint32_t MW = 16u * MT, OCT = TAPS == 1 ? 8u : 4u, CHUNK = 8u * OCT;
-  constexpr uint32_t PP = pt_pixels(SAMPLE, TAPS, NT);
+  constexpr uint32_t PP = pt_pixels(SAMPLE, TAPS, NT, 1);
   constexpr bool SINGLE = SAMPLE == kDown && TAPS == 1;  // of a pair only the first pixel is of use
   constexpr int XU = (OCT * PP / (SINGLE ? 1u : 2u) + kPtThreads - 1u) / kPtThreads;  // (pair, octet) units a thread stages
   constexpr int WU = (MW * OCT + kPtThreads - 1u) / kPtThreads;                       // (m, octet) units
@@ -122,7 +102,7 @@ __global__ __launch_bounds__(kPtThreads, 2) void conv_bf16_patch_kernel(const Pa
   constexpr uint32_t DOWN = SAMPLE == kDown ? 2u : 1u, UP = SAMPLE == kUp ? 2u : 1u;
   __shared__ __align__(16) uintx4 xl[OCT * PP];
   __shared__ __align__(16) uintx4 wl[TAPS * OCT * MW];
-  __shared__ const uint16_t *tab[2 * ADH_MAX_TILES];
+  __shared__ const void *tab[2 * ADH_MAX_TILES];
   const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
   const uint32_t wave = (uint32_t)__builtin_amdgcn_readfirstlane((int)(tid >> 6));
 
@@ -231,7 +211,7 @@ __global__ __launch_bounds__(kPtThreads, 2) void conv_bf16_patch_kernel(const Pa
   uintx4 rv[READY ? RU : 1];
   auto load_w = [&](uint32_t ch) {
     if constexpr (READY) {
-      const uintx4 *base = reinterpret_cast<const uintx4 *>(P.w) + (size_t)(mg * MW / 64u * P.nchunks + ch) * (TAPS * OCT * 64u) + mg * MW % 64u;
+      const uintx4 *base = static_cast<const uintx4 *>(P.w) + (size_t)(mg * MW / 64u * P.nchunks + ch) * (TAPS * OCT * 64u) + mg * MW % 64u;
 #pragma unroll
       for (int j = 0; j < RU; ++j) {
         const uint32_t u = tid + (uint32_t)j * kPtThreads;
@@ -244,7 +224,7 @@ __global__ __launch_bounds__(kPtThreads, 2) void conv_bf16_patch_kernel(const Pa
         if (wave * 64u + (uint32_t)j * kPtThreads >= MW * OCT) break;
         const FilterUnit F = w_unit(j);
         const uint32_t c0 = ch * CHUNK + 8u * F.o;
-        const uint16_t *p = P.w + (size_t)min(mg * MW + F.m, P.M - 1u) * P.w_m_stride + (size_t)min(c0, P.C - 1u) * P.w_c_stride;
+        const uint16_t *p = static_cast<const uint16_t *>(P.w) + (size_t)min(mg * MW + F.m, P.M - 1u) * P.w_m_stride + (size_t)min(c0, P.C - 1u) * P.w_c_stride;
         pt_load_filter<TAPS>(p, c0, P.C, P.w_c_stride, wv[j]);
       }
     }
@@ -386,13 +366,19 @@ __global__ __launch_bounds__(kPtThreads, 2) void conv_bf16_patch_kernel(const Pa
 
 // ---- host side ----
 
-struct PatchPlan {
-  PatchParams P;
-  int MT, NT;
-  bool ready;    // the filter is put in order first
-  uint64_t units;  // of eight channels' taps in it
-  double us;     // what the launches are expected to take
-};
+// fp32: what `blocks` blocks of patches of `staged` pixels are expected to take, as fitted to 230 launches at stride 1 (rms error 6 %).
+static double f32_patch_us(const Conv3x3Problem &q, int taps, int MT, int NT, uint32_t chunks, uint64_t blocks, uint32_t staged) {
+  const bool two = taps == 1 || (MT == 1 && NT == 1 && q.sample != kDown);  // workgroups on a compute unit
+  const double fit = two ? 512.0 : 256.0, rounds = std::max(1.0, 0.77 * std::ceil(blocks / fit) + 0.23 * blocks / fit);
+  const double shared = two && blocks > 256u ? 1.0 + 0.336 * std::min(1.0, (blocks - 256.0) / 256.0) : 1.0;
+  const double multiply = taps * (taps == 1 ? 2.0 : 1.0) * std::max(96.0 * MT * NT, 55.0 * (MT + NT));  // cycles, or operands' way out of LDS
+  const double filter = (taps == 1 ? 0.17 : 0.757) * MT * (q.flip ? 0.534 : 1.0);
+  return 2.8 + rounds * (1.7 + chunks * shared * (0.00096 * multiply + (taps == 1 ? 0.0053 : 0.00267) * staged + filter + 0.37));
+}
+// a chunk's multiplications, or their operands' way out of LDS
+static double patch_multiply(int taps, uint32_t chunk, int MT, int NT) {
+  return taps * (chunk / 32u) * std::max(16.0 * MT * NT, 32.0 * (MT + NT));
+}
 
 // Blocks of BR x BC output pixels (of NB images) by 16 MT channels, two workgroups per compute unit.  The tile is chosen by a model of
 // a block's cycles: a chunk's multiplications (or their operands' way out of LDS), its staging, and a load's latency.
@@ -402,7 +388,7 @@ struct PatchPlan {
 //   put in order first   2.1 + rounds (5.4 + n 0.00096 multiply (1 + 1.06 f)) us
 // (from 20 us on the second: forward, the caller's filter costs a line of cache per lane and load.  64 -> 64 channels, 8 tiles of
 // 128 x 2048 717 -> 578 us, 16 -> 32 on 72 x 16 4.7 -> 7.3.)
-static int patch_plan(const Conv3x3Problem &q, int taps, size_t workspace_bytes, PatchPlan *plan) {
+int patch_plan(const Conv3x3Problem &q, int taps, int parts, size_t workspace_bytes, PatchPlan *plan) {
   PatchParams &P = plan->P;
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
   P.NI = q.stacked ? q.N : q.N * q.num_tiles;
@@ -431,13 +417,14 @@ static int patch_plan(const Conv3x3Problem &q, int taps, size_t workspace_bytes,
   double best = 1e300;
   uint32_t nbi = 0, nbj = 0;
   const uint64_t grid_pixels = (uint64_t)P.NI * P.grid_VH * P.grid_W;
-  for (int MT = P.M <= 16u ? 1 : P.M <= 32u ? 2 : 4; MT >= 1; MT /= 2) {
+  for (int MT = P.M <= 16u ? 1 : P.M <= 32u || parts == 3 ? 2 : 4; MT >= 1; MT /= 2) {
     const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
-    for (int NT = q.sample == kUnit || taps == 1 ? 4 : 2; NT >= 1; NT /= 2) {
-      const uint32_t slots = 64u * NT, pixels = pt_pixels(q.sample, taps, NT);
-      const double multiply = taps * (chunk / 32u) * std::max(16.0 * MT * NT, 32.0 * (MT + NT));
+    for (int NT = parts == 3 ? (q.sample == kUnit || taps == 1 ? 2 : 1) : q.sample == kUnit || taps == 1 ? 4 : 2; NT >= 1; NT /= 2) {
+      const uint32_t slots = 64u * NT, pixels = pt_pixels(q.sample, taps, NT, parts);
+      const double multiply = patch_multiply(taps, chunk, MT, NT);
       // what `blocks` blocks of patches of `staged` pixels cost: a chunk's staging is instructions per unit, and its way through the cache
       auto price = [&](uint64_t blocks, uint32_t staged) {
+        if (parts == 3) return f32_patch_us(q, taps, MT, NT, P.nchunks, blocks, staged);
         const double stage = 300.0 + 0.6 * staged + 4.0 * taps * MT;
         const double alone = 5000.0 + P.nchunks * (multiply + stage + 1000.0), both = 3000.0 + P.nchunks * std::max(2.0 * multiply + stage, multiply + stage + 1000.0);
         return (blocks <= 256u ? alone : std::max(alone, (double)((blocks + 511u) / 512u) * both)) + 1e-3 * (double)blocks;
@@ -480,7 +467,11 @@ static int patch_plan(const Conv3x3Problem &q, int taps, size_t workspace_bytes,
   P.div_pairs = FastDiv(pairs); P.div_pairs_img = FastDiv(P.image / per_pair); P.div_pairs_row = FastDiv(P.pitch / per_pair);
   P.div_in = FastDiv(P.in_step); P.div_out = FastDiv(P.out_step);
   const double full = std::min(1.0, blocks / 512.0), rounds = std::max(1.0, blocks / 512.0);
-  const double multiply = taps * (chunk / 32u) * std::max(16.0 * plan->MT * plan->NT, 32.0 * (plan->MT + plan->NT));
+  if (parts == 3) {
+    plan->us = best;
+    return ADH_OK;
+  }
+  const double multiply = patch_multiply(taps, chunk, plan->MT, plan->NT);
   plan->us = rounds * (4.1 + P.nchunks * (0.00032 * multiply * (1.0 + 5.3 * full) + 0.52 * plan->MT));
   plan->units = (uint64_t)((P.M + 63u) / 64u) * P.nchunks * 256u;
   const double ready_us = 2.1 + rounds * (5.4 + P.nchunks * 0.00096 * multiply * (1.0 + 1.06 * full));
@@ -517,26 +508,26 @@ static void launch_patch_mt(const PatchPlan &plan, hipStream_t st) {
 
 bool conv_bf16_patch_name(const Conv3x3Problem &q, int taps, size_t workspace_bytes, double most_us, char *name, size_t name_bytes) {
   PatchPlan plan = {};
-  if (patch_plan(q, taps, workspace_bytes, &plan) || plan.us > most_us) return false;
+  if (patch_plan(q, taps, 1, workspace_bytes, &plan) || plan.us > most_us) return false;
   snprintf(name, name_bytes, "conv_bf16_patch_kernel<%d, %d, %d, %d, %s>", plan.MT, plan.NT, (int)q.sample, taps, plan.ready ? "true" : "false");
   return true;
 }
 
 int conv_bf16_patch(const Conv3x3Problem &q, int taps, void *workspace, size_t workspace_bytes, double most_us, hipStream_t st) {
   PatchPlan plan = {};
-  const int e = patch_plan(q, taps, workspace ? workspace_bytes : 0u, &plan);
+  const int e = patch_plan(q, taps, 1, workspace ? workspace_bytes : 0u, &plan);
   if (e) return e;
   if (plan.us > most_us) return ADH_EUNIMPL;
   for (uint32_t t = 0; t < q.num_tiles; ++t) {
-    plan.P.in[t] = reinterpret_cast<const uint16_t *>(q.in[t]);
-    plan.P.out[t] = reinterpret_cast<uint16_t *>(q.out[t]);
+    plan.P.in[t] = q.in[t];
+    plan.P.out[t] = q.out[t];
   }
-  plan.P.w = reinterpret_cast<const uint16_t *>(q.w);
+  plan.P.w = q.w;
   if (plan.ready) {
-    hipLaunchKernelGGL(conv_bf16_patch_filter_kernel, dim3((uint32_t)((plan.units + kPtThreads - 1u) / kPtThreads)), dim3(kPtThreads), 0, st, plan.P.w,
+    hipLaunchKernelGGL(conv_bf16_patch_filter_kernel, dim3((uint32_t)((plan.units + kPtThreads - 1u) / kPtThreads)), dim3(kPtThreads), 0, st, reinterpret_cast<const uint16_t *>(q.w),
                        reinterpret_cast<uintx4 *>(workspace), plan.P.M, plan.P.C, plan.P.nchunks, plan.P.w_m_stride, plan.P.w_c_stride, plan.P.flip,
                        (uint32_t)plan.units);
-    plan.P.w = reinterpret_cast<const uint16_t *>(workspace);
+    plan.P.w = workspace;
   }
   if (taps == 9) {
     if (q.sample == kUnit) launch_patch_mt<kUnit, 9>(plan, st);
