@@ -36,13 +36,9 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t v) {
   return __uint_as_float(((uint32_t)v) << 16);
 }
 
-// round-to-nearest-even; NaN stays a quiet NaN
-__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) {
-  uint32_t u = __float_as_uint(f);
-  if ((u & 0x7fffffffu) > 0x7f800000u) return (uint16_t)((u >> 16) | 0x0040u);
-  u += 0x7fffu + ((u >> 16) & 1u);
-  return (uint16_t)(u >> 16);
-}
+// round-to-nearest-even; NaN stays a quiet NaN (one instruction; for all 2^32 floats the bits of adding 0x7fff and the last bit and
+// shifting, which takes seven)
+__device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
 // A thread's vector (16 bytes, or one element) at element alignment.  STREAM: non-temporal, for data that the on-package
 // cache would not keep anyway.  Reads of 537 MB reach 6.9 to 7.1 TB/s that way against 5.7 to 6.4, whatever the order and the
