@@ -29,6 +29,7 @@ __global__ __launch_bounds__(256) void wgrad_sums_kernel(const WgradSums P) {
   const uint32_t group = quad / kQuads, e = quad - group * kQuads;
   const floatx4 *p = reinterpret_cast<const floatx4 *>(P.part) + (size_t)group * P.splits * kQuads + e;
   doublex4 sum = {0.0, 0.0, 0.0, 0.0};
+#pragma unroll 4  // (eight, the compiler's choice: 16 -> 17 channels on 7 tiles of 24 x 440, 8 images, 46 us with the sums' kernel, 36 with four)
   for (uint32_t k = slice; k < P.splits; k += 16u) sum += __builtin_convertvector(*reinterpret_cast<const floatx4 *>(p + (size_t)k * kQuads), doublex4);
   sums[slice][threadIdx.x & 15u] = sum;
   __syncthreads();
