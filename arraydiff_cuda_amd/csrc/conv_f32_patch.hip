@@ -400,7 +400,7 @@ bool conv_f32_patch_ahead(const Conv3x3Problem &q, bool workspace) {
   if (patch_plan(q, 9, 3, 0u, &plan)) return false;
   const double split = conv3x3_split_us(q, workspace);
   if (q.sample == kDown) return 1.2 * plan.us - 1.3 < 2.0 + 1.23 * split;
-  if (q.sample == kUp) return 1.07 * plan.us < 0.7 + 1.1 * split;
+  if (q.sample == kUp) return 1.13 * plan.us < 0.7 + 1.1 * split;  // (1.07 as fitted; 512 -> 512 channels on 4 x 16 tiles lost 4 % by it)
   return plan.us < 3.5 + 1.09 * split;
 }
 
