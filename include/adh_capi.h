@@ -537,7 +537,7 @@ int adh_stat_step_f32(uint64_t n, float rate, const float *avg_stat, float *runn
 /* Op::store_val / store_grad (src/op.cc:170-194) and Op::load_val (src/op.cc:148-158) for one flat
  * vector: the arrays, in the order given, occupy consecutive ranges of `flat` starting at element
  * flat_offset (array i of lens[i] floats; a zero length is skipped).  store copies arrays -> flat,
- * load copies flat -> arrays.  One launch per 48 arrays instead of one copy per array. */
+ * load copies flat -> arrays.  One launch per 64 arrays instead of one copy per array. */
 int adh_flat_store_f32(uint32_t num_arrays, const float *const *arrays, const uint64_t *lens, uint64_t flat_offset,
                        float *flat, void *stream);
 int adh_flat_load_f32(uint32_t num_arrays, float *const *arrays, const uint64_t *lens, uint64_t flat_offset,
