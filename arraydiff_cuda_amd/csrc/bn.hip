@@ -464,7 +464,7 @@ static dim3 bn_apply_grid(BnParams *P, uint32_t groups_per_plane, bool backward)
     while ((1u << P->slots_log2) < groups_per_plane) ++P->slots_log2;
   }
   const uint32_t planes = P->tiles * P->N * P->C, along = 4u * kBnThreads;
-  P->along = backward && groups_per_plane >= along;
+  P->along = backward && groups_per_plane >= along && planes < (1u << 24);  // (a launch has less than 2^32 threads)
   if (P->along) return dim3(planes, (groups_per_plane + along - 1u) / along);
   const uint32_t per_block = 4u * (kBnThreads >> P->slots_log2);
   return dim3((planes + per_block - 1u) / per_block, (groups_per_plane + kBnThreads - 1u) / kBnThreads);

@@ -81,3 +81,23 @@ def test_splits(K, N, C):
 @pytest.mark.parametrize("dtype,W", [(torch.float32, 1100), (torch.float32, 1099), (torch.bfloat16, 2200), (torch.bfloat16, 2199)])
 def test_larger_than_the_cache(dtype, W):
     _run(dtype, 2, 2, 33, 512, W)
+
+
+def test_more_planes_than_workgroups_of_a_launch():
+    """2^24 planes of more than 1024 groups (16 tiles that share their memory): a workgroup per plane would be 2^32 threads."""
+    K, N, C, H, W = capi.ADH_MAX_TILES, 1024, 1024, 94, 11
+    g = torch.Generator(device="cuda").manual_seed(2)
+    x = torch.randn((N, C, H, W), device="cuda", generator=g, dtype=torch.bfloat16)
+    dy = torch.randn((N, C, H + 2, W + 2), device="cuda", generator=g, dtype=torch.bfloat16)
+    dx = torch.full((N, C, H, W), 7.0, device="cuda", dtype=torch.bfloat16)
+    scale, mean, invstd = torch.rand(C, device="cuda", generator=g) + 0.5, torch.randn(C, device="cuda", generator=g) * 0.1, torch.rand(C, device="cuda", generator=g) + 0.5
+    dscale, dshift = torch.empty(C, device="cuda"), torch.empty(C, device="cuda")
+    ws = torch.empty(capi.batchnorm_workspace_bytes(K, N, C) // 4, device="cuda")
+    capi.check(capi.batchnorm_bwd_tiles([x] * K, [dy] * K, [scale] * K, [scale] * K, [mean] * K, [invstd] * K, [dx] * K, [dscale] * K, [dshift] * K, N, C, H, W,
+                                        dy_halo=1, ws=ws))
+    for c in (0, 1, 700, C - 1):
+        xc, d = x[:, c].double() - mean[c].double(), dy[:, c, 1:-1, 1:-1].double()
+        i, m = invstd[c].double(), N * H * W
+        want = scale[c].double() * i * (d - d.sum() / m - xc * i * (d * xc * i).sum() / m)
+        # rounded to bf16, and sums of a million fp32 terms behind the small corrections
+        assert ((dx[:, c].double() - want).abs() <= 2.0 ** -8 * want.abs() + 1e-5).all()
