@@ -40,28 +40,32 @@ __device__ __forceinline__ float bf16_bits_to_f32(uint16_t v) {
 // shifting, which takes seven)
 __device__ __forceinline__ uint16_t f32_to_bf16_bits(float f) { return __builtin_bit_cast(uint16_t, (__bf16)f); }
 
-// A thread's vector (16 bytes, or one element) at element alignment.  STREAM: non-temporal, for data that the on-package
-// cache would not keep anyway.  Reads of 537 MB reach 6.9 to 7.1 TB/s that way against 5.7 to 6.4, whatever the order and the
-// loads in flight.
+// A thread's vector (16 bytes, or less at its type's own alignment) at element alignment.  STREAM: non-temporal, for data that the
+// on-package cache would not keep anyway.  Reads of 537 MB reach 6.9 to 7.1 TB/s that way against 5.7 to 6.4, whatever the order and
+// the loads in flight.
+typedef uint32_t Raw16 __attribute__((ext_vector_type(4), aligned(2)));
 template <bool STREAM, typename V, typename T>
 __device__ __forceinline__ V load_vec(const T *p) {
-  typedef uint32_t Raw __attribute__((ext_vector_type(4), aligned(2)));
-  V v;
-  if constexpr (STREAM && sizeof(V) == 16) {
-    const Raw r = __builtin_nontemporal_load(reinterpret_cast<const Raw *>(p));
+  if constexpr (sizeof(V) == 16) {
+    const Raw16 *q = reinterpret_cast<const Raw16 *>(p);
+    Raw16 r;
+    if constexpr (STREAM) r = __builtin_nontemporal_load(q);
+    else r = *q;
+    V v;
     __builtin_memcpy(&v, &r, 16);
+    return v;
   } else {
-    v = *reinterpret_cast<const V *>(p);
+    return *reinterpret_cast<const V *>(p);
   }
-  return v;
 }
 template <bool STREAM, typename V, typename T>
 __device__ __forceinline__ void store_vec(T *p, const V &v) {
-  typedef uint32_t Raw __attribute__((ext_vector_type(4), aligned(2)));
-  if constexpr (STREAM && sizeof(V) == 16) {
-    Raw r;
+  if constexpr (sizeof(V) == 16) {
+    Raw16 *q = reinterpret_cast<Raw16 *>(p);
+    Raw16 r;
     __builtin_memcpy(&r, &v, 16);
-    __builtin_nontemporal_store(r, reinterpret_cast<Raw *>(p));
+    if constexpr (STREAM) __builtin_nontemporal_store(r, q);
+    else *q = r;
   } else {
     *reinterpret_cast<V *>(p) = v;
   }
