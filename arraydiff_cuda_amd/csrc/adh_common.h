@@ -15,8 +15,7 @@ struct FastDiv {
   uint32_t d, mul, shift;
   FastDiv() : d(1), mul(1), shift(0) {}
   explicit FastDiv(uint32_t div) : d(div ? div : 1) {
-    shift = 0;
-    while ((1ull << shift) < d) ++shift;
+    shift = d > 1u ? 32u - (uint32_t)__builtin_clz(d - 1u) : 0u;
     mul = (uint32_t)(((1ull << 32) * ((1ull << shift) - d)) / d + 1);
   }
   __host__ __device__ __forceinline__ uint32_t div(uint32_t n) const {

@@ -1319,19 +1319,21 @@ int conv2d_fwd(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_FWD, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = x_tiles; q.out = y_tiles; q.w = w;
-    if (conv_f32_patch_ahead(q, workspace != nullptr)) {
-      e = conv_f32_patch(q, 9, as_stream(stream));
-      if (e != ADH_EUNIMPL) return e;
+    PatchPlan patch = {};
+    const double beyond = conv_f32_patch_beyond(q, &patch);
+    if (g.sh == 2u) {
+      if (beyond < 1e300 && conv3x3_split_exceeds(q, workspace != nullptr, beyond)) return conv_f32_patch(q, 9, patch, as_stream(stream));
+      // The two kernels stand as 0.85 - 0.91 to 1 in time where the split one's rounds are full, from 64 to 1024 channels on either
+      // side; its blocks are coarse, and with more than an eighth of the rounds idle the fp32 one is ahead (of full rounds:
+      // 9/16 1.08 - 1.13, 3/4 1.08 - 1.15, 5/6 1.06, 9/10 0.97 - 1.0).  A single round is the split one's: 0.15 - 0.85 with chunks
+      // dealt out.
+      if (conv3x3_split_idles(q)) {
+        e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
+        if (e != ADH_EUNIMPL) return e;
+      }
     }
-    // Stride 2: the two kernels stand as 0.85 - 0.91 to 1 in time where the split one's rounds are full, from 64 to 1024 channels
-    // on either side; its blocks are coarse, and with more than an eighth of the rounds idle the fp32 one is ahead (of full
-    // rounds: 9/16 1.08 - 1.13, 3/4 1.08 - 1.15, 5/6 1.06, 9/10 0.97 - 1.0).  A single round is the split one's: 0.15 - 0.85 with
-    // chunks dealt out.
-    if (g.sh == 2u && conv3x3_split_idles(q)) {
-      e = conv3x3s2_fwd_try(num_tiles, N, Cin, Cout, g.HP - 2u, g.WP - 2u, x_tiles, w, y_tiles, beta, as_stream(stream));
-      if (e != ADH_EUNIMPL) return e;
-    }
-    e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
+    e = conv3x3_split(q, workspace, workspace_bytes, g.sh == 2u ? 1e300 : beyond, as_stream(stream));
+    if (e == ADH_EUNIMPL && g.sh != 2u && beyond < 1e300) e = conv_f32_patch(q, 9, patch, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   if (const int taps = dtype != ADH_BF16 ? 0 : gen_patch_taps(ADH_CONV_FWD, g, unpadded, pad_h, pad_w)) {
@@ -1391,11 +1393,10 @@ int conv2d_bwd_data(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, uin
     Conv3x3Problem q = gen_3x3_problem(ADH_CONV_BWD_DATA, g, num_tiles, unpadded, pad_h, pad_w);
     q.beta = beta;
     q.in = dy_tiles; q.out = dx_tiles; q.w = w;
-    if (conv_f32_patch_ahead(q, workspace != nullptr)) {
-      e = conv_f32_patch(q, 9, as_stream(stream));
-      if (e != ADH_EUNIMPL) return e;
-    }
-    e = conv3x3_split(q, workspace, workspace_bytes, as_stream(stream));
+    PatchPlan patch = {};
+    const double beyond = conv_f32_patch_beyond(q, &patch);
+    e = conv3x3_split(q, workspace, workspace_bytes, beyond, as_stream(stream));
+    if (e == ADH_EUNIMPL && beyond < 1e300) e = conv_f32_patch(q, 9, patch, as_stream(stream));
     if (e != ADH_EUNIMPL) return e;
   }
   if (const int taps = dtype != ADH_BF16 ? 0 : gen_patch_taps(ADH_CONV_BWD_DATA, g, unpadded, pad_h, pad_w)) {

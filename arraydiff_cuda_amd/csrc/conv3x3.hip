@@ -66,11 +66,17 @@ static int conv_direct(int which, int dtype, uint32_t num_tiles, uint32_t N, uin
   q.beta = res_tiles ? 1.f : beta;
   q.in = in_tiles; q.out = out_tiles; q.res = res_tiles; q.w = w;
   // (of the plain form, for all forms of a layer: their sums have the same bits)
-  if (conv_f32_patch_ahead(conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, unpadded), false)) {
+  PatchPlan patch = {};
+  if (rows_from_neighbours) {
+    const Conv3x3Problem plain = conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, unpadded);
+    const double beyond = conv_f32_patch_beyond(plain, &patch);
+    if (beyond == 1e300 || !conv3x3_split_exceeds(plain, false, beyond)) return conv3x3_split(q, nullptr, 0, 1e300, st);
     const int e = conv_f32_patch(q, 9, st);
-    if (e != ADH_EUNIMPL) return e;
+    return e == ADH_EUNIMPL ? conv3x3_split(q, nullptr, 0, 1e300, st) : e;
   }
-  return conv3x3_split(q, nullptr, 0, st);
+  const double beyond = conv_f32_patch_beyond(q, &patch);
+  const int e = conv3x3_split(q, nullptr, 0, beyond, st);
+  return e == ADH_EUNIMPL && beyond < 1e300 ? conv_f32_patch(q, 9, patch, st) : e;
 }
 
 // the patches' kernel name, where they serve the call
@@ -98,7 +104,10 @@ int adh_conv3x3_kernel_name(int which, int dtype, uint32_t num_tiles, uint32_t N
   }
   if (dtype != ADH_F32) return ADH_EINVAL;
   const Conv3x3Problem q = conv3x3_problem(which, num_tiles, N, Cin, Cout, H, W, false, false);
-  if (!conv_f32_patch_ahead(q, false) || !conv_f32_patch_name(q, 9, name, name_bytes)) conv3x3_split_name(q, name, name_bytes);
+  PatchPlan patch = {};
+  const double beyond = conv_f32_patch_beyond(q, &patch);
+  if (beyond < 1e300 && conv3x3_split_exceeds(q, false, beyond)) conv_f32_patch_name(q, 9, patch, name, name_bytes);
+  else conv3x3_split_name(q, name, name_bytes);
   return ADH_OK;
 }
 

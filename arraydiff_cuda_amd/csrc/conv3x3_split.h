@@ -35,10 +35,11 @@ Conv3x3Problem conv3x3_problem(int which, uint32_t num_tiles, uint32_t N, uint32
 
 // fp32 sums of channel chunks that are dealt to several workgroups (0: none are)
 size_t conv3x3_split_workspace(const Conv3x3Problem &q);
-// The workspace may be null: then no chunks are dealt out.
-int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st);
-// expected time (1e300: a shape it does not take)
-double conv3x3_split_us(const Conv3x3Problem &q, bool workspace);
+// The workspace may be null: then no chunks are dealt out.  ADH_EUNIMPL: nothing launched, as it is expected to take more than
+// most_us, or as the shape is none that it takes.
+int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, double most_us, hipStream_t st);
+// whether it is expected to take more than most_us (or does not take the shape)
+bool conv3x3_split_exceeds(const Conv3x3Problem &q, bool workspace, double most_us);
 // more than one round of workgroups, and more than an eighth of all rounds idle
 bool conv3x3_split_idles(const Conv3x3Problem &q);
 void conv3x3_split_name(const Conv3x3Problem &q, char *name, size_t name_bytes);

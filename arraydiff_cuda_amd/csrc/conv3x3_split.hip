@@ -598,6 +598,10 @@ struct SplitPlan {
 // The choice is made anew on every call, so tiles that cannot win are passed over by their least number of blocks before they are
 // priced: 64 channels on 4 x 32 x 128 5.8 -> 1.2 us of host time, on 8 x 128 x 2048 10.8 -> 1.6, the median of random shapes
 // 3.9 -> 1.5, with the same choices.
+static double split_chunk_cycles(int MT, int NT) { return 9.0 * (std::max(192.0 * MT * NT, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT; }
+static double split_results_cycles(SplitSample sample, int MT, int NT) { return 2000.0 + 500.0 * MT * NT * (sample == kUp ? 4 : 1); }
+constexpr double kSplitDealtCycles = 9000.0;  // the second kernel's launch
+
 static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) {
   SplitParams &P = plan->P;
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
@@ -634,14 +638,12 @@ static int split_plan(const Conv3x3Problem &q, bool workspace, SplitPlan *plan) 
       // (what the registers hold of two sets of sums: at stride 1 the largest such tile of each height)
       if (plan->low == kLowApart && (q.sample == kUnit ? NT != (MT == 1 ? 4 : 2) : q.sample == kUp && NT > 1 && MT * NT > 2)) continue;
       const uint32_t slots = 128u * NT;
-      const double matrix = 192.0 * MT * NT;
-      const double chunk = 9.0 * (std::max(matrix, 1300.0) + 300.0) + 1500.0 + 2000.0 * NT;
-      const double results = 2000.0 + 500.0 * MT * NT * (q.sample == kUp ? 4 : 1);
+      const double chunk = split_chunk_cycles(MT, NT), results = split_results_cycles(q.sample, MT, NT);
       // What `blocks` blocks cost, their chunks undealt or (where they leave compute units idle) as dealt at best.  It grows with
       // their number, so that tiles whose least possible number costs more than the best plan so far are passed over.
       auto undealt = [&](uint64_t blocks) { return (double)((blocks + 255u) / 256u) * (P.nchunks * chunk + results) + 1e-3 * (double)blocks; };
       auto dealt = [&](uint64_t blocks, uint32_t cps, uint32_t ks) {
-        return cps * chunk + results + 9000.0 + out_bytes * (ks + 1) / 1200.0 + 1e-3 * (double)blocks;
+        return cps * chunk + results + kSplitDealtCycles + out_bytes * (ks + 1) / 1200.0 + 1e-3 * (double)blocks;
       };
       auto worse = [&](uint64_t least) {
         if (undealt(least) < best) return false;
@@ -709,9 +711,19 @@ size_t conv3x3_split_workspace(const Conv3x3Problem &q) {
   return split_plan(q, true, &plan) ? 0u : (plan.part_bytes + 255u) & ~(size_t)255u;
 }
 
-double conv3x3_split_us(const Conv3x3Problem &q, bool workspace) {
+constexpr double kSplitCyclesPerUs = 2100.0;
+// No plan is expected to take less than a block of the smallest tile, of all chunks or (with a workspace) of one of them: what tells
+// small launches, which go to conv_f32_patch.hip, without a plan.
+static double split_least_us(const Conv3x3Problem &q, bool workspace) {
+  const uint32_t nchunks = (q.C + kSpChunk - 1u) / kSpChunk;
+  const double chunk = split_chunk_cycles(1, 1), results = split_results_cycles(q.sample, 1, 1), whole = nchunks * chunk + results;
+  return (workspace ? std::min(whole, chunk + results + kSplitDealtCycles) : whole) / kSplitCyclesPerUs;
+}
+
+bool conv3x3_split_exceeds(const Conv3x3Problem &q, bool workspace, double most_us) {
+  if (split_least_us(q, workspace) > most_us) return true;
   SplitPlan plan = {};
-  return split_plan(q, workspace, &plan) ? 1e300 : plan.cycles / 2100.0;
+  return split_plan(q, workspace, &plan) || plan.cycles / kSplitCyclesPerUs > most_us;
 }
 
 bool conv3x3_split_idles(const Conv3x3Problem &q) {
@@ -753,9 +765,11 @@ static void launch_split_nt(const SplitPlan &plan, SplitSample sample, hipStream
   }
 }
 
-int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, hipStream_t st) {
+int conv3x3_split(const Conv3x3Problem &q, void *workspace, size_t workspace_bytes, double most_us, hipStream_t st) {
+  if (split_least_us(q, workspace != nullptr) > most_us) return ADH_EUNIMPL;
   SplitPlan plan = {};
   int e = split_plan(q, workspace != nullptr, &plan);
+  if (e == ADH_OK && plan.cycles / kSplitCyclesPerUs > most_us) return ADH_EUNIMPL;
   if (e == ADH_OK && plan.part_bytes > workspace_bytes) {
     plan = {};
     e = split_plan(q, false, &plan);

@@ -390,6 +390,25 @@ static double f32_patch_us(const Conv3x3Problem &q, int taps, int MT, int NT, ui
 static double patch_multiply(int taps, uint32_t chunk, int MT, int NT) {
   return taps * (chunk / 32u) * std::max(16.0 * MT * NT, 32.0 * (MT + NT));
 }
+// bf16: as fitted (see patch_plan); ready: the filter put in order first
+static double bf16_patch_us(int taps, int MT, int NT, uint32_t chunks, uint64_t blocks, bool ready) {
+  const double full = std::min(1.0, blocks / 512.0), rounds = std::max(1.0, blocks / 512.0), multiply = patch_multiply(taps, taps == 1 ? 64u : 32u, MT, NT);
+  return ready ? 2.1 + rounds * (5.4 + chunks * 0.00096 * multiply * (1.0 + 1.06 * full))
+               : rounds * (4.1 + chunks * (0.00032 * multiply * (1.0 + 5.3 * full) + 0.52 * MT));
+}
+// 3x3 at stride 1: whether no tile can be expected to take less than most_us, by its least number of blocks.  Tells large launches,
+// which are the strips', without a plan.
+static bool bf16_patch_exceeds(const Conv3x3Problem &q, double most_us) {
+  if (most_us >= 1e30 || q.sample != kUnit) return false;
+  const uint64_t pixels = (uint64_t)q.num_tiles * q.N * (q.stacked ? q.step : q.out_H) * q.out_W;
+  const uint32_t chunks = (q.C + 31u) / 32u;
+  for (int MT = q.M <= 16u ? 1 : q.M <= 32u ? 2 : 4; MT >= 1; MT /= 2)
+    for (int NT = 4; NT >= 1; NT /= 2) {
+      const uint64_t blocks = (pixels + 64u * NT - 1u) / (64u * NT) * ((q.M + 16u * MT - 1u) / (16u * MT));
+      if (bf16_patch_us(9, MT, NT, chunks, blocks, false) <= most_us || bf16_patch_us(9, MT, NT, chunks, blocks, true) <= most_us) return false;
+    }
+  return true;
+}
 
 // Blocks of BR x BC output pixels (of NB images) by 16 MT channels, two workgroups per compute unit.  The tile is chosen by a model of
 // a block's cycles: a chunk's multiplications (or their operands' way out of LDS), its staging, and a load's latency.
@@ -428,43 +447,50 @@ int patch_plan(const Conv3x3Problem &q, int taps, int parts, size_t workspace_by
   double best = 1e300;
   uint32_t nbi = 0, nbj = 0;
   const uint64_t grid_pixels = (uint64_t)P.NI * P.grid_VH * P.grid_W;
-  for (int MT = P.M <= 16u ? 1 : P.M <= 32u || parts == 3 ? 2 : 4; MT >= 1; MT /= 2) {
-    const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT);
+  // what `blocks` blocks of patches of `staged` pixels cost: a chunk's staging is instructions per unit, and its way through the cache
+  auto price = [&](int MT, int NT, uint64_t blocks, uint32_t staged) {
+    if (parts == 3) return f32_patch_us(q, taps, MT, NT, P.nchunks, blocks, staged);
+    const double multiply = patch_multiply(taps, chunk, MT, NT), stage = 300.0 + 0.6 * staged + 4.0 * taps * MT;
+    const double alone = 5000.0 + P.nchunks * (multiply + stage + 1000.0), both = 3000.0 + P.nchunks * std::max(2.0 * multiply + stage, multiply + stage + 1000.0);
+    return (blocks <= 256u ? alone : std::max(alone, (double)((blocks + 511u) / 512u) * both)) + 1e-3 * (double)blocks;
+  };
+  // The tiles by what they cost with their least number of blocks, so that most are passed over (the plan is made anew on every call:
+  // 16 -> 16 channels on 2 tiles of 4 x 2000 1.2 -> 0.5 us of host time, with the same choices).
+  struct Tile { double least; int MT, NT; } tiles[9];
+  int num_tiles = 0;
+  for (int MT = P.M <= 16u ? 1 : P.M <= 32u || parts == 3 ? 2 : 4; MT >= 1; MT /= 2)
     for (int NT = parts == 3 ? (q.sample == kUnit || taps == 1 ? 2 : 1) : q.sample == kUnit || taps == 1 ? 4 : 2; NT >= 1; NT /= 2) {
-      const uint32_t slots = 64u * NT, pixels = pt_pixels(q.sample, taps, NT, parts);
-      const double multiply = patch_multiply(taps, chunk, MT, NT);
-      // what `blocks` blocks of patches of `staged` pixels cost: a chunk's staging is instructions per unit, and its way through the cache
-      auto price = [&](uint64_t blocks, uint32_t staged) {
-        if (parts == 3) return f32_patch_us(q, taps, MT, NT, P.nchunks, blocks, staged);
-        const double stage = 300.0 + 0.6 * staged + 4.0 * taps * MT;
-        const double alone = 5000.0 + P.nchunks * (multiply + stage + 1000.0), both = 3000.0 + P.nchunks * std::max(2.0 * multiply + stage, multiply + stage + 1000.0);
-        return (blocks <= 256u ? alone : std::max(alone, (double)((blocks + 511u) / 512u) * both)) + 1e-3 * (double)blocks;
-      };
-      // (tiles that cannot win by their least number of blocks are passed over)
-      if (price((grid_pixels + slots - 1u) / slots * MG, (uint32_t)std::min<uint64_t>(slots, grid_pixels)) >= best) continue;
-      uint32_t last_BC = 0;
-      for (uint32_t parts = (P.grid_W + slots - 1u) / slots; parts <= P.grid_W; parts += 1u + parts / 4u) {
-        const uint32_t BC = ((P.grid_W + parts - 1u) / parts + 3u) & ~3u;
-        if (parts > 1u && BC < 8u) break;
-        const uint32_t pitch = pairs_of(BC) * per_pair;
-        if (BC > slots || BC == last_BC || rows_of(1u) * pitch > pixels) continue;
-        last_BC = BC;
-        // (rows_of is linear)
-        const uint32_t held = pixels / pitch, one = rows_of(1u), more = rows_of(2u) - one;
-        const uint32_t max_BR = std::min(std::min(P.grid_VH, slots / BC), 1u + (held - one) / more);
-        const uint32_t nc = (P.grid_W + BC - 1u) / BC, nr = (P.grid_VH + max_BR - 1u) / max_BR, BR = (P.grid_VH + nr - 1u) / nr;
-        const uint32_t image = rows_of(BR) * pitch;
-        uint32_t NB = std::min(std::min(slots / (BR * BC), pixels / image), P.NI);
-        const uint32_t groups = (P.NI + NB - 1u) / NB;
-        NB = (P.NI + groups - 1u) / groups;
-        const uint64_t blocks = (uint64_t)groups * nc * nr * MG;
-        const double cost = price(blocks, NB * image);
-        if (cost >= best) continue;
-        best = cost;
-        plan->MT = MT; plan->NT = NT;
-        P.BR = BR; P.BC = BC; P.NB = NB; P.pitch = pitch; P.image = image;
-        nbi = nr; nbj = nc;
-      }
+      const uint32_t slots = 64u * NT;
+      const Tile tile = {price(MT, NT, (grid_pixels + slots - 1u) / slots * ((P.M + 16u * MT - 1u) / (16u * MT)), (uint32_t)std::min<uint64_t>(slots, grid_pixels)), MT, NT};
+      int k = num_tiles++;
+      for (; k > 0 && tiles[k - 1].least > tile.least; --k) tiles[k] = tiles[k - 1];
+      tiles[k] = tile;
+    }
+  for (int k = 0; k < num_tiles && tiles[k].least < best; ++k) {
+    const int MT = tiles[k].MT, NT = tiles[k].NT;
+    const uint32_t MG = (P.M + 16u * MT - 1u) / (16u * MT), slots = 64u * NT, pixels = pt_pixels(q.sample, taps, NT, parts);
+    uint32_t last_BC = 0;
+    for (uint32_t cuts = (P.grid_W + slots - 1u) / slots; cuts <= P.grid_W; cuts += 1u + cuts / 4u) {
+      const uint32_t BC = ((P.grid_W + cuts - 1u) / cuts + 3u) & ~3u;
+      if (cuts > 1u && BC < 8u) break;
+      const uint32_t pitch = pairs_of(BC) * per_pair;
+      if (BC > slots || BC == last_BC || rows_of(1u) * pitch > pixels) continue;
+      last_BC = BC;
+      // (rows_of is linear)
+      const uint32_t held = pixels / pitch, one = rows_of(1u), more = rows_of(2u) - one;
+      const uint32_t max_BR = std::min(std::min(P.grid_VH, slots / BC), 1u + (held - one) / more);
+      const uint32_t nc = (P.grid_W + BC - 1u) / BC, nr = (P.grid_VH + max_BR - 1u) / max_BR, BR = (P.grid_VH + nr - 1u) / nr;
+      const uint32_t image = rows_of(BR) * pitch;
+      uint32_t NB = std::min(std::min(slots / (BR * BC), pixels / image), P.NI);
+      const uint32_t groups = (P.NI + NB - 1u) / NB;
+      NB = (P.NI + groups - 1u) / groups;
+      const uint64_t blocks = (uint64_t)groups * nc * nr * MG;
+      const double cost = price(MT, NT, blocks, NB * image);
+      if (cost >= best) continue;
+      best = cost;
+      plan->MT = MT; plan->NT = NT;
+      P.BR = BR; P.BC = BC; P.NB = NB; P.pitch = pitch; P.image = image;
+      nbi = nr; nbj = nc;
     }
   }
   if (nbi == 0u) return ADH_EUNIMPL;
@@ -477,15 +503,13 @@ int patch_plan(const Conv3x3Problem &q, int taps, int parts, size_t workspace_by
   P.div_BC = FastDiv(P.BC); P.div_live = FastDiv(P.BR * P.BC);
   P.div_pairs = FastDiv(pairs); P.div_pairs_img = FastDiv(P.image / per_pair); P.div_pairs_row = FastDiv(P.pitch / per_pair);
   P.div_in = FastDiv(P.in_step); P.div_out = FastDiv(P.out_step);
-  const double full = std::min(1.0, blocks / 512.0), rounds = std::max(1.0, blocks / 512.0);
   if (parts == 3) {
     plan->us = best;
     return ADH_OK;
   }
-  const double multiply = patch_multiply(taps, chunk, plan->MT, plan->NT);
-  plan->us = rounds * (4.1 + P.nchunks * (0.00032 * multiply * (1.0 + 5.3 * full) + 0.52 * plan->MT));
+  plan->us = bf16_patch_us(taps, plan->MT, plan->NT, P.nchunks, blocks, false);
   plan->units = (uint64_t)((P.M + 63u) / 64u) * P.nchunks * 256u;
-  const double ready_us = 2.1 + rounds * (5.4 + P.nchunks * 0.00096 * multiply * (1.0 + 1.06 * full));
+  const double ready_us = bf16_patch_us(taps, plan->MT, plan->NT, P.nchunks, blocks, true);
   plan->ready = taps == 9 && ready_us < plan->us && plan->units * 144u <= workspace_bytes && plan->units < (1ull << 31);
   if (plan->ready) plan->us = ready_us;
   return ADH_OK;
@@ -519,12 +543,13 @@ static void launch_patch_mt(const PatchPlan &plan, hipStream_t st) {
 
 bool conv_bf16_patch_name(const Conv3x3Problem &q, int taps, size_t workspace_bytes, double most_us, char *name, size_t name_bytes) {
   PatchPlan plan = {};
-  if (patch_plan(q, taps, 1, workspace_bytes, &plan) || plan.us > most_us) return false;
+  if (bf16_patch_exceeds(q, most_us) || patch_plan(q, taps, 1, workspace_bytes, &plan) || plan.us > most_us) return false;
   snprintf(name, name_bytes, "conv_bf16_patch_kernel<%d, %d, %d, %d, %s>", plan.MT, plan.NT, (int)q.sample, taps, plan.ready ? "true" : "false");
   return true;
 }
 
 int conv_bf16_patch(const Conv3x3Problem &q, int taps, void *workspace, size_t workspace_bytes, double most_us, hipStream_t st) {
+  if (bf16_patch_exceeds(q, most_us)) return ADH_EUNIMPL;
   PatchPlan plan = {};
   const int e = patch_plan(q, taps, 1, workspace ? workspace_bytes : 0u, &plan);
   if (e) return e;

@@ -3,16 +3,18 @@
 #ifndef ADH_CONV_F32_PATCH_H
 #define ADH_CONV_F32_PATCH_H
 
-#include "conv3x3_split.h"
+#include "conv_patch_plan.h"
 
 namespace adh {
 
 // taps: 9, or 1 for a 1x1 window (padding 0, at kDown and kUp the even rows and columns).
-// Whether the 3x3 window is expected to be faster here than in conv3x3_split.hip (workspace: with one).
-bool conv_f32_patch_ahead(const Conv3x3Problem &q, bool workspace);
+// The expected time of conv3x3_split.hip beyond which the 3x3 window is expected to be faster here, and the plan for that
+// (1e300: it never is, and there is none).
+double conv_f32_patch_beyond(const Conv3x3Problem &q, PatchPlan *plan);
+int conv_f32_patch(const Conv3x3Problem &q, int taps, const PatchPlan &plan, hipStream_t st);
 // ADH_EUNIMPL: nothing launched, rows of fewer than two elements
 int conv_f32_patch(const Conv3x3Problem &q, int taps, hipStream_t st);
-bool conv_f32_patch_name(const Conv3x3Problem &q, int taps, char *name, size_t name_bytes);
+void conv_f32_patch_name(const Conv3x3Problem &q, int taps, const PatchPlan &plan, char *name, size_t name_bytes);
 
 }  // namespace adh
 #endif

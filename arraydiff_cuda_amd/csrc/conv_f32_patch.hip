@@ -22,7 +22,6 @@
 
 #include <algorithm>
 
-#include "conv_patch_plan.h"
 #include "split_bf16.h"
 
 namespace adh {
@@ -393,28 +392,26 @@ static void launch_f32_patch_mt(const PatchPlan &plan, const F32PatchParams &P, 
 // 3 times at the smallest, where the other kernel's nine barriers a chunk and its filter tap by tap stand in a row (480 -> 160
 // channels on 9 x 15, forward 108 -> 38 us); persistent workgroups of twice the waves where blocks are many.
 // (Beyond four rounds of the smallest blocks they are 0.5 to 1.1 times as fast and not priced: the choice is made on every call.)
-bool conv_f32_patch_ahead(const Conv3x3Problem &q, bool workspace) {
+// Host time: planned once a call and the other kernel not where its least time says enough: 16 -> 16 channels on 2 tiles of 4 x 2000 2.7 -> 0.5 us.
+double conv_f32_patch_beyond(const Conv3x3Problem &q, PatchPlan *plan) {
   const uint64_t pixels = (uint64_t)q.num_tiles * q.N * (q.sample == kUp ? (uint64_t)q.in_H * q.in_W : (uint64_t)q.out_H * q.out_W);
-  if (pixels * q.M > 2048ull * 64u * 16u) return false;
-  PatchPlan plan = {};
-  if (patch_plan(q, 9, 3, 0u, &plan)) return false;
-  const double split = conv3x3_split_us(q, workspace);
-  if (q.sample == kDown) return 1.2 * plan.us - 1.3 < 2.0 + 1.23 * split;
-  if (q.sample == kUp) return 1.13 * plan.us < 0.7 + 1.1 * split;  // (1.07 as fitted; 512 -> 512 channels on 4 x 16 tiles lost 4 % by it)
-  return plan.us < 3.5 + 1.09 * split;
+  if (pixels * q.M > 2048ull * 64u * 16u || patch_plan(q, 9, 3, 0u, plan)) return 1e300;
+  if (q.sample == kDown) return (1.2 * plan->us - 3.3) / 1.23;
+  if (q.sample == kUp) return (1.13 * plan->us - 0.7) / 1.1;  // (1.07 as fitted; 512 -> 512 channels on 4 x 16 tiles lost 4 % by it)
+  return (plan->us - 3.5) / 1.09;
 }
 
-bool conv_f32_patch_name(const Conv3x3Problem &q, int taps, char *name, size_t name_bytes) {
-  PatchPlan plan = {};
-  if (patch_plan(q, taps, 3, 0u, &plan)) return false;
+void conv_f32_patch_name(const Conv3x3Problem &q, int taps, const PatchPlan &plan, char *name, size_t name_bytes) {
   snprintf(name, name_bytes, "conv_f32_patch_kernel<%d, %d, %d, %d>", plan.MT, plan.NT, (int)q.sample, taps);
-  return true;
 }
 
 int conv_f32_patch(const Conv3x3Problem &q, int taps, hipStream_t st) {
   PatchPlan plan = {};
   const int e = patch_plan(q, taps, 3, 0u, &plan);
-  if (e) return e;
+  return e ? e : conv_f32_patch(q, taps, plan, st);
+}
+
+int conv_f32_patch(const Conv3x3Problem &q, int taps, const PatchPlan &plan, hipStream_t st) {
   F32PatchParams P = {};
   static_cast<PatchParams &>(P) = plan.P;
   for (uint32_t t = 0; t < q.num_tiles; ++t) {

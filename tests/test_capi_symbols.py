@@ -132,3 +132,27 @@ def test_the_choice_of_a_tile_is_made_in_microseconds():
             best = min(best, (time.perf_counter() - t) / 20)
         assert name.value == b"conv3x3_split_kernel" + kernel
         assert best < 6e-6, (K, N, Cin, Cout, H, W, best)
+
+
+def test_small_layers_are_planned_once():
+    """The choice between patches and persistent workgroups or strips costs a small layer less than one plan of the latter takes (it
+    took two to seven times as much while both sides were planned, the patches twice)."""
+    l = capi.lib()
+    name = ctypes.create_string_buffer(256)
+
+    def cost(dtype, K, N, Cin, Cout, H, W):
+        best = 1e9
+        for _ in range(50):
+            t = time.perf_counter()
+            for _ in range(20):
+                assert l.adh_conv3x3_kernel_name(capi.ADH_CONV_FWD, dtype, K, N, Cin, Cout, H, W, 0.0, name, 256) == capi.ADH_OK
+            best = min(best, (time.perf_counter() - t) / 20)
+        return best
+
+    plan = cost(capi.ADH_F32, 4, 32, 64, 64, 14, 56)
+    assert b"split" in name.value and plan < 20e-6
+    for dtype in (capi.ADH_F32, capi.ADH_BF16):
+        for shape in ((2, 1, 16, 16, 4, 2000), (2, 3, 20, 36, 9, 130), (4, 1, 32, 64, 14, 56)):
+            us = cost(dtype, *shape)
+            assert b"patch" in name.value
+            assert us < plan + 0.4e-6, (dtype, shape, us, plan)
