@@ -17,7 +17,8 @@
 // Measured (32 images, 4 tiles; before: v_mfma_f32 kernels, in bf16 over widened values): fp32 3x3, 128 -> 256 channels on 16 x 64 tiles
 // 0.202 -> 0.128 ms (150 TFLOP/s), 64 -> 128 on 32 x 128 0.217 -> 0.148, 256 -> 512 on 8 x 32 0.206 -> 0.129; bf16 3x3, 128 -> 256
 // 0.341 -> 0.068, 1x1 0.143 -> 0.025; 56 -> 112, 2 images, 2 tiles of 22 x 124: 36 -> 16 us.  Relative error against double
-// precision over the former kernels': fp32 0.2 - 0.8 (rectified inputs up to 1.0), bf16 0.35 - 1.0.
+// precision over the former kernels': fp32 0.2 - 0.7 (up to 1.9 with the products below h*h in the same sums: six roundings a step in place of
+// one, at no less time: 0.0 - 0.3 % of a projection block), bf16 0.35 - 1.0.
 // Bound: fp32 by splitting and storing four rows' worth of x per output row beside 1728 matrix cycles a wave and step; bf16 by
 // the staging alone; short layers by the workgroups' sums.
 #include "conv_s2_wgrad.h"
@@ -237,11 +238,14 @@ __global__ __launch_bounds__(64 * WO * WC, 2) void conv_s2_wgrad_kernel(const S2
   const uint32_t a_c = wo * OT * 16u + l16;
   const uint32_t b_base = ((wc * 16u + l16) * pitch + 8u * qo) * 2u;
 
-  floatx4 acc[OT][TAPS];
+  floatx4 acc[OT][TAPS], low[PARTS == 3 ? OT : 1][PARTS == 3 ? TAPS : 1];  // (fp32: low, the products below h*h)
 #pragma unroll
   for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
-    for (int t = 0; t < TAPS; ++t) acc[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < TAPS; ++t) {
+      acc[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (PARTS == 3) low[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
 
   // base: ring slot of the step's first x row
   auto multiply = [&](uint32_t base, uint32_t buf) {
@@ -274,16 +278,16 @@ __global__ __launch_bounds__(64 * WO * WC, 2) void conv_s2_wgrad_kernel(const S2
           w[k][0] = even;
         }
       }
-      auto products = [&](int ka, int kb) {
+      auto products = [&](auto &sum, int ka, int kb) {
 #pragma unroll
         for (int col = 0; col < COLS; ++col)
 #pragma unroll
-          for (int ot = 0; ot < OT; ++ot) acc[ot][r * 3 + col] = mfma_bf16(a[ot][ka], w[kb][col], acc[ot][r * 3 + col]);
+          for (int ot = 0; ot < OT; ++ot) sum[ot][r * 3 + col] = mfma_bf16(a[ot][ka], w[kb][col], sum[ot][r * 3 + col]);
       };
-      if constexpr (PARTS == 3) {  // small products first
-        products(0, 2); products(1, 1); products(2, 0); products(0, 1); products(1, 0);
+      if constexpr (PARTS == 3) {
+        products(low, 0, 2); products(low, 1, 1); products(low, 2, 0); products(low, 0, 1); products(low, 1, 0);
       }
-      products(0, 0);
+      products(acc, 0, 0);
     }
   };
 
@@ -338,7 +342,8 @@ __global__ __launch_bounds__(64 * WO * WC, 2) void conv_s2_wgrad_kernel(const S2
   for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
     for (int t = 0; t < TAPS; ++t) {
-      const floatx4 sum = acc[ot][t];
+      floatx4 sum = acc[ot][t];
+      if constexpr (PARTS == 3) sum += low[ot][t];
       nan |= __builtin_isunordered(sum[0], sum[1]) || __builtin_isunordered(sum[2], sum[3]);
       *(ADH_GLOBAL floatx4_u *)(out + (ot * TAPS + t) * 256) = sum;
     }
