@@ -18,7 +18,8 @@
 // Measured in bf16, both kernels and, at odd widths before, the copies (before: conv3x3_bf16_wgrad.hip alone), us: 512 -> 512 channels, 32 images,
 // 4 tiles of 4 x 16 591 -> 71; 128 -> 128, 8 images, 4 tiles of 64 x 255 247 -> 168 (900 TFLOP/s); 208 -> 433, 27 images, 3 tiles of
 // 9 x 16 221 -> 54; 18 -> 16, 2 tiles of 42 x 24 43 -> 8; 300 layers of 16 to 512 channels 1.65 times as fast (geometric mean).
-// Relative error against double precision over the former kernel's: 0.54 in the mean of 240 layers, 1.0 and below but for four (1.11).
+// Relative error against double precision over the former kernel's: 1.0 and below in 900 layers (steps_plan; up to 1.9 while layers of several channel groups
+// had no more splits than run at once).
 // Bound: long layers by the waits between a step's LDS accesses, products and staging (two workgroups a compute unit, 40 % of the
 // matrix cores' cycles); short ones by the two launches and the sums.
 #include "conv3x3_wgrad_steps.h"
@@ -457,7 +458,8 @@ struct StepsCost {
 static double steps_us(const StepsCost &c, uint32_t TW, uint32_t groups, uint32_t splits, uint32_t total, size_t split_bytes) {
   const double wg = (double)groups * splits / 256.0, on = std::min(std::max(wg, 1.0), (double)c.fit);
   const double step = c.step * (1.0 + c.more * (on - 1.0)) * (TW == 8u ? 1.3 : TW == 16u ? 1.03 : 1.0);
-  return 8.4 + ((total + splits - 1u) / splits) * step * std::max(1.0, wg / c.fit) + 0.29e-6 * (double)split_bytes * splits;
+  const double rounds = std::max(1.0, 0.8 * std::ceil(wg / c.fit) + 0.2 * wg / c.fit);
+  return 8.4 + ((total + splits - 1u) / splits) * step * rounds + 0.29e-6 * (double)split_bytes * splits;
 }
 
 static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
@@ -482,18 +484,22 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   const uint64_t planes = (uint64_t)q.N * (q.stacked ? 1u : q.num_tiles);
   static const StepsCost costs[4] = {{1.15, 0.54, 4}, {1.55, 0.33, 2}, {1.4, 0.34, 3}, {1.8, 0.11, 2}};  // [co64][ci64]
   const StepsCost &cost = costs[(plan->co64 ? 2 : 0) + (plan->ci64 ? 1 : 0)];
-  // The step's shape and the number of splits: the shortest expected time, steps per split going up by a quarter, with no longer chains
-  // of additions than a walk down 64 columns of every tile makes where tiles are short (those sums would be more accurate).
+  // The step's shape and the number of splits: the shortest expected time, steps per split going up by a quarter.  However few workgroups
+  // run at once, as many splits as conv3x3_bf16_wgrad.hip has workgroups that walk down 64 columns of images: no sum is of more
+  // pixels (four times as many are 1.9 times as far from double precision; narrow images, whose walks multiply zeros for the most
+  // part, are 1.1 times as far at as many).  Half as many pixels where enough workgroups run at once.
   const uint64_t strips = (uint64_t)q.num_tiles * q.N * ((q.W + 63u) / 64u), rows = (strips + 255u) / 256u * q.H * (q.W > 32u ? 2u : 1u);
   const uint64_t longest = (rows + 8u) / (2u * kb);
+  const uint64_t walks = std::min<uint64_t>(strips, 256u) * (q.W > 32u ? 4u : 5u) / 4u;
   double best = 1e300;
   for (uint32_t TW = 32u * kb; TW >= steps_narrowest(!plan->co64 || !plan->ci64); TW /= 2u) {
     const uint32_t RS = 32u * kb / TW, row_steps = (P.rows + RS - 1u) / RS, cols = (q.W + TW - 1u) / TW;
     const uint64_t total = planes * cols * row_steps;
     if (total >= (1ull << 31)) continue;
     const uint32_t most = std::max(1u, std::min((uint32_t)total, 256u * cost.fit / std::min(groups, 256u * cost.fit)));
-    const uint64_t least = (total + most - 1u) / most;
-    for (uint64_t per = least; per <= std::max(least, std::min(total, longest)); per += 1u + per / 4u) {
+    const uint64_t fit = (total + most - 1u) / most, cap = std::max<uint64_t>(1u, total / walks);
+    const uint64_t least = fit <= cap ? fit : (cap + 1u) / 2u, upper = fit <= cap ? std::max(fit, std::min(total, longest)) : cap;
+    for (uint64_t per = least; per <= upper; per = per < upper && upper == cap ? std::min(upper, per + 1u + per / 8u) : per + 1u + per / 4u) {
       const uint32_t splits = (uint32_t)((total + per - 1u) / per);
       const double us = steps_us(cost, TW, groups, splits, (uint32_t)total, plan->split_bytes);
       if (us >= best) {

@@ -106,3 +106,27 @@ def test_small_workspaces(stacked, W):
         served += 1
         assert (got - want).norm() <= 1e-6 * want.norm()
     assert served
+
+
+def _error(K, N, Ci, Co, H, W):
+    """Relative error against double precision, computed on the GPU."""
+    g = torch.Generator(device="cuda").manual_seed(1)
+    xs = [(torch.rand((N, Ci, H + 2, W + 2), device="cuda", generator=g) * 2 - 1).bfloat16() for _ in range(K)]
+    dys = [torch.randn((N, Co, H, W), device="cuda", generator=g).bfloat16() for _ in range(K)]
+    want = torch.zeros((Co, Ci, 3, 3), device="cuda", dtype=torch.float64)
+    for x, dy in zip(xs, dys):
+        d = dy.double().transpose(0, 1).reshape(Co, -1)
+        for a in range(3):
+            for b in range(3):
+                want[:, :, a, b] += d @ x[:, :, a:a + H, b:b + W].double().permute(0, 2, 3, 1).reshape(-1, Ci)
+    dw = torch.empty((Co, Ci, 3, 3), device="cuda")
+    ws = torch.empty(capi.conv_workspace_bytes(capi.ADH_CONV_BWD_FILTER, capi.ADH_BF16, K, N, Ci, Co, H, W) // 4, device="cuda")
+    capi.check(capi.conv_bwd_filter_tiles(xs, dys, dw, N, Ci, Co, H, W, ws=ws), "filter gradient")
+    return ((dw.double() - want).norm() / want.norm()).item()
+
+
+@pytest.mark.parametrize("shape,walks", [((3, 7, 263, 135, 11, 272), 1.58e-7), ((7, 31, 103, 287, 13, 50), 1.64e-7), ((8, 24, 48, 256, 10, 170), 2.27e-7)])
+def test_sums_of_no_more_pixels_than_walks_down_64_columns(shape, walks):
+    """Layers of several channel groups, of which few splits run at once.  walks: the error of conv3x3_bf16_wgrad.hip's sums (measured; 2.48e-7, 3.16e-7
+    and 2.39e-7 where the splits are as many as run at once)."""
+    assert _error(*shape) <= 1.02 * walks
