@@ -860,20 +860,22 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
 
 // Strips or patches: strips are ahead on large images of 64 or 128 channels (64 -> 64 on 8 tiles of 128 x 2048 258 against 578 us, 128 ->
 // 128 on 4 tiles of 64 x 256 109 and 190), patches where a launch is small, the channels are no whole 64, or more than one launch of
-// strips would follow another (21 -> 400 on 6 tiles of 6 x 171, backward-data, 372 against 25 us; 566 random shapes: 2.25 times as fast
-// over all, 2.48 with this choice, 2.51 with the better of both each time).
-// What the strips' launches take, fitted to those shapes (rms error 20 %): each its start and its waves' steps; padded to whole 64 (or
-// 128) channels and 64 (32) columns the multiplications; the copies of odd rows, and the sums between launches.
+// strips would follow another (21 -> 400 on 6 tiles of 6 x 171, backward-data, 372 against 25 us).  5000 passes of random layers take 0.8 %
+// more over all than with the better of both each time; 47 lose more than 3 % by patches, up to 27 % (107 and 53 % before forward's even
+// widths, which are not copied, were priced without a copy, and a round of patches that is begun like a whole one).
+// What the strips' launches take, fitted to 5600 passes (rms error 14 % of a single launch, 20 % of several): each its start and its
+// waves' steps; padded to whole 64 (or 128) channels and 64 (32) columns the multiplications, slower by the four-wave kernel; the results;
+// the copies of odd rows, and the sums between launches.
 static double conv_bf16_strips_us(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, bool halofree) {
   const bool fwd = which == ADH_CONV_FWD, wide = conv_bf16_uses_k128(which, Cin, Cout);
+  const bool copies = !halofree && conv_bf16_repitches(which, Cin, Cout, H, W), four_waves = !halofree && !copies && !conv_bf16_w8_width(which, W);
   const double images = (double)num_tiles * N, C = fwd ? Cin : Cout, M = fwd ? Cout : Cin;
   const double oh = H + (fwd || halofree ? 0.0 : 2.0), ow = W + (fwd || halofree ? 0.0 : 2.0), ih = H + (fwd && !halofree ? 2.0 : 0.0), iw = W + (fwd && !halofree ? 2.0 : 0.0);
-  const double unit = wide ? 128.0 : 64.0, cols = wide ? 32.0 : 64.0, launches = std::ceil(C / unit), groups = std::ceil(M / unit);
+  const double unit = wide ? 128.0 : 64.0, cols = wide ? 32.0 : 64.0, launches = std::ceil(C / unit), groups = std::ceil(M / unit), pixels = images * oh * ow;
   const double flops = images * oh * std::ceil(ow / cols) * cols * 18.0 * launches * groups * unit * unit;
-  const double steps = std::ceil(std::max(1.0, images * std::ceil(ow / 64.0) * std::ceil(oh / 4.0) * std::ceil(M / 64.0) / 256.0));
-  double us = launches * (wide ? 22.7 : 18.2) + (wide ? 0.49e-9 : 0.81e-9) * flops + 0.69 * steps * std::ceil(C / 64.0);
-  if (!halofree && W % 8u != 0u) us += 0.74e-6 * images * C * ih * iw;
-  return us + 2e-6 * (launches - 1.0) * images * M * oh * ow;
+  const double steps = std::ceil(std::max(1.0, images * std::ceil(ow / 64.0) * std::ceil(oh / 4.0) * std::ceil(M / 64.0) / 256.0)) * std::ceil(C / 64.0);
+  if (wide) return 19.0 * launches + 0.459e-9 * flops + 0.082e-9 * 18.0 * pixels * C * groups * unit + 0.89 * steps + 1.7e-6 * (launches - 1.0) * pixels * M + (copies ? 4.7 + 0.68e-6 * images * C * ih * iw : 0.0);
+  return 16.0 * launches + (four_waves ? 0.66e-9 : 0.48e-9) * flops + 1.78 * steps + 0.15e-6 * pixels * M + 2e-6 * (launches - 1.0) * pixels * M + (copies ? 11.0 + 1.06e-6 * images * C * ih * iw : 0.0);
 }
 constexpr double kPatchAhead = 1.15;  // by which patches have to be expected ahead
 

@@ -390,11 +390,11 @@ static double f32_patch_us(const Conv3x3Problem &q, int taps, int MT, int NT, ui
 static double patch_multiply(int taps, uint32_t chunk, int MT, int NT) {
   return taps * (chunk / 32u) * std::max(16.0 * MT * NT, 32.0 * (MT + NT));
 }
-// bf16: as fitted (see patch_plan); ready: the filter put in order first
+// bf16: what the launches are expected to take (see patch_plan); ready: the filter put in order first
 static double bf16_patch_us(int taps, int MT, int NT, uint32_t chunks, uint64_t blocks, bool ready) {
-  const double full = std::min(1.0, blocks / 512.0), rounds = std::max(1.0, blocks / 512.0), multiply = patch_multiply(taps, taps == 1 ? 64u : 32u, MT, NT);
-  return ready ? 2.1 + rounds * (5.4 + chunks * 0.00096 * multiply * (1.0 + 1.06 * full))
-               : rounds * (4.1 + chunks * (0.00032 * multiply * (1.0 + 5.3 * full) + 0.52 * MT));
+  const double round = blocks / 512.0, full = std::min(1.0, round), multiply = patch_multiply(taps, taps == 1 ? 64u : 32u, MT, NT);
+  return ready ? 3.2 + std::max(1.0, 0.6 * std::ceil(round) + 0.4 * round) * (5.9 + chunks * (0.001 * multiply * (0.033 + 1.62 * std::sqrt(full)) + 0.11 * MT))
+               : 0.8 + std::ceil(round) * (3.1 + chunks * (0.00039 * multiply * (1.0 + 5.1 * std::pow(full, 1.7)) + 0.54 * MT));
 }
 // 3x3 at stride 1: whether no tile can be expected to take less than most_us, by its least number of blocks.  Tells large launches,
 // which are the strips', without a plan.
@@ -412,12 +412,13 @@ static bool bf16_patch_exceeds(const Conv3x3Problem &q, double most_us) {
 
 // Blocks of BR x BC output pixels (of NB images) by 16 MT channels, two workgroups per compute unit.  The tile is chosen by a model of
 // a block's cycles: a chunk's multiplications (or their operands' way out of LDS), its staging, and a load's latency.
-// The launch's time is then expected as fitted to 566 shapes (rms error 15 %), rounds of 512 workgroups of n chunks each,
+// Whether the filter is put in order first, is decided by times as fitted to 566 shapes, rounds of 512 workgroups of n chunks each,
 // `multiply` cycles of matrix work a chunk, f the part of a round's workgroups that exist:
 //   the caller's filter        rounds (4.1 + n (0.00032 multiply (1 + 5.3 f) + 0.52 MT)) us
 //   put in order first   2.1 + rounds (5.4 + n 0.00096 multiply (1 + 1.06 f)) us
 // (from 20 us on the second: forward, the caller's filter costs a line of cache per lane and load.  64 -> 64 channels, 8 tiles of
-// 128 x 2048 717 -> 578 us, 16 -> 32 on 72 x 16 4.7 -> 7.3.)
+// 128 x 2048 717 -> 578 us, 16 -> 32 on 72 x 16 4.7 -> 7.3.)  The launch's time is then expected as fitted to 5000 passes served here (bf16_patch_us;
+// rms error 14 %): a round that is begun takes most of a whole one's time.
 int patch_plan(const Conv3x3Problem &q, int taps, int parts, size_t workspace_bytes, PatchPlan *plan) {
   PatchParams &P = plan->P;
   P.N = q.N; P.C = q.C; P.M = q.M; P.num_tiles = q.num_tiles;
@@ -507,11 +508,12 @@ int patch_plan(const Conv3x3Problem &q, int taps, int parts, size_t workspace_by
     plan->us = best;
     return ADH_OK;
   }
-  plan->us = bf16_patch_us(taps, plan->MT, plan->NT, P.nchunks, blocks, false);
+  const double full = std::min(1.0, blocks / 512.0), rounds = std::max(1.0, blocks / 512.0), multiply = patch_multiply(taps, chunk, plan->MT, plan->NT);
+  const double first_us = 2.1 + rounds * (5.4 + P.nchunks * 0.00096 * multiply * (1.0 + 1.06 * full));
   plan->units = (uint64_t)((P.M + 63u) / 64u) * P.nchunks * 256u;
-  const double ready_us = bf16_patch_us(taps, plan->MT, plan->NT, P.nchunks, blocks, true);
-  plan->ready = taps == 9 && ready_us < plan->us && plan->units * 144u <= workspace_bytes && plan->units < (1ull << 31);
-  if (plan->ready) plan->us = ready_us;
+  plan->ready = taps == 9 && first_us < rounds * (4.1 + P.nchunks * (0.00032 * multiply * (1.0 + 5.3 * full) + 0.52 * plan->MT)) &&
+                plan->units * 144u <= workspace_bytes && plan->units < (1ull << 31);
+  plan->us = bf16_patch_us(taps, plan->MT, plan->NT, P.nchunks, blocks, plan->ready);
   return ADH_OK;
 }
 

@@ -156,3 +156,12 @@ def test_small_layers_are_planned_once():
             us = cost(dtype, *shape)
             assert b"patch" in name.value
             assert us < plan + 0.4e-6, (dtype, shape, us, plan)
+
+
+@pytest.mark.parametrize("shape,strips_us,patches_us", [((6, 10, 64, 64, 80, 324), 143, 247), ((5, 29, 64, 32, 34, 566), 181, 278), ((8, 7, 64, 32, 34, 660), 88, 116),
+                                                        ((6, 6, 64, 128, 12, 153), 26, 35), ((2, 16, 128, 128, 4, 930), 43, 62)])
+def test_bf16_layers_that_strips_take_faster(shape, strips_us, patches_us):
+    """Forward of layers that went to patches: even widths priced with copies that are not made, rounds that are begun as parts of one."""
+    name = ctypes.create_string_buffer(256)
+    assert capi.lib().adh_conv3x3_kernel_name(capi.ADH_CONV_FWD, capi.ADH_BF16, *shape, 0.0, name, 256) == capi.ADH_OK
+    assert b"patch" not in name.value
