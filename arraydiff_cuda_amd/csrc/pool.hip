@@ -672,14 +672,13 @@ __device__ __forceinline__ S2Row<NC> s2_load_row(const PoolS2Params &P, uint32_t
     for (int k = 0; k < NC; ++k) q.v[k] = 0.f;
   return q;
 }
-template <typename T, bool TAILS, int V>
-__device__ __forceinline__ void s2_store(T *p, const float (&f)[V], uint32_t count, bool stream) {
+template <typename T, bool TAILS, bool STREAM, int V>
+__device__ __forceinline__ void s2_store(T *p, const float (&f)[V], uint32_t count) {
   S2Pack<T, V> v;
 #pragma unroll
   for (int k = 0; k < V; ++k) st_f(v.e, k, f[k]);
   if (!TAILS || count >= (uint32_t)V) {
-    if (stream) store_vec<true>(p, v);
-    else store_vec<false>(p, v);
+    store_vec<STREAM>(p, v);
   } else {
 #pragma unroll
     for (int k = 0; k < V - 1; ++k)
@@ -731,7 +730,7 @@ __global__ __launch_bounds__(kPoolThreads) void pool_fwd_max3s2_kernel(const Poo
     arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l);
     uint32_t t, r;
     P.div_OH.divmod(o, t, r);
-    s2_store<T, TAILS, NW>(reinterpret_cast<T *>(P.out[t]) + ((size_t)plane * P.OH + r) * P.OW + c / 2u, f, P.OW - c / 2u, false);
+    s2_store<T, TAILS, false, NW>(reinterpret_cast<T *>(P.out[t]) + ((size_t)plane * P.OH + r) * P.OW + c / 2u, f, P.OW - c / 2u);
     top = bot;
     r0 = n0; r1 = n1;
   }
@@ -818,7 +817,7 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
       for (int k = 0; k < NC; ++k)
         if (!TAILS || c + (uint32_t)k < P.W) f[k] += ld_f(p, k);
     }
-    s2_store<T, TAILS, NC>(p, f, P.W - c, STREAM);
+    s2_store<T, TAILS, STREAM, NC>(p, f, P.W - c);
   };
 
   const uint32_t o_lo = blockIdx.y * P.steps, o_hi = min(VO + 1u, o_lo + P.steps);  // (step VO: the last input row)
