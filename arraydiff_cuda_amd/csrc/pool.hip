@@ -611,18 +611,19 @@ static void launch_bwd_band(int dtype, bool max, const PoolParams &P, uint32_t b
 }
 
 // 3x3 max pooling at stride 2, padding 1, over tiles of even height without halo (rows of at least one group of columns).
-// A thread owns NC columns (16 bytes of a row) and marches down a band of window rows of the stacked tensor.  No LDS, no
+// A thread owns NC columns and marches down a band of window rows of the stacked tensor.  No LDS, no
 // barrier; the next step's loads are in flight during this one's work (and have arrived before its stores go out, or the
-// next step would wait for those too: 82 against 102 us).  Bound by memory.  Bands of 32 window rows; 8: 8 % slower, 64: no faster.
-// Measured against the LDS bands, which stage rows that are no whole 16-byte groups one element at a time: 18 x 482 planes of
-// 6 x 350, fp32: forward 33 -> 19.5 us, backward 82 -> 41; bf16, 36 x 100 planes of 14 x 333: 31 -> 13, 62 -> 35.  32 x 64 planes,
-// 4 tiles of 48 x 128, fp32: forward 80 -> 43, and at 64 x 256: forward 126 -> 138, backward 389 -> 247; bf16: 127 -> 83, 194
-// (four columns a thread) -> 145.
+// next step would wait for those too: 82 against 102 us; the last step has none, and does not wait: 4 to 12 % of a small
+// tensor's pass).  Bound by memory.  Bands of 32 window rows; 8: 8 % slower, 64: no faster.
+// Measured against the LDS bands, which stage rows that are no whole 16-byte groups one element at a time (bands -> here): 4 tiles of 32 x 64
+// planes, fp32: 48 x 128 forward 63 -> 37 us, backward 123 -> 93; 64 x 255 270 -> 160, 675 -> 313; 64 x 256 backward 389 -> 234 (5.2 TB/s);
+// bf16: 64 x 512 forward 171 -> 143, backward 936 -> 251; 64 x 516 (four columns a thread) 370 -> 167, 1920 -> 355.
 struct PoolS2Params {
   const void *x[ADH_MAX_TILES], *dy[ADH_MAX_TILES];
   void *out[ADH_MAX_TILES];  // y (forward) or dx
   uint32_t items;  // planes x groups of columns
-  uint32_t K, H, W, OH, OW, steps;  // steps: window rows per band
+  uint32_t K, H, W, OH, OW, steps, nc;  // steps: window rows per band; nc: a thread's columns
+  bool stream;
   float beta;
   FastDiv div_groups, div_H, div_OH;
 };
@@ -693,9 +694,9 @@ __device__ __forceinline__ void arrived(const float (&f)[V]) {
   for (int k = 0; k < V; ++k) asm volatile("" ::"v"(f[k]));
 }
 
-template <typename T, bool TAILS, bool STREAM>
+template <typename T, int NC, bool TAILS, bool STREAM>
 __global__ __launch_bounds__(kPoolThreads) void pool_fwd_max3s2_kernel(const PoolS2Params P) {
-  constexpr int NC = 16 / sizeof(T), NW = NC / 2;
+  constexpr int NW = NC / 2;
   const uint32_t id = blockIdx.x * kPoolThreads + threadIdx.x;
   if (id >= P.items) return;
   uint32_t plane, c;
@@ -718,8 +719,12 @@ __global__ __launch_bounds__(kPoolThreads) void pool_fwd_max3s2_kernel(const Poo
   if (o_lo >= o_hi) return;
   Best top = best_of(load_row(2u * o_lo - 1u));  // (row -1: none)
   S2Row<NC> r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
-  for (uint32_t o = o_lo; o < o_hi; ++o) {
-    const S2Row<NC> n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
+  auto step = [&](uint32_t o, auto more) {  // more: the band goes on, and wants the next rows
+    S2Row<NC> n0, n1;
+    if constexpr (more) {
+      n0 = load_row(2u * o + 2u);
+      n1 = load_row(2u * o + 3u);
+    }
     const Best mid = best_of(r0), bot = best_of(r1);
     float f[NW];
 #pragma unroll
@@ -727,21 +732,26 @@ __global__ __launch_bounds__(kPoolThreads) void pool_fwd_max3s2_kernel(const Poo
       f[w] = mid.b[w] > top.b[w] ? mid.b[w] : top.b[w];
       f[w] = bot.b[w] > f[w] ? bot.b[w] : f[w];
     }
-    arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l);
+    if constexpr (more) { arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l); }
     uint32_t t, r;
     P.div_OH.divmod(o, t, r);
     s2_store<T, TAILS, false, NW>(reinterpret_cast<T *>(P.out[t]) + ((size_t)plane * P.OH + r) * P.OW + c / 2u, f, P.OW - c / 2u);
-    top = bot;
-    r0 = n0; r1 = n1;
-  }
+    if constexpr (more) {
+      top = bot;
+      r0 = n0; r1 = n1;
+    }
+  };
+  uint32_t o = o_lo;
+  for (; o + 1u < o_hi; ++o) step(o, std::true_type{});
+  step(o, std::false_type{});
 }
 
 // A step loads two input rows, finds where the windows of this row that touch the thread's columns (the last one with its
 // first column only) have their first maximum (a row's own is shared by the window rows above and below it) and stores the
 // two input rows that no later window touches.
-template <typename T, bool TAILS, bool STREAM>
+template <typename T, int NC, bool TAILS, bool STREAM>
 __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const PoolS2Params P) {
-  constexpr int NC = 16 / sizeof(T), NW = NC / 2;
+  constexpr int NW = NC / 2;
   const uint32_t id = blockIdx.x * kPoolThreads + threadIdx.x;
   if (id >= P.items) return;
   uint32_t plane, c;
@@ -835,9 +845,14 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
   }
   S2Row<NC> r0 = load_row(2u * o_lo), r1 = load_row(2u * o_lo + 1u);
   Grad g = load_dy(o_lo);
-  for (uint32_t o = o_lo; o < o_hi; ++o) {
-    const S2Row<NC> n0 = load_row(2u * o + 2u), n1 = load_row(2u * o + 3u);
-    const Grad ng = load_dy(o + 1u);
+  auto step = [&](uint32_t o, auto more) {
+    S2Row<NC> n0, n1;
+    Grad ng;
+    if constexpr (more) {
+      n0 = load_row(2u * o + 2u);
+      n1 = load_row(2u * o + 3u);
+      ng = load_dy(o + 1u);
+    }
     const Best bot = best_of(r1);
     const Windows here = windows_of(top, best_of(r0), bot, g);
     float f0[NC] = {}, f1[NC] = {};  // rows 2 o - 1 and 2 o
@@ -851,23 +866,42 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
       add(f0, above, 2u);
     }
     add(f1, here, 1u);
-    arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l); arrived(n0.r); arrived(n1.r); arrived(ng.v); arrived(ng.n);
+    if constexpr (more) { arrived(n0.v); arrived(n1.v); arrived(n0.l); arrived(n1.l); arrived(n0.r); arrived(n1.r); arrived(ng.v); arrived(ng.n); }
     if (o > 0u) store_row(2u * o - 1u, f0);
     if (o < VO) store_row(2u * o, f1);
-    above = here;
-    top = bot;
-    r0 = n0; r1 = n1; g = ng;
-  }
+    if constexpr (more) {
+      above = here;
+      top = bot;
+      r0 = n0; r1 = n1; g = ng;
+    }
+  };
+  uint32_t o = o_lo;
+  for (; o + 1u < o_hi; ++o) step(o, std::true_type{});
+  step(o, std::false_type{});
 }
 
-// 3x3 / 2, padding 1, rows of at least a group of columns; anything else takes the bands, and so do the smallest tensors: a
-// thread's chain of loads is longer than a band's (16 to 20 k pixels: 4.1 us a pass there, 5 to 9 here; 72 k: the other way round)
-static bool pool_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
-  const uint32_t nc = (uint32_t)(16u / es), groups = (P.W + nc - 1u) / nc;
+// 3x3 / 2, padding 1, rows of at least a group of columns; anything else takes the bands, and so do
+//   * the smallest tensors, a thread's chain of loads being longer than a band's (16 to 20 k pixels: 4.1 us a pass there, 5 to 9 here;
+//     72 k: the other way round; backward, where bands would stage element by element or not: rows of whole groups of four 4.9 us here at
+//     15 k pixels, 5.3 there);
+//   * forward, fp32 tensors larger than the on-package cache in long rows of whole 16-byte groups (64 x 260: 133 us there, 158 here; 64 x 700
+//     177 and 206; 64 x 256 130 and 132; but 64 x 128 158 and 117, 64 x 222 262 and 132).
+// bf16: eight columns a thread are 16 bytes; four where only that many are whole groups (64 x 516: backward 355 us, 383 by eights), and for
+// tensors below 24 MB, which want the threads (5 x 29 x 141 planes of 8 x 12: 7.1 us, 11.3; 7 x 31 x 72 of 14 x 63, 28 MB, 25.6 and 26.8).
+// Non-temporal accesses where the input is larger than the cache and the rows are whole lines of 128 bytes (fp32 64 x 256: backward 234
+// us, 260 without); else lines that two rows share would come twice (64 x 260 313 and 305), which is not worth giving up bf16's
+// forward (64 x 520 178 and 188) and backward's ragged rows (64 x 255 313 and 335) for.
+static bool pool_max3s2(const PoolParams &P, size_t es, bool fwd, PoolS2Params *q) {
+  const uint64_t rows = (uint64_t)P.num_tiles * P.H, pixels = P.planes * rows * P.W;
+  const bool large = pixels * es > (256ull << 20);  // than the on-package cache
+  const uint32_t nc = q->nc = es == 4u || P.W < 8u || P.W % 8u == 4u || pixels * es < (24ull << 20) ? 4u : 8u;
+  const uint32_t groups = (P.W + nc - 1u) / nc;
   if (P.wh != 3u || P.ww != 3u || P.sh != 2u || P.sw != 2u || P.pad_h != 1u || P.pad_w != 1u || P.W < nc) return false;
-  const uint64_t items = (uint64_t)P.planes * groups, rows = (uint64_t)P.num_tiles * P.H;
+  const uint64_t items = (uint64_t)P.planes * groups;
   if (items >= (1ull << 31) || rows >= (1ull << 31)) return false;
-  if (P.planes * rows * P.W < (1u << 15)) return false;
+  if (pixels < (1u << 15) && (fwd || P.W % 4u != 0u)) return false;
+  if (fwd && es == 4u && large && P.W % 4u == 0u && P.W >= 160u) return false;
+  q->stream = large && (P.W * es % 128u == 0u || (fwd ? es == 2u : P.W % nc != 0u));
   for (uint32_t t = 0; t < P.num_tiles; ++t) {
     q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->out[t] = P.out[t];
   }
@@ -882,23 +916,22 @@ static bool pool_max3s2(const PoolParams &P, size_t es, PoolS2Params *q) {
   q->div_groups = FastDiv(groups); q->div_H = FastDiv(P.H); q->div_OH = FastDiv(P.OH);
   return true;
 }
-// non-temporal accesses where the input is larger than the on-package cache
-template <bool FWD>
-static int launch_max3s2(int dtype, const PoolParams &P, const PoolS2Params &q, hipStream_t st) {
-  const size_t es = dtype_size(dtype);
-  const bool tails = q.W % (16u / es) != 0u, stream = (uint64_t)P.planes * q.K * q.H * q.W * es > (256ull << 20);
+template <typename T, int NC, bool FWD>
+static void launch_max3s2_nc(const PoolS2Params &q, hipStream_t st) {
+  const bool tails = q.W % NC != 0u;
   const dim3 grid((q.items + kPoolThreads - 1u) / kPoolThreads, (q.K * q.OH + q.steps) / q.steps), block(kPoolThreads);
   auto go = [&](auto tl, auto sm) {
-    auto kernel = [&](auto t) {
-      typedef decltype(t) T;
-      if constexpr (FWD) hipLaunchKernelGGL((pool_fwd_max3s2_kernel<T, tl, sm>), grid, block, 0, st, q);
-      else hipLaunchKernelGGL((pool_bwd_max3s2_kernel<T, tl, sm>), grid, block, 0, st, q);
-    };
-    if (dtype == ADH_F32) kernel(0.f);
-    else kernel(uint16_t(0));
+    if constexpr (FWD) hipLaunchKernelGGL((pool_fwd_max3s2_kernel<T, NC, tl, sm>), grid, block, 0, st, q);
+    else hipLaunchKernelGGL((pool_bwd_max3s2_kernel<T, NC, tl, sm>), grid, block, 0, st, q);
   };
-  if (tails) stream ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
-  else stream ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+  if (tails) q.stream ? go(std::true_type{}, std::true_type{}) : go(std::true_type{}, std::false_type{});
+  else q.stream ? go(std::false_type{}, std::true_type{}) : go(std::false_type{}, std::false_type{});
+}
+template <bool FWD>
+static int launch_max3s2(int dtype, const PoolS2Params &q, hipStream_t st) {
+  if (dtype == ADH_F32) launch_max3s2_nc<float, 4, FWD>(q, st);
+  else if (q.nc == 8u) launch_max3s2_nc<uint16_t, 8, FWD>(q, st);
+  else launch_max3s2_nc<uint16_t, 4, FWD>(q, st);
   return launch_status();
 }
 
@@ -1073,7 +1106,7 @@ int adh_pool2d_unpadded_fwd_tiles(int dtype, int mode, uint32_t num_tiles, uint3
   const uint32_t band_rows = pick_band_rows(P, num_tiles, kPoolBandBytes, [&](uint32_t r) { return fwd_band_lds(P, es, r); });
   if (!band_rows) return ADH_EUNIMPL;  // rows too wide for a band in LDS: use the padded entry points
   PoolS2Params q = {};
-  if (mode == ADH_POOL_MAX && pool_max3s2(P, es, &q)) return launch_max3s2<true>(dtype, P, q, as_stream(stream));
+  if (mode == ADH_POOL_MAX && pool_max3s2(P, es, true, &q)) return launch_max3s2<true>(dtype, q, as_stream(stream));
   set_bands(&P, band_rows);
   launch_fwd_band_u<true>(dtype, mode == ADH_POOL_MAX, P, P.planes * num_tiles * P.bands, fwd_band_lds(P, es, band_rows),
                           as_stream(stream));
@@ -1113,7 +1146,7 @@ int adh_pool2d_unpadded_bwd_tiles(int dtype, int mode, uint32_t num_tiles, uint3
       wh * ww > 256u ? 0u : pick_band_rows(P, num_tiles, bwd_band_aim(P, es, is_max), [&](uint32_t r) { return bwd_band_lds(P, es, is_max, r); });
   if (!band_rows) return ADH_EUNIMPL;
   PoolS2Params q = {};
-  if (is_max && pool_max3s2(P, es, &q)) return launch_max3s2<false>(dtype, P, q, as_stream(stream));
+  if (is_max && pool_max3s2(P, es, false, &q)) return launch_max3s2<false>(dtype, q, as_stream(stream));
   set_bands(&P, band_rows);
   launch_bwd_band_u<true>(dtype, is_max, P, P.planes * num_tiles * P.bands, bwd_band_lds(P, es, is_max, band_rows),
                           as_stream(stream));

@@ -67,3 +67,28 @@ def test_larger_than_the_cache(dtype):
         capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, small, None, sdy, d1, 1, C, Ht, W, *WINDOW, 1, 1), "backward")
         for t in range(K):
             assert _same(ys[t][n:n + 1], y1[t]) and _same(dxs[t][n:n + 1], d1[t])
+
+
+@pytest.mark.parametrize("W", [8, 9, 11, 13, 15, 16, 17, 22, 255, 520])
+def test_eight_columns_a_thread(W):
+    """bf16 tensors of 24 MB and more: the same bits as image by image, by fours."""
+    N, K, Ht = 3, 2, 10
+    C = (26 << 20) // (2 * N * K * Ht * W) + 1
+    g = torch.Generator(device="cuda").manual_seed(W)
+    x = torch.randint(-2, 3, (N, C, K * Ht, W), device="cuda", generator=g).bfloat16()
+    special = torch.tensor([float("inf"), -float("inf"), float("nan"), torch.finfo(torch.bfloat16).min, -0.0], device="cuda").bfloat16()
+    x = torch.where(torch.rand(x.shape, device="cuda", generator=g) < 0.2, special[torch.randint(0, 5, x.shape, device="cuda", generator=g)], x)
+    dy = torch.randn((N, C, K * Ht // 2, (W - 1) // 2 + 1), device="cuda", generator=g).bfloat16()
+
+    def run(x, dy, old):
+        xs, dys, dxs = ([t.clone(memory_format=torch.contiguous_format) for t in v.chunk(K, 2)] for v in (x, dy, old))
+        ys = [torch.full_like(t, 7.0) for t in dys]
+        capi.check(capi.pool_unpadded_fwd_tiles(capi.ADH_POOL_MAX, xs, ys, x.shape[0], C, Ht, W, *WINDOW, 1, 1), "forward")
+        capi.check(capi.pool_unpadded_bwd_tiles(capi.ADH_POOL_MAX, xs, None, dys, dxs, x.shape[0], C, Ht, W, *WINDOW, 1, 1, beta=1.0), "backward")
+        return torch.cat(ys, 2), torch.cat(dxs, 2)
+
+    old = torch.randint(-4, 5, x.shape, device="cuda", generator=g).bfloat16()
+    y, dx = run(x, dy, old)
+    for n in range(N):
+        y1, dx1 = run(x[n:n + 1], dy[n:n + 1], old[n:n + 1])
+        assert _same(y[n:n + 1], y1) and _same(dx[n:n + 1], dx1)
