@@ -165,3 +165,10 @@ def test_bf16_layers_that_strips_take_faster(shape, strips_us, patches_us):
     name = ctypes.create_string_buffer(256)
     assert capi.lib().adh_conv3x3_kernel_name(capi.ADH_CONV_FWD, capi.ADH_BF16, *shape, 0.0, name, 256) == capi.ADH_OK
     assert b"patch" not in name.value
+
+
+@pytest.mark.parametrize("shape,persistent_us,patches_us", [((8, 2, 512, 256, 36, 6), 124, 153), ((2, 2, 512, 512, 44, 11), 125, 154), ((3, 10, 512, 128, 24, 10), 124, 152)])
+def test_fp32_layers_that_persistent_workgroups_take_faster(shape, persistent_us, patches_us):
+    name = ctypes.create_string_buffer(256)
+    assert capi.lib().adh_conv3x3_kernel_name(capi.ADH_CONV_FWD, capi.ADH_F32, *shape, 0.0, name, 256) == capi.ADH_OK
+    assert b"split" in name.value
