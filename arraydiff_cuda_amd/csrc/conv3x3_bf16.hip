@@ -172,7 +172,7 @@ int repitch_bf16_tiles(uint32_t num_tiles, uint64_t rows, uint32_t w_src, uint32
 }
 
 static StepsWgradProblem wgrad_problem(bool stacked, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
-  return StepsWgradProblem{ADH_BF16, stacked, num_tiles, N, Cin, Cout, H, W, nullptr, nullptr, nullptr, 0.f};
+  return StepsWgradProblem{stacked, num_tiles, N, Cin, Cout, H, W, nullptr, nullptr, nullptr, 0.f};
 }
 static int wgrad_steps(StepsWgradProblem q, const void *const *x_tiles, const void *const *dy_tiles, float *dw, float beta, void *workspace,
                        size_t workspace_bytes, hipStream_t st) {

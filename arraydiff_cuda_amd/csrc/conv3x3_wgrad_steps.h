@@ -1,4 +1,4 @@
-// Filter gradients of 3x3 windows at stride 1: what conv3x3_wgrad_steps.hip gives the entry points.
+// Filter gradients of 3x3 windows at stride 1 over bf16 tensors, dw in fp32: what conv3x3_wgrad_steps.hip gives the entry points.
 #ifndef ADH_CONV3X3_WGRAD_STEPS_H
 #define ADH_CONV3X3_WGRAD_STEPS_H
 
@@ -9,7 +9,6 @@ namespace adh {
 // dw[co][ci][a][b] = beta*dw + sum over images, h, w of dy[co][h][w] * x[ci][h + a][w + b], x with a halo of one (H + 2 x W + 2, tiles of
 // their own), or (stacked) x[ci][h + a - 1][w + b - 1] with zeros outside, the tiles being the row tiles of one tensor in rank order.
 struct StepsWgradProblem {
-  int dtype;
   bool stacked;
   uint32_t num_tiles, N, Cin, Cout, H, W;
   const void *const *x, *const *dy;

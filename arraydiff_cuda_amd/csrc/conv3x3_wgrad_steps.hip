@@ -1,21 +1,21 @@
-// Filter gradient of the 3x3 stride-1 window on the bf16 matrix cores, over padded tiles or row tiles without halo, at any width from eight
-// and any number of channels; fp32 tensors in three parts and six products (split_bf16.h):
+// Filter gradient of the 3x3 stride-1 window over bf16 tensors on the matrix cores, over padded tiles or row tiles without halo, at any
+// width from eight and any number of channels:
 //   dw[co][ci][a][b] = beta*dw + sum over images, R, Q of dy[co][R][Q] * x[ci][R + a - halo][Q + b - halo]
 //
 // Mapping.  Per tap D[co][ci] += A[co][pixel] B[pixel][ci] on v_mfma_f32_16x16x32_bf16, k = 32 pixels: four octets of neighbouring
 // pixels of a row.
 //   * A workgroup owns 16*OT*WO output channels x 16*WC input channels x all taps and a run of steps; a step is RS rows of TW output
-//     columns, 64 pixels in bf16 (1 x 64 .. 8 x 8), 32 in fp32.  A wave keeps 16*OT x 16 x 9 sums: the octets of x that it shifts for
+//     columns, 64 pixels (1 x 64 .. 8 x 8).  A wave keeps 16*OT x 16 x 9 sums: the octets of x that it shifts for
 //     the three columns of a window's row feed 3*OT products.  Unlike a walk down whole columns of an image this splits small and narrow
 //     images over the chip as finely as their sums are worth, and has no columns beyond an image's end to speak of.
 //   * x rows go through a ring: a row is read once per run (an image's column of steps), its two columns behind the step's twice.  Rows
-//     are loaded from wherever they start (2 or 4 bytes' alignment), so that neither odd widths nor missing halos want copies.
+//     are loaded from wherever they start (2 bytes' alignment), so that neither odd widths nor missing halos want copies.
 //   * Rows lie in LDS as [octet][channel], exchanged so that neither side's accesses meet in a bank (with channels 144 bytes apart
 //     half of all cycles went there).  A step's rows are asked for two steps ahead, stored one ahead.  One barrier a step.
 //   * Past dy's last row and column dy is zero and x need not be there or finite: sums that come out as NaN are computed over again in
 //     plain fp32 from the pixels that exist.
 //   * The workgroups' sums are added by a second kernel in a fixed order (reproducible).
-// Measured in bf16, both kernels and, at odd widths before, the copies (before: conv3x3_bf16_wgrad.hip alone), us: 512 -> 512 channels, 32 images,
+// Measured, both kernels and, at odd widths before, the copies (before: conv3x3_bf16_wgrad.hip alone), us: 512 -> 512 channels, 32 images,
 // 4 tiles of 4 x 16 591 -> 71; 128 -> 128, 8 images, 4 tiles of 64 x 255 247 -> 168 (900 TFLOP/s); 208 -> 433, 27 images, 3 tiles of
 // 9 x 16 221 -> 54; 18 -> 16, 2 tiles of 42 x 24 43 -> 8; 300 layers of 16 to 512 channels 1.65 times as fast (geometric mean).
 // Relative error against double precision over the former kernel's: 1.0 and below in 900 layers (steps_plan; up to 1.9 while layers of several channel groups
@@ -40,15 +40,14 @@ struct StepsParams : WgradSums {
   FastDiv div_row_steps, div_cols, div_H, div_N, div_groups, div_splits;
 };
 
-// k blocks (of 32 pixels) a step, the widest step
-constexpr uint32_t steps_k(int parts) { return parts == 3 ? 1u : 2u; }
+constexpr uint32_t kStepBlocks = 2;  // k blocks (of 32 pixels) a step
 // the ring holds a step's rows and the most that the next one brings (its run may be another)
 constexpr uint32_t steps_ring(uint32_t rs) { return 2u * rs + 4u; }
 // the narrowest step of 32 channels: a wave's units of eight columns are of one row
 constexpr uint32_t steps_narrowest(bool few) { return few ? 16u : 8u; }
-// of one part: x rows with an octet behind them (whose first two columns exist), dy rows, twice
-constexpr uint32_t steps_x_bytes(uint32_t tw, uint32_t ci, uint32_t kb) { return steps_ring(kb * 32u / tw) * (tw / 8u + 1u) * ci * 16u; }
-constexpr uint32_t steps_dy_bytes(uint32_t co, uint32_t kb) { return 2u * kb * 4u * co * 16u; }
+// x rows with an octet behind them (whose first two columns exist), dy rows, twice
+constexpr uint32_t steps_x_bytes(uint32_t tw, uint32_t ci) { return steps_ring(kStepBlocks * 32u / tw) * (tw / 8u + 1u) * ci * 16u; }
+constexpr uint32_t steps_dy_bytes(uint32_t co) { return 2u * kStepBlocks * 4u * co * 16u; }
 // How THREADS threads take a row's units of eight columns, columns first, then channels, then rows (a wave's units are of one row):
 // unit j of a thread is channel pass j % passes of row (j / passes) * rows + the thread's.
 template <uint32_t THREADS, uint32_t U, uint32_t C>
@@ -62,19 +61,11 @@ struct StepsUnits {
   __device__ uint32_t row_of(int j) const { return (uint32_t)j / passes * rows + row; }
 };
 
-// eight neighbouring columns, and the two behind a step's, as loaded
-template <typename T> struct StepsRaw;
-template <> struct StepsRaw<float> { floatx4 v[2]; };
-template <> struct StepsRaw<uint16_t> { uintx4 v; };
-template <typename T> struct StepsTail;
-template <> struct StepsTail<float> { floatx2 v; };
-template <> struct StepsTail<uint16_t> { uint32_t v; };
 typedef uintx4 steps_u32x4 __attribute__((aligned(2)));
 typedef uint32_t steps_u32 __attribute__((aligned(2)));
-typedef floatx2 steps_f32x2 __attribute__((aligned(4)));
 
-// Values from column Q on of a row of W were loaded from column min(max(Q, 0), W - 8) on (floats: each half by itself): to their places,
-// zeros where none exists.
+// Values from column Q on of a row of W were loaded from column min(max(Q, 0), W - 8) on: to their places, zeros
+// where none exists.
 __device__ __forceinline__ uintx4 steps_place(uintx4 v, int32_t Q, int32_t W) {
   const int32_t d = Q - min(max(Q, 0), W - 8);
   if (d != 0) {
@@ -89,34 +80,20 @@ __device__ __forceinline__ uintx4 steps_place(uintx4 v, int32_t Q, int32_t W) {
   }
   return v;
 }
-__device__ __forceinline__ floatx4 steps_place(floatx4 v, int32_t Q, int32_t W) {
-  const int32_t d = Q - min(max(Q, 0), W - 4);
-  if (d != 0) {
-    if (d < 0) {
-      v = floatx4{0.f, v[0], v[1], v[2]};
-    } else {
-      if (d & 2) v = floatx4{v[2], v[3], 0.f, 0.f};
-      if (d & 1) v = floatx4{v[1], v[2], v[3], 0.f};
-      if (d >= 4) v = floatx4{0.f, 0.f, 0.f, 0.f};
-    }
-  }
-  return v;
-}
 
 // A step: RS rows of TW columns.
-template <typename T, uint32_t TW, int OT, int WO, int WC>
-__global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2 && WC == 4 && TW == 64u) ? 2 : OT == 2 ? 3 : 4) void conv3x3_wgrad_steps_kernel(const StepsParams P) {
+template <uint32_t TW, int OT, int WO, int WC>
+__global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW == 64u) ? 2 : OT == 2 ? 3 : 4) void conv3x3_wgrad_steps_kernel(const StepsParams P) {
   constexpr uint32_t THREADS = 64u * WO * WC, CO = 16u * OT * WO, CI = 16u * WC;
-  constexpr int PARTS = sizeof(T) == 4 ? 3 : 1;
-  constexpr uint32_t KB = steps_k(PARTS), RS = KB * 32u / TW, NR = steps_ring(RS), U = TW / 8u;
-  constexpr uint32_t XB = steps_x_bytes(TW, CI, KB), LDS = XB + steps_dy_bytes(CO, KB);
+  constexpr uint32_t KB = kStepBlocks, RS = KB * 32u / TW, NR = steps_ring(RS), U = TW / 8u;
+  constexpr uint32_t XB = steps_x_bytes(TW, CI);
   typedef StepsUnits<THREADS, U, CI> XUnits;
   typedef StepsUnits<THREADS, U, CO> DyUnits;
   // units that a thread stages per step (x: of all rows, where a run begins), and the two columns behind
   constexpr int XU = XUnits::count(RS + 2u), DU = DyUnits::count(RS), XS = XUnits::sure(RS), DS = DyUnits::sure(RS);
   constexpr uint32_t tail_per = THREADS / CI;
   constexpr int TU = (int)((RS + 2u + tail_per - 1u) / tail_per);
-  __shared__ __align__(16) char lds[PARTS * LDS];
+  __shared__ __align__(16) char lds[XB + steps_dy_bytes(CO)];
   __shared__ uint32_t nan_sums;
   char *const dyl = lds + XB;
   const uint32_t tid = threadIdx.x, lane = tid & 63u, l16 = lane & 15u, g = lane >> 4;
@@ -162,8 +139,8 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
   // the step whose rows are on their way
   struct Flight {
     Step s;
-    StepsRaw<T> x[XU], dy[DU];
-    StepsTail<T> tail[TU];
+    uintx4 x[XU], dy[DU];
+    uint32_t tail[TU];
   } f;
 
   // Row r of the plane, of the group's first channel.  The tiles' addresses come from lanes: a table in memory would be waited for
@@ -175,21 +152,15 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
   };
   auto x_at = [&](const Step &s, int32_t r) {
     const uint32_t t = P.div_H.div((uint32_t)r);  // (not stacked: 0)
-    return (const ADH_GLOBAL T *)of_lane(x_tile, s.tile + t) + (s.x_from + ((uint32_t)r - t * P.H) * P.x_W);
+    return (const ADH_GLOBAL uint16_t *)of_lane(x_tile, s.tile + t) + (s.x_from + ((uint32_t)r - t * P.H) * P.x_W);
   };
   auto dy_at = [&](const Step &s, uint32_t R) {
     const uint32_t t = P.div_H.div(R);
-    return (const ADH_GLOBAL T *)of_lane(dy_tile, s.tile + t) + (s.dy_from + (R - t * P.H) * P.W);
+    return (const ADH_GLOBAL uint16_t *)of_lane(dy_tile, s.tile + t) + (s.dy_from + (R - t * P.H) * P.W);
   };
   // (images are below 2^31 bytes)
-  auto load8 = [&](const ADH_GLOBAL T *row, uint32_t channel, int32_t Q, int32_t W, StepsRaw<T> &u) {
-    const ADH_GLOBAL char *p = (const ADH_GLOBAL char *)row;
-    if constexpr (PARTS == 3) {
-      u.v[0] = *(const ADH_GLOBAL floatx4_u *)(p + (channel + (uint32_t)min(max(Q, 0), W - 4)) * 4u);
-      u.v[1] = *(const ADH_GLOBAL floatx4_u *)(p + (channel + (uint32_t)min(Q + 4, W - 4)) * 4u);
-    } else {
-      u.v = *(const ADH_GLOBAL steps_u32x4 *)(p + (channel + (uint32_t)min(max(Q, 0), W - 8)) * 2u);
-    }
+  auto load8 = [&](const ADH_GLOBAL uint16_t *row, uint32_t channel, int32_t Q, int32_t W) {
+    return *(const ADH_GLOBAL steps_u32x4 *)(row + (channel + (uint32_t)min(max(Q, 0), W - 8)));
   };
   // Channels that do not exist are taken as the group's first: what they add to is not used.
   uint32_t x_chan[XUnits::passes], dy_chan[DyUnits::passes];
@@ -204,18 +175,16 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
     const Step &s = f.s;
     const int32_t x0 = (int32_t)(s.rs * RS) - halo + (s.first ? 0 : 2), Q0 = (int32_t)s.c0 - halo;
     const uint32_t nx = s.first ? RS + 2u : RS;
-    auto load_x = [&](int j) { load8(x_at(s, min(max(x0 + (int32_t)xu.row_of(j), 0), x_rows - 1)), x_chan[j % XUnits::passes], Q0 + (int32_t)q8, xW, f.x[j]); };
-    auto load_dy = [&](int j) { load8(dy_at(s, min(s.rs * RS + du.row_of(j), P.rows - 1u)), dy_chan[j % DyUnits::passes], (int32_t)(s.c0 + q8), dW, f.dy[j]); };
+    auto load_x = [&](int j) { f.x[j] = load8(x_at(s, min(max(x0 + (int32_t)xu.row_of(j), 0), x_rows - 1)), x_chan[j % XUnits::passes], Q0 + (int32_t)q8, xW); };
+    auto load_dy = [&](int j) { f.dy[j] = load8(dy_at(s, min(s.rs * RS + du.row_of(j), P.rows - 1u)), dy_chan[j % DyUnits::passes], (int32_t)(s.c0 + q8), dW); };
 #pragma unroll
     for (int j = 0; j < TU; ++j) {
       const uint32_t i = (uint32_t)j * tail_per + tail_row;
       if (i < nx) {
-        auto row = [&](uint32_t of_wave) { return (const ADH_GLOBAL char *)x_at(s, min(max(x0 + (int32_t)((uint32_t)j * tail_per + wave * 64u / CI + of_wave), 0), x_rows - 1)); };
-        const ADH_GLOBAL char *p = row(0u);
+        auto row = [&](uint32_t of_wave) { return x_at(s, min(max(x0 + (int32_t)((uint32_t)j * tail_per + wave * 64u / CI + of_wave), 0), x_rows - 1)); };
+        const ADH_GLOBAL uint16_t *p = row(0u);
         if (CI < 64u && lane >= CI) p = row(1u);
-        p += (tail_chan + (uint32_t)min(Q0 + (int32_t)TW, xW - 2)) * (uint32_t)sizeof(T);
-        if constexpr (PARTS == 3) f.tail[j].v = *(const ADH_GLOBAL steps_f32x2 *)p;
-        else f.tail[j].v = *(const ADH_GLOBAL steps_u32 *)p;
+        f.tail[j] = *(const ADH_GLOBAL steps_u32 *)(p + (tail_chan + (uint32_t)min(Q0 + (int32_t)TW, xW - 2)));
       }
     }
 #pragma unroll
@@ -230,22 +199,10 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
     for (int j = 0; j < DS; ++j) load_dy(j);
   };
   // eight values in their places, or none, to p
-  auto store8 = [&](char *p, uint32_t part_bytes, const StepsRaw<T> &u, int32_t Q, int32_t W, bool ok) {
-    if constexpr (PARTS == 3) {
-      floatx4 a = steps_place(u.v[0], Q, W), b = steps_place(u.v[1], Q + 4, W);
-      if (!ok) a = b = floatx4{0.f, 0.f, 0.f, 0.f};
-      uint32_t part[3][4];
-      split_pair(a[0], a[1], part[0][0], part[1][0], part[2][0]);
-      split_pair(a[2], a[3], part[0][1], part[1][1], part[2][1]);
-      split_pair(b[0], b[1], part[0][2], part[1][2], part[2][2]);
-      split_pair(b[2], b[3], part[0][3], part[1][3], part[2][3]);
-#pragma unroll
-      for (int k = 0; k < 3; ++k) *reinterpret_cast<uintx4 *>(p + k * part_bytes) = uintx4{part[k][0], part[k][1], part[k][2], part[k][3]};
-    } else {
-      uintx4 v = steps_place(u.v, Q, W);
-      if (!ok) v = uintx4{0u, 0u, 0u, 0u};
-      *reinterpret_cast<uintx4 *>(p) = v;
-    }
+  auto store8 = [&](char *p, uintx4 u, int32_t Q, int32_t W, bool ok) {
+    uintx4 v = steps_place(u, Q, W);
+    if (!ok) v = uintx4{0u, 0u, 0u, 0u};
+    *reinterpret_cast<uintx4 *>(p) = v;
   };
   // slot0: ring slot of the first row; buf: the dy buffer
   auto store = [&](uint32_t slot0, uint32_t buf) {
@@ -261,7 +218,7 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
       const uint32_t i = xu.row_of(j), c = xu.channel(j);
       if (j < XS || i < nx) {
         const int32_t r = x0 + (int32_t)i;
-        store8(lds + slot_of(i) * ((U + 1u) * CI * 16u) + (xu.q * CI + (c ^ swap)) * 16u, LDS, f.x[j], Q0 + (int32_t)q8, xW, r >= 0 && r < x_rows);
+        store8(lds + slot_of(i) * ((U + 1u) * CI * 16u) + (xu.q * CI + (c ^ swap)) * 16u, f.x[j], Q0 + (int32_t)q8, xW, r >= 0 && r < x_rows);
       }
     }
 #pragma unroll
@@ -270,26 +227,14 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
       if (i < nx) {
         const int32_t r = x0 + (int32_t)i, d = Q0 + (int32_t)TW - min(Q0 + (int32_t)TW, xW - 2);
         const bool none = r < 0 || r >= x_rows || d >= 2;
-        char *p = lds + slot_of(i) * ((U + 1u) * CI * 16u) + tail_to;
-        if constexpr (PARTS == 3) {
-          floatx2 v = f.tail[j].v;
-          if (d == 1) v = floatx2{v[1], 0.f};
-          if (none) v = floatx2{0.f, 0.f};
-          uint32_t h, m, l;
-          split_pair(v[0], v[1], h, m, l);
-          *reinterpret_cast<uint32_t *>(p) = h;
-          *reinterpret_cast<uint32_t *>(p + LDS) = m;
-          *reinterpret_cast<uint32_t *>(p + 2u * LDS) = l;
-        } else {
-          *reinterpret_cast<uint32_t *>(p) = none ? 0u : d == 1 ? f.tail[j].v >> 16 : f.tail[j].v;
-        }
+        *reinterpret_cast<uint32_t *>(lds + slot_of(i) * ((U + 1u) * CI * 16u) + tail_to) = none ? 0u : d == 1 ? f.tail[j] >> 16 : f.tail[j];
       }
     }
 #pragma unroll
     for (int j = 0; j < DU; ++j) {
       const uint32_t i = du.row_of(j), c = du.channel(j);
       if (j < DS || i < RS)
-        store8(dyl + (buf * RS + i) * (U * CO * 16u) + (du.q * CO + (c ^ swap)) * 16u, LDS, f.dy[j], (int32_t)(s.c0 + q8), dW, s.rs * RS + i < P.rows);
+        store8(dyl + (buf * RS + i) * (U * CO * 16u) + (du.q * CO + (c ^ swap)) * 16u, f.dy[j], (int32_t)(s.c0 + q8), dW, s.rs * RS + i < P.rows);
     }
   };
   auto advance = [&]() {
@@ -312,29 +257,23 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
     constexpr int kReads = 3 * (int)KB;  // (k block, window row)
     constexpr int ABUF = OT == 4 ? 1 : 2;  // (registers)
     struct Row { uintx4 d; uintx2 e; };  // an octet, the next one's first four columns
-    uintx4 a[ABUF][OT][PARTS];
-    Row x[2][PARTS];
+    uintx4 a[ABUF][OT];
+    Row x[2];
     // this lane group's octet of k block kb: row io of the step, octet qo of the row
     auto row_of = [&](uint32_t kb) { return U >= 4u ? kb * 4u / U : kb * (4u / U) + g / U; };
     auto octet_of = [&](uint32_t kb) { return U >= 4u ? kb * 4u % U + g : g % U; };
     auto lane_at = [&](uint32_t octet, uint32_t C, uint32_t c0) { return (octet * C + c0 + (l16 ^ octet_swap(octet))) * 16u; };
-    auto read_dy = [&](uint32_t kb, uintx4 (&v)[OT][PARTS]) {
+    auto read_dy = [&](uint32_t kb, uintx4 (&v)[OT]) {
       const char *p = dyl + (buf * RS + row_of(kb)) * (U * CO * 16u) + lane_at(octet_of(kb), CO, wo * OT * 16u);
 #pragma unroll
-      for (int ot = 0; ot < OT; ++ot)
-#pragma unroll
-        for (int k = 0; k < PARTS; ++k) v[ot][k] = *reinterpret_cast<const uintx4 *>(p + k * LDS + ot * 256u);
+      for (int ot = 0; ot < OT; ++ot) v[ot] = *reinterpret_cast<const uintx4 *>(p + ot * 256u);
     };
-    auto read_x = [&](int i, Row (&v)[PARTS]) {
+    auto read_x = [&](int i, Row &v) {
       uint32_t slot = base + row_of(i / 3) + (uint32_t)(i % 3);
       slot -= slot >= NR ? NR : 0u;
       const char *p = lds + slot * ((U + 1u) * CI * 16u);
-      const uint32_t d = lane_at(octet_of(i / 3), CI, wc * 16u), e = lane_at(octet_of(i / 3) + 1u, CI, wc * 16u);
-#pragma unroll
-      for (int k = 0; k < PARTS; ++k) {
-        v[k].d = *reinterpret_cast<const uintx4 *>(p + d + k * LDS);
-        v[k].e = *reinterpret_cast<const uintx2 *>(p + e + k * LDS);
-      }
+      v.d = *reinterpret_cast<const uintx4 *>(p + lane_at(octet_of(i / 3), CI, wc * 16u));
+      v.e = *reinterpret_cast<const uintx2 *>(p + lane_at(octet_of(i / 3) + 1u, CI, wc * 16u));
     };
     read_dy(0, a[0]);
     read_x(0, x[0]);
@@ -345,28 +284,18 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
         read_x(i + 1, x[(i + 1) & 1]);
       }
       const int r = i % 3;
-      const uintx4(&av)[OT][PARTS] = a[i / 3 % ABUF];
-      uintx4 w[PARTS][3];
+      const uintx4(&av)[OT] = a[i / 3 % ABUF];
+      uintx4 d = x[i & 1].d;
+      asm volatile("" : "+v"(d));  // (the compiler would read the shifted columns from LDS again, dword by dword)
+      const uint32_t e = x[i & 1].e[0];
+      const uintx4 w[3] = {d,
+                           uintx4{__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
+                                  __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(e, d[3], 16)},
+                           uintx4{d[1], d[2], d[3], e}};
 #pragma unroll
-      for (int k = 0; k < PARTS; ++k) {
-        uintx4 d = x[i & 1][k].d;
-        asm volatile("" : "+v"(d));  // (the compiler would read the shifted columns from LDS again, dword by dword)
-        const uint32_t e = x[i & 1][k].e[0];
-        w[k][0] = d;
-        w[k][1] = uintx4{__builtin_amdgcn_alignbit(d[1], d[0], 16), __builtin_amdgcn_alignbit(d[2], d[1], 16),
-                         __builtin_amdgcn_alignbit(d[3], d[2], 16), __builtin_amdgcn_alignbit(e, d[3], 16)};
-        w[k][2] = uintx4{d[1], d[2], d[3], e};
-      }
-      auto products = [&](int ka, int kb) {
+      for (int b = 0; b < 3; ++b)
 #pragma unroll
-        for (int b = 0; b < 3; ++b)
-#pragma unroll
-          for (int ot = 0; ot < OT; ++ot) acc[ot][r * 3 + b] = mfma_bf16(av[ot][ka], w[kb][b], acc[ot][r * 3 + b]);
-      };
-      if constexpr (PARTS == 3) {  // small products first
-        products(0, 2); products(1, 1); products(2, 0); products(0, 1); products(1, 0);
-      }
-      products(0, 0);
+        for (int ot = 0; ot < OT; ++ot) acc[ot][r * 3 + b] = mfma_bf16(av[ot], w[b], acc[ot][r * 3 + b]);
       if (ABUF == 1 && i % 3 == 2 && i + 1 < kReads) read_dy((i + 1) / 3, a[0]);
       __builtin_amdgcn_sched_barrier(0);
     }
@@ -411,10 +340,6 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
   __syncthreads();
   if (nan_sums == 0u) return;
   // sums that are NaN once more in plain fp32, straight from memory
-  auto value = [](T v) {
-    if constexpr (PARTS == 3) return v;
-    else return bf16_bits_to_f32(v);
-  };
   for (uint32_t at = tid; at < WO * WC * kWave; at += THREADS) {
     if (part[at] == part[at]) continue;
     const uint32_t i = at & 3u, ln = at >> 2 & 63u, rest = at >> 8, tap = rest % 9u, ot = rest / 9u % OT, wt = rest / 9u / OT;
@@ -428,9 +353,9 @@ __global__ __launch_bounds__(64 * WO * WC, sizeof(T) == 4 || OT == 4 || (OT == 2
         for (uint32_t R = s.rs * RS; R < min((s.rs + 1u) * RS, P.rows) && sum == sum; ++R)
           for (uint32_t Q = s.c0; Q < min(s.c0 + TW, P.W) && sum == sum; ++Q) {
             const int32_t r = (int32_t)(R + tap / 3u) - halo, c = (int32_t)(Q + tap % 3u) - halo;
-            const float dyv = value(((const ADH_GLOBAL T *)P.dy[s.tile + P.div_H.div(R)] + ((size_t)s.n * P.Cout + co) * dy_plane + (size_t)(R - P.div_H.div(R) * P.div_H.d) * P.W)[Q]);
+            const float dyv = bf16_bits_to_f32(((const ADH_GLOBAL uint16_t *)P.dy[s.tile + P.div_H.div(R)] + ((size_t)s.n * P.Cout + co) * dy_plane + (size_t)(R - P.div_H.div(R) * P.div_H.d) * P.W)[Q]);
             float xe = 0.f;
-            if (r >= 0 && r < x_rows && c >= 0 && c < xW) xe = value(((const ADH_GLOBAL T *)P.x[s.tile + P.div_H.div((uint32_t)r)] + ((size_t)s.n * P.Cin + ci) * x_plane + (size_t)((uint32_t)r - P.div_H.div((uint32_t)r) * P.div_H.d) * P.x_W)[c]);
+            if (r >= 0 && r < x_rows && c >= 0 && c < xW) xe = bf16_bits_to_f32(((const ADH_GLOBAL uint16_t *)P.x[s.tile + P.div_H.div((uint32_t)r)] + ((size_t)s.n * P.Cin + ci) * x_plane + (size_t)((uint32_t)r - P.div_H.div((uint32_t)r) * P.div_H.d) * P.x_W)[c]);
             sum = __builtin_fmaf(dyv, xe, sum);
           }
       }
@@ -466,8 +391,7 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   StepsParams &P = plan->P;
   if (q.W < 8u || (uint64_t)(q.H + 2ull) * q.num_tiles >= (1ull << 30) || (uint64_t)q.W >= (1ull << 30)) return false;
   if ((uint64_t)q.Cin * q.Cout * 9u >= (1ull << 31)) return false;
-  const int parts = q.dtype == ADH_F32 ? 3 : 1;
-  if ((uint64_t)std::max(q.Cin, q.Cout) * (q.H + 2ull) * (q.W + 2ull) * (parts == 3 ? 4u : 2u) >= (1ull << 31)) return false;
+  if ((uint64_t)std::max(q.Cin, q.Cout) * (q.H + 2ull) * (q.W + 2ull) * 2u >= (1ull << 31)) return false;
   P.N = q.N; P.Cin = q.Cin; P.Cout = q.Cout;
   P.stacked = q.stacked ? 1u : 0u;
   P.H = q.H; P.W = q.W;
@@ -475,7 +399,7 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   P.rows = q.stacked ? q.H * q.num_tiles : q.H;
   P.x_rows = q.stacked ? P.rows : P.x_H;
   P.beta = q.beta;
-  const uint32_t kb = steps_k(parts);
+  const uint32_t kb = kStepBlocks;
   plan->co64 = q.Cout > 32u; plan->ci64 = q.Cin > 32u;
   const uint32_t co = plan->co64 ? 64u : 32u, ci = plan->ci64 ? 64u : 32u;
   P.ci_groups = (q.Cin + ci - 1u) / ci;
@@ -518,7 +442,7 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   plan->us = steps_us(cost, plan->TW, groups, P.splits, P.total_steps, plan->split_bytes);
   // From half of what the XCDs' caches hold (8 x 4 MB): 240 -> 16 channels on 4 tiles of 20 x 104, 81 MB, 85 -> 59 us, 1.08 in the mean from 32 MB,
   // 1.02 from 16; smaller ones lose 1 to 4 % (up to 16 %), as the partial sums' order suits the second kernel less.
-  P.by_xcd = (uint64_t)q.num_tiles * q.N * q.H * q.W * (q.Cin + q.Cout) * (parts == 3 ? 4u : 2u) > (16ull << 20) ? 1u : 0u;
+  P.by_xcd = (uint64_t)q.num_tiles * q.N * q.H * q.W * (q.Cin + q.Cout) * 2u > (16ull << 20) ? 1u : 0u;
   P.div_row_steps = FastDiv(P.row_steps); P.div_cols = FastDiv(P.cols); P.div_H = FastDiv(q.stacked ? P.H : 1u << 31); P.div_N = FastDiv(P.N);
   P.div_cig = FastDiv(P.ci_groups);
   return true;
@@ -534,28 +458,21 @@ double conv3x3_wgrad_steps_us(const StepsWgradProblem &q) {
   return steps_plan(q, &plan) ? plan.us : 0.0;
 }
 
-template <typename T, int OT, int WO, int WC>
+template <int OT, int WO, int WC>
 static void launch_steps(const StepsPlan &plan, hipStream_t st) {
   const dim3 grid(plan.groups * plan.P.splits), block(64 * WO * WC);
   switch (plan.TW) {
     case 64:
-      if constexpr (sizeof(T) == 2) hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<T, 64, OT, WO, WC>), grid, block, 0, st, plan.P);
+      hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<64, OT, WO, WC>), grid, block, 0, st, plan.P);
       break;
-    case 32: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<T, 32, OT, WO, WC>), grid, block, 0, st, plan.P); break;
-    case 16: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<T, 16, OT, WO, WC>), grid, block, 0, st, plan.P); break;
+    case 32: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<32, OT, WO, WC>), grid, block, 0, st, plan.P); break;
+    case 16: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<16, OT, WO, WC>), grid, block, 0, st, plan.P); break;
     default:
-      if constexpr (16 * OT * WO == 64 && WC == 4) hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<T, 8, OT, WO, WC>), grid, block, 0, st, plan.P);
+      if constexpr (16 * OT * WO == 64 && WC == 4) hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<8, OT, WO, WC>), grid, block, 0, st, plan.P);
       break;
   }
   hipLaunchKernelGGL((wgrad_sums_kernel<9, OT, WO, WC>), dim3(plan.groups * (WO * WC * OT * 9u * 64u / 16u)), dim3(256), 0, st, static_cast<const WgradSums &>(plan.P));
 }
-template <typename T>
-static void launch_steps_channels(const StepsPlan &plan, hipStream_t st) {
-  constexpr bool wide = sizeof(T) == 2;
-  if (plan.co64) plan.ci64 ? launch_steps<T, wide ? 4 : 2, wide ? 1 : 2, 4>(plan, st) : launch_steps<T, wide ? 2 : 1, wide ? 2 : 4, 2>(plan, st);
-  else plan.ci64 ? launch_steps<T, wide ? 2 : 1, wide ? 1 : 2, 4>(plan, st) : launch_steps<T, 1, 2, 2>(plan, st);
-}
-
 int conv3x3_wgrad_steps(const StepsWgradProblem &q, void *workspace, size_t workspace_bytes, hipStream_t st) {
   StepsPlan plan = {};
   if (!steps_plan(q, &plan) || workspace_bytes < plan.split_bytes) return ADH_EUNIMPL;
@@ -568,8 +485,8 @@ int conv3x3_wgrad_steps(const StepsWgradProblem &q, void *workspace, size_t work
   }
   P.part = reinterpret_cast<float *>(workspace);
   P.dw = q.dw;
-  if (q.dtype == ADH_F32) launch_steps_channels<float>(plan, st);
-  else launch_steps_channels<uint16_t>(plan, st);
+  if (plan.co64) plan.ci64 ? launch_steps<4, 1, 4>(plan, st) : launch_steps<2, 2, 2>(plan, st);
+  else plan.ci64 ? launch_steps<2, 1, 4>(plan, st) : launch_steps<1, 2, 2>(plan, st);
   return launch_status();
 }
 

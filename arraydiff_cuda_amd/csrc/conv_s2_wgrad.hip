@@ -475,7 +475,7 @@ int conv_s2_wgrad(const S2WgradProblem &q, void *workspace, size_t workspace_byt
   }
   P.part = reinterpret_cast<float *>(workspace);
   P.dw = q.dw;
-  if (q.dtype == ADH_F32) q.taps == 9 ? launch_s2wg_channels<float, 9>(plan, st) : launch_s2wg_channels<float, 1>(plan, st);
+  if (q.dtype == ADH_F32) launch_s2wg_channels<float, 9>(plan, st);
   else q.taps == 9 ? launch_s2wg_channels<uint16_t, 9>(plan, st) : launch_s2wg_channels<uint16_t, 1>(plan, st);
   return launch_status();
 }
