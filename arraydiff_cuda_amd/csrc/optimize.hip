@@ -243,9 +243,11 @@ static int flat_copy(uint32_t num, const float *const *arrays, const uint64_t *l
     if (!aligned_to(arrays[s], 4)) return ADH_EALIGN;
     total += lens[s];
   }
-  // Gradients are read once: non-temporal from 32 MB on, where several ranks' and their flat vectors would not all stay in
-  // the on-package cache.  A step of 11.7 M parameters: 160 us, 177 without; 8.7 M on 4 ranks 118 and 128, on one 57 and 55;
-  // below (4 M): 40 and 37 on 2 ranks, 105 and 114 on 8.
+  // Gradients are read once a step, after a backward pass that has moved more than the on-package cache holds since it wrote the
+  // first of them: non-temporal from 32 MB on, all that a call knows of.  8.7 M floats that are not in the cache, in one array 15.1 us
+  // (16.6 without), in 56 16.0 (23.2 by 48 arrays a launch, without); that are in it, 14.4 (12.1) and 15.1 (15.6).  A step of 11.7 M
+  // parameters on 4 ranks, over and over on the same gradients: 160 us, 177 without; 8.7 M on 4 ranks 118 and 128, on one 57 and 55.
+  // Smaller ones are no slower than before either way, but for a single array of 4 M (8.5 -> 9.2 us not in the cache; in eight arrays 10.0 -> 10.1).
   const bool stream_data = TO_FLAT && total * sizeof(float) >= (32ull << 20);
   float *base = flat + flat_offset;
   uint32_t s = 0;

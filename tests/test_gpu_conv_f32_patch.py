@@ -62,6 +62,22 @@ def test_images_and_tiles(which, k, s, K, N, H):
     _close(*_unpadded(which, k, s, K, N, 24, 40, H, 12))
 
 
+# What the larger tiles serve (two tiles of H x W): 16 MT channels by 64 NT pixels, MT and NT of 1 and 2 as the plan takes them there
+LARGER_TILES = [(FWD, 3, 1, 2, 20, 24, 30, 130), (FWD, 3, 1, 4, 33, 31, 14, 130), (BWD, 3, 1, 2, 24, 20, 30, 130), (BWD, 3, 1, 4, 31, 33, 14, 130),
+                (FWD, 3, 2, 4, 16, 24, 30, 130), (FWD, 3, 2, 8, 33, 17, 14, 130), (FWD, 1, 1, 4, 16, 16, 30, 130), (FWD, 1, 1, 2, 16, 24, 30, 130),
+                (FWD, 1, 1, 8, 70, 17, 14, 130), (FWD, 1, 2, 16, 16, 16, 30, 130), (FWD, 1, 2, 16, 16, 24, 14, 130), (FWD, 1, 2, 16, 20, 33, 30, 88),
+                (BWD, 1, 1, 4, 16, 16, 30, 130), (BWD, 1, 1, 4, 24, 16, 14, 130), (BWD, 1, 1, 8, 24, 70, 14, 130), (BWD, 1, 2, 16, 16, 16, 30, 130),
+                (BWD, 1, 2, 16, 24, 16, 14, 130), (BWD, 1, 2, 16, 33, 20, 30, 88)]
+
+
+@pytest.mark.parametrize("which,k,s,N,Ci,Co,H,W", LARGER_TILES)
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+def test_larger_tiles(which, k, s, N, Ci, Co, H, W, beta):
+    if k == 3 and s == 1:  # (which the name is of)
+        assert "conv_f32_patch_kernel<2, 2, 0, 9>" in capi.conv_kernel_name(which, capi.ADH_F32, 2, N, Ci, Co, H, W)
+    _close(*_unpadded(which, k, s, 2, N, Ci, Co, H, W, beta=beta), beta=beta)
+
+
 @pytest.mark.parametrize("which,k,s", FORMS)
 def test_accumulates(which, k, s):
     _close(*_unpadded(which, k, s, 2, 3, 40, 24, 8, 22, beta=1.0), beta=1.0)
@@ -112,6 +128,21 @@ def test_not_finite_values_stay_in_their_windows(which, k, s, value):
         near = touched & (want.abs() < 3.3e38)
         assert ((got - want)[near].abs() <= 1e-6 * want[near].abs()).all()
     fine = ~touched
+    assert (got - want)[fine].norm() <= 3e-7 * want[fine].norm()
+
+
+@pytest.mark.parametrize("which,k,s,N,Ci,Co,H,W", LARGER_TILES[1::3])
+@pytest.mark.parametrize("value", [float("nan"), float("inf")])
+def test_not_finite_values_in_larger_tiles(which, k, s, N, Ci, Co, H, W, value):
+    def spoil(w, t):
+        t[0, 3, 1, 2] = value
+        t[1, 5, -1, -1] = value
+        t[-1, 7, 0, 64 // s] = value  # (a pixel that every form reads)
+
+    got, want = _unpadded(which, k, s, 2, N, Ci, Co, H, W, spoil=spoil)
+    assert torch.equal(got.isnan(), want.isnan()) and torch.equal(got.isinf(), want.isinf())
+    fine = want.isfinite()
+    assert fine.any() and not fine.all()
     assert (got - want)[fine].norm() <= 3e-7 * want[fine].norm()
 
 

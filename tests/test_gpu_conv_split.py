@@ -104,6 +104,73 @@ def test_values_without_finite_bf16_parts(bad):
         assert fine.any() and not torch.equal(want, torch.nn.functional.conv2d(x, w, padding=1))
 
 
+# Layers just beyond what conv_f32_patch.hip takes: chunks of channels and groups of 16, 32 and 64 that are not full, rows of any width,
+# every number of channels on which the order of additions hangs
+BEYOND = [(2, 3, 33, 70, 30, 187), (3, 2, 40, 90, 41, 96), (1, 4, 4, 96, 61, 90), (2, 9, 17, 16, 80, 92), (2, 9, 16, 33, 80, 91), (4, 9, 64, 130, 14, 33), (2, 4, 100, 72, 30, 124)]
+
+
+def _slab(which, K, N, Cin, Cout, H, W, beta=0.0, spoil=None):
+    """A pass over padded tiles by the persistent workgroups, and its sums in double precision, both with the padding as data."""
+    assert "conv3x3_split_kernel" in capi.conv_kernel_name(which, capi.ADH_F32, K, N, Cin, Cout, H, W)
+    g = torch.Generator(device="cuda").manual_seed(Cin + W)
+    fwd = which == capi.ADH_CONV_FWD
+    w = torch.randn((Cout, Cin, 3, 3), device="cuda", generator=g) * (2.0 / (Cin * 9)) ** 0.5
+    t = torch.rand((K * N, Cin if fwd else Cout, H + 2 if fwd else H, W + 2 if fwd else W), device="cuda", generator=g) * 2 - 1
+    if spoil:
+        spoil(w, t)
+    M, OH, OW = (Cout, H, W) if fwd else (Cin, H + 2, W + 2)
+    tp = t.double() if fwd else torch.nn.functional.pad(t, (2,) * 4).double()
+    wd = (w if fwd else w.transpose(0, 1).flip(2, 3)).double()
+    want = torch.zeros((M, K * N * OH * OW), device="cuda", dtype=torch.float64)
+    for a in range(3):
+        for b in range(3):
+            want += wd[:, :, a, b].contiguous() @ tp[:, :, a:a + OH, b:b + OW].transpose(0, 1).reshape(t.shape[1], -1)
+    want = want.reshape(M, K * N, OH, OW).transpose(0, 1)
+    outs = [torch.full((N, M, OH, OW), 2.0, device="cuda") for _ in range(K)]
+    tiles = [v.contiguous() for v in t.chunk(K, 0)]
+    if fwd:
+        capi.check(capi.conv_fwd_tiles(tiles, w, outs, N, Cin, Cout, H, W, beta=beta), "fwd")
+    else:
+        capi.check(capi.conv_bwd_data_tiles(w, tiles, outs, N, Cin, Cout, H, W, beta=beta), "bwd-data")
+    return torch.cat(outs).double() - (2.0 if beta else 0.0), want
+
+
+@pytest.mark.parametrize("which", [capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA])
+@pytest.mark.parametrize("beta", [0.0, 1.0])
+@pytest.mark.parametrize("shape", BEYOND)
+def test_persistent_workgroups_vs_double(which, beta, shape):
+    if which == capi.ADH_CONV_BWD_DATA:
+        K, N, Cin, Cout, H, W = shape
+        shape = (K, N, Cout, Cin, H, W)  # (as many results)
+    got, want = _slab(which, *shape, beta=beta)
+    # 24 bits of every factor and fp32 sums: 2^-24 a term, random in sign; the old output's rounding
+    assert (got - want).norm() <= 3e-7 * want.norm() + (2e-7 * want.numel() ** 0.5 if beta else 0.0)
+
+
+@pytest.mark.parametrize("which", [capi.ADH_CONV_FWD, capi.ADH_CONV_BWD_DATA])
+@pytest.mark.parametrize("bad", [float("inf"), -float("inf"), 3.4e38, float("nan")])
+@pytest.mark.parametrize("where", ["input", "filter"])
+def test_persistent_workgroups_of_values_without_finite_bf16_parts(which, bad, where):
+    def spoil(w, t):
+        w.copy_(w.sign() * w.abs().clamp(min=0.01))
+        if where == "input":
+            t[0, 3, 4, 10] = t[-1, 5, -1, -1] = bad
+        else:
+            w[5, 7, 1, 2] = bad
+
+    got, want = _slab(which, 2, 3, 70, 70, 30, 187, spoil=spoil)
+    want32 = want.float().double()  # beyond fp32: infinite
+    assert torch.equal(got.isnan(), want32.isnan())
+    far = want32.isinf() | (want.abs() > 3.3e38)  # (which side of the largest number a sum near it falls on is its rounding's)
+    assert torch.equal(got[want32.isinf() & (bad != 3.4e38)], want32[want32.isinf() & (bad != 3.4e38)])
+    large = (want.abs() > 1e30) & ~far
+    assert ((got - want)[large].abs() <= 2e-6 * want[large].abs()).all()
+    fine = want.abs() <= 1e30
+    assert fine.any() and (~fine).any()
+    # 630 terms of 24 bits in one chain of 27 sums, each rounded (2^-24, random in sign) at the size it has by then
+    assert (got - want)[fine].norm() <= 2.0 ** -24 * 27 ** 0.5 * 2 * want[fine].norm()
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 def test_filter_gradient_of_values_without_finite_bf16_parts(bad):
     N, Cin, Cout, H, W = 1, 20, 40, 6, 21

@@ -56,7 +56,8 @@ def _passes(x, w, dy, k, s, pad):
 
 @pytest.mark.parametrize("kind", ["uniform", "rectified"])
 @pytest.mark.parametrize("Cin,Cout,k,s,pad", [(1, 64, 3, 1, 1), (3, 40, 3, 1, 1), (5, 33, 3, 1, 1), (16, 16, 3, 1, 1), (40, 20, 3, 1, 1), (64, 64, 3, 1, 1),
-                                              (2, 3, 3, 2, 1), (16, 48, 3, 2, 1), (64, 16, 3, 2, 1), (3, 64, 7, 1, 0), (3, 48, 7, 2, 0), (1, 16, 3, 1, 0)])
+                                              (2, 3, 3, 2, 1), (16, 48, 3, 2, 1), (64, 16, 3, 2, 1), (3, 64, 7, 1, 0), (3, 48, 7, 2, 0), (1, 16, 3, 1, 0),
+                                              (20, 48, 1, 1, 0), (70, 33, 1, 2, 0)])
 def test_sums_are_as_close_to_double_precision_as_fp32_ones(Cin, Cout, k, s, pad, kind):
     x, w, dy = _data(2, Cin, Cout, 16, 24, k, s, pad, kind)
     want, plain, got = _sums(x, w, dy, s, pad, torch.float64), _sums(x, w, dy, s, pad, torch.float32), _passes(x, w, dy, k, s, pad)
@@ -67,7 +68,36 @@ def test_sums_are_as_close_to_double_precision_as_fp32_ones(Cin, Cout, k, s, pad
         assert err(v, t) <= err(p, t), (name, err(v, t), err(p, t))
 
 
-@pytest.mark.parametrize("Cin,Cout,k,s,pad", [(5, 33, 3, 1, 1), (64, 64, 3, 1, 1), (16, 48, 3, 2, 1), (3, 48, 7, 2, 0)])
+@pytest.mark.parametrize("kind", ["uniform", "rectified"])
+@pytest.mark.parametrize("Cin,Cout", [(3, 64), (33, 40), (40, 33), (64, 64), (100, 64)])
+def test_persistent_workgroups_sums(Cin, Cout, kind):
+    """Layers beyond what conv_f32_patch.hip takes (2.1 M results), forward and backward-data."""
+    H = W = 96
+    N = 2100000 // (min(Cin, Cout) * H * W) + 1
+    x, w, dy = _data(N, Cin, Cout, H, W, 3, 1, 1, kind)
+    geo = (3, 3, 1, 1, 1, 1, 1, 1)
+    for name, which, t, out, M in (("fwd", capi.ADH_CONV_FWD, x, dy, Cout), ("bwd-data", capi.ADH_CONV_BWD_DATA, dy, x, Cin)):
+        assert "conv3x3_split_kernel" in capi.conv_kernel_name(which, capi.ADH_F32, 1, N, Cin, Cout, H, W)
+        f = (w if which == capi.ADH_CONV_FWD else w.transpose(0, 1).flip(2, 3)).reshape(M, -1).double()
+        sums = {}
+        for dtype in (torch.float64, torch.float32):
+            at = sums[dtype] = torch.zeros((N, M, H * W), dtype=dtype, device="cuda")
+            tp = torch.nn.functional.pad(t, (1,) * 4).double()
+            for c in range(t.shape[1]):
+                for a in range(9):
+                    col = tp[:, c, a // 3:a // 3 + H, a % 3:a % 3 + W].reshape(N, 1, -1)
+                    at.copy_((at.double() + f[None, :, c * 9 + a, None] * col).to(dtype))
+        got = torch.empty((N, M, H, W), device="cuda")
+        ws = torch.empty(capi.conv2d_unpadded_workspace_bytes(which, capi.ADH_F32, 1, N, Cin, Cout, H, W, *geo) // 4 + 64, device="cuda")
+        if which == capi.ADH_CONV_FWD:
+            capi.check(capi.conv2d_unpadded_fwd_tiles([x], w, [got], N, Cin, Cout, H, W, *geo, ws=ws), name)
+        else:
+            capi.check(capi.conv2d_unpadded_bwd_data_tiles(w, [dy], [got], N, Cin, Cout, H, W, *geo, ws=ws), name)
+        err = lambda v: ((v.double().reshape(N, M, -1) - sums[torch.float64]).norm() / sums[torch.float64].norm()).item()
+        assert err(got) <= err(sums[torch.float32]), (name, err(got), err(sums[torch.float32]))
+
+
+@pytest.mark.parametrize("Cin,Cout,k,s,pad", [(5, 33, 3, 1, 1), (64, 64, 3, 1, 1), (16, 48, 3, 2, 1), (3, 48, 7, 2, 0), (20, 48, 1, 1, 0), (70, 33, 1, 2, 0)])
 @pytest.mark.parametrize("scale", [2.0 ** -109, 2.0 ** -118])
 def test_values_near_the_smallest(Cin, Cout, k, s, pad, scale):
     """Three bf16 parts hold a value down to 2^-134: an input of 2^-110 and more whole, a smaller one to that much."""
