@@ -185,14 +185,14 @@ static int wgrad_steps(StepsWgradProblem q, const void *const *x_tiles, const vo
 // Whether conv3x3_wgrad_steps.hip is expected to be faster than conv3x3_bf16_wgrad.hip, which walks whole columns of an image 64 wide:
 // that one where such strips fill the chip and are long (64 channels on 32 images of 4 tiles of 32 x 128: 49 us against 62), the steps where they
 // do not, where channels are few or the filter is large (512 on 4 x 16: 591 -> 71), and at odd widths, which they
-// take as they are (128 on 8 images of 4 tiles of 64 x 255: 247 -> 168).  By a fifth, which is what the two models may be off (7 and
-// 10 %): 2 of 900 layers lose more than 3 % to the strips (without: 20, up to a half), and in the mean nothing is given away.
+// take as they are (128 on 8 images of 4 tiles of 64 x 255: 243 -> 165).  By 8 %, as the two models may be off by as much: 4 of 900
+// layers lose more than 3 % to the strips, up to 13 % (without: 20, up to a half), and in the mean nothing is given away.
 static bool takes_steps(const StepsWgradProblem &q) {
   const uint32_t Wd = (q.W + 7u) & ~7u;
   double strips = conv_bf16_wgrad_mfma_us(q.num_tiles, q.N, q.Cin, q.Cout, q.H, Wd);
   if (Wd != q.W) strips += 8.0 + 0.106e-6 * 4.0 * q.num_tiles * q.N * ((double)q.Cin * (q.H + 2.0) * (Wd + 2.0) + (double)q.Cout * q.H * Wd);
   const double steps = conv3x3_wgrad_steps_us(q);
-  return steps > 0.0 && 1.2 * steps < strips;
+  return steps > 0.0 && 1.08 * steps < strips;
 }
 
 // what a call has to bring

@@ -16,10 +16,9 @@
 //     plain fp32 from the pixels that exist.
 //   * The workgroups' sums are added by a second kernel in a fixed order (reproducible).
 // Measured, both kernels and, at odd widths before, the copies (before: conv3x3_bf16_wgrad.hip alone), us: 512 -> 512 channels, 32 images,
-// 4 tiles of 4 x 16 591 -> 71; 128 -> 128, 8 images, 4 tiles of 64 x 255 247 -> 168 (900 TFLOP/s); 208 -> 433, 27 images, 3 tiles of
-// 9 x 16 221 -> 54; 18 -> 16, 2 tiles of 42 x 24 43 -> 8; 300 layers of 16 to 512 channels 1.65 times as fast (geometric mean).
-// Relative error against double precision over the former kernel's: 1.0 and below in 900 layers (steps_plan; up to 1.9 while layers of several channel groups
-// had no more splits than run at once).
+// 4 tiles of 4 x 16 575 -> 147; 128 -> 128, 8 images, 4 tiles of 64 x 255 243 -> 165 (920 TFLOP/s); 208 -> 433, 27 images, 3 tiles of
+// 9 x 16 218 -> 110; 18 -> 16, 2 tiles of 42 x 24 40 -> 9; 900 layers of 16 to 512 channels 1.62 times as fast (geometric mean).
+// Relative error against double precision over the former kernel's in those: 0.61 in the mean, nowhere above 1 (steps_plan).
 // Bound: long layers by the waits between a step's LDS accesses, products and staging (two workgroups a compute unit, 40 % of the
 // matrix cores' cycles); short ones by the two launches and the sums.
 #include "conv3x3_wgrad_steps.h"
@@ -37,6 +36,7 @@ struct StepsParams : WgradSums {
   uint32_t H, W, x_H, x_W;         // a tile's dy and x
   uint32_t rows, x_rows;           // of a plane (an image; stacked: of all tiles): of dy and x
   uint32_t row_steps, cols, total_steps, ci_groups;
+  uint32_t chain;  // (HI) steps whose products go into one chain of additions
   FastDiv div_row_steps, div_cols, div_H, div_N, div_groups, div_splits;
 };
 
@@ -81,9 +81,11 @@ __device__ __forceinline__ uintx4 steps_place(uintx4 v, int32_t Q, int32_t W) {
   return v;
 }
 
-// A step: RS rows of TW columns.
-template <uint32_t TW, int OT, int WO, int WC>
-__global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW == 64u) ? 2 : OT == 2 ? 3 : 4) void conv3x3_wgrad_steps_kernel(const StepsParams P) {
+// A step: RS rows of TW columns.  HI: a chain's sums are added to others, and what that addition rounds off begins the next chain, so that
+// hi + acc is the exact sum of the chains, and a split may be of any number of them (16 output channels a wave: 72 sums and as many
+// others are more registers than there are).
+template <uint32_t TW, int OT, int WO, int WC, bool HI>
+__global__ __launch_bounds__(64 * WO * WC, HI ? 2 : OT == 4 || (OT == 2 && WC == 4 && TW == 64u) ? 2 : OT == 2 ? 3 : 4) void conv3x3_wgrad_steps_kernel(const StepsParams P) {
   constexpr uint32_t THREADS = 64u * WO * WC, CO = 16u * OT * WO, CI = 16u * WC;
   constexpr uint32_t KB = kStepBlocks, RS = KB * 32u / TW, NR = steps_ring(RS), U = TW / 8u;
   constexpr uint32_t XB = steps_x_bytes(TW, CI);
@@ -246,11 +248,29 @@ __global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW 
     }
   };
 
-  floatx4 acc[OT][9];
+  floatx4 acc[OT][9], hi[HI ? OT : 1][HI ? 9 : 1];
 #pragma unroll
   for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
-    for (int t = 0; t < 9; ++t) acc[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    for (int t = 0; t < 9; ++t) {
+      acc[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+      if constexpr (HI) hi[ot][t] = floatx4{0.f, 0.f, 0.f, 0.f};
+    }
+  uint32_t chain = P.chain;  // steps that this one still takes
+  auto link = [&]() {
+    if constexpr (HI) {
+      if (--chain != 0u) return;
+      chain = P.chain;
+#pragma unroll
+      for (int ot = 0; ot < OT; ++ot)
+#pragma unroll
+        for (int t = 0; t < 9; ++t) {
+          const floatx4 sum = hi[ot][t] + acc[ot][t];
+          acc[ot][t] -= sum - hi[ot][t];
+          hi[ot][t] = sum;
+        }
+    }
+  };
 
   // base: ring slot of the step's first x row
   auto multiply = [&](uint32_t base, uint32_t buf) {
@@ -312,6 +332,7 @@ __global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW 
     multiply(base, buf);
     __builtin_amdgcn_sched_barrier(0);
     if (k + 1u == steps) break;
+    link();
     store(next, buf ^ 1u);
     base = f.s.first ? next : next + NR - 2u;
     base -= base >= NR ? NR : 0u;
@@ -332,7 +353,10 @@ __global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW 
   for (int ot = 0; ot < OT; ++ot)
 #pragma unroll
     for (int t = 0; t < 9; ++t) {
-      const floatx4 sum = acc[ot][t];
+      floatx4 sum = acc[ot][t];
+      if constexpr (HI) {
+        sum += hi[ot][t];
+      }
       nan |= __builtin_isunordered(sum[0], sum[1]) || __builtin_isunordered(sum[2], sum[3]);
       *(ADH_GLOBAL floatx4_u *)(out + (ot * 9 + t) * 256) = sum;
     }
@@ -367,7 +391,7 @@ __global__ __launch_bounds__(64 * WO * WC, OT == 4 || (OT == 2 && WC == 4 && TW 
 
 struct StepsPlan {
   StepsParams P;
-  bool co64, ci64;
+  bool co64, ci64, hi;
   uint32_t TW, groups;
   double us;
   size_t split_bytes;  // a split's sums over all channel groups
@@ -404,14 +428,20 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
   const uint32_t co = plan->co64 ? 64u : 32u, ci = plan->ci64 ? 64u : 32u;
   P.ci_groups = (q.Cin + ci - 1u) / ci;
   const uint32_t groups = plan->groups = P.ci_groups * ((q.Cout + co - 1u) / co);
-  plan->split_bytes = (size_t)groups * co * ci * 9u * 4u;
+  const uint32_t hi_co = plan->ci64 ? 32u : co, hi_groups = P.ci_groups * ((q.Cout + hi_co - 1u) / hi_co);
+  plan->split_bytes = (size_t)groups * co * ci * 9u * 4u;  // (HI: no more)
   const uint64_t planes = (uint64_t)q.N * (q.stacked ? 1u : q.num_tiles);
   static const StepsCost costs[4] = {{1.15, 0.54, 4}, {1.55, 0.33, 2}, {1.4, 0.34, 3}, {1.8, 0.11, 2}};  // [co64][ci64]
-  const StepsCost &cost = costs[(plan->co64 ? 2 : 0) + (plan->ci64 ? 1 : 0)];
-  // The step's shape and the number of splits: the shortest expected time, steps per split going up by a quarter.  However few workgroups
-  // run at once, as many splits as conv3x3_bf16_wgrad.hip has workgroups that walk down 64 columns of images: no sum is of more
-  // pixels (four times as many are 1.9 times as far from double precision; narrow images, whose walks multiply zeros for the most
-  // part, are 1.1 times as far at as many).  Half as many pixels where enough workgroups run at once.
+  const int tile = (plan->co64 ? 2 : 0) + (plan->ci64 ? 1 : 0);
+  const StepsCost &cost = costs[tile];
+  const StepsCost linked = {1.26, 0.0, 1};  // (HI: and 0.84 a link; from 25 layers, rms error 6 %)
+  const double link_us = 0.84;
+  // The step's shape and the number of splits: the shortest expected time, steps per split going up by a quarter.  No chain of additions
+  // is of more pixels than conv3x3_bf16_wgrad.hip's, whose workgroups walk down 64 columns of images (four times as many are 1.9 times
+  // as far from double precision; narrow images, whose walks multiply zeros for the most part, are 1.1 times as far at as many):
+  // as many splits as there were walks, or, where so many don't run at once, linked chains (HI: 512 -> 512 channels on 4 tiles of 4 x 16, 32
+  // images, 486 and 150 us, relative error 4.7e-8 and 5.7e-8, by walks 576 us and 8.8e-8; with chains as long as splits 78 us and 1.8e-7).
+  // Half as many pixels where enough workgroups run at once.
   const uint64_t strips = (uint64_t)q.num_tiles * q.N * ((q.W + 63u) / 64u), rows = (strips + 255u) / 256u * q.H * (q.W > 32u ? 2u : 1u);
   const uint64_t longest = (rows + 8u) / (2u * kb);
   const uint64_t walks = std::min<uint64_t>(strips, 256u) * (q.W > 32u ? 4u : 5u) / 4u;
@@ -431,15 +461,32 @@ static bool steps_plan(const StepsWgradProblem &q, StepsPlan *plan) {
         continue;
       }
       best = us;
+      plan->hi = false;
       plan->TW = TW;
       P.splits = splits;
       P.row_steps = row_steps;
       P.cols = cols;
       P.total_steps = (uint32_t)total;
     }
+    // or no more splits than run at once, as chains of as many steps
+    if (fit <= cap || (!plan->co64 && !plan->ci64)) continue;  // (a single group of 32 x 32 channels has splits enough)
+    const uint32_t at_once = std::max(1u, std::min((uint32_t)total, 256u * linked.fit / std::min(hi_groups, 256u * linked.fit)));
+    const uint64_t per = (total + at_once - 1u) / at_once;
+    const uint32_t splits = (uint32_t)((total + per - 1u) / per);
+    const double us = steps_us({linked.step + link_us / (double)cap, linked.more, linked.fit}, TW, hi_groups, splits, (uint32_t)total, plan->split_bytes);
+    if (TW < 16u || us >= best) continue;
+    best = us;
+    plan->hi = true;
+    plan->TW = TW;
+    P.splits = splits;
+    P.row_steps = row_steps;
+    P.cols = cols;
+    P.total_steps = (uint32_t)total;
+    P.chain = (uint32_t)cap;
   }
-  if (best == 1e300 || (uint64_t)groups * P.splits >= (1ull << 22)) return false;
-  plan->us = steps_us(cost, plan->TW, groups, P.splits, P.total_steps, plan->split_bytes);
+  if (plan->hi) plan->groups = hi_groups;
+  if (best == 1e300 || (uint64_t)plan->groups * P.splits >= (1ull << 22)) return false;
+  plan->us = best;
   // From half of what the XCDs' caches hold (8 x 4 MB): 240 -> 16 channels on 4 tiles of 20 x 104, 81 MB, 85 -> 59 us, 1.08 in the mean from 32 MB,
   // 1.02 from 16; smaller ones lose 1 to 4 % (up to 16 %), as the partial sums' order suits the second kernel less.
   P.by_xcd = (uint64_t)q.num_tiles * q.N * q.H * q.W * (q.Cin + q.Cout) * 2u > (16ull << 20) ? 1u : 0u;
@@ -458,17 +505,17 @@ double conv3x3_wgrad_steps_us(const StepsWgradProblem &q) {
   return steps_plan(q, &plan) ? plan.us : 0.0;
 }
 
-template <int OT, int WO, int WC>
+template <int OT, int WO, int WC, bool HI>
 static void launch_steps(const StepsPlan &plan, hipStream_t st) {
   const dim3 grid(plan.groups * plan.P.splits), block(64 * WO * WC);
   switch (plan.TW) {
     case 64:
-      hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<64, OT, WO, WC>), grid, block, 0, st, plan.P);
+      hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<64, OT, WO, WC, HI>), grid, block, 0, st, plan.P);
       break;
-    case 32: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<32, OT, WO, WC>), grid, block, 0, st, plan.P); break;
-    case 16: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<16, OT, WO, WC>), grid, block, 0, st, plan.P); break;
+    case 32: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<32, OT, WO, WC, HI>), grid, block, 0, st, plan.P); break;
+    case 16: hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<16, OT, WO, WC, HI>), grid, block, 0, st, plan.P); break;
     default:
-      if constexpr (16 * OT * WO == 64 && WC == 4) hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<8, OT, WO, WC>), grid, block, 0, st, plan.P);
+      if constexpr (!HI && 16 * OT * WO == 64 && WC == 4) hipLaunchKernelGGL((conv3x3_wgrad_steps_kernel<8, OT, WO, WC, HI>), grid, block, 0, st, plan.P);
       break;
   }
   hipLaunchKernelGGL((wgrad_sums_kernel<9, OT, WO, WC>), dim3(plan.groups * (WO * WC * OT * 9u * 64u / 16u)), dim3(256), 0, st, static_cast<const WgradSums &>(plan.P));
@@ -485,8 +532,13 @@ int conv3x3_wgrad_steps(const StepsWgradProblem &q, void *workspace, size_t work
   }
   P.part = reinterpret_cast<float *>(workspace);
   P.dw = q.dw;
-  if (plan.co64) plan.ci64 ? launch_steps<4, 1, 4>(plan, st) : launch_steps<2, 2, 2>(plan, st);
-  else plan.ci64 ? launch_steps<2, 1, 4>(plan, st) : launch_steps<1, 2, 2>(plan, st);
+  if (plan.hi) {
+    if (plan.ci64) launch_steps<1, 2, 4, true>(plan, st);
+    else launch_steps<1, 4, 2, true>(plan, st);
+  } else {
+    if (plan.co64) plan.ci64 ? launch_steps<4, 1, 4, false>(plan, st) : launch_steps<2, 2, 2, false>(plan, st);
+    else plan.ci64 ? launch_steps<2, 1, 4, false>(plan, st) : launch_steps<1, 2, 2, false>(plan, st);
+  }
   return launch_status();
 }
 

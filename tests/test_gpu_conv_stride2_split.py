@@ -45,7 +45,9 @@ def _want(x, w, dy):
 
 @pytest.mark.parametrize("K,N,Cin,Cout,Ht,W", [
     (1, 1, 1, 1, 2, 2), (2, 3, 31, 17, 2, 10), (1, 2, 5, 70, 18, 6), (3, 1, 33, 16, 4, 626), (4, 9, 32, 65, 4, 16), (4, 5, 64, 64, 2, 8),
-    (1, 2, 65, 33, 34, 34), (2, 1, 96, 130, 16, 64), (5, 2, 16, 48, 6, 24), (2, 7, 48, 16, 14, 14), (3, 3, 512, 256, 2, 8)])
+    (1, 2, 65, 33, 34, 34), (2, 1, 96, 130, 16, 64), (5, 2, 16, 48, 6, 24), (2, 7, 48, 16, 14, 14), (3, 3, 512, 256, 2, 8),
+    # 2.1 M results and more, which conv_f32_patch.hip takes no part of: forward, backward-data
+    (2, 9, 33, 70, 58, 116), (1, 9, 4, 140, 64, 122), (2, 9, 70, 33, 58, 116), (1, 9, 140, 17, 64, 122)])
 def test_passes_vs_double_precision(K, N, Cin, Cout, Ht, W):
     x, w, dy = _inputs(N, Cin, Cout, K * Ht, W, 60 + Cin + W)
     y, g = _want(x, w, dy)
@@ -65,19 +67,19 @@ def test_sums_are_as_close_to_double_precision_as_fp32_ones():
         assert err <= max(2 * ref, 1.5e-6), (err, ref)  # 2304 terms: fp32 sums in order are 1e-6 off
 
 
+@pytest.mark.parametrize("N,C,H,W", [(1, 40, 10, 20), (16, 44, 100, 128)])  # the second beyond what conv_f32_patch.hip takes
 @pytest.mark.parametrize("bad", [float("inf"), -float("inf"), 3.4e38, float("nan")])
-def test_values_without_finite_bf16_parts(bad):
+def test_values_without_finite_bf16_parts(bad, N, C, H, W):
     """What an infinity or a number that rounds to an infinite bf16 touches is what plain sums over the zero-padded tensor give."""
-    N, C, H, W = 1, 40, 10, 20
     x, w, dy = _inputs(N, C, C, H, W, 3)
-    x, w, dy = x.abs() + 0.5, w.abs() + 0.01, dy.abs() + 0.5
+    x, w, dy = (x.abs() + 0.5).cuda(), (w.abs() + 0.01).cuda(), (dy.abs() + 0.5).cuda()
     for where in ("data", "filter"):
         xb, wb, db = x.clone(), w.clone(), dy.clone()
         if where == "data":
             xb[0, 3, 4, 10] = db[0, 3, 2, 7] = bad
         else:
             wb[5, 7, 1, 2] = bad
-        y, g = torch.zeros((N, C, H // 2, W // 2)), torch.zeros((N, C, H + 2, W + 2))
+        y, g = torch.zeros((N, C, H // 2, W // 2), device="cuda"), torch.zeros((N, C, H + 2, W + 2), device="cuda")
         xp, dp = torch.nn.functional.pad(xb, (1, 1, 1, 1)), torch.nn.functional.pad(db, (0, 1, 0, 1))
         for a in range(3):
             for b in range(3):
@@ -85,7 +87,6 @@ def test_values_without_finite_bf16_parts(bad):
                 # gradient row 2i + a - 1 from gradient row i: quads past the last one read the zero padding, as data
                 g[:, :, a:a + H + 1:2, b:b + W + 1:2] += (dp[:, :, None] * wb[None, :, :, a, b, None, None]).sum(1)[..., :(H + 3 - a) // 2, :(W + 3 - b) // 2]
         for got, want in zip(_passes(xb, wb, db, 1), (y, g[:, :, 1:-1, 1:-1])):
-            got = got.cpu()
             assert torch.equal(torch.isnan(got), torch.isnan(want))
             assert torch.equal(torch.isinf(got), torch.isinf(want))
             fine = torch.isfinite(want)

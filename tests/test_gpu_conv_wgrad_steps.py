@@ -125,8 +125,39 @@ def _error(K, N, Ci, Co, H, W):
     return ((dw.double() - want).norm() / want.norm()).item()
 
 
-@pytest.mark.parametrize("shape,walks", [((3, 7, 263, 135, 11, 272), 1.58e-7), ((7, 31, 103, 287, 13, 50), 1.64e-7), ((8, 24, 48, 256, 10, 170), 2.27e-7)])
-def test_sums_of_no_more_pixels_than_walks_down_64_columns(shape, walks):
-    """Layers of several channel groups, of which few splits run at once.  walks: the error of conv3x3_bf16_wgrad.hip's sums (measured; 2.48e-7, 3.16e-7
-    and 2.39e-7 where the splits are as many as run at once)."""
+@pytest.mark.parametrize("shape,walks", [((3, 7, 263, 135, 11, 272), 1.58e-7), ((7, 31, 103, 287, 13, 50), 1.64e-7), ((8, 24, 48, 256, 10, 170), 2.27e-7),
+                                         ((6, 3, 339, 228, 5, 342), 1.18e-7), ((5, 25, 38, 377, 3, 295), 1.46e-7)])
+def test_chains_of_no_more_pixels_than_walks_down_64_columns(shape, walks):
+    """Layers of several channel groups, of which few splits run at once.  walks: the error of conv3x3_bf16_wgrad.hip's sums (measured; 2.48e-7,
+    3.16e-7, 2.39e-7, 2.19e-7 and 2.09e-7 with chains as long as such splits)."""
     assert _error(*shape) <= 1.02 * walks
+
+
+# (few rows and many channels: chains of 1, 2, 3, 4 and 5 steps, one group of 32 channels on either side, groups and splits that are not full)
+LINKED = [(8, 6, 206, 148, 3, 29), (6, 23, 54, 226, 3, 79), (3, 21, 128, 32, 2, 507), (4, 17, 16, 256, 2, 92), (6, 2, 85, 203, 4, 551), (8, 11, 29, 212, 5, 145),
+          (7, 22, 375, 95, 4, 12)]
+
+
+@pytest.mark.parametrize("shape", LINKED)
+def test_linked_chains(shape):
+    # the rounding of a split's sum and of the result (2^-24 each), and of chains of at most 1024 pixels, 32 of an addition
+    assert _error(*shape) <= 2.0 ** -24 * (2 + 32 / 3) ** 0.5
+
+
+@pytest.mark.parametrize("shape", [LINKED[1], LINKED[2], LINKED[3]])
+@pytest.mark.parametrize("value", [float("nan"), float("inf"), -float("inf"), 3e38])
+def test_not_finite_values_in_linked_chains(shape, value):
+    """What is not finite, or becomes so in a chain, is summed again in plain fp32."""
+    K, N, Ci, Co, H, W = shape
+    x, dy = _tensors(K, N, Ci, Co, H, W, False, 3)
+    x[1, 3, 2, 5] = value
+    x[-1, 7, 1, 40] = value
+    got, want = _run(x, dy, K, False, beta=1.0), _reference(x, dy, K, False)
+    if value == 3e38:
+        want = torch.where(want.abs() > 3.4e38, want.sign() * float("inf"), want)
+    assert torch.equal(got.isnan(), want.isnan())
+    sure = want.isinf() if value != 3e38 else want.abs() > 1e39
+    assert torch.equal(got[sure], want[sure])
+    fine = want.abs() < 1e30
+    assert fine.any() and not fine.all()
+    assert (got - want)[fine].norm() <= 1e-6 * want[fine].norm()
