@@ -89,10 +89,10 @@ __device__ __forceinline__ float2 block_sum2(float a, float b) {
 // VEC > 1: H*W (and, backward, W) are whole numbers of VEC-element groups, one 16-byte access per group.
 // U groups a thread are loaded before the first is added (with one, the latency of a load bounds it), and are added in the
 // order of a thread that takes one at a time: what a sum rounds to decides where activations tie in a pooling window.
-template <typename T, bool BWD, int VEC, bool STREAM>
+// (U = 1 where a split has no U groups a thread: 136 channels of 1 x 46 on 8 tiles, 3 images, 4.2 us, with 8 5.6)
+template <typename T, bool BWD, int VEC, int U, bool STREAM>
 __global__ __launch_bounds__(kBnThreads) void bn_reduce_kernel(const BnParams P) {
   typedef BnVec<T, VEC> Vec;
-  constexpr int U = VEC > 1 ? 4 : 8;
   uint32_t tc, sp, tile, c;
   P.div_split.divmod(blockIdx.x, tc, sp);
   P.div_C.divmod(tc, tile, c);
@@ -479,9 +479,15 @@ static void bn_items(BnParams *P, uint32_t items, uint32_t rows) {
 
 // The backward apply pass: a plane is `runs` runs of `run` elements, each moved as groups of `vec`.  False: one element at a
 // time, where the last groups, stored element by element, are more than an eighth of all (5.6 us against 8.9 over bf16
-// planes of 22).
+// planes of 22), and, at row lengths that are no whole groups, where groups would be less than a workgroup per compute unit (140 tensors:
+// 1.04 to 1.17 times as long by groups, up to 1.4; from 256 workgroups on 0.92, from 512 0.82).
 static bool bn_runs(BnParams *P, uint32_t run, uint32_t runs, uint32_t vec) {
-  const bool wide = run % vec == 0u || run >= 8u * vec;
+  bool wide = run % vec == 0u || run >= 8u * vec;
+  if (wide && P->W % vec != 0u) {
+    BnParams Q = *P;
+    const dim3 grid = bn_apply_grid(&Q, (run + vec - 1u) / vec * runs, true);
+    wide = (uint64_t)grid.x * grid.y >= 256u;
+  }
   const uint32_t groups = wide ? (run + vec - 1u) / vec : run;
   P->run = run;
   P->groups_per_plane = groups * runs;
@@ -491,6 +497,15 @@ static bool bn_runs(BnParams *P, uint32_t run, uint32_t runs, uint32_t vec) {
 
 // `bytes`: what a pass reads.  Non-temporal where the on-package cache (256 MB) cannot keep it for the second pass.
 static bool bn_stream(uint64_t bytes) { return bytes > (256ull << 20); }
+
+template <typename T, bool BWD, int VEC, bool STREAM>
+static void bn_reduce(const BnParams &P, dim3 grid, hipStream_t st) {
+  constexpr int U = VEC > 1 ? 4 : 8;
+  if ((uint64_t)P.n_per_split * P.div_groups.d >= (uint64_t)U * kBnThreads)
+    hipLaunchKernelGGL((bn_reduce_kernel<T, BWD, VEC, U, STREAM>), grid, dim3(kBnThreads), 0, st, P);
+  else
+    hipLaunchKernelGGL((bn_reduce_kernel<T, BWD, VEC, 1, false>), grid, dim3(kBnThreads), 0, st, P);
+}
 
 template <typename F>
 static void bn_launch(bool stream_data, int dtype, F f) {
@@ -559,8 +574,8 @@ int adh_batchnorm2d_fwd_tiles(int dtype, int training, uint32_t num_tiles, uint3
     bn_items(&P, H * W / (wide ? vec : 1u), 1u);
     bn_launch(stream_data, dtype, [&](auto s, auto t) {
       typedef decltype(t) T;
-      if (wide) hipLaunchKernelGGL((bn_reduce_kernel<T, false, 16 / sizeof(T), s>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
-      else hipLaunchKernelGGL((bn_reduce_kernel<T, false, 1, false>), dim3(tc * P.split), dim3(kBnThreads), 0, st, P);
+      if (wide) bn_reduce<T, false, 16 / sizeof(T), s>(P, dim3(tc * P.split), st);
+      else bn_reduce<T, false, 1, false>(P, dim3(tc * P.split), st);
     });
   }
   P.div_cols = FastDiv(W + 2u * out_halo);  // the apply kernel walks the padded output plane
@@ -620,8 +635,8 @@ int adh_batchnorm2d_bwd_tiles(int dtype, uint32_t num_tiles, uint32_t N, uint32_
   const dim3 rgrid(tc * P.split);
   bn_launch(stream_data, dtype, [&](auto s, auto t) {
     typedef decltype(t) T;
-    if (rwide) hipLaunchKernelGGL((bn_reduce_kernel<T, true, 16 / sizeof(T), s>), rgrid, dim3(kBnThreads), 0, st, P);
-    else hipLaunchKernelGGL((bn_reduce_kernel<T, true, 1, false>), rgrid, dim3(kBnThreads), 0, st, P);
+    if (rwide) bn_reduce<T, true, 16 / sizeof(T), s>(P, rgrid, st);
+    else bn_reduce<T, true, 1, false>(P, rgrid, st);
   });
   P.div_cols = apply_cols;
   const dim3 agrid = bn_apply_grid(&P, apply_groups, true);

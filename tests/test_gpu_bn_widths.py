@@ -73,6 +73,26 @@ def test_gradient_over_its_input(dtype, H, W):
     _run(dtype, 2, 3, 5, H, W, over_dy=True)
 
 
+def _many(H, W, dtype):
+    """Channels of 2 tiles of 16 images that are more than a workgroup per compute unit by 16-byte groups (as the apply pass deals them)."""
+    groups = -(-H * W // (4 if dtype is torch.float32 else 8))
+    threads = 256 if groups > 128 else max(16, 1 << (groups - 1).bit_length())
+    return 256 * 4 * (256 // threads) // 32 + 3
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,W", [(5, 13), (1, 65), (2, 33), (4, 129), (64, 67), (3, 257)])
+@pytest.mark.parametrize("p,beta", [(0, 0.0), (0, 1.0), (1, 1.0)])
+def test_lengths_by_groups(dtype, H, W, p, beta):
+    _run(dtype, 2, 16, _many(H, W, dtype), H, W, p, beta)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("H,W", [(5, 13), (4, 129), (64, 67)])
+def test_gradient_over_its_input_by_groups(dtype, H, W):
+    _run(dtype, 2, 16, _many(H, W, dtype), H, W, over_dy=True)
+
+
 @pytest.mark.parametrize("K,N,C", [(1, 37, 1), (1, 70, 3), (2, 9, 130)])
 def test_splits(K, N, C):
     _run(torch.float32, K, N, C, 6, 11)
