@@ -679,7 +679,7 @@ def main():
                                                                        gwu.data_ptr(), 0.0, wsu.data_ptr(), wsb, stream)
             add("conv fwd over tiles without halo, fp32, N=32, 4 tiles: " + nm, f, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
             add("conv bwd-data into tiles without halo, fp32: " + nm, b, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
-            add("conv bwd-filter over tiles without halo, fp32: " + nm, wgf, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS if su == 1 else MFMA_F32_PEAK_TFLOPS, "TFLOP/s")
+            add("conv bwd-filter over tiles without halo, fp32: " + nm, wgf, "mfma", flop, MFMA_SPLIT_PEAK_TFLOPS, "TFLOP/s")
             del xu, yu, wu_, gwu, wsu
         # the 1x1 stride-2 projection shortcuts of the same net (matrix-product kernels of their own): the first is
         # sized by memory (priced by the bytes of the pixels it uses and writes), the third by the matrix cores
