@@ -184,7 +184,7 @@ static int wgrad_steps(StepsWgradProblem q, const void *const *x_tiles, const vo
 }
 // Whether conv3x3_wgrad_steps.hip is expected to be faster than conv3x3_bf16_wgrad.hip, which walks whole columns of an image 64 wide:
 // that one where such strips fill the chip and are long (64 channels on 32 images of 4 tiles of 32 x 128: 49 us against 62), the steps where they
-// do not, where channels are few or the filter is large (512 on 4 x 16: 591 -> 71), and at odd widths, which they
+// do not, where channels are few or the filter is large (512 on 4 x 16: 575 -> 147), and at odd widths, which they
 // take as they are (128 on 8 images of 4 tiles of 64 x 255: 243 -> 165).  By 8 %, as the two models may be off by as much: 4 of 900
 // layers lose more than 3 % to the strips, up to 13 % (without: 20, up to a half), and in the mean nothing is given away.
 static bool takes_steps(const StepsWgradProblem &q) {

@@ -100,7 +100,8 @@ struct SplitBlock {
 // LOW.  Six products of parts go into a sum per tap and chunk, and each addition is rounded at the size of the sum; all but h*h
 // are below 2^-8 of it.  kLowApart: they have sums of their own, added at the block's end, and cost no digit.  Where registers
 // are short, the small products of LOW of the nine taps are summed up from zero and added at once; 0: every product is added
-// by itself.  The choice hangs on the channels alone, so that all tiles give the same bits (split_low).
+// by itself.  The choice hangs on the channels alone, not on the block's shape or the images it holds (split_low); small launches go
+// to conv_f32_patch.hip, which adds in another order: the forms of one layer have the same bits, not a layer and a part of it.
 template <int MT, int NT, bool VEC, int SAMPLE, int LOW>
 __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const SplitParams P) {
   constexpr uint32_t MW = 16u * MT;
