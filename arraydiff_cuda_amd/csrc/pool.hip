@@ -884,8 +884,10 @@ __global__ __launch_bounds__(kPoolThreads) void pool_bwd_max3s2_kernel(const Poo
 //   * the smallest tensors, a thread's chain of loads being longer than a band's (16 to 20 k pixels: 4.1 us a pass there, 5 to 9 here;
 //     72 k: the other way round; backward, where bands would stage element by element or not: rows of whole groups of four 4.9 us here at
 //     15 k pixels, 5.3 there);
-//   * forward, fp32 tensors larger than the on-package cache in long rows of whole 16-byte groups (64 x 260: 133 us there, 158 here; 64 x 700
-//     177 and 206; 64 x 256 130 and 132; but 64 x 128 158 and 117, 64 x 222 262 and 132).
+//   * forward, fp32 tensors larger than the on-package cache in long rows of whole 16-byte groups that are no whole lines of 128 bytes
+//     (64 x 260: 134 us there, 159 here; 64 x 700 136 and 157; but 64 x 128 158 and 117, 64 x 222 262 and 132; off 16 bytes 64 x 260
+//     292 and 160).  Rows of whole lines stay here: over and over on one tensor 64 x 192 takes 101 and 109, 64 x 256 132 and 134, 64 x 384 108 and
+//     106, but within a training step 179 and 175 (64 images, 3 tiles), 164 and 145, 187 and 176 (16 images, 6 tiles).
 // bf16: eight columns a thread are 16 bytes; four where only that many are whole groups (64 x 516: backward 355 us, 383 by eights), and for
 // tensors below 24 MB, which want the threads (5 x 29 x 141 planes of 8 x 12: 7.1 us, 11.3; 7 x 31 x 72 of 14 x 63, 28 MB, 25.6 and 26.8).
 // Non-temporal accesses where the input is larger than the cache and the rows are whole lines of 128 bytes (fp32 64 x 256: backward 234
@@ -900,7 +902,7 @@ static bool pool_max3s2(const PoolParams &P, size_t es, bool fwd, PoolS2Params *
   const uint64_t items = (uint64_t)P.planes * groups;
   if (items >= (1ull << 31) || rows >= (1ull << 31)) return false;
   if (pixels < (1u << 15) && (fwd || P.W % 4u != 0u)) return false;
-  if (fwd && es == 4u && large && P.W % 4u == 0u && P.W >= 160u) return false;
+  if (fwd && es == 4u && large && P.x_vec != 0u && P.W % 32u != 0u && P.W >= 160u) return false;
   q->stream = large && (P.W * es % 128u == 0u || (fwd ? es == 2u : P.W % nc != 0u));
   for (uint32_t t = 0; t < P.num_tiles; ++t) {
     q->x[t] = P.x[t]; q->dy[t] = P.dy[t]; q->out[t] = P.out[t];

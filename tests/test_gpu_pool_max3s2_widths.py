@@ -92,3 +92,42 @@ def test_eight_columns_a_thread(W):
     for n in range(N):
         y1, dx1 = run(x[n:n + 1], dy[n:n + 1], old[n:n + 1])
         assert _same(y[n:n + 1], y1) and _same(dx[n:n + 1], dx1)
+
+
+@pytest.mark.parametrize("W", [256, 260])
+@pytest.mark.parametrize("offset", [0, 1])
+def test_larger_than_the_cache_at_any_alignment(W, offset):
+    """Forward, fp32, rows of whole lines and of whole 16-byte groups: off 16 bytes the same bits as image by image, and no more
+    than 1.7 times as long (1.1 and 1.2 without LDS; the bands, which would stage element by element, 2.1 times)."""
+    N, C, Ht, K = 18, 64, 64, 4
+
+    def off(t, by):
+        flat = torch.empty(t.numel() + 4, device="cuda")[by:by + t.numel()].view(t.shape)
+        return flat.copy_(t)
+
+    def run(xs, ys):
+        capi.check(capi.pool_unpadded_fwd_tiles(capi.ADH_POOL_MAX, xs, ys, xs[0].shape[0], C, Ht, W, *WINDOW, 1, 1), "forward")
+
+    def fastest(xs, ys):
+        run(xs, ys)
+        events = [(torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)) for _ in range(10)]
+        for a, b in events:
+            a.record()
+            run(xs, ys)
+            b.record()
+        torch.cuda.synchronize()
+        return min(a.elapsed_time(b) for a, b in events)
+
+    x, _ = _inputs(torch.float32, K, N, C, Ht, W, 5)
+    assert x.numel() * 4 > 256 << 20
+    aligned = [t.contiguous() for t in x.chunk(K, 2)]
+    xs = [off(t, offset) for t in aligned]
+    ys = [off(torch.full((N, C, Ht // 2, W // 2), 7.0, device="cuda"), offset) for _ in xs]
+    run(xs, ys)
+    for n in range(0, N, 5):
+        small = [t[n:n + 1].contiguous() for t in aligned]
+        y1 = [torch.empty_like(y[n:n + 1]).contiguous() for y in ys]
+        run(small, y1)
+        assert all(_same(ys[t][n:n + 1], y1[t]) for t in range(K))
+    if offset:
+        assert fastest(xs, ys) < 1.7 * fastest(aligned, [torch.empty_like(y).contiguous() for y in ys])
