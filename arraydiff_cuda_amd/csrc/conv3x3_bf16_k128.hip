@@ -51,7 +51,9 @@ static __device__ __forceinline__ uint32_t k2_wrap(uint32_t s) { return s >= (ui
 // P.part and added.  POUT: the sums go to P.part as fp32 instead of to the output as bf16 (a later pass follows).
 // HF (P.pad == 1): neither the input nor the output carries a halo; rows -1 and IH come from the neighbouring
 // tiles (P.neighbour_rows), and a row is staged from eight columns left of the strip in six granules.
-template <bool BETA, bool PIN, bool POUT, bool HF>
+// ROWS: 0, every input row starts on a 4-byte boundary (pad 0) or on 16 bytes and is whole granules; kOddRows (forward) and kAnyRows
+// (backward-data): conv3x3_bf16_mfma.h.
+template <bool BETA, bool PIN, bool POUT, bool HF, int ROWS = 0>
 __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf16Params P) {
   static_assert(!(BETA && PIN), "the old output is added in the first pass, which reads no sums");
   constexpr int G = HF ? 6 : 5;                 // granules of a staged row = copies per row group
@@ -125,6 +127,9 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
   // padded slab); the ring holds staged pixels xoff .. xoff + 33 as its pixels 0 .. 33
   const int32_t xoff = P.pad ? 8 - P.pad : 0;
   const int32_t col_back = P.pad ? 8 : 0;
+  // odd rows of an odd width are staged from one element back (forward) or on (backward-data): their ring pixel is that
+  // much further on
+  const int32_t odd_px = ROWS == kOddRows ? -1 : ROWS == kAnyRows ? (int32_t)(P.IW & 1u) : 0;
 
   // ---- requests: copy q of a group moves staging slots 64 q + lane; slot = (row * 16 + channel) * G + granule
   uint32_t ld_off[6];  // G of them are used
@@ -136,7 +141,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
     const uint32_t row = slot / (16u * G), rem = slot - row * (16u * G), ch = rem / (uint32_t)G, gran = rem - ch * (uint32_t)G;
     const uint32_t chan = 16u * wv + ch;
     const bool ok = chan < P.cred_pass;
-    ld_off[q] = (P.chan0 + chan) * plane_bytes + row * P.IW * 2u + gran * 16u;
+    ld_off[q] = (P.chan0 + chan) * plane_bytes + row * P.IW * 2u + gran * 16u + (ROWS && (row & 1u) ? (uint32_t)(odd_px * 2) : 0u);
     ld_rows |= ((row & 3u) | (ok ? 4u : 0u)) << (3 * q);
     ld_gran |= gran << (3 * q);
   }
@@ -168,20 +173,26 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
     T.lo = k2_read_tr(src);
     T.hi = k2_read_tr(src + 4 * kChanBytes);
   };
+  int32_t colT = 0;  // input column of staged pixel 0 of the group to transpose
   auto tr_write = [&](auto tag, const TrPair &T) {
     constexpr int t = decltype(tag)::value;
-    const u32x4 v = {T.lo[0], T.lo[1], T.hi[0], T.hi[1]};
+    u32x4 v = {T.lo[0], T.lo[1], T.hi[0], T.hi[1]};
     int32_t px;
     uint32_t row;
     if constexpr (HF) {
       px = (t % 3) * 16 + (int32_t)l16 - xoff;
       row = 2u * (t / 3) + (g >> 1);
     } else if constexpr (t < 4) {
-      px = (int32_t)((g >> 1) * 16u + l16) - xoff;
+      px = (int32_t)((g >> 1) * 16u + l16) - xoff + (t & 1 ? odd_px : 0);
       row = (uint32_t)t;
     } else {
-      px = 32 + (int32_t)(l16 & 7u) - xoff;
+      px = 32 + (int32_t)(l16 & 7u) - xoff + (ROWS && l16 >= 8u ? odd_px : 0);
       row = 2u * (g >> 1) + (l16 >> 3);
+    }
+    if constexpr (ROWS == kAnyRows) {  // granules that straddle the row's ends hold the neighbouring rows' pixels
+      const bool inside = (uint32_t)(colT + xoff + px) < P.IW;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = inside ? v[j] : 0u;
     }
     uint8_t *const dst = ring + k2_wrap(tb + row) * kK2RowBytes + (uint32_t)px * kK2PxBytes + wr_chan;
     *reinterpret_cast<u32x4 *>((px >= 0 && px < kK2RowPx) ? dst : wr_dummy) = v;
@@ -235,7 +246,9 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
 #pragma unroll
     for (int q = 0; q < G; ++q) {
       const int32_t col = colL + 8 * (int32_t)((ld_gran >> (3 * q)) & 7u);
-      const bool ok = ((ld_rows >> (3 * q)) & 4u) && col >= 0 && col < (int32_t)P.IW;
+      // (backward-data: the granule left of an odd row that is staged one element on ends with the row's first pixel)
+      const int32_t first = ROWS == kAnyRows && (ld_rows >> (3 * q) & 1u) ? -8 * odd_px : 0;
+      const bool ok = ((ld_rows >> (3 * q)) & 4u) && col >= first && col < (int32_t)P.IW;
       okL |= (ok ? 1u : 0u) << q;
     }
     grpL = -1;
@@ -542,6 +555,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
   uint32_t sb = 4;  // ring slot of the first input row of the step multiplied in this phase
   loader_open();
   for_each_int(std::make_integer_sequence<int, G>(), [&](auto tag) { request(tag, IntTag<HF ? 1 : 0>()); });
+  colT = colL;
   loader_advance();
   auto phase_barrier = [&]() {
     __builtin_amdgcn_s_waitcnt(0xC07F);  // lgkmcnt(0): LDS only
@@ -572,6 +586,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
       phase_barrier();
       after_plain = true;
     }
+    colT = colL;
     loader_advance();
     sb = k2_wrap(sb + kStepRows);
     tb = k2_wrap(tb + kStepRows);
@@ -595,10 +610,15 @@ bool conv_bf16_k128_takes(const ConvBf16Params &P, uint32_t num_tiles) {
 int conv_bf16_k128_launch(const ConvBf16Params &P, uint32_t gx, uint32_t groups128, hipStream_t st) {
   const dim3 grid(gx, groups128), block(kK2Threads);
   const bool first = P.first_pass != 0u, last = P.last_pass != 0u, beta = P.beta != 0.f;
+  const int rows = conv_bf16_rows(P);
 #define ADH_K128(B, PI, PO)                                                                                       \
   do {                                                                                                            \
     if (P.pad == 1)                                                                                               \
       hipLaunchKernelGGL((conv3x3_bf16_k128_kernel<B, PI, PO, true>), grid, block, 0, st, P);                     \
+    else if (rows == kOddRows)                                                                                    \
+      hipLaunchKernelGGL((conv3x3_bf16_k128_kernel<B, PI, PO, false, kOddRows>), grid, block, 0, st, P);          \
+    else if (rows == kAnyRows)                                                                                    \
+      hipLaunchKernelGGL((conv3x3_bf16_k128_kernel<B, PI, PO, false, kAnyRows>), grid, block, 0, st, P);          \
     else                                                                                                          \
       hipLaunchKernelGGL((conv3x3_bf16_k128_kernel<B, PI, PO, false>), grid, block, 0, st, P);                    \
   } while (0)

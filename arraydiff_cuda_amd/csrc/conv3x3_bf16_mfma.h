@@ -64,6 +64,20 @@ __device__ __forceinline__ uint32_t pack_bf16x2(float a, float b) {
   return __builtin_bit_cast(uint32_t, __builtin_convertvector(f, bf16x2));
 }
 
+// How the eight-wave kernels stage rows that start anywhere.  A copy to LDS needs 4-byte alignment.  At an odd width every other
+// row is 2 bytes off it; with an even height the same ones in every channel and image (a group of four rows begins with an even one).
+//   kOddRows (forward, odd width): odd rows are staged from one element back, and written to the ring one pixel back.
+//   kAnyRows (backward-data, a width that is no whole granules): odd rows of an odd width are staged from one element on (staging
+//   begins eight columns left of the strip and has six to spare); pixels outside the row, which share granules with it, are zeroed
+//   on their way to the ring.
+constexpr int kNoRows = -1, kOddRows = 1, kAnyRows = 2;
+inline int conv_bf16_rows(int32_t pad, uint32_t IH, uint32_t IW) {
+  if (pad ? IW % 8u == 0u : IW % 2u == 0u) return 0;
+  if (pad == 0) return IH % 2u == 0u ? kOddRows : kNoRows;
+  return pad == 2 && IW >= 8u && (IH % 2u == 0u || IW % 2u == 0u) ? kAnyRows : kNoRows;
+}
+inline int conv_bf16_rows(const ConvBf16Params &P) { return conv_bf16_rows(P.pad, P.IH, P.IW); }
+
 // the eight-wave kernel: shapes it takes, and its launch (grid.x workgroups per output group)
 bool conv_bf16_w8_takes(const ConvBf16Params &P, uint32_t num_tiles);
 // launches the pass of up to 64 reduction channels from P.chan0 on

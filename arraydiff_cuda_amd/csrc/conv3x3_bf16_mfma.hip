@@ -561,9 +561,9 @@ static int num_cus() {
 
 // Up to 64 reduction channels: any shape.  More: several launches with fp32 sums between them, which the
 // eight-wave kernels address through a buffer resource: the sums of one image have to lie inside 2 GiB.
-// (The eight-wave kernels need input rows on a 4-byte boundary (forward: even width) or whole 16-byte granules
-// (backward-data: a width that is a multiple of 8) and aligned tiles; at other widths they run over a copy of the
-// input with wider rows.  The four-wave kernel, once per 64 reduction channels, takes what is left.)
+// (The eight-wave kernels need aligned tiles, and an odd width an even height (conv_bf16_rows).  Where those are missing and more than 64
+// channels are summed they run over a copy of the input with wider rows.  The four-wave kernel, once per 64 reduction channels,
+// takes what is left.)
 bool conv_bf16_mfma_supported(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W) {
   const uint32_t cred = which == ADH_CONV_FWD ? Cin : Cout;
   if (cred <= 64u) return true;
@@ -571,9 +571,13 @@ bool conv_bf16_mfma_supported(int which, uint32_t Cin, uint32_t Cout, uint32_t H
   const uint64_t oh = which == ADH_CONV_FWD ? H : H + 2ull, ow = which == ADH_CONV_FWD ? W : W + 2ull;
   return cout_k * oh * ow * 4u < (1ull << 31);
 }
-// widths whose rows the eight-wave kernels take
+// widths whose rows the eight-wave kernels stage as whole 4-byte (backward-data: 16-byte) pieces, at any height and, forward, alignment
 static bool conv_bf16_w8_width(int which, uint32_t W) { return which == ADH_CONV_FWD ? (W % 2u) == 0u : (W % 8u) == 0u; }
-// At the other widths the input is copied into rows of the next multiple of 8, zeros behind, and the eight-wave kernels
+// other shapes whose rows they stage as they lie, from tiles on 16 bytes (128 -> 128 channels, 8 images of 4 tiles of 64x255, over copies before:
+// forward 233 -> 178 us, backward-data 209 -> 166; 64 -> 64, 2 images of 8 tiles of 128x1023, by the four-wave kernel before: 261 -> 198 and
+// 208 -> 194)
+static bool conv_bf16_any_rows(int which, uint32_t H, uint32_t W) { return (which == ADH_CONV_FWD ? conv_bf16_rows(0, H + 2u, W + 2u) : conv_bf16_rows(2, H, W)) > 0; }
+// Elsewhere the input is copied into rows of the next multiple of 8, zeros behind, and the eight-wave kernels
 // run on the copy: where more than 64 channels are summed, which the four-wave kernel takes in one launch per 64 with
 // fp32 sums through memory (128 -> 128 channels, 8 images of 4 tiles of 64x255: forward 455 -> 212 us, backward-data
 // 357 -> 199, the copy included; 512 -> 512, 4 images of 14x13: 258 -> 125).  Up to 64 channels the copy costs what the
@@ -594,11 +598,10 @@ static uint32_t conv_bf16_passes(int which, uint32_t Cin, uint32_t Cout) {
 // conv3x3_bf16_k128.hip while more than 64 are left, then at most 64 by the eight-wave kernel.  Otherwise one
 // launch of the eight-wave kernel per 64.
 static bool conv_bf16_uses_k128(int which, uint32_t Cin, uint32_t Cout) { return Cin > 64u && Cout > 64u; }
-// (a width the eight-wave kernels do not take: one launch of the four-wave kernel per 64)
-static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, bool may_copy = true) {
+// (not by the eight-wave kernels: one launch of the four-wave kernel per 64)
+static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, bool eight_waves) {
   const uint32_t cred = which == ADH_CONV_FWD ? Cin : Cout;
-  if (!conv_bf16_uses_k128(which, Cin, Cout) || !(conv_bf16_w8_width(which, W) || (may_copy && conv_bf16_repitches(which, Cin, Cout, H, W))))
-    return (cred + 63u) / 64u;
+  if (!conv_bf16_uses_k128(which, Cin, Cout) || !eight_waves) return (cred + 63u) / 64u;
   uint32_t n = 0, rem = cred;
   while (rem > 64u) {
     rem -= rem < 128u ? rem : 128u;
@@ -608,17 +611,18 @@ static uint32_t conv_bf16_launches(int which, uint32_t Cin, uint32_t Cout, uint3
 }
 
 // name of the kernel a bf16 forward / backward-data call over padded tiles runs, for tiles aligned to 16 bytes
-// (template arguments: old output added, sums of earlier passes read, sums written for a later pass, tiles without halo)
+// (template arguments: old output added, sums of earlier passes read, sums written for a later pass, tiles without halo; the last one,
+// how rows are staged, is left out)
 const char *conv_bf16_kernel_name(int which, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, float beta) {
   if (!conv_bf16_mfma_supported(which, Cin, Cout, H, W)) return "widen_bf16_kernel + conv3x3_split_kernel + narrow_bf16_kernel";
-  if (!conv_bf16_w8_width(which, W) && !conv_bf16_repitches(which, Cin, Cout, H, W)) {
+  if (!conv_bf16_w8_width(which, W) && !conv_bf16_any_rows(which, H, W) && !conv_bf16_repitches(which, Cin, Cout, H, W)) {
     if (conv_bf16_passes(which, Cin, Cout) > 1u)
       return beta != 0.f ? "conv3x3_bf16_kernel<true, false, true> + <false, true, true> per middle 64 reduction channels + <false, true, false>"
                          : "conv3x3_bf16_kernel<false, false, true> + <false, true, true> per middle 64 reduction channels + <false, true, false>";
     return beta != 0.f ? "conv3x3_bf16_kernel<true, false, false>" : "conv3x3_bf16_kernel<false, false, false>";
   }
   if (conv_bf16_uses_k128(which, Cin, Cout)) {
-    if (conv_bf16_launches(which, Cin, Cout, H, W) == 1u)
+    if (conv_bf16_launches(which, Cin, Cout, true) == 1u)
       return beta != 0.f ? "conv3x3_bf16_k128_kernel<true, false, false, false>" : "conv3x3_bf16_k128_kernel<false, false, false, false>";
     return "conv3x3_bf16_k128_kernel per 128 reduction channels (fp32 sums between the launches) + conv3x3_bf16_w8_kernel for a rest of at most 64";
   }
@@ -669,7 +673,7 @@ struct CopyTurn {
 };
 static CopyTurn conv_bf16_copy_turn(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                                     uint64_t room) {
-  const bool sums = conv_bf16_launches(which, Cin, Cout, H, W) > 1u;
+  const bool sums = conv_bf16_launches(which, Cin, Cout, true) > 1u;
   auto bytes = [&](uint32_t images) {
     return (uint64_t)conv_bf16_repitch_bytes(which, images, Cin, Cout, H, W) + (sums ? part_region_bytes(which, images, Cin, Cout, H, W) : 0u);
   };
@@ -684,10 +688,11 @@ static CopyTurn conv_bf16_copy_turn(int which, uint32_t num_tiles, uint32_t N, u
   t.bytes = t.tiles * bytes(t.images);
   return t;
 }
-// may_copy: with room for copies of the input with wider rows where there is a route over them
+// may_copy: with room for copies of the input with wider rows where there is a route over them (tiles off 16 bytes need them also
+// where rows are staged as they lie otherwise)
 size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H,
                                       uint32_t W, bool may_copy) {
-  size_t bytes = conv_bf16_launches(which, Cin, Cout, H, W, false) > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : (size_t)0;
+  size_t bytes = conv_bf16_launches(which, Cin, Cout, conv_bf16_w8_width(which, W)) > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : (size_t)0;
   if (may_copy && conv_bf16_repitches(which, Cin, Cout, H, W))
     bytes = std::max<size_t>(bytes, conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, kMostCopies).bytes);
   return filter_region_bytes(which, Cin, Cout) + bytes;
@@ -699,10 +704,11 @@ size_t conv_bf16_mfma_workspace_bytes(int which, uint32_t num_tiles, uint32_t N,
 // and a tile's rows -1 and H are its neighbours' last and first rows (zeros at the tensor's own border): the
 // unsplit convolution with zero padding, restricted to the tile.  Only shapes the eight-wave kernel takes
 // (ADH_EUNIMPL otherwise).
-// may_copy: the workspace has room for copies of the tiles with wider rows.  filter_ready: it holds the reordered filter already.
+// may_copy: over copies of the tiles with wider rows, for which the workspace has room.  as_they_lie: conv_bf16_any_rows from tiles
+// on 16 bytes.  filter_ready: it holds the reordered filter already.
 static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W,
                                const void *const *in_tiles, const void *w, void *const *out_tiles, float beta, void *workspace,
-                               hipStream_t st, bool halofree, bool may_copy, bool filter_ready) {
+                               hipStream_t st, bool halofree, bool may_copy, bool as_they_lie, bool filter_ready) {
   ConvBf16Params P = {};
   for (uint32_t t = 0; t < num_tiles; ++t) {
     P.in[t] = reinterpret_cast<const uint16_t *>(in_tiles[t]);
@@ -732,13 +738,13 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
   P.chan0 = 0;
   P.cred_pass = P.Cred < 64u ? P.Cred : 64u;
   P.first_pass = P.last_pass = 1;
-  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, H, W, may_copy);
+  const uint32_t launches = conv_bf16_launches(which, Cin, Cout, conv_bf16_w8_width(which, W) || may_copy || as_they_lie);
   if (launches > 1u) {
     uint8_t *part = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout);
     const size_t per_tile = part_region_bytes(which, N, Cin, Cout, H, W);
     for (uint32_t t = 0; t < num_tiles; ++t) P.part[t] = reinterpret_cast<float *>(part + t * per_tile);
   }
-  if (!halofree && may_copy && conv_bf16_repitches(which, Cin, Cout, H, W)) {
+  if (may_copy) {
     uint8_t *copy = reinterpret_cast<uint8_t *>(workspace) + filter_region_bytes(which, Cin, Cout) +
                     (launches > 1u ? num_tiles * part_region_bytes(which, N, Cin, Cout, H, W) : 0u);
     const size_t per_tile = conv_bf16_repitch_bytes(which, N, Cin, Cout, H, W);
@@ -752,7 +758,7 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
   }
   if (halofree && !conv_bf16_w8_takes(P, num_tiles)) return ADH_EUNIMPL;
   // the forward pass of the eight-wave kernel can read the caller's filter itself
-  const bool direct = which == ADH_CONV_FWD && (Cin % 64u) == 0u && aligned_to(w, 16) && (P.IW % 2u) == 0u;
+  const bool direct = which == ADH_CONV_FWD && (Cin % 64u) == 0u && aligned_to(w, 16) && conv_bf16_rows(P) != kNoRows;
   int e = ADH_OK;
   if (!direct && !filter_ready) {
     const uint32_t total = groups * P.passes * kWtGroupElems;
@@ -812,7 +818,7 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
   }
   if (P.passes > 1u) {
     if (!w8) {
-      // odd widths, tiles off the eight-wave kernels' alignment: the four-wave kernel once per 64 channels.  The
+      // an odd width and height, tiles off the eight-wave kernels' alignment: the four-wave kernel once per 64 channels.  The
       // workspace holds the sums between the launches unless the width promised one launch of 128 channels: then
       // it is the tiles' alignment that keeps the eight-wave kernels away, and there is no room for the sums.
       if (launches <= 1u) return ADH_EALIGN;
@@ -868,14 +874,16 @@ static int conv_bf16_mfma_some(int which, uint32_t num_tiles, uint32_t N, uint32
 // the copies of odd rows, and the sums between launches.
 static double conv_bf16_strips_us(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint32_t Cout, uint32_t H, uint32_t W, bool halofree) {
   const bool fwd = which == ADH_CONV_FWD, wide = conv_bf16_uses_k128(which, Cin, Cout);
-  const bool copies = !halofree && conv_bf16_repitches(which, Cin, Cout, H, W), four_waves = !halofree && !copies && !conv_bf16_w8_width(which, W);
   const double images = (double)num_tiles * N, C = fwd ? Cin : Cout, M = fwd ? Cout : Cin;
+  // (rows as they lie: as dear as copies where several launches follow, whose error is the largest; in one, the loads of odd rows)
+  const bool eight = halofree || conv_bf16_w8_width(which, W), any = !eight && conv_bf16_any_rows(which, H, W);
+  const bool copies = !eight && (!any || C > (wide ? 128.0 : 64.0)) && conv_bf16_repitches(which, Cin, Cout, H, W), four_waves = !eight && !any && !copies;
   const double oh = H + (fwd || halofree ? 0.0 : 2.0), ow = W + (fwd || halofree ? 0.0 : 2.0), ih = H + (fwd && !halofree ? 2.0 : 0.0), iw = W + (fwd && !halofree ? 2.0 : 0.0);
   const double unit = wide ? 128.0 : 64.0, cols = wide ? 32.0 : 64.0, launches = std::ceil(C / unit), groups = std::ceil(M / unit), pixels = images * oh * ow;
   const double flops = images * oh * std::ceil(ow / cols) * cols * 18.0 * launches * groups * unit * unit;
   const double steps = std::ceil(std::max(1.0, images * std::ceil(ow / 64.0) * std::ceil(oh / 4.0) * std::ceil(M / 64.0) / 256.0)) * std::ceil(C / 64.0);
-  if (wide) return 19.0 * launches + 0.459e-9 * flops + 0.082e-9 * 18.0 * pixels * C * groups * unit + 0.89 * steps + 1.7e-6 * (launches - 1.0) * pixels * M + (copies ? 4.7 + 0.68e-6 * images * C * ih * iw : 0.0);
-  return 16.0 * launches + (four_waves ? 0.66e-9 : 0.48e-9) * flops + 1.78 * steps + 0.15e-6 * pixels * M + 2e-6 * (launches - 1.0) * pixels * M + (copies ? 11.0 + 1.06e-6 * images * C * ih * iw : 0.0);
+  if (wide) return 19.0 * launches + 0.459e-9 * flops + 0.082e-9 * 18.0 * pixels * C * groups * unit + 0.89 * steps + 1.7e-6 * (launches - 1.0) * pixels * M + (copies ? 4.7 + 0.68e-6 * images * C * ih * iw : any ? 4.7 + (fwd ? 0.3e-6 * images * C * ih * iw : 0.0) : 0.0);
+  return 16.0 * launches + (four_waves ? 0.66e-9 : 0.48e-9) * flops + 1.78 * steps + 0.15e-6 * pixels * M + 2e-6 * (launches - 1.0) * pixels * M + (copies ? 11.0 + 1.06e-6 * images * C * ih * iw : any ? (fwd ? 0.25e-6 * images * C * ih * iw : 4.0) : 0.0);
 }
 constexpr double kPatchAhead = 1.15;  // by which patches have to be expected ahead
 
@@ -898,10 +906,11 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
     const int e = conv_bf16_patch(q, 9, workspace, workspace_bytes, conv_bf16_strips_us(which, num_tiles, N, Cin, Cout, H, W, halofree) / kPatchAhead, st);
     if (e != ADH_EUNIMPL) return e;
   }
+  const bool as_they_lie = aligned && !halofree && conv_bf16_any_rows(which, H, W);
   const uint64_t room = workspace_bytes > filter_region_bytes(which, Cin, Cout) ? workspace_bytes - filter_region_bytes(which, Cin, Cout) : 0u;
-  if (halofree || !conv_bf16_repitches(which, Cin, Cout, H, W) ||
+  if (halofree || as_they_lie || !conv_bf16_repitches(which, Cin, Cout, H, W) ||
       room < conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, kLeastCopies).bytes)
-    return conv_bf16_mfma_some(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, halofree, false, false);
+    return conv_bf16_mfma_some(which, num_tiles, N, Cin, Cout, H, W, in_tiles, w, out_tiles, beta, workspace, st, halofree, false, as_they_lie, false);
   const CopyTurn turn = conv_bf16_copy_turn(which, num_tiles, N, Cin, Cout, H, W, std::min<uint64_t>(room, kMostCopies));
   const uint64_t slab = (H + 2ull) * (W + 2ull) * 2u, inner = (uint64_t)H * W * 2u;  // bytes of a channel
   const uint64_t in_image = which == ADH_CONV_FWD ? Cin * slab : Cout * inner, out_image = which == ADH_CONV_FWD ? Cout * inner : Cin * slab;
@@ -915,7 +924,7 @@ int conv_bf16_mfma(int which, uint32_t num_tiles, uint32_t N, uint32_t Cin, uint
         in[k] = reinterpret_cast<const char *>(in_tiles[t + k]) + n * in_image;
         out[k] = reinterpret_cast<char *>(out_tiles[t + k]) + n * out_image;
       }
-      const int e = conv_bf16_mfma_some(which, tiles, images, Cin, Cout, H, W, in, w, out, beta, workspace, st, false, true, filter_ready);
+      const int e = conv_bf16_mfma_some(which, tiles, images, Cin, Cout, H, W, in, w, out, beta, workspace, st, false, true, false, filter_ready);
       if (e) return e;
       filter_ready = true;
     }

@@ -65,11 +65,13 @@ static __device__ __forceinline__ uint32_t wrap_slot(uint32_t s) { return s >= (
 // leaves idle fetch the tenth granule of every row and channel into the idle tail of the staging area, and a
 // sixth transposing read turns its first pixel into ring pixel 72 (rows of 73 pixels).  Rows -1 and IH come
 // from the neighbouring tiles (P.neighbour_rows).
-template <bool BETA, bool PIN = false, bool POUT = false, bool HF = false>
+// ROWS: 0, every input row starts on a 4-byte boundary (pad 0) or on 16 bytes and is whole granules; kOddRows (forward) and kAnyRows
+// (backward-data): conv3x3_bf16_mfma.h.
+template <bool BETA, bool PIN = false, bool POUT = false, bool HF = false, int ROWS = 0>
 __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16Params P) {
   static_assert(!(BETA && PIN), "the old output is added in the first pass, which reads no sums");
   constexpr int kRowBytes = (HF ? kW8RowPx + 1 : kW8RowPx) * kW8PxBytes;
-  constexpr int kRingBytes = kW8RingRows * kRowBytes;
+  constexpr int kRingBytes = kW8RingRows * kRowBytes + (ROWS ? kW8PxBytes : 0);  // (ROWS: a row's last pixel may be one on)
   constexpr int kGroups = HF ? 6 : 5;  // transposing read pairs (and ring writes) per row group
   __shared__ __attribute__((aligned(16))) uint8_t raw[kW8RawBytes];
   __shared__ __attribute__((aligned(16))) uint8_t ring[kRingBytes];
@@ -139,7 +141,10 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   const uint32_t image_bytes = P.Cred * plane_bytes;
   // ring pixel of the strip's first output column at tap column 0: the staged row starts eight columns left of
   // the strip whenever the input has no halo of its own (pad 1: unpadded in and out; pad 2: backward-data into a padded slab)
-  const uint32_t xoff = P.pad ? 8u - (uint32_t)P.pad : 0u;
+  // Odd rows of an odd width are staged from one element back (forward) or on (backward-data); so that no ring pixel is below 0,
+  // forward writes the even rows one pixel on, backward-data the odd ones.
+  const uint32_t xoff = P.pad ? 8u - (uint32_t)P.pad : (ROWS ? 1u : 0u);
+  const uint32_t on_odd = ROWS == kAnyRows ? (P.IW & 1u) : 0u, on_even = ROWS == kOddRows ? 1u : 0u;
   const int32_t col_back = P.pad ? 8 : 0;       // the staged row starts this many columns left of the strip
 
   // ---- requests: copy q of a group moves staging slots 64 q + lane; slot = (row * 8 + channel) * 9 + granule
@@ -157,7 +162,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
     }
     const uint32_t chan = 8u * wv + ch;
     const bool ok = (HF || slot < 288u) && chan < P.cred_pass;
-    ld_off[q] = (P.chan0 + chan) * plane_bytes + row * P.IW * 2u + gran * 16u;
+    ld_off[q] = (P.chan0 + chan) * plane_bytes + row * P.IW * 2u + gran * 16u + (ROWS && (row & 1u) ? 2u * (on_odd - on_even) : 0u);
     ld_rows |= ((row & 3u) | (ok ? 4u : 0u)) << (3 * q);
     ld_gran |= gran << (4 * q);
   }
@@ -172,7 +177,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   const uint8_t *const tr03 = raw_wave + tr_lane + g * 32u;                  // + t * 8 * kW8RawCh
   const uint8_t *const tr4 = raw_wave + tr_lane + g * 8u * kW8RawCh + 128u;
   const uint32_t wr03 = (16u * g + l16) * kW8PxBytes + wv * 16u;             // + slot(row t) * kRowBytes
-  const uint32_t wr4 = (64u + l16) * kW8PxBytes + wv * 16u;                  // + slot(row g) * kRowBytes
+  const uint32_t wr4 = (64u + l16 + (g & 1u ? on_odd : on_even)) * kW8PxBytes + wv * 16u;  // + slot(row g) * kRowBytes
   uint8_t *const wr4_dummy = raw_wave + 288 * 16 + ((l16 & 7u) + 8u * g) * 16u;
   // HF, round 5: row g's tenth granule, [channel][8 pixels] at slot 288 + 8 g + channel; lane 0 of the group
   // receives its first pixel (the reads of the other lanes run on into the next slots and are not used)
@@ -194,11 +199,18 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
       T.hi = lds_read_tr(tr5 + 4 * 16);
     }
   };
+  int32_t colT = 0;  // input column of staged pixel 0 of the group to transpose
   auto tr_write = [&](auto tag, const TrPair &T) {
     constexpr int t = decltype(tag)::value;
-    const u32x4 v = {T.lo[0], T.lo[1], T.hi[0], T.hi[1]};
+    u32x4 v = {T.lo[0], T.lo[1], T.hi[0], T.hi[1]};
+    if constexpr (ROWS == kAnyRows) {  // granules that straddle the row's ends hold the neighbouring rows' pixels
+      const uint32_t px = t < 4 ? 16u * g + l16 + (t & 1 ? on_odd : 0u) : 64u + l16 + (g & 1u ? on_odd : 0u);
+      const bool inside = (uint32_t)colT + px < P.IW;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) v[j] = inside ? v[j] : 0u;
+    }
     if constexpr (t < 4) {
-      *reinterpret_cast<u32x4 *>(ring + wrap_slot(tb + (uint32_t)t) * kRowBytes + wr03) = v;
+      *reinterpret_cast<u32x4 *>(ring + wrap_slot(tb + (uint32_t)t) * kRowBytes + (t & 1 ? on_odd : on_even) * kW8PxBytes + wr03) = v;
     } else if constexpr (t == 4) {
       uint8_t *const dst = ring + wrap_slot(tb + g) * kRowBytes + wr4;
       *reinterpret_cast<u32x4 *>(l16 < 8u ? dst : wr4_dummy) = v;
@@ -259,7 +271,9 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
 #pragma unroll
     for (int q = 0; q < kW8Copies; ++q) {
       const int32_t col = colL + 8 * (int32_t)((ld_gran >> (4 * q)) & 15u);
-      const bool ok = ((ld_rows >> (3 * q)) & 4u) && col >= 0 && col < (int32_t)P.IW;
+      // (backward-data: the granule left of an odd row that is staged one element on ends with the row's first pixel)
+      const int32_t first = ROWS == kAnyRows && (ld_rows >> (3 * q) & 1u) ? -8 * (int32_t)on_odd : 0;
+      const bool ok = ((ld_rows >> (3 * q)) & 4u) && col >= first && col < (int32_t)P.IW;
       okL |= (ok ? 1u : 0u) << q;
     }
     grpL = -1;
@@ -614,6 +628,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   uint32_t sb = 4;  // ring slot of the first input row of the step multiplied in this phase
   loader_open();
   for_each_int(std::make_integer_sequence<int, 5>(), [&](auto tag) { request(tag, IntTag<HF ? 1 : 0>()); });
+  colT = colL;
   loader_advance();
   // Every wave passes one barrier per phase, after its last ring access of the phase.
   auto phase_barrier = [&]() {
@@ -668,6 +683,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
       move_rows_plain();
       after_plain = true;
     }
+    colT = colL;
     loader_advance();
     if (!barrier_done) {
       if (rp == 0u)
@@ -687,11 +703,10 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   if (barrier_owed) phase_barrier();
 }
 
-// Shapes of the eight-wave kernel: input rows that start on a 4-byte boundary (on 16 bytes for
-// backward-data, whose granules must lie wholly inside or outside a row; output rows may start
-// anywhere), images whose byte offsets fit the buffer range check's 31 bits.
+// Shapes of the eight-wave kernel: rows as conv_bf16_rows takes them, over tiles without halo of whole granules (output rows
+// may start anywhere), images whose byte offsets fit the buffer range check's 31 bits.
 bool conv_bf16_w8_takes(const ConvBf16Params &P, uint32_t num_tiles) {
-  if (P.pad ? (P.IW % 8u) != 0u : (P.IW % 2u) != 0u) return false;
+  if (conv_bf16_rows(P) == kNoRows) return false;
   if (P.neighbour_rows && P.IH == 0u) return false;
   const uint64_t image_bytes = (uint64_t)P.Cred * P.IH * P.IW * 2u;
   if (image_bytes >= (1ull << 31)) return false;
@@ -711,39 +726,29 @@ bool conv_bf16_w8_takes(const ConvBf16Params &P, uint32_t num_tiles) {
 int conv_bf16_w8_launch(const ConvBf16Params &P, uint32_t gx, uint32_t groups, hipStream_t st) {
   const dim3 grid(gx, groups), block(kW8Threads);
   const bool first = P.first_pass != 0u, last = P.last_pass != 0u;
-  if (P.pad == 1) {  // no halo on either side
-    if (first && last) {
-      if (P.beta != 0.f)
-        hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<true, false, false, true>), grid, block, 0, st, P);
-      else
-        hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, false, false, true>), grid, block, 0, st, P);
-    } else if (first) {
-      if (P.beta != 0.f)
-        hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<true, false, true, true>), grid, block, 0, st, P);
-      else
-        hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, false, true, true>), grid, block, 0, st, P);
-    } else if (!last) {
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, true, true, true>), grid, block, 0, st, P);
-    } else {
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, true, false, true>), grid, block, 0, st, P);
-    }
-    return launch_status();
-  }
+  const bool beta = P.beta != 0.f;
+  const int rows = conv_bf16_rows(P);
+#define ADH_W8(B, PI, PO)                                                                               \
+  do {                                                                                                  \
+    if (P.pad == 1)                                                                                     \
+      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<B, PI, PO, true>), grid, block, 0, st, P);             \
+    else if (rows == kOddRows)                                                                          \
+      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<B, PI, PO, false, kOddRows>), grid, block, 0, st, P);  \
+    else if (rows == kAnyRows)                                                                          \
+      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<B, PI, PO, false, kAnyRows>), grid, block, 0, st, P);  \
+    else                                                                                                \
+      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<B, PI, PO, false>), grid, block, 0, st, P);            \
+  } while (0)
   if (first && last) {
-    if (P.beta != 0.f)
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<true>), grid, block, 0, st, P);
-    else
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false>), grid, block, 0, st, P);
+    if (beta) ADH_W8(true, false, false); else ADH_W8(false, false, false);
   } else if (first) {
-    if (P.beta != 0.f)
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<true, false, true>), grid, block, 0, st, P);
-    else
-      hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, false, true>), grid, block, 0, st, P);
+    if (beta) ADH_W8(true, false, true); else ADH_W8(false, false, true);
   } else if (!last) {
-    hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, true, true>), grid, block, 0, st, P);
+    ADH_W8(false, true, true);
   } else {
-    hipLaunchKernelGGL((conv3x3_bf16_w8_kernel<false, true, false>), grid, block, 0, st, P);
+    ADH_W8(false, true, false);
   }
+#undef ADH_W8
   return launch_status();
 }
 
