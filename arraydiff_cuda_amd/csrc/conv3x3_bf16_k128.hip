@@ -384,8 +384,9 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
   // input rows 0 and 1 in turn (one and two MFMAs), rounds 48-71 row 2, rounds 72-95 row 3 (three each), rounds
   // 96-143 rows 4 and 5 in turn (two and one): output row 0 is complete after round 71, row 1 after round 95.
   // With SIDE everything else a wave does in a phase is dealt out between the rounds one instruction at a time.
+  // SIDE 2: a strip whose last columns, or output channels, don't exist.
   auto compute = [&](uint32_t sb, auto side_tag, auto nbr_tag, uint32_t row0, uint32_t nrows, bool after_plain) {
-    constexpr bool SIDE = decltype(side_tag)::value != 0;
+    constexpr bool SIDE = decltype(side_tag)::value != 0, RAGGED = decltype(side_tag)::value == 2;
     const uint32_t cur_off = ooff_lane + (row0 * P.OW + c0C) * 2u;
     const uint32_t pcur = poff_lane + (row0 * P.OW + c0C) * 4u;
     uint32_t off[4], poff[4];
@@ -394,6 +395,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
       off[r] = nrows > (uint32_t)r ? cur_off + (uint32_t)r * orow_bytes : kOutOfRange;
       poff[r] = nrows > (uint32_t)r ? pcur + (uint32_t)r * prow_bytes : kOutOfRange;
     }
+    const RaggedStore ragged(cur_off, okc, c0C + ocol_lane, P.OW);
     floatx4 acc[4][2];  // [row][column tile]
 #pragma unroll
     for (int r = 0; r < 4; ++r)
@@ -423,7 +425,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
       if (after_plain)
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       else
-        __builtin_amdgcn_s_waitcnt(POUT ? 0x0F78 : 0x0F74);  // vmcnt(8) : vmcnt(4)
+        __builtin_amdgcn_s_waitcnt(RAGGED ? 0x4F70 : POUT ? 0x0F78 : 0x0F74);  // vmcnt(16) : vmcnt(8) : vmcnt(4)
     }
     // packs output row r back to store order through the swap between lane rows and stores it
     auto pack_row = [&](auto tag) {
@@ -468,7 +470,9 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
       const u32x2 q0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v1[0], v1[1]), false, false);
       const u32x2 q1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[2], v0[3]), pack_bf16x2(v1[2], v1[3]), false, false);
       const u32x4 pk = {q0[0], q1[0], q0[1], q1[1]};
-      if constexpr (SIDE) {
+      if constexpr (RAGGED) {
+        ragged.store(rsrcC, pk, nrows > (uint32_t)r, (uint32_t)r * orow_bytes, 0, P.OW);
+      } else if constexpr (SIDE) {
         __builtin_amdgcn_raw_buffer_store_b128(pk, rsrcC, off[r], 0, 0);
       } else {
         if ((uint32_t)r < nrows) store_guarded(pk, row0 + r);
@@ -521,7 +525,7 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
         // output rows 0 and 1 are packed and stored while rows 2 and 3 are still being multiplied
         if constexpr (t == 80 || t == 106) {
           pack_row(IntTag<t == 80 ? 0 : 1>());
-          __builtin_amdgcn_sched_group_barrier(0x010, POUT ? 2 : 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x010, RAGGED ? 4 : POUT ? 2 : 1, 0);
         }
       }
     };
@@ -539,7 +543,8 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
     }
   };
 
-  // the same side work in one piece, for the phases that cannot take the interleaved form
+  // the same side work in one piece, for the phases that cannot take the interleaved form: those without MFMAs, and (the old output
+  // added, or sums of several passes) ragged strips
   auto move_rows_plain = [&]() {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     TrPair T[6];
@@ -575,6 +580,9 @@ __global__ __launch_bounds__(kK2Threads, 1) void conv3x3_bf16_k128_kernel(ConvBf
         } else {
           compute(sb, IntTag<1>(), IntTag<0>(), row0, nrows, after_plain);
         }
+        after_plain = false;
+      } else if constexpr (!BETA && !PART) {
+        compute(sb, IntTag<2>(), IntTag<HF ? 1 : 0>(), row0, nrows, after_plain);
         after_plain = false;
       } else {
         move_rows_plain();

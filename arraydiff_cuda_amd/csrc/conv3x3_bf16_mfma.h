@@ -78,6 +78,31 @@ inline int conv_bf16_rows(int32_t pad, uint32_t IH, uint32_t IW) {
 }
 inline int conv_bf16_rows(const ConvBf16Params &P) { return conv_bf16_rows(P.pad, P.IH, P.IW); }
 
+// Stores a strip's ragged end: sixteen bytes from lanes whose eight columns exist, and from the one that holds the row's last
+// `tail` (1 to 7) columns four, two and one of them.  Four stores, always: lanes and pieces that don't exist have an offset out of range, so that a
+// ragged strip's steps interleave their side work like any other's (with the side work in one piece and stores element by element, where
+// every workgroup has one strip, the ragged ones set the time: 128 -> 128 channels, 8 images of 4 tiles, forward at 64x255 178 -> 149 us, at
+// 64x250 138 -> 124, backward-data 166 -> 159 and 144 -> 128; 64 -> 64, 2 images of 8 tiles of 128x1020, 170 -> 151 and 199 -> 158).
+struct RaggedStore {
+  uint32_t full, piece4, piece2, piece1;  // byte offsets
+  __device__ __forceinline__ RaggedStore(uint32_t off, bool exists, uint32_t col, uint32_t width) {
+    const uint32_t tail = width & 7u;  // (strips and lanes start at multiples of eight columns)
+    const bool part = exists && col < width && col + 8u > width;
+    full = exists && col + 8u <= width ? off : kOutOfRange;
+    piece4 = part && (tail & 4u) ? off : kOutOfRange;
+    piece2 = part && (tail & 2u) ? off + 2u * (tail & 4u) : kOutOfRange;
+    piece1 = part && (tail & 1u) ? off + 2u * (tail & 6u) : kOutOfRange;
+  }
+  // `live`: the row exists
+  __device__ __forceinline__ void store(const __amdgpu_buffer_rsrc_t &rsrc, const u32x4 &v, bool live, uint32_t row_off, uint32_t soff, uint32_t width) const {
+    const uint32_t two = (width & 4u) ? v[2] : v[0], one = (width & 2u) ? ((width & 4u) ? v[3] : v[1]) : two;
+    __builtin_amdgcn_raw_buffer_store_b128(v, rsrc, live ? full + row_off : kOutOfRange, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b64((u32x2){v[0], v[1]}, rsrc, live ? piece4 + row_off : kOutOfRange, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b32(two, rsrc, live ? piece2 + row_off : kOutOfRange, soff, 0);
+    __builtin_amdgcn_raw_buffer_store_b16((uint16_t)one, rsrc, live ? piece1 + row_off : kOutOfRange, soff, 0);
+  }
+};
+
 // the eight-wave kernel: shapes it takes, and its launch (grid.x workgroups per output group)
 bool conv_bf16_w8_takes(const ConvBf16Params &P, uint32_t num_tiles);
 // launches the pass of up to 64 reduction channels from P.chan0 on

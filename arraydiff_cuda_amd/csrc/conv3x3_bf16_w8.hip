@@ -437,9 +437,10 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
   // of the row group that has landed, the five copies of the next group, and for beta = 1 the
   // four loads of old values (buffer loads and stores: a row that does not exist gets an
   // out-of-range offset, so the sequence has no branches).
+  // SIDE 2: a strip whose last columns, or output channels, don't exist.
   auto compute = [&](uint32_t sb, auto side_tag, auto bar_tag, auto nbr_tag, uint32_t row0, uint32_t nrows, bool barrier_owed,
                      bool after_plain) {
-    constexpr bool SIDE = decltype(side_tag)::value != 0;
+    constexpr bool SIDE = decltype(side_tag)::value != 0, RAGGED = decltype(side_tag)::value == 2;
     // 1: this phase's barrier comes between the rounds and the packing; 2: the previous phase's barrier, if still
     // owed, comes after the first operand fetches (row pair 0 only: they read rows that step shares with this one)
     constexpr int BAR = decltype(bar_tag)::value;
@@ -488,7 +489,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
       if (after_plain)
         __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
       else
-        __builtin_amdgcn_s_waitcnt(POUT ? 0x0F78 : 0x0F74);  // vmcnt(8) : vmcnt(4)
+        __builtin_amdgcn_s_waitcnt(RAGGED ? 0x4F70 : POUT ? 0x0F78 : 0x0F74);  // vmcnt(16) : vmcnt(8) : vmcnt(4)
     }
     // packs tile i (row i / 2 of the pair, channel tile i % 2) back to store order through the
     // swap between lane rows and, in the interleaved form, stores it
@@ -526,7 +527,10 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
       const u32x2 q0 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[0], v0[1]), pack_bf16x2(v1[0], v1[1]), false, false);
       const u32x2 q1 = __builtin_amdgcn_permlane16_swap(pack_bf16x2(v0[2], v0[3]), pack_bf16x2(v1[2], v1[3]), false, false);
       pk[ct][r] = (u32x4){q0[0], q1[0], q0[1], q1[1]};
-      if constexpr (SIDE)
+      if constexpr (RAGGED)
+        RaggedStore(cur_off, okct[ct], c0C + ocol_lane, P.OW)
+            .store(rsrcC, pk[ct][r], nrows > (uint32_t)r, (uint32_t)r * orow_bytes, ct ? ct_bytes : 0u, P.OW);
+      else if constexpr (SIDE)
         __builtin_amdgcn_raw_buffer_store_b128(pk[ct][r], rsrcC, r ? off1 : off0, ct ? ct_bytes : 0u, 0);
     };
     auto round = [&](auto tag) {
@@ -566,7 +570,7 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
         // rounds 38 and 42: output row 0, complete since round 35, is packed and stored
         if constexpr (t == 38 || t == 42) {
           pack_tile(IntTag<(t - 38) / 4>());
-          __builtin_amdgcn_sched_group_barrier(0x010, POUT ? 2 : 1, 0);
+          __builtin_amdgcn_sched_group_barrier(0x010, RAGGED ? 4 : POUT ? 2 : 1, 0);
         }
         // the earlier passes' sums: output row 0 in rounds 24, 27, 30, 33; row 1 once row 0's have been used
         // (rounds 39, 40 after the packing in round 38; rounds 43, 44 after the one in round 42)
@@ -611,7 +615,8 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
     }
   };
 
-  // the same side work in one piece, for the phases that cannot take the interleaved form
+  // the same side work in one piece, for the phases that cannot take the interleaved form: those without MFMAs, and (the old output
+  // added, or sums of several passes) ragged strips
   auto move_rows_plain = [&]() {
     __builtin_amdgcn_s_waitcnt(0x0F70);  // vmcnt(0)
     TrPair T[kGroups];
@@ -672,6 +677,10 @@ __global__ __launch_bounds__(kW8Threads, 1) void conv3x3_bf16_w8_kernel(ConvBf16
           }
           barrier_done = true;
         }
+        after_plain = false;
+      } else if constexpr (!BETA && !PART) {
+        compute(sb, IntTag<2>(), IntTag<1>(), IntTag<HF ? 1 : 0>(), row0, nrows, false, after_plain);
+        barrier_done = true;
         after_plain = false;
       } else {
         if (BETA) load_old_guarded(row0, nrows);
