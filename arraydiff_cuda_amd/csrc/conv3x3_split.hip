@@ -27,7 +27,9 @@
 // from the chunk's first step on (stride 1 has the registers for them from the fourth): 0.202 -> 0.187 and 0.126 -> 0.118.
 // Measured (32 images, 4 tiles without halo, forward / backward-data; v_mfma_f32 kernels before): 64 channels on 32 x 128
 // tiles 0.309 -> 0.209 / 0.197 ms (196 TFLOP/s), 128 on 16 x 64 0.297 -> 0.182, 256 on 8 x 32 0.292 -> 0.175 (221), 512 on
-// 4 x 16 0.39 -> 0.215 / 0.212.  Bound: the matrix pipe is busy 0.6 of the cycles; a step of 3072 matrix cycles takes 3700 to 4400
+// 4 x 16 0.39 -> 0.215 / 0.212; with the arguments read where they are used (from_memory; 130 to 200 scalar registers were spilled) 512 on 4 x 16
+// 0.246 -> 0.237, backward-data at stride 2, 128 -> 256 on 16 x 64, 0.131 -> 0.120, 60 random padded layers 0.967 / 0.974 of the time, up to
+// 0.88 where a block has 32 channels.  Bound: the matrix pipe is busy 0.6 of the cycles; a step of 3072 matrix cycles takes 3700 to 4400
 // (the loads' address arithmetic and the splitting compete for issue slots), the patch's change of chunk 4500, and a block's
 // results leave at the rate of the memory, all workgroups at once.
 #include "conv3x3_split.h"
@@ -103,7 +105,8 @@ struct SplitBlock {
 // by itself.  The choice hangs on the channels alone, not on the block's shape or the images it holds (split_low); small launches go
 // to conv_f32_patch.hip, which adds in another order: the forms of one layer have the same bits, not a layer and a part of it.
 template <int MT, int NT, bool VEC, int SAMPLE, int LOW>
-__global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const SplitParams P) {
+__global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const SplitParams args) {
+  const SplitParams &P = args;
   constexpr uint32_t MW = 16u * MT;
   constexpr int SETS = SAMPLE == kUp ? 4 : 1;  // of sums
   constexpr uint32_t DOWN = SAMPLE == kDown ? 2u : 1u, UP = SAMPLE == kUp ? 2u : 1u;
@@ -124,6 +127,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   const uint32_t end_vid = min(P.blocks, ((blockIdx.x & 7u) + 1u) * P.xcd_chunk);
   if (next_vid >= end_vid) return;
   auto next_block = [&]() {
+    const SplitParams &P = from_memory(args);
     SplitBlock B;
     uint32_t bid, outer, inner, group;
     P.div_ksplit.divmod(next_vid, bid, B.ks);
@@ -147,8 +151,8 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   lds_barrier();
 
   // tile of row R of the stacked tensor
-  auto in_tile = [&](uint32_t R) { return R < P.in_lead ? 0u : min(P.div_in.div(R - P.in_lead), P.last_tile); };
-  auto out_tile = [&](uint32_t R) { return R < P.out_lead ? 0u : min(P.div_out.div(R - P.out_lead), P.last_tile); };
+  auto in_tile = [&](const SplitParams &P, uint32_t R) { return R < P.in_lead ? 0u : min(P.div_in.div(R - P.in_lead), P.last_tile); };
+  auto out_tile = [&](const SplitParams &P, uint32_t R) { return R < P.out_lead ? 0u : min(P.div_out.div(R - P.out_lead), P.last_tile); };
 
   // ---- the patch: this thread stages units tid + j * kSpThreads of its pixels' octets (octet 0 of all pixels first);
   // element e of octet o is channel 4e + o of the chunk, the filter's order below ----
@@ -169,6 +173,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   const ADH_GLOBAL char *src = nullptr;  // the next element to load, and how many there are of the unit
   uint32_t src_n = 0;
   auto set_unit = [&](const SplitBlock &B, uint32_t ch, int j) {
+    const SplitParams &P = from_memory(args);
     uint32_t o, p, b, e, r, c;
     P.div_PPn.divmod(unit(j), o, p);
     P.div_PPI.divmod(p, b, e);
@@ -179,7 +184,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     const bool ok = o < 4u && c0 < P.C && img < P.NI && R >= 0 && R < (int32_t)P.in_VH && Q >= 0 && Q < (int32_t)P.in_W;
     uint32_t tile0, n;
     P.div_N.divmod(ok ? img : 0u, tile0, n);
-    const uint32_t Ru = ok ? (uint32_t)R : P.in_lead, t = in_tile(Ru);
+    const uint32_t Ru = ok ? (uint32_t)R : P.in_lead, t = in_tile(P, Ru);
     src_n = ok ? min(8u, (P.C - c0 + 3u) >> 2) : 0u;
     xn = (j == 0 ? 0u : xn) | src_n << (4 * j);
     // (a unit that does not exist loads an existing place; its values are replaced by zero)
@@ -196,6 +201,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     }
   };
   auto store_x = [&]() {
+    const SplitParams &P = from_memory(args);
     float mx = 0.f;
 #pragma unroll
     for (int j = 0; j < XU; ++j) {
@@ -242,6 +248,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   };
   float wrow[12];
   auto load_wrow = [&](uint32_t mg, uint32_t ch, int kh) {
+    const SplitParams &P = from_memory(args);
     const FilterLane L = w_lane();
     const float *base = P.w + (size_t)min(mg * MW + L.m, P.M - 1u) * P.w_m_stride + (P.flip ? 6 - 3 * kh : 3 * kh);
 #pragma unroll
@@ -293,6 +300,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   const size_t out_plane = (size_t)P.out_H * P.out_W;
   struct Place { bool ok; uint32_t img, i, j, tile; size_t at; };
   auto place_of = [&](const SplitBlock &B, uint32_t f) {  // pixel slot f of the block
+    const SplitParams &P = from_memory(args);
     Place pl;
     uint32_t b, e, r, c, tile0, n;
     asm volatile("" : "+v"(f));  // (worked out where it is used, not kept)
@@ -303,12 +311,13 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
     pl.j = B.bj * P.BC + c;
     pl.ok = b < P.NB && pl.img < P.NI && pl.i < P.grid_VH && pl.j < P.grid_W;
     P.div_N.divmod(pl.ok ? pl.img : 0u, tile0, n);
-    const uint32_t R = pl.ok ? pl.i : P.out_lead, t = out_tile(R);
+    const uint32_t R = pl.ok ? pl.i : P.out_lead, t = out_tile(P, R);
     pl.tile = tile0 + t;
     pl.at = (size_t)n * P.M * out_plane + (size_t)((R - t * P.out_step) * UP) * P.out_W + (pl.ok ? pl.j * UP : 0u);
     return pl;
   };
   auto emit_all = [&](const SplitBlock &B) {
+    const SplitParams &P = from_memory(args);
     // channel of accumulator (mt, i) above m0: 16 mt (VEC) or 16 mt + i
     const uint32_t m0 = B.mg * MW + (VEC ? l16 : g * 4u), m_top = P.M - 1u - min(m0, P.M - 1u);
     const bool whole = (B.mg + 1u) * MW <= P.M;
@@ -382,6 +391,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
   };
   // something staged has parts that are not finite: the wave's outputs as plain fp32 sums, straight from memory
   auto emit_plain = [&](const SplitBlock &B) {
+    const SplitParams &P = from_memory(args);
     for (uint32_t of = lane; of < 16u * NT * MW * SETS; of += 64u) {
       const uint32_t at = of / SETS, set = of % SETS, m = B.mg * MW + at / (16u * NT);
       const Place pl = place_of(B, wave * (16u * NT) + at % (16u * NT));
@@ -396,7 +406,7 @@ __global__ __launch_bounds__(kSpThreads, 2) void conv3x3_split_kernel(const Spli
           const int32_t R = (int32_t)(pl.i * DOWN + a * P.dil) - P.pad_r, Q = (int32_t)(pl.j * DOWN + b * P.dil) - P.pad_c;
           float x = 0.f;  // the padding is data: an infinite filter element times it is NaN
           if (R >= 0 && R < (int32_t)P.in_VH && Q >= 0 && Q < (int32_t)P.in_W) {
-            const uint32_t ti = in_tile((uint32_t)R);
+            const uint32_t ti = in_tile(P, (uint32_t)R);
             x = tab[tile0 + ti][((size_t)n * P.C + c) * plane + ((uint32_t)R - ti * P.in_step) * (size_t)P.in_W + (uint32_t)Q];
           }
           v = __builtin_fmaf(P.w[(size_t)m * P.w_m_stride + (size_t)c * P.w_c_stride + (P.flip ? 8u - t : t)], x, v);

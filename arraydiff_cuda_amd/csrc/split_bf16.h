@@ -56,6 +56,17 @@ __device__ __forceinline__ floatx4 mfma_bf16(uintx4 a, uintx4 b, floatx4 c) {
   return __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
 }
 
+// A kernel's only argument, read where it is used, through the scalar cache.  What a kernel with many reads once and keeps
+// runs out of scalar registers, and the compiler then keeps them in lanes of vector registers, an instruction of the vector units for
+// each use: 300 to 350 of 1300 to 1640 a chunk in conv3x3_split_kernel, which has none now.  The values are not known to be invariant
+// to the compiler: what is used in a loop that stores is copied first.
+template <typename Params>
+__device__ __forceinline__ const Params &from_memory(const Params &) {
+  const __attribute__((address_space(4))) Params *p = (const __attribute__((address_space(4))) Params *)__builtin_amdgcn_kernarg_segment_ptr();
+  asm volatile("" : "+s"(p));
+  return *(const Params *)p;
+}
+
 // barrier over LDS only: memory operations in flight stay in flight
 __device__ __forceinline__ void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 
