@@ -22,7 +22,8 @@
 // Measured (32 images, 4 tiles without halo; the v_mfma_f32 kernel before): 64 channels on 32 x 128 tiles 0.351 -> 0.197 ms
 // (196 TFLOP/s), 128 on 16 x 64 0.354 -> 0.193, 256 on 8 x 32 0.361 -> 0.195, 512 on 4 x 16 0.456 -> 0.21 (0.61 through the
 // general entry point before); with [octet][channel] rows in place of [channel][pixel] ones, where bank conflicts took 0.41 of all cycles,
-// 0.181, 0.173, 0.175, 0.192, and 1.08 times as fast in the mean of 115 layers (176 -> 16 channels on 3 tiles of 7 x 391 116 -> 91 us).  Staging: with rows, channels and tiles worked out per group of four values the kernel took
+// 0.181, 0.173, 0.175, 0.192, and 1.08 times as fast in the mean of 115 layers (176 -> 16 channels on 3 tiles of 7 x 391 116 -> 91 us); with what a step's loads need read where it is used (from_memory), 0.989 of the
+// time over 60 random padded layers.  Staging: with rows, channels and tiles worked out per group of four values the kernel took
 // 0.45 ms; a thread's channel and column fixed and a wave's row uniform it is a load, a split and three writes.  Bound: a
 // step of 6912 matrix cycles takes about 11000, the splitting and the shifts (a third of the issue slots) and the clock,
 // which the power limit holds at 1.8 - 2.1 GHz; and on short layers the workgroups' sums, 38 MB written and read back.
@@ -53,7 +54,8 @@ struct WgradSplitParams {
 };
 
 template <int OT, int CT>
-__global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(const WgradSplitParams P) {
+__global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(const WgradSplitParams args) {
+  const WgradSplitParams &P = args;
   constexpr uint32_t CO = 32u * OT, CI = 32u * CT;
   __shared__ __align__(16) char lds[kWsLdsBytes];
   __shared__ uint32_t nan_sums;
@@ -77,7 +79,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   const size_t x_plane = (size_t)P.x_H * P.x_W, dy_plane = (size_t)P.dy_H * P.dy_W;
   // tile and row of the stacked tensor's row R; of x row R where the halo rows are the neighbours' interior rows
   struct Row { uint32_t tile, r; };
-  auto row_of = [&](uint32_t R, bool is_x) {
+  auto row_of = [&](const WgradSplitParams &P, uint32_t R, bool is_x) {
     const uint32_t t = min(P.div_step.div(R), P.last_tile);
     Row w = {tile0 + t, R - t * P.step};
     if (P.neighbours && is_x) {
@@ -115,12 +117,13 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   };
   // x rows x0 .. x0 + nx - 1 (of the padded numbering), dy rows d0 .. d0 + nd - 1
   auto load = [&](uint32_t x0, uint32_t nx, uint32_t d0, uint32_t nd) {
+    const WgradSplitParams &P = from_memory(args);
 #pragma unroll
     for (int j = 0; j < XR; ++j) {
       const uint32_t i = (uint32_t)j * x_rows + x_row;
       const int32_t R = (int32_t)(x0 + i) - P.pad_r;
       if (i < nx && R >= 0 && R < (int32_t)P.x_VH) {
-        const Row w = row_of((uint32_t)R, true);
+        const Row w = row_of(P, (uint32_t)R, true);
         vx[j] = load4(P.x[w.tile] + ((size_t)n * P.Cin * x_plane + (size_t)w.r * P.x_W) + x_chan, x_from, xW);
       } else {
         vx[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -130,7 +133,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
     for (int j = 0; j < DR; ++j) {
       const uint32_t i = (uint32_t)j * dy_rows + dy_row, R = d0 + i;
       if (i < nd && R < P.dy_VH) {
-        const Row w = row_of(R, false);
+        const Row w = row_of(P, R, false);
         vd[j] = load4(P.dy[w.tile] + ((size_t)n * P.Cout * dy_plane + (size_t)w.r * P.dy_W) + dy_chan, dy_from, dW);
       } else {
         vd[j] = floatx4{0.f, 0.f, 0.f, 0.f};
@@ -139,7 +142,7 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
     const int32_t R = (int32_t)(x0 + wave) - P.pad_r, Q = (int32_t)(c0 + P.TW) - P.pad_c;
     tail[0] = tail[1] = 0.f;
     if (wave < nx && R >= 0 && R < (int32_t)P.x_VH) {
-      const Row w = row_of((uint32_t)R, true);
+      const Row w = row_of(P, (uint32_t)R, true);
       const ADH_GLOBAL float *p = (const ADH_GLOBAL float *)P.x[w.tile] + ((size_t)n * P.Cin * x_plane + (size_t)w.r * P.x_W) + tail_chan;
       if (Q < xW) tail[0] = p[Q];
       if (Q + 1 < xW) tail[1] = p[Q + 1];
@@ -260,12 +263,13 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
 
   while (s < s_end) {
     // a run: steps of one image (pair) and column tile
+    const WgradSplitParams &M = from_memory(args);
     uint32_t run, rs, img, ctile;
-    P.div_row_steps.divmod(s, run, rs);
-    P.div_cols.divmod(run, img, ctile);
-    P.div_N.divmod(img, tile0, n);
+    M.div_row_steps.divmod(s, run, rs);
+    M.div_cols.divmod(run, img, ctile);
+    M.div_N.divmod(img, tile0, n);
     c0 = ctile * P.TW;
-    const uint32_t steps = min(s_end - s, P.row_steps - rs);
+    const uint32_t steps = min(s_end - s, M.row_steps - rs);
     place((int32_t)(c0 + 4u * q) - P.pad_c, xW, c_x_ok, x_from, x_shift);
     place((int32_t)(c0 + 4u * q), dW, c_dy_ok, dy_from, dy_shift);
     uint32_t r0 = rs * P.RS, base = 0, buf = 0;
@@ -332,29 +336,30 @@ __global__ __launch_bounds__(kWsThreads, 2) void conv3x3_wgrad_split_kernel(cons
   __syncthreads();
   if (nan_sums == 0u) return;
   // sums that are NaN once more in plain fp32, straight from memory
-  s = (uint32_t)((uint64_t)P.total_steps * split / P.splits);
+  const WgradSplitParams &M = from_memory(args);
+  s = (uint32_t)((uint64_t)M.total_steps * split / M.splits);
   for (uint32_t at = tid; at < 4u * OT * CT * kTile; at += kWsThreads) {
     if (part[at] == part[at]) continue;
     const uint32_t i = at & 3u, ln = at >> 2 & 63u, rest = at >> 8, tap = rest % 9u, ct = rest / 9u % CT, ot = rest / 9u / CT % OT;
     const uint32_t wt = rest / 9u / CT / OT;
     const uint32_t co = co0 + ((wt & 1u) * OT + ot) * 16u + (ln >> 4) * 4u + i, ci = ci0 + ((wt >> 1) * CT + ct) * 16u + (ln & 15u);
     float sum = 0.f;
-    if (co < P.Cout && ci < P.Cin)
+    if (co < M.Cout && ci < M.Cin)
       for (uint32_t st = s; st < s_end && sum == sum; ++st) {  // (a NaN stays one)
         uint32_t run, rs, img, ctile;
-        P.div_row_steps.divmod(st, run, rs);
-        P.div_cols.divmod(run, img, ctile);
-        P.div_N.divmod(img, tile0, n);
-        for (uint32_t R = rs * P.RS; R < min((rs + 1u) * P.RS, P.dy_VH) && sum == sum; ++R)
-          for (uint32_t Q = ctile * P.TW; Q < min((ctile + 1u) * P.TW, P.dy_W) && sum == sum; ++Q) {
-            const int32_t xr = (int32_t)(R + tap / 3u) - P.pad_r, xc = (int32_t)(Q + tap % 3u) - P.pad_c;
+        M.div_row_steps.divmod(st, run, rs);
+        M.div_cols.divmod(run, img, ctile);
+        M.div_N.divmod(img, tile0, n);
+        for (uint32_t R = rs * M.RS; R < min((rs + 1u) * M.RS, M.dy_VH) && sum == sum; ++R)
+          for (uint32_t Q = ctile * M.TW; Q < min((ctile + 1u) * M.TW, M.dy_W) && sum == sum; ++Q) {
+            const int32_t xr = (int32_t)(R + tap / 3u) - M.pad_r, xc = (int32_t)(Q + tap % 3u) - M.pad_c;
             float xe = 0.f;
-            if (xr >= 0 && xr < (int32_t)P.x_VH && xc >= 0 && xc < (int32_t)P.x_W) {
-              const Row w = row_of((uint32_t)xr, true);
-              xe = P.x[w.tile][((size_t)n * P.Cin + ci) * x_plane + (size_t)w.r * P.x_W + (uint32_t)xc];
+            if (xr >= 0 && xr < (int32_t)M.x_VH && xc >= 0 && xc < (int32_t)M.x_W) {
+              const Row w = row_of(M, (uint32_t)xr, true);
+              xe = M.x[w.tile][((size_t)n * M.Cin + ci) * x_plane + (size_t)w.r * M.x_W + (uint32_t)xc];
             }
-            const Row w = row_of(R, false);
-            sum = __builtin_fmaf(P.dy[w.tile][((size_t)n * P.Cout + co) * dy_plane + (size_t)w.r * P.dy_W + Q], xe, sum);
+            const Row w = row_of(M, R, false);
+            sum = __builtin_fmaf(M.dy[w.tile][((size_t)n * M.Cout + co) * dy_plane + (size_t)w.r * M.dy_W + Q], xe, sum);
           }
       }
     part[at] = sum;
