@@ -639,12 +639,12 @@ static int gen_patch_taps(int which, const GenShape &g, bool unpadded, uint32_t 
   }
   return gen_is_3x3_split(ADH_F32, g, unpadded, pad_h, pad_w) ? 9 : 0;
 }
-// conv_s2_wgrad.hip: the filter gradient at stride 2 over tiles of even height and width without halo, 3x3 in either type and 1x1 in
-// bf16 (conv1x1.hip has fp32's).  Whether the shape is such a one.
+// conv_s2_wgrad.hip: the filter gradient at stride 2 over tiles of even height and width without halo, 3x3 and 1x1.  Whether the shape
+// is such a one.
 static bool gen_s2_wgrad_problem(int dtype, const GenShape &g, uint32_t num_tiles, bool unpadded, uint32_t pad_h, uint32_t pad_w, S2WgradProblem *q) {
   if (!unpadded || g.sh != 2u || g.sw != 2u || g.HP % 2u != 0u || g.WP % 2u != 0u) return false;
   const bool three = gen_is_3x3s2_unpadded(ADH_F32, g, unpadded, pad_h, pad_w);
-  if (!three && (dtype != ADH_BF16 || g.kh != 1u || g.kw != 1u || pad_h != 0u || pad_w != 0u)) return false;
+  if (!three && (g.kh != 1u || g.kw != 1u || pad_h != 0u || pad_w != 0u)) return false;
   *q = S2WgradProblem{dtype, three ? 9 : 1, num_tiles, g.N, g.Cin, g.Cout, g.OH, g.OW, nullptr, nullptr, nullptr, 0.f};
   return true;
 }
@@ -1457,6 +1457,12 @@ int conv2d_bwd_filter(int dtype, uint32_t num_tiles, uint32_t N, uint32_t Cin, u
     const size_t need = conv1x1_wgrad_workspace(num_tiles, N, Cin, Cout, g.OH, g.OW);
     if (need != 0) {
       if (workspace_bytes < need) return ADH_EWORKSPACE;
+      S2WgradProblem s2;
+      if (gen_s2_wgrad_problem(dtype, g, num_tiles, unpadded, pad_h, pad_w, &s2)) {
+        s2.x = x_tiles; s2.dy = dy_tiles; s2.dw = dwt; s2.beta = beta;
+        e = conv_s2_wgrad(s2, workspace, workspace_bytes, st);
+        if (e != ADH_EUNIMPL) return e;
+      }
       e = conv1x1_wgrad_try(num_tiles, N, Cin, Cout, g.HP, g.WP, g.OH, g.OW, g.sh, g.sw, x_tiles, dy_tiles, dwt, beta,
                             workspace, st);
       if (e != ADH_EUNIMPL) return e;

@@ -16,7 +16,8 @@
 //   * The workgroups' sums are added by a second kernel in a fixed order (reproducible).
 // Measured (32 images, 4 tiles; before: v_mfma_f32 kernels, in bf16 over widened values): fp32 3x3, 128 -> 256 channels on 16 x 64 tiles
 // 0.202 -> 0.128 ms (150 TFLOP/s), 64 -> 128 on 32 x 128 0.217 -> 0.148, 256 -> 512 on 8 x 32 0.206 -> 0.129; bf16 3x3, 128 -> 256
-// 0.341 -> 0.068, 1x1 0.143 -> 0.025; 56 -> 112, 2 images, 2 tiles of 22 x 124: 36 -> 16 us.  Relative error against double
+// 0.341 -> 0.068, 1x1 0.143 -> 0.025; fp32 1x1, 128 -> 256 on 16 x 64 39 -> 33 us, 96 -> 96, 4 images, 8 tiles of 6 x 88, 19.5 -> 10.7, 24 shapes 0.68
+// of the time (one workgroup per compute unit in place of two 50 and 10.8) at 0.2 - 0.5 of the error; 56 -> 112, 2 images, 2 tiles of 22 x 124: 36 -> 16 us.  Relative error against double
 // precision over the former kernels': fp32 0.2 - 0.7 (up to 1.9 with the products below h*h in the same sums: six roundings a step in place of
 // one, at no less time: 0.0 - 0.3 % of a projection block), bf16 0.35 - 1.0.
 // Bound: fp32 by splitting and storing four rows' worth of x per output row beside 1728 matrix cycles a wave and step; bf16 by
@@ -421,7 +422,7 @@ static bool s2wg_plan(const S2WgradProblem &q, S2WgPlan *plan) {
   // One workgroup per compute unit over all groups (two where the registers and the LDS hold them: a projection block of 80 -> 80 channels
   // on 4 tiles of 56 x 102 in bf16 takes 153 us with one of 64 x 64 channels and 169 with two, which run in turn), and no more than the reduction kernel pays for: the
   // square root is where a step's time saved is a split's sums added (8 to 60 in place of 25: 0 to 6 % slower).
-  const bool both = plan->co64 && plan->ci64, twice = q.dtype == ADH_BF16 ? q.taps == 1 || !both : !plan->co64 && !plan->ci64;
+  const bool both = plan->co64 && plan->ci64, twice = q.taps == 1 || (q.dtype == ADH_BF16 ? !both : !plan->co64 && !plan->ci64);
   const uint32_t most = twice ? 512u : 256u;
   P.splits = std::min(most / std::min(plan->groups, most), std::min(P.total_steps, (uint32_t)std::sqrt(25.0 * P.total_steps)));
   if ((uint64_t)plan->groups * P.splits >= (1ull << 22)) return false;
@@ -475,7 +476,7 @@ int conv_s2_wgrad(const S2WgradProblem &q, void *workspace, size_t workspace_byt
   }
   P.part = reinterpret_cast<float *>(workspace);
   P.dw = q.dw;
-  if (q.dtype == ADH_F32) launch_s2wg_channels<float, 9>(plan, st);
+  if (q.dtype == ADH_F32) q.taps == 9 ? launch_s2wg_channels<float, 9>(plan, st) : launch_s2wg_channels<float, 1>(plan, st);
   else q.taps == 9 ? launch_s2wg_channels<uint16_t, 9>(plan, st) : launch_s2wg_channels<uint16_t, 1>(plan, st);
   return launch_status();
 }
