@@ -495,8 +495,10 @@ static bool bn_runs(BnParams *P, uint32_t run, uint32_t runs, uint32_t vec) {
   return wide;
 }
 
-// `bytes`: what a pass reads.  Non-temporal where the on-package cache (256 MB) cannot keep it for the second pass.
-static bool bn_stream(uint64_t bytes) { return bytes > (256ull << 20); }
+// `bytes`: what a pass reads.  Non-temporal where the on-package cache (256 MB, which the results go through too) cannot keep it for the
+// second pass: batch norm and pooling, both passes, 32 images, 64 channels, 4 tiles, fp32 32 x 128 (134 and 268 MB) 302 us with the line at 256 MB
+// and beyond, 281 from 128 to 224, 285 at 96; bf16 64 x 256 (268 and 537 MB) 616 and 608; fp32 28 and 24 images of 64 x 128 the same.
+static bool bn_stream(uint64_t bytes) { return bytes > (192ull << 20); }
 
 template <typename T, bool BWD, int VEC, bool STREAM>
 static void bn_reduce(const BnParams &P, dim3 grid, hipStream_t st) {
