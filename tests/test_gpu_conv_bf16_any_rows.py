@@ -10,7 +10,7 @@ pytestmark = pytest.mark.gpu
 # (strips: the smallest tiles that patches don't take; one and several launches, channels off 64 and 128, heights off four rows)
 FWD = [(4, 4, 64, 64, 34, 255), (4, 8, 61, 64, 34, 127), (2, 3, 1, 144, 64, 255), (8, 2, 128, 128, 34, 127), (8, 2, 128, 128, 64, 65),
        (8, 8, 128, 256, 16, 33), (4, 1, 66, 320, 34, 255), (8, 4, 96, 96, 34, 127), (4, 1, 128, 128, 64, 257)]
-BWD = [(4, 6, 64, 64, 16, 255), (4, 6, 61, 64, 64, 127), (4, 6, 64, 64, 64, 132), (4, 8, 48, 48, 64, 130), (8, 3, 128, 128, 16, 127),
+BWD = [(4, 6, 64, 64, 16, 255), (4, 12, 61, 64, 16, 127), (8, 12, 64, 64, 16, 132), (4, 8, 48, 48, 64, 130), (8, 3, 128, 128, 16, 127),
        (4, 6, 128, 128, 34, 65), (4, 6, 128, 128, 34, 70), (4, 8, 192, 128, 34, 33), (4, 4, 130, 128, 16, 132), (2, 3, 320, 66, 16, 255),
        (8, 1, 384, 256, 16, 255), (8, 3, 384, 256, 16, 132), (4, 6, 128, 128, 33, 132)]
 
