@@ -7,8 +7,9 @@
 //   conv_bias_grad_kernel  workgroup (channel, split): adds its share of the channel's planes, every thread a
 //                          fixed subsequence, then a tree over the workgroup; one number per workgroup.
 //                          Four groups in flight and non-temporal loads: 537 MB in 120 -> 80 us (6.7 TB/s)
-//   conv_bias_grad_final   one thread per channel adds the splits in order (double) and applies beta:
-//                          the sum does not depend on timing, repeated calls give the same bits
+//   conv_bias_grad_final   a wave per channel adds the splits in a fixed order (double) and applies beta: the sum does
+//                          not depend on timing, repeated calls give the same bits (a thread per channel, whose
+//                          loads follow each other: 64 splits of 16 channels 6.0 us, 1.8 now)
 #include "adh_common.h"
 
 #include <algorithm>
@@ -91,12 +92,14 @@ __global__ __launch_bounds__(kBiasThreads) void conv_bias_grad_kernel(const Bias
   if (threadIdx.x == 0) P.partial[(size_t)c * P.split + s] = (red[0] + red[1]) + (red[2] + red[3]);
 }
 
-__global__ void conv_bias_grad_final(const float *partial, uint32_t C, uint32_t split, float beta, float *db) {
-  const uint32_t c = blockIdx.x * blockDim.x + threadIdx.x;
+__global__ __launch_bounds__(kBiasThreads) void conv_bias_grad_final(const float *partial, uint32_t C, uint32_t split, float beta, float *db) {
+  const uint32_t c = blockIdx.x * (kBiasThreads / 64u) + (threadIdx.x >> 6), lane = threadIdx.x & 63u;
   if (c >= C) return;
   double a = 0.0;
-  for (uint32_t s = 0; s < split; ++s) a += (double)partial[(size_t)c * split + s];
-  db[c] = (float)(beta != 0.0f ? a + (double)beta * (double)db[c] : a);
+  for (uint32_t s = lane; s < split; s += 64u) a += (double)partial[(size_t)c * split + s];
+#pragma unroll
+  for (int o = 32; o > 0; o >>= 1) a += __shfl_xor(a, o);
+  if (lane == 0u) db[c] = (float)(beta != 0.0f ? a + (double)beta * (double)db[c] : a);
 }
 
 static uint32_t bias_grad_split(uint32_t tiles, uint32_t N, uint32_t C) {
@@ -186,7 +189,7 @@ extern "C" int adh_conv_bwd_bias_tiles(int dtype, uint32_t num_tiles, uint32_t N
   const hipStream_t st = as_stream(stream);
   if (N == 0 || H == 0 || W == 0) {  // an empty sum
     if (beta == 0.0f) {
-      hipLaunchKernelGGL(conv_bias_grad_final, dim3((C + 255) / 256), dim3(256), 0, st, (const float *)nullptr, C, 0u,
+      hipLaunchKernelGGL(conv_bias_grad_final, dim3((C + 3u) / 4u), dim3(kBiasThreads), 0, st, (const float *)nullptr, C, 0u,
                          beta, db);
       return launch_status();
     }
@@ -211,7 +214,7 @@ extern "C" int adh_conv_bwd_bias_tiles(int dtype, uint32_t num_tiles, uint32_t N
   P.div_N = FastDiv(N);
   const int rc = dtype == ADH_F32 ? bias_grad_launch<float>(P, true, st) : bias_grad_launch<uint16_t>(P, true, st);
   if (rc != ADH_OK) return rc;
-  hipLaunchKernelGGL(conv_bias_grad_final, dim3((C + 255) / 256), dim3(256), 0, st, (const float *)P.partial, C, P.split,
+  hipLaunchKernelGGL(conv_bias_grad_final, dim3((C + 3u) / 4u), dim3(kBiasThreads), 0, st, (const float *)P.partial, C, P.split,
                      beta, db);
   return launch_status();
 }
